@@ -19,6 +19,26 @@ extern "C" {
  * does not serve a shape makes the matmul return MGN_EINVAL ("... does not support this shape"). */
 mgn_status mgn_ctx_set_route(mgn_ctx* ctx, mgn_route route);
 
+/* Whether the automatic choice gives a shape to the blocked kernel (MGN_ROUTE_BLOCK_MFMA), and how it
+ * would launch it, without a device: arguments as mgn_matmul_q_plan, whose answer for such a shape is
+ * the kernel that serves it where the blocked one is not to be had.  MGN_EUNSUPPORTED when the
+ * blocked kernel does not serve the shape at all. */
+typedef struct mgn_block_plan {
+  uint32_t taken; /* 1: the automatic choice */
+  uint32_t rows;  /* outputs per workgroup: rows x cols */
+  uint32_t cols;
+  uint32_t threads; /* per workgroup */
+  uint32_t lds_bytes;
+  uint32_t row_groups;
+  uint32_t col_groups;
+  uint32_t k_parts;    /* > 1: partial results through the workspace, added up by a second launch */
+  uint32_t launches;   /* blocks of rows that run one after the other (the workspace's room) */
+  float us;            /* what the planner expects the call to take */
+  uint64_t workspace_bytes;
+} mgn_block_plan;
+mgn_status mgn_matmul_q_block_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus,
+                                   mgn_block_plan* out);
+
 /* How many times a wave polls for another workgroup's partial sums before it gives up (kernels whose
  * K parts meet without counters; default 2^20, far beyond any wait of a healthy launch).  With 0 a
  * reading wave looks at nothing and gives up at once, which is how a test makes that path run: the

@@ -62,10 +62,13 @@ typedef enum mgn_route {
   MGN_ROUTE_GEMV_MFMA = 3, /* streaming dequant-GEMV, raw quants x split-fp16 activations on MFMA, M <= 4 */
   MGN_ROUTE_GEMM_MFMA = 4, /* tiled dequant-GEMM on MFMA (32x32x16 tiles), larger M: the fast form, for weights whose
                               block minima stay below 2047 (Q8: scales below 15.99) and f32 activations below 65504 */
-  MGN_ROUTE_TILE_MFMA = 5  /* tiled dequant-GEMM on MFMA (16x16x32 tiles, activations rescaled per row and 256-element
+  MGN_ROUTE_TILE_MFMA = 5, /* tiled dequant-GEMM on MFMA (16x16x32 tiles, activations rescaled per row and 256-element
                               K slice): any finite weight, activations below 2^100 in magnitude (a slice that holds a
                               larger one gives its row non-finite results), larger M; the automatic choice for weights
                               outside the range of the form above */
+  MGN_ROUTE_BLOCK_MFMA = 6 /* blocked dequant-GEMM on MFMA (32x32x16 tiles, up to 256 x 256 outputs per workgroup,
+                              activations prepared once per call: f32 split on one power-of-two scale per row):
+                              any finite weight, activations below 2^100 in magnitude; many rows */
 } mgn_route;
 
 typedef struct mgn_ctx mgn_ctx;
@@ -248,7 +251,8 @@ mgn_status mgn_matmul_q_at(mgn_ctx* ctx, const mgn_buf* a_t, const mgn_weight* w
  * `num_cus` is the device's compute-unit count (256 on MI355X); the workspace is assumed to be
  * the one every context owns.  a_is_f16: 0 = f32 activations of any magnitude (a context's
  * default), 1 = fp16 activations, 2 = f32 activations promised to lie in the fp16 range
- * (MGN_ACT_FP16_RANGE).  MGN_EINVAL for shapes no weight can have. */
+ * (MGN_ACT_FP16_RANGE).  MGN_EINVAL for shapes no weight can have.  For the many-row shapes that the
+ * blocked kernel takes (mgn_matmul_q_block_plan in mgn_bench.h tells), this is the kernel behind it. */
 typedef struct mgn_plan_info {
   int route;              /* mgn_route (never MGN_ROUTE_AUTO) */
   uint32_t grid[3];       /* workgroups: GEMV (column groups, K parts, 1); tiled routes (K parts, column groups, row

@@ -15,10 +15,10 @@ OK, EINVAL, ENOMEM, EHIP, ENOTFOUND, ENODEVICE, EUNSUPPORTED, ERANGE, ETIMEOUT =
 FMT_Q4, FMT_Q8 = 0, 1
 ACT_ANY, ACT_FP16_RANGE = 0, 1
 STATIC_WORKSPACE_BYTES = 4 << 20  # MGN_STATIC_WORKSPACE_BYTES
-ROUTE_AUTO, ROUTE_GENERIC, ROUTE_GEMV_VALU, ROUTE_GEMV_MFMA, ROUTE_GEMM_MFMA, ROUTE_TILE_MFMA = range(6)
+ROUTE_AUTO, ROUTE_GENERIC, ROUTE_GEMV_VALU, ROUTE_GEMV_MFMA, ROUTE_GEMM_MFMA, ROUTE_TILE_MFMA, ROUTE_BLOCK_MFMA = range(7)
 
 # every symbol include/mgn_hip.h, include/mgn_bench.h and include/mgn_session.h declare
-BENCH_SYMBOLS = ["mgn_ctx_set_route", "mgn_ctx_set_spin_limit", "mgn_engine_clock_mhz", "mgn_matmul_q_loop", "mgn_weight_read_loop"]
+BENCH_SYMBOLS = ["mgn_ctx_set_route", "mgn_matmul_q_block_plan", "mgn_ctx_set_spin_limit", "mgn_engine_clock_mhz", "mgn_matmul_q_loop", "mgn_weight_read_loop"]
 HIP_SYMBOLS = [
     "mgn_ctx_create", "mgn_ctx_destroy", "mgn_last_error", "mgn_sync", "mgn_ctx_set_activation_range", "mgn_ctx_set_shared_device",
     "mgn_buf_alloc", "mgn_buf_free", "mgn_buf_size", "mgn_buf_device_ptr", "mgn_buf_upload",
@@ -121,6 +121,7 @@ def load():
         "mgn_matmul_q_epilogue": (C.c_int, [vp, vp, vp, vp, vp, C.c_uint32, vp, C.c_size_t]),
         "mgn_matmul_q_at": (C.c_int, [vp, vp, vp, vp, vp, C.c_uint32, vp, C.c_size_t]),
         "mgn_matmul_q_plan": (C.c_int, [C.c_int, C.c_uint32, C.c_uint64, C.c_uint64, C.c_int, C.c_int, vp]),
+        "mgn_matmul_q_block_plan": (C.c_int, [C.c_int, C.c_uint32, C.c_uint64, C.c_uint64, C.c_int, C.c_int, vp]),
         "mgn_matmul_q_loop": (C.c_int, [vp, vp, C.c_int, vp, C.c_size_t, vp, vp, C.c_uint32, C.c_uint32]),
         "mgn_weight_read_loop": (C.c_int, [vp, vp, C.c_size_t, C.c_uint32, C.c_int]),
         "mgn_matmul_q_rms_norm": (C.c_int, [vp, vp, vp, C.c_float, vp, vp, vp, C.c_uint32]),
@@ -204,6 +205,19 @@ def matmul_plan(fmt, m, k, n, a_is_f16=False, num_cus=256, fp16_range=False):
     if st != OK:
         raise MgnError(st, "matmul_plan: no weight has this shape")
     return info
+
+
+class BlockPlan(C.Structure):
+    _fields_ = [("taken", C.c_uint32), ("rows", C.c_uint32), ("cols", C.c_uint32), ("threads", C.c_uint32), ("lds_bytes", C.c_uint32),
+                ("row_groups", C.c_uint32), ("col_groups", C.c_uint32), ("k_parts", C.c_uint32), ("launches", C.c_uint32),
+                ("us", C.c_float), ("workspace_bytes", C.c_uint64)]
+
+
+def matmul_block_plan(fmt, m, k, n, a_is_f16=False, num_cus=256):
+    """How the blocked kernel would launch this shape (no device needed); None if it does not serve it."""
+    plan = BlockPlan()
+    st = load().mgn_matmul_q_block_plan(fmt, m, k, n, 1 if a_is_f16 else 0, num_cus, C.byref(plan))
+    return plan if st == OK else None
 
 
 def quantize_ref(fmt, w):

@@ -1,0 +1,932 @@
+// Blocked dequant-GEMM on the matrix cores for many rows: C[M,N] = A[M,K] x W (+ D), f32 or fp16 activations
+// (prefill, and decode batches of more than some 32 rows on large weights).
+//
+// The arithmetic is that of the other tiled kernels (raw quants as the B operand of the matrix
+// instructions, block scales on their results, block minima as a product of their own), so the vector
+// ALU owes 16 multiply-adds per 32 x 32 outputs and quant block whatever the tiling; with the matrix
+// instructions (two of 32 cycles; four with f32 activations, which enter as fp16 pairs hi + lo) that is
+// the bound: measured on one SIMD, v_mfma_f32_32x32x16_f16 occupies its pipe for 32 cycles and the vector
+// issue port for about 8, a v_fma_f32 the port for 4, and two waves overlap the two almost fully.  The
+// kernels this one takes over from ran far from it: a 32-row tile per wave unpacks the quants for
+// every tile, stages activations through registers in every column group and keeps the matrix pipe
+// 16 % busy.  What is different here:
+//   * a wave owns 32 RT x 64 outputs (up to 128 x 64: 128 accumulator registers), so the 14 instructions that
+//     unpack a column tile's quants serve RT row tiles, and the tiles' multiply-adds are woven between
+//     the next tile's matrix instructions by hand;
+//   * activations and quants travel from memory into LDS without touching registers (buffer loads with
+//     the LDS bit), several substeps ahead, in rings; one barrier per substep.  What a lane reads
+//     together is spread over the banks by an exclusive-or of its 16-byte unit with the row;
+//   * everything the multiplication wants to know about the activations is worked out once per call by
+//     a small launch in front (prepare_*): the blocks' means, and for f32 the fp16 pairs on a scale per
+//     row.  One scale for the whole row, so that no accumulator is rescaled on the way: a slice of
+//     256 elements that would keep fewer than 22 bits on it gets its own, and the waves that meet
+//     such a row move their sums from scale to scale;
+//   * K parts for different workgroups, where the tiles do not fill the chip, meet in the workspace and are added
+//     in part order by a third launch.
+// Measured (one box, weights from memory; before -> now, us): fp16 2048 x 4096 x 14336 589 -> 299 (805 TFLOP/s),
+// f32 the same 1034 -> 467; f32 512 x 4096 x 14336 295 -> 123; f32 77 x 4096 x 14336 82 -> 44, 77 x 14336 x 4096
+// 98 -> 46.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.4
+// times its issue cycles (LDS and barrier waits).
+#include <algorithm>
+#include <cmath>
+
+#include <type_traits>
+#include <utility>
+
+#include "kernels_operand.hip.h"
+
+namespace mgn {
+namespace {
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+// f(0), f(1), .. f(N - 1) with compile-time indices
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_each(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_each(f, std::make_integer_sequence<int, N>{});
+}
+
+constexpr int kCT = 2;  // column tiles of 32 columns per wave
+
+constexpr int stage_blocks(int fmt) { return fmt == MGN_FMT_Q4 ? 4 : 2; }  // 64 bytes of quants per column
+
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
+}
+
+// 64 x 16 bytes from memory straight into LDS: lane i's bytes land at lds + 16 i.  (In assembly, with the
+// waits counted by hand: the compiler waits for every such load before any LDS read that might alias it.)
+__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t src, uint32_t lane_off, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(lane_off), "s"(src), "s"(__builtin_amdgcn_readfirstlane(off)) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// one dword of nibbles -> 8 fp16 in element order, each n * 2^-20
+__device__ __forceinline__ half8 nibbles_in_order(uint32_t w) {
+  const uint32_t ev = (w << 4) & 0xF0F0F0F0u, od = w & 0xF0F0F0F0u;
+  return as_half8(__builtin_amdgcn_perm(od, ev, 0x0c040c00u), __builtin_amdgcn_perm(od, ev, 0x0c050c01u),
+                  __builtin_amdgcn_perm(od, ev, 0x0c060c02u), __builtin_amdgcn_perm(od, ev, 0x0c070c03u));
+}
+
+// the j-th of NM equal shares of acc += dq * d
+template <int NM, int j>
+__device__ __forceinline__ void scale_part(floatx16& acc, const floatx16& d, float dq) {
+  static_for<16 / NM>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = j * (16 / NM) + I;
+    acc[i] = __fmaf_rn(dq, d[i], acc[i]);
+  });
+}
+
+struct BlockArgs {
+  const void* a;      // fp16 activations, or the prepared f32 ones
+  const void* means;  // [stages][mpad]{hi x SB, lo x SB}
+  const float* inv;   // [slices][mpad] inverse scales (f32 activations)
+  const float* row_scale;  // [mpad] the inverse scale of a row's last slice; NaN for a row that holds a magnitude of 2^100 or more
+  const uint32_t* mixed;  // [mpad] nonzero: the row's slices do not share one scale
+  const void* meta;
+  const void* quants;
+  uint32_t a_pitch, a_bytes, quant_bytes, meta_bytes, means_bytes;
+  uint32_t m, mpad, n, bpc, stages, rowgroups, colgroups, parts;
+  uint32_t add_hi, add_lo;  // fp16 pairs: 2^lift and 2^(lift - 11)
+  float unit;               // 2^-lift times the inverse operand scale
+  float dscale;             // what a block scale is multiplied by: operand scale * 2^lift
+  const float* dres;
+  float* c;
+  float* partial;  // [parts][m][n] when parts > 1
+  uint32_t epilogue;
+};
+
+__device__ __forceinline__ float group_max32(float v) {
+  v = fmaxf(v, dpp_move<kDppQuadXor1>(v));
+  v = fmaxf(v, dpp_move<kDppQuadXor2>(v));
+  v = fmaxf(v, dpp_move<kDppRowHalfMirror>(v));
+  v = fmaxf(v, dpp_move<kDppRowMirror>(v));
+  return fmaxf(v, __shfl_xor(v, 16, 64));
+}
+
+// Geometry of a workgroup: WM x WN waves side by side, each RT row tiles of 32 rows x 64 columns, and
+// WK streams of them that take the stages (64 bytes of quants per column) in turn; substeps of SUBB
+// blocks of activations, requested PD substeps ahead; stages requested SD stages ahead.
+template <int FMT, bool F32A, int RT, int WM, int WN, int WK, int SUBB, int PD, int SD>
+struct BlockShape {
+  static constexpr int SB = stage_blocks(FMT);
+  static constexpr int NSUB = SB / SUBB;
+  static constexpr int WAVES = WM * WN * WK;
+  static constexpr int ROWS = WM * RT * 32, COLS = WN * kCT * 32;
+  static constexpr int PANELS = SUBB * (F32A ? 128 : 64) / 128;  // 128 bytes of activations per row each
+  static constexpr int ARING = PD + 1, SRING = SD + 1;
+  static constexpr uint32_t A_BYTES = WK * PANELS * ROWS * 128u, B_BYTES = WK * COLS * 64u, M_BYTES = WK * COLS * 16u;
+  static constexpr uint32_t MEAN_STREAM = (ROWS * SB * 4 + 1023) / 1024 * 1024, S_BYTES = WK * MEAN_STREAM;
+  static constexpr uint32_t STAGE_BYTES = B_BYTES + M_BYTES + S_BYTES;
+  static constexpr int NA = (int)(A_BYTES / 1024), NST = (int)(STAGE_BYTES / 1024);  // loads of 1 KiB
+  static constexpr int NAW = (NA + WAVES - 1) / WAVES, NSTW = (NST + WAVES - 1) / WAVES;
+  static constexpr size_t PIPE = (size_t)ARING * A_BYTES + (size_t)SRING * STAGE_BYTES;
+  static constexpr size_t RED = WK > 1 ? (size_t)WM * WN * RT * kCT * 4096 : 0, STRIP = (size_t)WAVES * 4096;
+  static constexpr size_t LDS = PIPE > RED ? (PIPE > STRIP ? PIPE : STRIP) : (RED > STRIP ? RED : STRIP);
+  // A wave's loads in issue order: in substep i the activations of substep i + PD, then, where it is a
+  // stage's first, the stage SD ahead.  At its end everything that substep i + 1 reads, and the first
+  // block of i + 2, must have landed; the loads issued after the last of those may be in flight.
+  static constexpr int issued(int i) { return NAW + (i % NSUB == 0 ? NSTW : 0); }
+  static constexpr int since(int from, int to) {
+    int n = 0;
+    for (int i = from; i <= to; i++) n += issued(i);
+    return n;
+  }
+  static constexpr int in_flight(int u) {
+    const int i = u + 64 * NSUB;
+    const int after_a = (i + 2 - PD) % NSUB == 0 ? NSTW + since(i + 3 - PD, i) : since(i + 3 - PD, i);
+    const int after_stage = since(((i + 2) / NSUB - SD) * NSUB + 1, i);
+    return after_a < after_stage ? after_a : after_stage;
+  }
+  static_assert(PD >= 2 && 2 / NSUB <= SD && (NSUB > 1 || SD >= 2), "what a substep waits for has been requested");
+};
+
+template <int FMT, bool F32A, int RT, int WM, int WN, int WK, int SUBB, int PD, int SD>
+__global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x) {
+  using S = BlockShape<FMT, F32A, RT, WM, WN, WK, SUBB, PD, SD>;
+  constexpr int SB = S::SB, NSUB = S::NSUB, ROWS = S::ROWS, COLS = S::COLS, PANELS = S::PANELS, ARING = S::ARING, SRING = S::SRING;
+  constexpr int NAW = S::NAW, NSTW = S::NSTW;
+  constexpr uint32_t A_BYTES = S::A_BYTES, B_BYTES = S::B_BYTES, M_BYTES = S::M_BYTES, STAGE_BYTES = S::STAGE_BYTES;
+  constexpr uint32_t MEAN_STREAM = S::MEAN_STREAM;
+  constexpr int QB = FMT == MGN_FMT_Q4 ? 16 : 32, MB = FMT == MGN_FMT_Q4 ? 4 : 2;
+  constexpr int NM = F32A ? 4 : 2;             // matrix instructions per tile and block
+  constexpr int TILES = RT * kCT;
+  static_assert(F32A || SUBB % 2 == 0, "fp16 activations: two blocks per 128 bytes");
+  extern __shared__ uint4 lds4[];
+  uint8_t* const lds = (uint8_t*)lds4;
+  uint8_t* const lds_st = lds + ARING * A_BYTES;  // [SRING]{quants, block constants, means}
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t ks = wave / (WM * WN), wm = (wave / WN) % WM, wn = wave % WN;
+  const uint32_t c = lane & 31, h = lane >> 5;
+
+  // the eight XCDs take workgroups in turn: each gets a contiguous run of tiles, row groups first
+  const uint32_t tiles = x.rowgroups * x.colgroups;
+  const uint32_t per = (tiles + 7) / 8;
+  const uint32_t part = blockIdx.x / (per * 8), id = blockIdx.x % (per * 8);
+  const uint32_t tile = (id & 7) * per + (id >> 3);
+  if (tile >= tiles) return;
+  const uint32_t rg = tile % x.rowgroups, cg = tile / x.rowgroups;
+  const uint32_t row0 = rg * ROWS, col0 = cg * COLS;
+
+  // this part's stages, dealt to the WK streams in turn
+  const uint32_t spp = (x.stages + x.parts - 1) / x.parts;
+  const uint32_t st0 = part * spp, st1 = min(st0 + spp, x.stages);
+  const uint32_t iters = (st1 - st0 + WK - 1) / WK;
+
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)x.a, 0, x.a_bytes, 0x00020000);
+  // A wave's share of the loads.  Activations: load q brings 8 rows of one panel; in LDS a row's unit u
+  // (16 bytes) lies at u ^ (row / 2 % 8), so that the operand reads of eight rows meet no bank twice.
+  // Stage: 16 columns of quants (unit u of a column at u ^ (column / 4 % 4)), 64 columns of constants, or
+  // 1 KiB of means, by load number.
+  uint32_t a_off[NAW], st_off[NSTW];
+#pragma unroll
+  for (int j = 0; j < NAW; j++) {
+    const uint32_t q = min(wave * NAW + j, (uint32_t)S::NA - 1) % (ROWS / 8);
+    const uint32_t row = q * 8 + (lane >> 3);
+    a_off[j] = min(row0 + row, x.m - 1) * x.a_pitch + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+  }
+  // (what a stage load reads is settled here, per load, so that the loop issues it without a branch)
+  constexpr uint32_t NBL = B_BYTES / 1024, NML = M_BYTES / 1024;
+  __amdgpu_buffer_rsrc_t st_src[NSTW];
+  uint32_t st_stream[NSTW], st_step[NSTW], st_base[NSTW];
+#pragma unroll
+  for (int j = 0; j < NSTW; j++) {
+    const uint32_t q = min(wave * NSTW + j, (uint32_t)S::NST - 1);
+    const void* base = x.quants;
+    uint32_t bytes = x.quant_bytes;
+    st_stream[j] = q / (COLS / 16), st_step[j] = 64, st_base[j] = 0;
+    const uint32_t bcol = q % (COLS / 16) * 16 + (lane >> 2);
+    st_off[j] = min(col0 + bcol, x.n - 1) * (x.bpc * QB) + (((lane & 3) ^ ((bcol >> 2) & 3)) << 4);
+    if (q >= NBL + NML) {
+      const uint32_t p = q - NBL - NML;
+      base = x.means, bytes = x.means_bytes;
+      st_stream[j] = p / (MEAN_STREAM / 1024), st_step[j] = x.mpad * (SB * 4), st_base[j] = row0 * (SB * 4);
+      st_off[j] = p % (MEAN_STREAM / 1024) * 1024u + lane * 16u;
+    } else if (q >= NBL) {
+      const uint32_t mcol = (q - NBL) % (COLS / 64) * 64 + lane;
+      base = x.meta, bytes = x.meta_bytes;
+      st_stream[j] = (q - NBL) / (COLS / 64), st_step[j] = SB * MB;
+      st_off[j] = (min(col0 + mcol, x.n - 1) * (x.bpc * MB)) & ~3u;  // (Q8: the aligned words around two blocks' scales)
+    }
+    st_src[j] = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000);
+  }
+  const uint32_t lds_a0 = lds_address(lds), lds_s0 = lds_address(lds_st);
+  // load j of this wave's share of the activations of (iteration it, substep u) into ring slot `slot`
+  auto load_a = [&](int j, uint32_t it, uint32_t u, uint32_t slot) __attribute__((always_inline)) {
+    const uint32_t q = min(wave * NAW + j, (uint32_t)S::NA - 1);
+    const uint32_t stream = q / (PANELS * ROWS / 8), panel = q / (ROWS / 8) % PANELS;
+    const uint32_t st = min(st0 + it * WK + stream, x.stages - 1);
+    load_to_lds(ra, a_off[j], ((st * NSUB + u) * PANELS + panel) * 128u, lds_a0 + slot * A_BYTES + q * 1024u);
+  };
+  // load j of its share of an iteration's stage
+  auto load_stage = [&](int j, uint32_t it, uint32_t slot) __attribute__((always_inline)) {
+    const uint32_t q = min(wave * NSTW + j, (uint32_t)S::NST - 1);
+    const uint32_t st = min(st0 + it * WK + st_stream[j], x.stages - 1);
+    load_to_lds(st_src[j], st_off[j], st_base[j] + st * st_step[j], lds_s0 + slot * STAGE_BYTES + q * 1024u);
+  };
+  floatx16 acc[RT][kCT];
+#pragma unroll
+  for (int r = 0; r < RT; r++)
+#pragma unroll
+    for (int t = 0; t < kCT; t++) acc[r][t] = (floatx16)(0.0f);
+
+  // lane addresses of the operand reads: unit q of a row or column is q ^ (its swizzle)
+  const uint32_t a_rd = (ks * PANELS * ROWS + wm * (RT * 32) + c) * 128u + ((2 * h) ^ ((c >> 1) & 7)) * 16u;
+  const uint32_t b_rd = (ks * COLS + wn * (kCT * 32) + c) * 64u + (FMT == MGN_FMT_Q4 ? ((c >> 2) & 3) * 16u + h * 8u : (h ^ ((c >> 2) & 3)) * 16u);
+  const uint32_t m_rd = B_BYTES + (ks * COLS + wn * (kCT * 32) + c) * 16u;
+  const uint32_t s_rd = B_BYTES + M_BYTES + ks * MEAN_STREAM + (wm * (RT * 32) + c) * (SB * 4u) + h * (SB * 2u);
+  const uint32_t addp = h ? x.add_lo : x.add_hi;
+
+  // (in the order of the loop's own requests: stages first that the first substeps read)
+#pragma unroll
+  for (int i = 0; i < SD; i++)
+#pragma unroll
+    for (int j = 0; j < NSTW; j++) load_stage(j, min((uint32_t)i, iters - 1), i);
+#pragma unroll
+  for (int i = 0; i < PD; i++)
+#pragma unroll
+    for (int j = 0; j < NAW; j++) load_a(j, min((uint32_t)(i / NSUB), iters - 1), i % NSUB, i);
+  bool mixed = false;
+  float row_scale[RT];  // of row c of each row tile
+  if constexpr (F32A) {
+    uint32_t any = 0;
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+      any |= x.mixed[row0 + (wm * RT + r) * 32 + c];
+      row_scale[r] = x.row_scale[row0 + (wm * RT + r) * 32 + c] * x.unit;
+    }
+    mixed = __builtin_amdgcn_ballot_w64(any != 0) != 0;
+  }
+  wait_loads<(PD - 2) * NAW>();
+  lds_barrier();
+
+  // What is in registers ahead of its use: the raw quants of the next block, the operands of its first
+  // row tile, and (d[1], dqp) the products of the last tile, which are scaled under the next block's
+  // first matrix instructions.
+  uint32_t braw[kCT][FMT == MGN_FMT_Q4 ? 2 : 4], mcur[kCT][FMT == MGN_FMT_Q4 ? 4 : 1];
+  half8 bop[kCT][2], aop[F32A ? 1 : 2][NM];
+  floatx16 d[2];
+  float dq[kCT], dqp = 0.0f;
+  auto read_b = [&](int t, const uint8_t* pb, int sb) __attribute__((always_inline)) {
+    if constexpr (FMT == MGN_FMT_Q4) {
+      const uint2 q = *(const uint2*)(pb + (b_rd ^ (sb * 16u)) + t * 2048);
+      braw[t][0] = q.x, braw[t][1] = q.y;
+    } else {
+      const uint4 q = *(const uint4*)(pb + (b_rd ^ (sb * 32u)) + t * 2048);
+      braw[t][0] = q.x, braw[t][1] = q.y, braw[t][2] = q.z, braw[t][3] = q.w;
+    }
+  };
+  auto unpack_b = [&](int t) __attribute__((always_inline)) {
+    if constexpr (FMT == MGN_FMT_Q4) {
+      bop[t][0] = nibbles_in_order(braw[t][0]);
+      bop[t][1] = nibbles_in_order(braw[t][1]);
+    } else {
+      bop[t][0] = bytes_to_operand(braw[t][0], braw[t][1]);
+      bop[t][1] = bytes_to_operand(braw[t][2], braw[t][3]);
+    }
+  };
+  // operand j of row tile r of block bl of a substep: fp16, k half j of block bl % 2 of panel bl / 2; f32,
+  // k half j % 2 of the high (j < 2) or low halves, panel bl
+  auto read_a = [&](int slot, int j, const uint8_t* pa, int bl, int r) __attribute__((always_inline)) {
+    const uint32_t unit = (j & 1) * 16u + (F32A ? j >> 1 : bl & 1) * 64u, panel = F32A ? bl : bl >> 1;
+    aop[slot][j] = __builtin_bit_cast(half8, *(const u32x4_t*)(pa + (a_rd ^ unit) + panel * (ROWS * 128u) + r * 4096));
+  };
+  d[1] = (floatx16)(0.0f);
+  read_b(0, lds_st, 0);
+  read_b(1, lds_st, 0);
+#pragma unroll
+  for (int j = 0; j < NM; j++) read_a(0, j, lds, 0, 0);
+  unpack_b(0);
+
+  uint32_t abuf = 0, sbuf = 0;  // ring slots in use
+  for (uint32_t it = 0; it < iters; it++) {
+    const uint32_t st = st0 + it * WK + ks;
+    const uint32_t valid = st < st1 ? min((uint32_t)SB, x.bpc - st * SB) : 0u;  // blocks of this stage (uniform)
+    // the block constants of the lane's own two columns
+#pragma unroll
+    for (int t = 0; t < kCT; t++) {
+      const uint8_t* const pm = lds_st + sbuf * STAGE_BYTES + m_rd + t * 512;
+      if constexpr (FMT == MGN_FMT_Q4) {
+        const uint4 v = *(const uint4*)pm;
+        mcur[t][0] = v.x, mcur[t][1] = v.y, mcur[t][2] = v.z, mcur[t][3] = v.w;
+      } else {
+        const uint2 v = *(const uint2*)pm;
+        const uint32_t odd = (min(col0 + (wn * kCT + t) * 32 + c, x.n - 1) * x.bpc) & 1u;  // (a stage starts at an even block)
+        mcur[t][0] = odd ? (v.x >> 16) | (v.y << 16) : v.x;
+      }
+    }
+    if (valid < SB) {
+#pragma unroll
+      for (int t = 0; t < kCT; t++) {
+        if constexpr (FMT == MGN_FMT_Q4) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) mcur[t][e] = (uint32_t)e < valid ? mcur[t][e] : 0u;
+        } else {
+          mcur[t][0] = valid == 1 ? mcur[t][0] & 0xFFFFu : 0u;
+        }
+      }
+    }
+    if (!F32A && valid > 0 && valid < SB) {
+      // What the loads brought in behind the row's last block is another row's, or nothing's.  (The two
+      // substeps that a stage of fp16 activations has at most have landed; each wave clears the rows that
+      // it reads, so that its own order suffices; waves that share rows write the same zeros.)
+      static_assert(F32A || NSUB <= 2, "one substep ahead has landed");
+      for (uint32_t i = lane; i < NSUB * PANELS * RT * 32 * 8; i += 64) {
+        const uint32_t unit = i & 7, row = i / 8 % (RT * 32), panel = i / (RT * 32 * 8);  // panels of the stage
+        const uint32_t buf = abuf + panel / PANELS >= ARING ? abuf + panel / PANELS - ARING : abuf + panel / PANELS;
+        const uint32_t at = (ks * PANELS + panel % PANELS) * ROWS + wm * (RT * 32) + row;
+        if (panel * 2 + unit / 4 >= valid) *(uint4*)(lds + buf * A_BYTES + at * 128u + ((unit ^ ((row >> 1) & 7)) << 4)) = make_uint4(0, 0, 0, 0);
+      }
+    }
+    if (F32A && mixed && it > 0 && valid > 0) {
+      // rows of very different magnitudes along K: the sums move on to the next slice's scale
+      const uint32_t sl = st * SB / 8, pl = (st - WK) * SB / 8;
+      if (sl != pl) {
+        acc[RT - 1][kCT - 1] = __builtin_elementwise_fma(d[1], (floatx16)(dqp), acc[RT - 1][kCT - 1]);
+        dqp = 0.0f;
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+          floatx16 f;
+#pragma unroll
+          for (int i = 0; i < 16; i++) {
+            const uint32_t row = row0 + (wm * RT + r) * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
+            const uint32_t now = __builtin_bit_cast(uint32_t, x.inv[(size_t)sl * x.mpad + row]);
+            const uint32_t was = __builtin_bit_cast(uint32_t, x.inv[(size_t)pl * x.mpad + row]);
+            f[i] = __builtin_bit_cast(float, 0x3F800000u + (was - now));
+          }
+#pragma unroll
+          for (int t = 0; t < kCT; t++) acc[r][t] *= f;
+        }
+      }
+    }
+    static_for<NSUB>([&](auto U) __attribute__((always_inline)) {
+      constexpr int u = U;
+      constexpr bool last = u == NSUB - 1;
+      constexpr int SLOTS = SUBB * TILES, LOADS = S::issued(u);
+      constexpr int ahead = (u + PD) / NSUB, usub = (u + PD) % NSUB;  // the activations requested here: iterations ahead, substep
+      const uint32_t anext = abuf + 1 == ARING ? 0 : abuf + 1, aload = abuf == 0 ? ARING - 1 : abuf - 1;
+      const uint32_t snext = sbuf + 1 == SRING ? 0 : sbuf + 1, sload = sbuf == 0 ? SRING - 1 : sbuf - 1;
+      const uint32_t ita = min(it + ahead, iters - 1), its = min(it + SD, iters - 1);
+      // The loads go out a few at a time between the tiles: all waves' loads at once hold every wave
+      // until the address unit has taken them.
+      auto issue_load = [&](auto Qn) __attribute__((always_inline)) {
+        constexpr int q = Qn;
+        if constexpr (q >= NAW) load_stage(q - NAW, its, sload);
+        else load_a(q, ita, usub, aload);
+      };
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<SUBB>([&](auto BL) __attribute__((always_inline)) {
+        constexpr int bl = BL, sb = u * SUBB + bl;
+        constexpr bool ends_sub = bl == SUBB - 1, ends_stage = sb == SB - 1;
+        const uint8_t* const pa = lds + abuf * A_BYTES;
+        const uint8_t* const pan = ends_sub ? lds + anext * A_BYTES : pa;
+        const uint8_t* const pbn = lds_st + (ends_stage ? snext : sbuf) * STAGE_BYTES;
+#pragma unroll
+        for (int t = 0; t < kCT; t++) {
+          if constexpr (FMT == MGN_FMT_Q4) dq[t] = half_bits_to_float(mcur[t][sb] & 0xFFFFu) * x.dscale;
+          else dq[t] = half_bits_to_float(sb ? mcur[t][0] >> 16 : mcur[t][0] & 0xFFFFu) * x.dscale;
+        }
+        // Tile T of the block: NM matrix instructions, and between them the scaling of tile T - 1
+        static_for<TILES>([&](auto TT) __attribute__((always_inline)) {
+          constexpr int T = TT, r = T / kCT, t = T % kCT, pr = T ? (T - 1) / kCT : RT - 1, pt = T ? (T - 1) % kCT : kCT - 1;
+          constexpr int slot = F32A ? 0 : (sb * RT + r) & 1;
+          static_for<NM>([&](auto J) __attribute__((always_inline)) {
+            constexpr int j = J;
+            d[T & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aop[slot][j], bop[t][j & 1], j == 0 ? (floatx16)(0.0f) : d[T & 1], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (F32A ? t == kCT - 1 : t == 0) {
+              // the next row tile's operands (f32: into the registers the instruction above was the last to read)
+              constexpr int ns = F32A ? 0 : slot ^ 1;
+              if constexpr (r + 1 < RT) read_a(ns, j, pa, bl, r + 1);
+              else read_a(ns, j, pan, ends_sub ? 0 : bl + 1, 0);
+            }
+            if constexpr (j == 0 && T == 0) unpack_b(1);
+            if constexpr (j == 0 && T == 1) read_b(0, pbn, ends_stage ? 0 : sb + 1), read_b(1, pbn, ends_stage ? 0 : sb + 1);
+            if constexpr (j == (TILES == 2 ? NM - 1 : 0) && T == TILES - 1) unpack_b(0);
+            scale_part<NM, j>(acc[pr][pt], d[(T + 1) & 1], T ? dq[pt] : dqp);
+            if constexpr (j == NM - 1) {
+              constexpr int from = (bl * TILES + T) * LOADS / SLOTS, to = (bl * TILES + T + 1) * LOADS / SLOTS;
+              static_for<to - from>([&](auto Qn) __attribute__((always_inline)) { issue_load(std::integral_constant<int, from + Qn>{}); });
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          });
+        });
+        dqp = dq[kCT - 1];
+      });
+      if constexpr (last) {
+        // the additive part of the stage's blocks: means times m (Q4) or the scale (Q8)
+        half8 bm[kCT];
+#pragma unroll
+        for (int t = 0; t < kCT; t++) {
+          uint32_t w0, w1 = 0;
+          const half2_t mulp = __builtin_bit_cast(half2_t, addp);
+          if constexpr (FMT == MGN_FMT_Q4) {
+            w0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(mcur[t][1], mcur[t][0], 0x07060302u)) * mulp);
+            w1 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(mcur[t][3], mcur[t][2], 0x07060302u)) * mulp);
+          } else {
+            w0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, mcur[t][0]) * mulp);
+          }
+          bm[t] = as_half8(w0, w1, 0u, 0u);
+        }
+        const uint8_t* const ps = lds_st + sbuf * STAGE_BYTES + s_rd;
+#pragma unroll
+        for (int r = RT - 1; r >= 0; r--) {
+          half8 am;
+          if constexpr (FMT == MGN_FMT_Q4) {
+            const uint2 v = *(const uint2*)(ps + r * (32 * SB * 4));
+            am = as_half8(v.x, v.y, 0u, 0u);
+          } else {
+            am = as_half8(*(const uint32_t*)(ps + r * (32 * SB * 4)), 0u, 0u, 0u);
+          }
+#pragma unroll
+          for (int t = kCT - 1; t >= 0; t--) acc[r][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm[t], acc[r][t], 0, 0, 0);
+        }
+      }
+      wait_loads<S::in_flight(u)>();
+      lds_barrier();
+      abuf = anext;
+      if constexpr (last) sbuf = snext;
+    });
+  }
+  acc[RT - 1][kCT - 1] = __builtin_elementwise_fma(d[1], (floatx16)(dqp), acc[RT - 1][kCT - 1]);
+  wait_loads<0>();
+  lds_barrier();
+
+  // ---- true units ----
+  if constexpr (F32A) {
+    // the rows' scales from the lanes that hold them to the lanes that hold the rows' sums
+    float* const sc = (float*)lds + wave * (RT * 32);
+#pragma unroll
+    for (int r = 0; r < RT; r++) sc[r * 32 + c] = row_scale[r];
+    const uint32_t mine = st1 > st0 + ks ? (st1 - 1 - st0 - ks) / WK * WK + st0 + ks : 0u;  // the stream's last stage
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+      floatx16 f;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        floatx4 v = *(const floatx4*)(sc + r * 32 + q * 8 + h * 4);
+        if (mixed) {
+          // the sums are on the scale of the stream's own last slice: from there to the row's last
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const uint32_t row = row0 + (wm * RT + r) * 32 + q * 8 + h * 4 + i;
+            const uint32_t own = __builtin_bit_cast(uint32_t, x.inv[(size_t)(mine * SB / 8) * x.mpad + row]);
+            const uint32_t end = __builtin_bit_cast(uint32_t, x.inv[(size_t)((x.bpc - 1) / 8) * x.mpad + row]);
+            v[i] *= __builtin_bit_cast(float, 0x3F800000u + (own - end));
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) f[q * 4 + i] = v[i];
+      }
+#pragma unroll
+      for (int t = 0; t < kCT; t++) acc[r][t] *= f;
+    }
+    if constexpr (WK > 1) lds_barrier();
+  } else {
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+      for (int t = 0; t < kCT; t++) acc[r][t] *= x.unit;
+  }
+  if constexpr (WK > 1) {
+    // the streams' sums meet in LDS, in stream order
+    float* const red = (float*)lds4;
+    constexpr int G = WM * WN;  // waves per stream
+    for (uint32_t s = 1; s < WK; s++) {
+      if (ks == s) {
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+#pragma unroll
+          for (int t = 0; t < kCT; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+              *(floatx4*)(red + ((((wave % G) * RT + r) * kCT + t) * 4 + i) * 256 + lane * 4) =
+                  floatx4{acc[r][t][4 * i], acc[r][t][4 * i + 1], acc[r][t][4 * i + 2], acc[r][t][4 * i + 3]};
+      }
+      lds_barrier();
+      if (ks == 0) {
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+#pragma unroll
+          for (int t = 0; t < kCT; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              const floatx4 v = *(const floatx4*)(red + ((((wave % G) * RT + r) * kCT + t) * 4 + i) * 256 + lane * 4);
+#pragma unroll
+              for (int e = 0; e < 4; e++) acc[r][t][4 * i + e] += v[e];
+            }
+      }
+      lds_barrier();
+    }
+    if (ks > 0) return;
+  }
+  // Stores through a buffer descriptor that ends with the last row: what lies past it is dropped.
+  const bool direct = x.parts == 1;
+  const uint32_t bytes = x.m * x.n * 4u;
+  const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc((void*)(direct ? x.c : x.partial + (size_t)part * x.m * x.n), 0, bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t res = __builtin_amdgcn_make_buffer_rsrc((void*)x.dres, 0, bytes, 0x00020000);
+  const uint32_t ops = direct ? x.epilogue : 0u;
+  const bool residual = direct && x.dres;
+  // (unary operations run in a loop over the lane's own words, parked in LDS: unrolled over the
+  // registers they would be most of the kernel)
+  float* const strip = (float*)lds4 + wave * 1024 + lane;
+  if (ops != 0) lds_barrier();
+#pragma unroll
+  for (int r = 0; r < RT; r++)
+#pragma unroll
+    for (int t = 0; t < kCT; t++) {
+      const uint32_t col = col0 + (wn * kCT + t) * 32 + c;
+      const uint32_t off = ((row0 + (wm * RT + r) * 32 + h * 4) * x.n + col) * 4u;
+      if (col >= x.n) continue;
+      if (residual) {
+        float dv[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) dv[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(res, off + ((i >> 2) * 8 + (i & 3)) * x.n * 4u, 0, 0));
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[r][t][i] += dv[i];
+      }
+      if (ops != 0) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) strip[i * 64] = acc[r][t][i];
+#pragma nounroll
+        for (int i = 0; i < 16; i++) strip[i * 64] = apply_epilogue(strip[i * 64], ops);
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[r][t][i] = strip[i * 64];
+      }
+#pragma unroll
+      for (int i = 0; i < 16; i++)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, (float)acc[r][t][i]), out, off + ((i >> 2) * 8 + (i & 3)) * x.n * 4u, 0, 0);
+    }
+}
+
+// ---- what the kernel needs to know about the activations, one workgroup per row ----
+constexpr uint32_t kMaxSlices = 256;
+constexpr int kTop = 14;  // a row's largest magnitude is brought into [2^14, 2^15)
+
+__device__ __forceinline__ void store_mean(uint16_t* means, int sb, uint32_t mpad, uint32_t row, uint32_t block, float mean) {
+  const uint32_t mh = pack_rtz(mean, 0.0f);
+  const uint32_t ml = pack_rtz((mean - half_lo(mh)) * 2048.0f, 0.0f);
+  uint16_t* const p = means + ((size_t)(block / sb) * mpad + row) * (sb * 2) + block % sb;
+  p[0] = (uint16_t)mh;
+  p[sb] = (uint16_t)ml;
+}
+
+// grid.x = mpad rows, 512 threads: half-wave w converts the row's slices w, w + 16, ..; HELD of them stay
+// in registers between the search for the row's largest magnitude and the conversion, the rest of a
+// longer row is read twice.
+template <int FMT, int HELD>
+__global__ __launch_bounds__(512) void prepare_f32_kernel(const float* __restrict__ a, uint8_t* __restrict__ out, uint16_t* __restrict__ means,
+                                                          float* __restrict__ inv, float* __restrict__ row_scale, uint32_t* __restrict__ mixed,
+                                                          uint32_t m, uint32_t k, uint32_t nslices, uint32_t mpad,
+                                                          uint32_t* __restrict__ range_flag) {
+  constexpr int SB = stage_blocks(FMT);
+  __shared__ float smax[kMaxSlices];
+  const uint32_t row = blockIdx.x, tid = threadIdx.x, l = tid & 31, hw = tid >> 5;
+  const float* const src = a + (size_t)min(row, m - 1) * k;
+  const bool live = row < m;
+  floatx4 held[HELD][2];
+  auto load = [&](uint32_t s, floatx4 (&v)[2]) __attribute__((always_inline)) {
+    const uint32_t k0 = s * 256 + l * 8;
+    const bool ok = live && k0 < k;
+    const floatx4* const p = (const floatx4*)(src + (ok ? k0 : 0));
+    v[0] = p[0], v[1] = p[1];
+    if (!ok) v[0] = v[1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  };
+  auto largest = [&](const floatx4 (&v)[2], uint32_t s) __attribute__((always_inline)) {
+    float am = fmaxf(fmaxf(fmaxf(fabsf(v[0].x), fabsf(v[0].y)), fmaxf(fabsf(v[0].z), fabsf(v[0].w))),
+                     fmaxf(fmaxf(fabsf(v[1].x), fabsf(v[1].y)), fmaxf(fabsf(v[1].z), fabsf(v[1].w))));
+    am = group_max32(am);
+    if (l == 0) smax[s] = am;
+  };
+#pragma unroll
+  for (int i = 0; i < HELD; i++) load(hw + 16 * i, held[i]);
+#pragma unroll
+  for (int i = 0; i < HELD; i++)
+    if (hw + 16 * i < nslices) largest(held[i], hw + 16 * i);
+  for (uint32_t s = hw + 16 * HELD; s < nslices; s += 16) {
+    floatx4 v[2];
+    load(s, v);
+    largest(v, s);
+  }
+  __syncthreads();
+  // (a NaN never wins fmaxf; an infinity does)
+  float rmax = 0.0f, rmin = __builtin_inff();  // the largest, and the smallest of the slices that hold anything
+  for (uint32_t s = l; s < nslices; s += 32) {
+    const float v = smax[s];
+    rmax = fmaxf(rmax, v);
+    if (((__builtin_bit_cast(uint32_t, v) >> 23) & 255) > 27) rmin = fminf(rmin, v);  // above 2^-100
+  }
+  rmax = group_max32(rmax);
+  rmin = -group_max32(-rmin);
+  const int er = (int)(__builtin_bit_cast(uint32_t, rmax) >> 23) - 127;
+  const bool bad = er >= 100;
+  const int shr = (er <= -100 || bad) ? 0 : kTop - er;
+  // One scale for the row, unless a slice would keep fewer than 22 bits of its largest magnitude on it
+  // (the low halves end at 2^-24, so below 2^-2): such slices get scales of their own.
+  auto shift = [&](float smx) __attribute__((always_inline)) {
+    const int es = (int)(__builtin_bit_cast(uint32_t, smx) >> 23) - 127;
+    return !bad && shr != 0 && es > -100 && es + shr < -2 ? min(kTop - es, shr + 60) : shr;
+  };
+  const bool any_mixed = shift(rmin) != shr;
+  auto convert = [&](const floatx4 (&v)[2], uint32_t s) __attribute__((always_inline)) {
+    const int sh = any_mixed ? shift(smax[s]) : shr;
+    const float scale = __builtin_bit_cast(float, (uint32_t)(127 + sh) << 23);
+    if (l == 0) {
+      const float back = __builtin_bit_cast(float, (uint32_t)(127 - sh) << 23);
+      inv[(size_t)s * mpad + row] = back;
+      if (s == nslices - 1) row_scale[row] = bad ? __builtin_nanf("") : back;
+    }
+    const floatx4 x0 = v[0] * scale, x1 = v[1] * scale;
+    const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    uint32_t hp[4], lp[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      hp[e] = pack_rtz(x[2 * e], x[2 * e + 1]);
+      lp[e] = pack_rtz(x[2 * e] - half_lo(hp[e]), x[2 * e + 1] - half_hi(hp[e]));
+    }
+    float sum = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+    if (live) {
+      uint8_t* const dst = out + ((size_t)row * nslices * 8 + s * 8 + (l >> 2)) * 128 + (l & 3) * 16;
+      *(uint4*)dst = make_uint4(hp[0], hp[1], hp[2], hp[3]);
+      *(uint4*)(dst + 64) = make_uint4(lp[0], lp[1], lp[2], lp[3]);
+    }
+    sum += dpp_move<kDppQuadXor1>(sum);
+    sum += dpp_move<kDppQuadXor2>(sum);
+    if ((l & 3) == 0) store_mean(means, SB, mpad, row, s * 8 + (l >> 2), sum * 0.03125f);
+  };
+#pragma unroll
+  for (int i = 0; i < HELD; i++)
+    if (hw + 16 * i < nslices) convert(held[i], hw + 16 * i);
+  for (uint32_t s = hw + 16 * HELD; s < nslices; s += 16) {
+    floatx4 v[2];
+    load(s, v);
+    convert(v, s);
+  }
+  if (tid == 0) {
+    mixed[row] = any_mixed ? 1u : 0u;
+    if (range_flag && rmax >= 65504.0f) *range_flag = 1u;  // a promise (MGN_ACT_FP16_RANGE) that does not hold
+  }
+}
+
+template <int FMT>
+__global__ __launch_bounds__(256) void prepare_f16_kernel(const _Float16* __restrict__ a, uint16_t* __restrict__ means, uint32_t m,
+                                                          uint32_t k, uint32_t nslices, uint32_t mpad) {
+  constexpr int SB = stage_blocks(FMT);
+  const uint32_t row = blockIdx.x;
+  for (uint32_t u = threadIdx.x; u < nslices * 32; u += 256) {
+    const uint32_t k0 = u * 8;
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (row < m && k0 < k) v = *(const uint4*)(a + (size_t)row * k + k0);
+    const half2_t ones = {(_Float16)1.0f, (_Float16)1.0f};
+    float s = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, v.x), ones, 0.0f, false);
+    s = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, v.y), ones, s, false);
+    s = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, v.z), ones, s, false);
+    s = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, v.w), ones, s, false);
+    s += dpp_move<kDppQuadXor1>(s);
+    s += dpp_move<kDppQuadXor2>(s);
+    if ((u & 3) == 0) store_mean(means, SB, mpad, row, u >> 2, s * 0.03125f);
+  }
+}
+
+// C = f(sum over the parts, in part order, + D); V words per thread and step
+template <int V>
+__global__ __launch_bounds__(256) void add_parts_kernel(const float* __restrict__ partial, const float* __restrict__ dres, float* __restrict__ c,
+                                                        uint64_t count, uint32_t parts, uint32_t epilogue) {
+  typedef float vec __attribute__((ext_vector_type(V)));
+  for (uint64_t i = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * V; i < count; i += (uint64_t)gridDim.x * 256 * V) {
+    vec s = *(const vec*)(partial + i);
+    uint32_t p = 1;
+    for (; p + 4 <= parts; p += 4) {
+      const vec a = *(const vec*)(partial + p * count + i), b = *(const vec*)(partial + (p + 1) * count + i);
+      const vec e = *(const vec*)(partial + (p + 2) * count + i), f = *(const vec*)(partial + (p + 3) * count + i);
+      s = s + a, s = s + b, s = s + e, s = s + f;
+    }
+    for (; p < parts; p++) s = s + *(const vec*)(partial + p * count + i);
+    if (dres) s = s + *(const vec*)(dres + i);
+    if (epilogue != 0) {
+#pragma unroll
+      for (int e = 0; e < V; e++) s[e] = apply_epilogue(s[e], epilogue);
+    }
+    *(vec*)(c + i) = s;
+  }
+}
+
+// ---- plans ----
+// The workgroup shapes that are built, by (format, activations): rows x columns per workgroup and what a
+// stage costs on them, in us per 128 elements of K: one workgroup per CU on all 256 (t1), and each
+// further round of 256 (tn; where two fit a CU, what the second costs beside the first).
+struct BlockConfig {
+  void (*kernel)(BlockArgs);
+  uint32_t rows, cols, threads;
+  size_t lds;
+  double t1, tn;
+};
+
+template <int FMT, bool F32A, int RT, int WM, int WN, int SUBB, int PD, int SD>
+BlockConfig block_config(double t1, double tn) {
+  using S = BlockShape<FMT, F32A, RT, WM, WN, 1, SUBB, PD, SD>;
+  static_assert(S::LDS <= 160 * 1024, "fits a CU");
+  return {block_kernel<FMT, F32A, RT, WM, WN, 1, SUBB, PD, SD>, (uint32_t)S::ROWS, (uint32_t)S::COLS, 64u * S::WAVES, S::LDS, t1, tn};
+}
+
+constexpr int kBlockConfigs = 7;
+const BlockConfig* block_configs(int fmt, bool f32a) {
+  static const BlockConfig q4_f16[kBlockConfigs] = {
+      block_config<0, false, 4, 2, 4, 2, 2, 1>(5.7, 4.1), block_config<0, false, 3, 2, 4, 2, 2, 2>(4.65, 3.1),
+      block_config<0, false, 2, 2, 4, 2, 2, 2>(3.6, 2.6), block_config<0, false, 3, 1, 4, 2, 2, 1>(2.9, 1.9),
+      block_config<0, false, 2, 1, 4, 2, 2, 1>(2.3, 1.5), block_config<0, false, 1, 1, 4, 2, 3, 2>(1.33, 0.9),
+      block_config<0, false, 1, 2, 2, 2, 2, 2>(1.45, 0.8)};
+  static const BlockConfig q4_f32[kBlockConfigs] = {
+      block_config<0, true, 4, 2, 4, 1, 2, 1>(7.6, 6.7), block_config<0, true, 3, 2, 4, 1, 2, 2>(6.3, 5.2),
+      block_config<0, true, 2, 2, 4, 1, 3, 1>(4.7, 3.2), block_config<0, true, 3, 1, 4, 1, 2, 1>(4.4, 2.4),
+      block_config<0, true, 2, 1, 4, 1, 3, 1>(2.95, 1.9), block_config<0, true, 1, 1, 4, 1, 4, 1>(2.0, 1.3),
+      block_config<0, true, 1, 2, 2, 1, 3, 1>(1.65, 1.2)};
+  static const BlockConfig q8_f16[kBlockConfigs] = {
+      block_config<1, false, 3, 2, 4, 2, 2, 3>(5.3, 3.5), block_config<1, false, 3, 2, 4, 2, 2, 2>(5.4, 3.8),
+      block_config<1, false, 2, 2, 4, 2, 2, 3>(4.35, 2.6), block_config<1, false, 3, 1, 4, 2, 2, 3>(3.3, 2.6),
+      block_config<1, false, 2, 1, 4, 2, 2, 3>(2.65, 2.2), block_config<1, false, 1, 1, 4, 2, 3, 2>(1.95, 1.9),
+      block_config<1, false, 1, 2, 2, 2, 2, 3>(1.6, 1.2)};
+  static const BlockConfig q8_f32[kBlockConfigs] = {
+      block_config<1, true, 4, 2, 4, 1, 2, 1>(8.4, 7.6), block_config<1, true, 3, 2, 4, 1, 2, 2>(6.9, 5.5),
+      block_config<1, true, 2, 2, 4, 1, 3, 2>(5.4, 3.9), block_config<1, true, 3, 1, 4, 1, 2, 1>(5.25, 2.6),
+      block_config<1, true, 2, 1, 4, 1, 3, 2>(3.6, 2.8), block_config<1, true, 1, 1, 4, 1, 4, 2>(2.4, 2.3),
+      block_config<1, true, 1, 2, 2, 1, 3, 2>(2.45, 1.4)};
+  return fmt == MGN_FMT_Q4 ? (f32a ? q4_f32 : q4_f16) : (f32a ? q8_f32 : q8_f16);
+}
+
+struct BlockPlan {
+  const BlockConfig* cfg;
+  uint32_t rows_per_launch, rowgroups, colgroups, parts, stages, nslices, mpad;
+  size_t a_bytes, means_bytes, inv_bytes, partial_bytes;  // in the workspace, in this order (row scales and flags behind inv)
+  double us;
+};
+
+size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+bool plan_block_rows(const LaunchArgs& x, uint32_t m, BlockPlan* out) {
+  const bool f32a = !x.a_is_f16;
+  const uint64_t k = x.w.k, n = x.w.n;
+  const uint32_t bpc = x.w.k / 32, sb = stage_blocks(x.w.fmt);
+  const uint32_t stages = (bpc + sb - 1) / sb, nslices = (bpc + 7) / 8;
+  if (m == 0 || bpc == 0 || nslices > kMaxSlices) return false;
+  if (n * bpc * 32 >= (1ull << 32)) return false;  // a lane's weight offsets are 32-bit
+  const BlockConfig* const cfgs = block_configs(x.w.fmt, f32a);
+  double best = 0;
+  for (int i = 0; i < kBlockConfigs; i++) {
+    const BlockConfig& c = cfgs[i];
+    const uint32_t rowgroups = (m + c.rows - 1) / c.rows, mpad = rowgroups * c.rows;
+    const uint64_t colgroups = (n + c.cols - 1) / c.cols;
+    const uint64_t tiles = rowgroups * colgroups;
+    if (tiles > (1u << 24) || (uint64_t)mpad * n * 4 >= (1ull << 32)) continue;
+    const size_t a_bytes = f32a ? align256((size_t)m * nslices * 1024) : 0;
+    const size_t a_read = f32a ? (size_t)m * nslices * 1024 : (size_t)m * k * 2;
+    if (a_read >= (1ull << 32)) continue;
+    const size_t means = align256((size_t)nslices * 8 * mpad * 4 + 4096);
+    const size_t inv = f32a ? align256((size_t)nslices * mpad * 4 + (size_t)mpad * 8) : 0;
+    for (uint32_t parts = 1; parts <= stages && parts <= 32; parts++) {
+      const uint32_t spp = (stages + parts - 1) / parts;
+      if ((stages + spp - 1) / spp != parts) continue;  // same split, already seen
+      const size_t partial = parts > 1 ? (size_t)parts * m * n * 4 : 0;
+      if (a_bytes + means + inv + partial > x.block_ws_bytes) break;
+      const uint64_t wgs = tiles * parts;
+      const double nk = spp * (double)sb / 4.0;
+      const double rounds = std::ceil((double)wgs / x.num_cus);
+      double us = nk * (c.t1 + (rounds - 1) * c.tn);
+      const double mem = (double)bpc * n * (x.w.fmt == MGN_FMT_Q4 ? 20 : 34) / 5.0e6 + (double)m * n * 4 / 4.0e6;
+      us = std::max(us, mem) + 3.5 + (double)m * n * 4 / 8.0e6;
+      if (parts > 1) us += 3.5 + (2.0 * parts + 1) * m * n * 4 / 5.0e6;
+      us += 2.2 + (double)m * k * (f32a ? 8 : 2) / 5.0e6;
+      if (best == 0 || us < best) {
+        best = us;
+        *out = BlockPlan{&c, m, rowgroups, (uint32_t)colgroups, parts, stages, nslices, mpad, a_bytes, means, inv, partial, us};
+      }
+    }
+  }
+  return best != 0;
+}
+
+// As many rows per launch as the workspace has room for: all of them, or blocks of rows one after the other.
+bool plan_block(const LaunchArgs& x, BlockPlan* out) {
+  if (!x.block_ws || x.n_more != 0 || x.pro_kind != kProNone) return false;
+  for (uint32_t rows = x.m;;) {
+    if (plan_block_rows(x, rows, out)) {
+      out->us *= (x.m + rows - 1) / rows;
+      return true;
+    }
+    if (rows <= 256) return false;
+    rows = (rows / 2 + 255) / 256 * 256;
+  }
+}
+
+uint32_t half_pair(float v) {
+  const uint16_t b = f32_to_f16_bits(v);
+  return b | ((uint32_t)b << 16);
+}
+
+template <int FMT>
+int launch_block_rows(ihipStream_t* s, const LaunchArgs& x, const BlockPlan& p) {
+  const bool f32a = !x.a_is_f16;
+  char* const ws = (char*)x.block_ws;
+  uint8_t* const prepared = (uint8_t*)ws;
+  uint16_t* const means = (uint16_t*)(ws + p.a_bytes);
+  float* const inv = (float*)(ws + p.a_bytes + p.means_bytes);
+  float* const row_scale = inv + (size_t)p.nslices * p.mpad;
+  uint32_t* const mixed = (uint32_t*)(row_scale + p.mpad);
+  float* const partial = (float*)(ws + p.a_bytes + p.means_bytes + p.inv_bytes);
+  if (f32a) {
+    auto prep = p.nslices <= 16 ? prepare_f32_kernel<FMT, 1> : prepare_f32_kernel<FMT, 4>;
+    hipLaunchKernelGGL(prep, dim3(p.mpad), dim3(512), 0, s, (const float*)x.a, prepared, means, inv, row_scale, mixed, x.m, x.w.k, p.nslices,
+                       p.mpad, x.promised_range ? x.range_flag : nullptr);
+  } else {
+    hipLaunchKernelGGL(prepare_f16_kernel<FMT>, dim3(p.mpad), dim3(256), 0, s, (const _Float16*)x.a, means, x.m, x.w.k, p.nslices, p.mpad);
+  }
+  MGN_HIP_LAUNCH_CHECK();
+  BlockArgs a{};
+  a.a = f32a ? (const void*)prepared : x.a;
+  a.means = means, a.inv = inv, a.row_scale = row_scale, a.mixed = mixed, a.meta = x.w.meta, a.quants = x.w.quants;
+  const size_t nb = (size_t)(x.w.k / 32) * x.w.n;
+  a.a_pitch = f32a ? p.nslices * 1024 : x.w.k * 2;
+  a.a_bytes = x.m * a.a_pitch;
+  // (256 zero blocks follow the weight's own, which a column's last stage may reach into)
+  a.quant_bytes = (uint32_t)std::min<size_t>((nb + 256) * (FMT == MGN_FMT_Q4 ? 16 : 32), 0xFFFFFFFFu);
+  a.meta_bytes = (uint32_t)((nb + 256) * (FMT == MGN_FMT_Q4 ? 4 : 2));
+  a.means_bytes = (uint32_t)p.means_bytes;
+  a.m = x.m, a.mpad = p.mpad, a.n = x.w.n, a.bpc = x.w.k / 32, a.stages = p.stages;
+  a.rowgroups = p.rowgroups, a.colgroups = p.colgroups, a.parts = p.parts;
+  // The sums run in units of 2^lift / 32 (Q4) or 2^lift / 4096 (Q8) of the result: the additive constants
+  // enter times 2^lift (WeightView::additive_lift), their means as they are.
+  const int lift = (int)std::min<uint32_t>(x.w.additive_lift, 15u);
+  const float sign = FMT == MGN_FMT_Q4 ? 1.0f : -1.0f;
+  a.add_hi = half_pair(sign * std::ldexp(1.0f, lift)), a.add_lo = half_pair(sign * std::ldexp(1.0f, lift - 11));
+  a.dscale = std::ldexp(1.0f, (FMT == MGN_FMT_Q4 ? 15 : 12) + lift);
+  a.unit = std::ldexp(1.0f, (FMT == MGN_FMT_Q4 ? 5 : 12) - lift);
+  a.dres = x.d, a.c = x.c, a.partial = partial, a.epilogue = x.epilogue;
+  if (p.cfg->lds > 64 * 1024) {
+    static std::atomic<uint64_t> big_lds_done[4][kBlockConfigs];
+    const BlockConfig* const first = block_configs(FMT, f32a);
+    if (int e = enable_big_lds(p.cfg->kernel, x.device, big_lds_done[FMT * 2 + f32a][p.cfg - first])) return e;
+  }
+  const uint32_t tiles = p.rowgroups * p.colgroups;
+  hipLaunchKernelGGL(p.cfg->kernel, dim3((tiles + 7) / 8 * 8 * p.parts), dim3(p.cfg->threads), p.cfg->lds, s, a);
+  MGN_HIP_LAUNCH_CHECK();
+  if (p.parts > 1) {
+    const uint64_t count = (uint64_t)x.m * x.w.n;
+    const bool wide = count % 4 == 0 && ((uintptr_t)x.c & 15) == 0 && ((uintptr_t)x.d & 15) == 0;
+    const uint64_t steps = wide ? count / 4 : count;
+    hipLaunchKernelGGL(wide ? add_parts_kernel<4> : add_parts_kernel<1>, dim3((unsigned)std::min<uint64_t>((steps + 255) / 256, 2048)), dim3(256), 0, s,
+                       partial, x.d, x.c, count, p.parts, x.epilogue);
+    MGN_HIP_LAUNCH_CHECK();
+  }
+  return 0;
+}
+
+}  // namespace
+
+bool block_mfma_supported(const LaunchArgs& x) {
+  BlockPlan p;
+  return plan_block(x, &p);
+}
+
+double block_mfma_us(const LaunchArgs& x) {
+  BlockPlan p;
+  return plan_block(x, &p) ? p.us : 0.0;
+}
+
+int launch_matmul_block_mfma(ihipStream_t* s, const LaunchArgs& x) {
+  BlockPlan p;
+  if (!plan_block(x, &p)) return (int)hipErrorInvalidValue;
+  const uint32_t rows = p.rows_per_launch;
+  for (uint32_t r0 = 0; r0 < x.m; r0 += rows) {
+    LaunchArgs y = x;
+    y.m = std::min(rows, x.m - r0);
+    y.a = (const char*)x.a + (size_t)r0 * x.w.k * (x.a_is_f16 ? 2 : 4);
+    y.c = x.c + (size_t)r0 * x.w.n;
+    y.d = x.d ? x.d + (size_t)r0 * x.w.n : nullptr;
+    if (y.m != rows && !plan_block_rows(y, y.m, &p)) return (int)hipErrorInvalidValue;
+    const int e = x.w.fmt == MGN_FMT_Q4 ? launch_block_rows<MGN_FMT_Q4>(s, y, p) : launch_block_rows<MGN_FMT_Q8>(s, y, p);
+    if (e) return e;
+  }
+  return 0;
+}
+
+bool describe_block_mfma(const LaunchArgs& x, mgn_block_plan* out) {
+  BlockPlan p;
+  if (!plan_block(x, &p)) return false;
+  out->rows = p.cfg->rows, out->cols = p.cfg->cols, out->threads = p.cfg->threads, out->lds_bytes = (uint32_t)p.cfg->lds;
+  out->row_groups = p.rowgroups, out->col_groups = p.colgroups, out->k_parts = p.parts;
+  out->launches = (x.m + p.rows_per_launch - 1) / p.rows_per_launch;
+  out->workspace_bytes = p.a_bytes + p.means_bytes + p.inv_bytes + p.partial_bytes;
+  out->us = (float)p.us;
+  return true;
+}
+
+}  // namespace mgn

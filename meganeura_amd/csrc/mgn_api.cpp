@@ -118,18 +118,49 @@ mgn_status weight_alloc(mgn_ctx* ctx, mgn_fmt fmt, size_t rows, size_t cols, mgn
   return MGN_OK;
 }
 
-// The automatic choice of a kernel family.  M <= 4: the MFMA GEMV.  Larger M: the resident
+// The automatic choice of a kernel family among those that need nothing prepared in a workspace of the
+// context's.  M <= 4: the MFMA GEMV.  Larger M: the resident
 // 16x16x32 kernel where it measured faster; the 32x32 tiled kernel for fp16 activations and
 // for f32 activations the caller has promised to keep in the fp16 range (it splits them
 // without rescaling), if the weight's block constants are in its range too; the rescaling
 // 16x16x32 kernels for everything else.
-mgn_route auto_route(const mgn::LaunchArgs& x, bool any_magnitude) {
+mgn_route basic_route(const mgn::LaunchArgs& x, bool any_magnitude) {
   if (mgn::gemv_mfma_supported(x)) return MGN_ROUTE_GEMV_MFMA;
   if (mgn::tile_mfma_preferred(x)) return MGN_ROUTE_TILE_MFMA;
   if ((x.a_is_f16 || !any_magnitude) && mgn::gemm_mfma_supported(x)) return MGN_ROUTE_GEMM_MFMA;
   if (mgn::tile_mfma_supported(x)) return MGN_ROUTE_TILE_MFMA;
   if (mgn::gemv_supported(x)) return MGN_ROUTE_GEMV_VALU;
   return MGN_ROUTE_GENERIC;
+}
+
+// What a call of more than 16 rows takes on the kernel of basic_route, in us, fitted to 480 measured
+// calls (M = 20 .. 2048 on twelve shapes from 576 x 1536 to 14336 x 4096 and 576 x 49152, both formats, f32 and fp16
+// activations).  The resident kernel: so much per round of workgroups; the others: a fixed part and a
+// rate over the rows they compute, a multiple of 32.
+double basic_us(const mgn::LaunchArgs& x, mgn_route route) {
+  const bool q4 = x.w.fmt == MGN_FMT_Q4;
+  const double flops = 2.0 * ((x.m + 31) / 32 * 32) * x.w.k * x.w.n;
+  if (route == MGN_ROUTE_GEMM_MFMA) return 7.0 + flops / (q4 ? 390e6 : 310e6);
+  mgn_plan_info p{};
+  if (route != MGN_ROUTE_TILE_MFMA || !mgn::describe_tile_mfma(x, &p)) return 1e9;  // scalar routes
+  if (p.quads_per_wave != 0) return 9.0 + flops / (q4 ? 175e6 : 165e6);
+  const double rounds = std::ceil((double)p.grid[0] * p.grid[1] * p.grid[2] / x.num_cus), parts = p.k_parts > 1 ? 1.0 : 0.0;
+  if (p.full_steps == 2) return 10.5 * rounds + parts;
+  if (p.waves_n <= 16) return (q4 ? 9.0 : 10.0) * (x.a_is_f16 ? 0.9 : 1.0) * rounds + parts;
+  return (q4 ? 15.5 : 22.0) * (x.a_is_f16 ? 0.9 : 1.0) * rounds + (q4 ? 1.0 : 9.0) * parts;
+}
+
+// The automatic choice: the above, or the blocked kernel where it is expected to be the faster one.  (It
+// costs a launch to prepare the activations, one to add up K parts if there are any, and about 5 us
+// besides, but multiplies two to three times as fast: f32 512 x 4096 x 14336 295 -> 123 us, fp16 2048 x 4096 x
+// 14336 527 -> 283, 77 x 14336 x 4096 83 -> 47 with Q8, while 128 x 1024 x 3072 stays at 10 against 15.  Its own estimate
+// is made for weights that come from memory, the fit above for weights in the caches: hence 0.92.
+// Of the 480 calls 22 end up on a kernel more than 6 % slower than the better one.)
+mgn_route auto_route(const mgn::LaunchArgs& x, bool any_magnitude) {
+  const mgn_route basic = basic_route(x, any_magnitude);
+  if (x.m <= 16 || (x.m <= 32 && x.w.fmt == MGN_FMT_Q4)) return basic;
+  const double us = mgn::block_mfma_us(x);
+  return us > 0 && us * 0.92 < basic_us(x, basic) ? MGN_ROUTE_BLOCK_MFMA : basic;
 }
 
 // After the stream has been synchronised: did a wave give up waiting for another workgroup's
@@ -278,6 +309,10 @@ mgn_status mgn_ctx_create(int device_id, mgn_ctx** out) {
     return hip_fail(nullptr, "hand-over workspace allocation", e);
   }
   ctx->handover_bytes = mgn::kHandoverBytes;
+  if ((e = hipMalloc(&ctx->block_ws, mgn::kBlockWsBytes)) != hipSuccess) {
+    mgn_ctx_destroy(ctx);
+    return hip_fail(nullptr, "workspace allocation", e);
+  }
   // one pinned, device-mapped word: a kernel that meets activations it cannot represent sets it
   // and the next synchronising call reports MGN_ERANGE
   if ((e = hipHostMalloc((void**)&ctx->range_flag_host, 2 * sizeof(uint32_t), hipHostMallocMapped)) != hipSuccess ||
@@ -298,6 +333,7 @@ void mgn_ctx_destroy(mgn_ctx* ctx) {
   }
   if (ctx->scratch) (void)hipFree(ctx->scratch);
   if (ctx->handover) (void)hipFree(ctx->handover);
+  if (ctx->block_ws) (void)hipFree(ctx->block_ws);
   if (ctx->at_stage) (void)hipFree(ctx->at_stage);
   if (ctx->range_flag_host) (void)hipHostFree(ctx->range_flag_host);
   if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
@@ -334,7 +370,7 @@ mgn_status mgn_ctx_set_spin_limit(mgn_ctx* ctx, uint32_t polls) {
 
 mgn_status mgn_ctx_set_route(mgn_ctx* ctx, mgn_route route) {
   if (!ctx) return MGN_EINVAL;
-  if (route < MGN_ROUTE_AUTO || route > MGN_ROUTE_TILE_MFMA) return fail(ctx, MGN_EINVAL, "unknown route");
+  if (route < MGN_ROUTE_AUTO || route > MGN_ROUTE_BLOCK_MFMA) return fail(ctx, MGN_EINVAL, "unknown route");
   ctx->route = route;
   return MGN_OK;
 }
@@ -710,6 +746,9 @@ static mgn_status matmul_impl(mgn_ctx* ctx, const mgn_buf* a, bool a_is_f16, con
   x.n_counters = ctx->n_counters;
   x.handover = ctx->handover;
   x.handover_bytes = ctx->handover_bytes;
+  x.block_ws = ctx->block_ws;
+  x.block_ws_bytes = mgn::kBlockWsBytes;
+  x.promised_range = !ctx->any_magnitude;
   x.pro_kind = pro_kind;
   x.pro_weight = norm_weight ? (const float*)norm_weight->ptr : nullptr;
   x.pro_eps = eps;
@@ -724,8 +763,12 @@ static mgn_status matmul_impl(mgn_ctx* ctx, const mgn_buf* a, bool a_is_f16, con
   if (route == MGN_ROUTE_AUTO) route = auto_route(x, ctx->any_magnitude);
   if (static_workspace) {
     // Same plan as the allocating entry point (the planners see the same workspace limits), run
-    // on the library's static array if the plan's partial sums fit it; refused otherwise.
+    // on the library's static array if the plan's partial sums fit it; refused otherwise.  (What the
+    // blocked kernel takes is refused or not by the plan behind it; it runs on the context's own
+    // workspace, which is there since the context was created.)
     mgn_plan_info plan{};
+    const mgn_route taken = route;
+    if (route == MGN_ROUTE_BLOCK_MFMA) route = basic_route(x, ctx->any_magnitude);
     const bool parts = route == MGN_ROUTE_GEMV_MFMA   ? mgn::describe_gemv_mfma(x, &plan)
                        : route == MGN_ROUTE_GEMM_MFMA ? mgn::describe_gemm_mfma(x, &plan)
                        : route == MGN_ROUTE_TILE_MFMA ? mgn::describe_tile_mfma(x, &plan)
@@ -736,11 +779,13 @@ static mgn_status matmul_impl(mgn_ctx* ctx, const mgn_buf* a, bool a_is_f16, con
                   "mgn_matmul_q_static: this shape's K parts need " + std::to_string(need) +
                       " bytes of workspace, the static one holds " + std::to_string(kStaticPartialBytes) +
                       "; use mgn_matmul_q");
+    const bool blocked = taken == MGN_ROUTE_BLOCK_MFMA;
+    route = taken;
     x.scratch = ctx->static_scratch;
     x.scratch_capacity = kStaticPartialBytes;  // a launch that would need more than was checked above is refused, not run
     x.counters = (uint32_t*)((char*)ctx->static_scratch + kStaticPartialBytes);
     x.handover = (char*)ctx->static_scratch + kStaticHandoverOffset;
-    if (need > 0) {
+    if (need > 0 && !blocked) {
       // every call on this device shares the array: the arrival counters must start at zero and
       // the hand-over words the plan uses must be empty, whatever an earlier call left (fill
       // kernels, not memset nodes: safe under graph capture)
@@ -770,6 +815,10 @@ static mgn_status matmul_impl(mgn_ctx* ctx, const mgn_buf* a, bool a_is_f16, con
     case MGN_ROUTE_GEMM_MFMA:
       if (!mgn::gemm_mfma_supported(x)) return fail(ctx, MGN_EINVAL, "GEMM_MFMA route does not support this shape");
       rc = mgn::launch_matmul_gemm_mfma(ctx->stream, x);
+      break;
+    case MGN_ROUTE_BLOCK_MFMA:
+      if (!mgn::block_mfma_supported(x)) return fail(ctx, MGN_EINVAL, "BLOCK_MFMA route does not support this shape");
+      rc = mgn::launch_matmul_block_mfma(ctx->stream, x);
       break;
     default:
       rc = mgn::launch_matmul_generic(ctx->stream, x);
@@ -887,29 +936,47 @@ mgn_status mgn_matmul_q_f16a(mgn_ctx* ctx, const mgn_buf* a_f16, const mgn_weigh
   return matmul_impl(ctx, a_f16, true, w, d, c, m);
 }
 
-mgn_status mgn_matmul_q_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus, mgn_plan_info* out) {
-  if (!out || !valid_fmt(fmt) || m == 0 || k == 0 || n == 0 || k % 32 != 0 || num_cus <= 0) return MGN_EINVAL;
-  if (k > 0xFFFFFFE0ull || n > 0xFFFFFFFFull || (k / 32) * n >= 0x7FFFFFFFull) return MGN_EINVAL;
-  *out = mgn_plan_info{};
-  mgn::LaunchArgs x{};
-  x.w = mgn::WeightView{nullptr, nullptr, (uint32_t)k, (uint32_t)n, (int)fmt, true};
-  x.m = m;
-  x.a_is_f16 = a_is_f16 == 1;
-  x.num_cus = num_cus;
-  // the planners only look at whether a workspace exists, never through the pointers
+// The launch arguments of a shape as the planners see them: they only look at whether a workspace
+// exists, never through the pointers.
+static bool planned_args(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus, mgn::LaunchArgs* x) {
+  if (!valid_fmt(fmt) || m == 0 || k == 0 || n == 0 || k % 32 != 0 || num_cus <= 0) return false;
+  if (k > 0xFFFFFFE0ull || n > 0xFFFFFFFFull || (k / 32) * n >= 0x7FFFFFFFull) return false;
+  if (a_is_f16 < 0 || a_is_f16 > 2) return false;
+  *x = mgn::LaunchArgs{};
+  x->w = mgn::WeightView{nullptr, nullptr, (uint32_t)k, (uint32_t)n, (int)fmt, true};
+  x->m = m;
+  x->a_is_f16 = a_is_f16 == 1;
+  x->num_cus = num_cus;
   static char workspace_stand_in;
-  x.scratch = &workspace_stand_in;
-  x.scratch_bytes = mgn::kWorkspaceBytes;
-  x.counters = (uint32_t*)&workspace_stand_in;
-  x.n_counters = mgn::kWorkspaceCounters;
-  x.handover = &workspace_stand_in;
-  x.handover_bytes = mgn::kHandoverBytes;
-  if (a_is_f16 < 0 || a_is_f16 > 2) return MGN_EINVAL;
-  const mgn_route route = auto_route(x, a_is_f16 == 0);
+  x->scratch = &workspace_stand_in;
+  x->scratch_bytes = mgn::kWorkspaceBytes;
+  x->counters = (uint32_t*)&workspace_stand_in;
+  x->n_counters = mgn::kWorkspaceCounters;
+  x->handover = &workspace_stand_in;
+  x->handover_bytes = mgn::kHandoverBytes;
+  x->block_ws = &workspace_stand_in;
+  x->block_ws_bytes = mgn::kBlockWsBytes;
+  return true;
+}
+
+mgn_status mgn_matmul_q_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus, mgn_plan_info* out) {
+  mgn::LaunchArgs x{};
+  if (!out || !planned_args(fmt, m, k, n, a_is_f16, num_cus, &x)) return MGN_EINVAL;
+  *out = mgn_plan_info{};
+  const mgn_route route = basic_route(x, a_is_f16 == 0);
   if (route == MGN_ROUTE_GEMV_MFMA && mgn::describe_gemv_mfma(x, out)) return MGN_OK;
   if (route == MGN_ROUTE_GEMM_MFMA && mgn::describe_gemm_mfma(x, out)) return MGN_OK;
   if (route == MGN_ROUTE_TILE_MFMA && mgn::describe_tile_mfma(x, out)) return MGN_OK;
   out->route = route;
+  return MGN_OK;
+}
+
+mgn_status mgn_matmul_q_block_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus, mgn_block_plan* out) {
+  mgn::LaunchArgs x{};
+  if (!out || !planned_args(fmt, m, k, n, a_is_f16, num_cus, &x)) return MGN_EINVAL;
+  *out = mgn_block_plan{};
+  if (!mgn::describe_block_mfma(x, out)) return MGN_EUNSUPPORTED;
+  out->taken = auto_route(x, a_is_f16 == 0) == MGN_ROUTE_BLOCK_MFMA ? 1u : 0u;
   return MGN_OK;
 }
 

@@ -86,6 +86,11 @@ struct LaunchArgs {
   void* handover = nullptr;
   size_t handover_bytes = 0;
   uint32_t spin_limit = 1u << 20;  // polls after which a reading wave gives up and sets fault_flag
+  // Third workspace, of the blocked kernel: prepared activations, their block means and scales, partial
+  // results.  Written and read within one call.
+  void* block_ws = nullptr;
+  size_t block_ws_bytes = 0;
+  bool promised_range = false;  // f32 activations were promised to lie in the fp16 range: report those that do not
   // host-visible word a kernel sets when f32 activations leave the range it can represent
   uint32_t* range_flag = nullptr;
   // host-visible word set by a wave that gave up waiting for another workgroup's partial sums
@@ -130,6 +135,7 @@ bool describe_gemm_mfma(const LaunchArgs& a, mgn_plan_info* out);
 constexpr size_t kWorkspaceBytes = (size_t)16 << 20;
 constexpr uint32_t kWorkspaceCounters = 4096;
 constexpr size_t kHandoverBytes = (size_t)16 << 20;  // the counter-free hand-over workspace of a context
+constexpr size_t kBlockWsBytes = (size_t)96 << 20;   // the blocked kernel's (LaunchArgs::block_ws)
 int launch_matmul_gemm_mfma(ihipStream_t* s, const LaunchArgs& a);
 // kernels_chain.hip: a chain of dependent one-row matmuls in one launch.  One stage as the kernel
 // reads it from its table in device memory.
@@ -159,6 +165,12 @@ bool tile_mfma_supported(const LaunchArgs& a);
 bool tile_mfma_preferred(const LaunchArgs& a);
 bool describe_tile_mfma(const LaunchArgs& a, mgn_plan_info* out);
 int launch_matmul_tile_mfma(ihipStream_t* s, const LaunchArgs& a);
+// kernels_block.hip: the blocked kernel for many rows (32x32x16 tiles, activations prepared once per call)
+bool block_mfma_supported(const LaunchArgs& a);
+// what it is expected to take on a shape (0: not served)
+double block_mfma_us(const LaunchArgs& a);
+bool describe_block_mfma(const LaunchArgs& a, mgn_block_plan* out);
+int launch_matmul_block_mfma(ihipStream_t* s, const LaunchArgs& a);
 
 }  // namespace mgn
 
@@ -181,6 +193,7 @@ struct mgn_ctx {
   uint32_t* range_flag_host = nullptr;  // pinned, mapped, two words: [0] range, [1] hand-over gave up; written by kernels, read at sync points
   uint32_t* range_flag_dev = nullptr;   // the same words as the device sees them
   void* static_scratch = nullptr;       // this device's copy of the library's static workspace (mgn_matmul_q_static)
+  void* block_ws = nullptr;             // the blocked kernel's workspace (LaunchArgs::block_ws)
   void* at_stage = nullptr;             // transposed activations of the A^T matmul forms, grown on demand
   size_t at_stage_bytes = 0;
   std::vector<struct mgn_chain*> chains;  // live chains: their workspaces are emptied again after a fault

@@ -52,6 +52,7 @@ pub const MGN_ROUTE_GEMV_VALU: mgn_route = 2;
 pub const MGN_ROUTE_GEMV_MFMA: mgn_route = 3;
 pub const MGN_ROUTE_GEMM_MFMA: mgn_route = 4;
 pub const MGN_ROUTE_TILE_MFMA: mgn_route = 5;
+pub const MGN_ROUTE_BLOCK_MFMA: mgn_route = 6;
 
 /// `mgn_unary`: the operations `fuse_epilogues` folds into a matmul (src/compile.rs:915-1035).
 pub type mgn_unary = c_int;
@@ -116,6 +117,22 @@ pub struct mgn_plan_info {
     pub workspace_bytes: u64,
 }
 
+#[repr(C)]
+#[derive(Clone, Copy, Debug, Default)]
+pub struct mgn_block_plan {
+    pub taken: u32,
+    pub rows: u32,
+    pub cols: u32,
+    pub threads: u32,
+    pub lds_bytes: u32,
+    pub row_groups: u32,
+    pub col_groups: u32,
+    pub k_parts: u32,
+    pub launches: u32,
+    pub us: f32,
+    pub workspace_bytes: u64,
+}
+
 #[link(name = "mgn_hip")]
 extern "C" {
     pub fn mgn_ctx_create(device_id: c_int, out: *mut *mut mgn_ctx) -> mgn_status;
@@ -170,7 +187,8 @@ pub mod bench {
 
     #[link(name = "mgn_hip")]
     extern "C" {
-        pub fn mgn_ctx_set_route(ctx: *mut mgn_ctx, route: mgn_route) -> mgn_status;
+        pub fn mgn_matmul_q_block_plan(fmt: mgn_fmt, m: u32, k: u64, n: u64, a_is_f16: c_int, num_cus: c_int, out: *mut mgn_block_plan) -> mgn_status;
+    pub fn mgn_ctx_set_route(ctx: *mut mgn_ctx, route: mgn_route) -> mgn_status;
         pub fn mgn_ctx_set_spin_limit(ctx: *mut mgn_ctx, polls: u32) -> mgn_status;
         pub fn mgn_engine_clock_mhz(ctx: *mut mgn_ctx, loaded: c_int, mhz: *mut f32, cycles_per_round: *mut f32) -> mgn_status;
         pub fn mgn_matmul_q_loop(ctx: *mut mgn_ctx, a: *const mgn_buf, a_is_f16: c_int, weights: *const *const mgn_weight, count: usize, d: *const mgn_buf, c: *mut mgn_buf, m: u32, steps: u32) -> mgn_status;

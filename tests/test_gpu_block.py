@@ -1,0 +1,137 @@
+"""The blocked many-row kernel (MGN_ROUTE_BLOCK_MFMA) against the oracle, at the edges of what it is built
+from: tiles of 32 rows and 64 columns, workgroups of 32 to 256 rows, blocks of 32 / stages of 64 or 128 / slices
+of 256 elements of K, K parts; and rows whose magnitudes change along K."""
+import numpy as np
+import pytest
+
+from helpers import Q4, Q8, bits
+from meganeura_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = capi.Context(0)
+    yield c
+    c.close()
+
+
+def run(ctx, x, wt, f16=False, d=None, ops=(), route=capi.ROUTE_BLOCK_MFMA):
+    m, n = x.shape[0], wt.cols
+    a, c = ctx.upload(x), ctx.buffer(m * n * 4)
+    dd = ctx.upload(d) if d is not None else None
+    ctx.set_route(route)
+    try:
+        if ops:
+            ctx.matmul_q_epilogue(a, wt, c, m, list(ops), d=dd)
+        else:
+            (ctx.matmul_q_f16a if f16 else ctx.matmul_q)(a, wt, c, m, d=dd)
+        return c.download(np.float32, m * n).reshape(m, n)
+    finally:
+        ctx.set_route(capi.ROUTE_AUTO)
+        for b in (a, c) + ((dd,) if dd is not None else ()):
+            b.free()
+
+
+def assert_rows_close(got, want, x, k):
+    """f32 accumulation of K products of 22-bit activations with exact weights: 2^-22 per product and 2^-24 per
+    addition, both of the row's magnitude times the weights' (0.02, minima included 0.06) and, the errors
+    being as good as independent, growing with sqrt(K); eight times that for the largest of many."""
+    scale = np.abs(x).max(axis=1, keepdims=True).astype(np.float64)
+    bound = 8 * (2.0**-22 + 2.0**-24) * 0.06 * np.sqrt(k) * scale
+    assert np.isfinite(got).all()
+    err = np.abs(got - want)
+    assert (err <= bound + 2.0**-23 * np.abs(want)).all(), float((err / bound).max())
+
+
+SHAPES = [(1, 32, 1), (31, 64, 63), (33, 96, 65), (32, 128, 64), (64, 160, 128), (65, 288, 257), (97, 992, 300), (129, 1056, 513),
+          (200, 4064, 192), (257, 2048, 96), (77, 4096, 1000), (40, 16416, 70), (513, 320, 130)]
+
+
+@pytest.mark.parametrize("fmt", [Q4, Q8])
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("m,k,n", SHAPES)
+def test_edges_of_tiles_stages_and_parts(ctx, orc, fmt, f16, m, k, n):
+    w = synth.normal(2000 + fmt, k * n, 0.02).reshape(k, n)
+    x = synth.normal(2001 + m, m * k).reshape(m, k)
+    x = x.astype(np.float16) if f16 else x
+    packed = orc.quantize(fmt, w)
+    want = np.asarray(orc.matmul_f64(x.astype(np.float32), orc.dequantize(fmt, packed, k, n)), np.float64)
+    wt = ctx.weight(fmt, w)
+    got = run(ctx, x, wt, f16)
+    assert_rows_close(got, want, x.astype(np.float32), k)
+    assert np.array_equal(bits(run(ctx, x, wt, f16)), bits(got)), "not repeatable"
+    wt.free()
+
+
+@pytest.mark.parametrize("fmt", [Q4, Q8])
+@pytest.mark.parametrize("m,k,n", [(70, 2048, 4096), (50, 96, 70)])  # K in parts, K in one part
+def test_residual_and_epilogue(ctx, orc, fmt, m, k, n):
+    w = synth.normal(2010, k * n, 0.02).reshape(k, n)
+    x, d = synth.normal(2011, m * k).reshape(m, k), synth.normal(2012, m * n).reshape(m, n)
+    wt = ctx.weight(fmt, w)
+    want = orc.matmul_f32(x, orc.dequantize(fmt, orc.quantize(fmt, w), k, n), d).astype(np.float64)
+    orc.assert_close(run(ctx, x, wt, d=d), want, 1e-3, 1e-4)
+    silu_of_negated = -want / (1 + np.exp(want))
+    orc.assert_close(run(ctx, x, wt, d=d, ops=(capi.UNARY_NEG, capi.UNARY_SILU)), silu_of_negated, 1e-3, 1e-4)
+    wt.free()
+
+
+@pytest.mark.parametrize("fmt", [Q4, Q8])
+@pytest.mark.parametrize("k", [1280, 4128])
+def test_magnitudes_that_change_along_k(ctx, orc, fmt, k):
+    """A row whose slices of 256 elements lie up to 2^70 apart keeps its relative accuracy where only the
+    small slices meet a weight: the large slices' columns of the weight are zero blocks in the last column."""
+    m, n = 35, 130
+    w = synth.normal(2020, k * n, 0.02).reshape(k, n)
+    w[:512, n - 1] = 0.0
+    x = synth.normal(2021, m * k).reshape(m, k)
+    x[3, 256:] *= np.float32(2.0**-30)
+    x[4, 512:] *= np.float32(2.0**-70)
+    x[5] *= np.float32(1e-25)
+    x[6] *= np.float32(1e20)
+    x[7, 300:700] = 0.0
+    wt = ctx.weight(fmt, w)
+    dq = orc.dequantize(fmt, orc.quantize(fmt, w), k, n)
+    want = np.asarray(orc.matmul_f64(x, dq), np.float64)
+    got = run(ctx, x, wt)
+    assert_rows_close(got, want, x, k)
+    small = np.abs(x[[3, 4]][:, 512:]).max(axis=1)
+    zero = dq[:512, n - 1] == 0  # (Q4 carries zero blocks exactly only up to its minimum's rounding)
+    if zero.all():
+        err = np.abs(got[[3, 4], n - 1] - want[[3, 4], n - 1])
+        assert (err <= 8 * 2.0**-21 * 0.06 * np.sqrt(k) * small).all(), err / small
+    # infinities, NaNs and magnitudes of 2^100 stay in their rows
+    y = x.copy()
+    y[0, 5], y[1, 700], y[2, 40] = np.inf, np.nan, np.float32(2.0**101)
+    bad = run(ctx, y, wt)
+    assert not np.isfinite(bad[:3]).any()
+    assert np.array_equal(bits(bad[3:]), bits(got[3:]))
+    wt.free()
+
+
+@pytest.mark.parametrize("fmt", [Q4, Q8])
+def test_infinite_rows_of_fp16_activations_stay_on_their_own(ctx, orc, fmt):
+    m, k, n = 40, 96, 70  # K ends in the middle of the 64 elements that are loaded at once
+    x = synth.normal(2030, m * k).reshape(m, k).astype(np.float16)
+    wt = ctx.weight(fmt, synth.normal(2031, k * n, 0.02).reshape(k, n))
+    clean = run(ctx, x, wt, True)
+    x[11, 0], x[12, 1] = np.inf, np.nan
+    got = run(ctx, x, wt, True)
+    rest = [r for r in range(m) if r not in (11, 12)]
+    assert np.array_equal(bits(got[rest]), bits(clean[rest])) and not np.isfinite(got[[11, 12]]).any()
+    wt.free()
+
+
+def test_rows_beyond_the_workspace_run_in_blocks(ctx, orc):
+    m, k, n = 2500, 16384, 64
+    assert capi.matmul_block_plan(Q4, m, k, n).launches > 1
+    w = synth.normal(2040, k * n, 0.02).reshape(k, n)
+    x = np.tile(synth.normal(2041, 50 * k).reshape(50, k), (m // 50, 1))
+    wt = ctx.weight(Q4, w)
+    got = run(ctx, x, wt)
+    want = np.asarray(orc.matmul_f64(x[:50], orc.dequantize(Q4, orc.quantize(Q4, w), k, n)), np.float64)
+    for r in range(0, m, 50):
+        assert_rows_close(got[r:r + 50], want, x[:50], k)
+    wt.free()
