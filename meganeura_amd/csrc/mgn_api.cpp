@@ -240,6 +240,14 @@ mgn_status reserve_at_stage(mgn_ctx* ctx, size_t bytes) {
   return MGN_OK;
 }
 
+// mgn_buf_upload without the wait: src may change on return, what follows on the stream sees the bytes.
+mgn_status queue_upload(mgn_ctx* ctx, mgn_buf* buf, size_t offset, const void* src, size_t bytes) {
+  if (!ctx || !buf || (!src && bytes)) return fail(ctx, MGN_EINVAL, "null argument");
+  if (offset > buf->bytes || bytes > buf->bytes - offset) return fail(ctx, MGN_EINVAL, "upload exceeds buffer size");
+  if (const int e = copy_in(ctx, (char*)buf->ptr + offset, src, bytes)) return hip_fail(ctx, "upload", (hipError_t)e);
+  return MGN_OK;
+}
+
 // Would one launch serve these weights together (mgn_matmul_q_batch's own check)?  The plan
 // depends on the column count of the whole batch, so a weight that plans alone need not plan
 // next to its siblings.
@@ -329,6 +337,7 @@ void mgn_ctx_destroy(mgn_ctx* ctx) {
   if (!ctx) return;
   if (ctx->stream) {
     (void)hipStreamSynchronize(ctx->stream);
+    mgn::release_host_stage(ctx);
     (void)hipStreamDestroy(ctx->stream);
   }
   if (ctx->scratch) (void)hipFree(ctx->scratch);
@@ -346,6 +355,7 @@ const char* mgn_last_error(const mgn_ctx* ctx) { return ctx ? ctx->err.c_str() :
 mgn_status mgn_sync(mgn_ctx* ctx) {
   if (!ctx) return MGN_EINVAL;
   MGN_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  ctx->stage.used = 0;
   return check_range_flag(ctx);
 }
 
@@ -410,11 +420,10 @@ size_t mgn_buf_size(const mgn_buf* buf) { return buf ? buf->bytes : 0; }
 void* mgn_buf_device_ptr(const mgn_buf* buf) { return buf ? buf->ptr : nullptr; }
 
 mgn_status mgn_buf_upload(mgn_ctx* ctx, mgn_buf* buf, size_t offset, const void* src, size_t bytes) {
-  if (!ctx || !buf || (!src && bytes)) return fail(ctx, MGN_EINVAL, "null argument");
-  if (offset > buf->bytes || bytes > buf->bytes - offset) return fail(ctx, MGN_EINVAL, "upload exceeds buffer size");
+  if (const mgn_status st = mgn::queue_upload(ctx, buf, offset, src, bytes)) return st;
   if (bytes == 0) return MGN_OK;
-  MGN_HIP(ctx, hipMemcpyAsync((char*)buf->ptr + offset, src, bytes, hipMemcpyHostToDevice, ctx->stream));
   MGN_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  ctx->stage.used = 0;
   return MGN_OK;
 }
 
@@ -422,8 +431,7 @@ mgn_status mgn_buf_download(mgn_ctx* ctx, const mgn_buf* buf, size_t offset, voi
   if (!ctx || !buf || (!dst && bytes)) return fail(ctx, MGN_EINVAL, "null argument");
   if (offset > buf->bytes || bytes > buf->bytes - offset) return fail(ctx, MGN_EINVAL, "download exceeds buffer size");
   if (bytes == 0) return mgn_sync(ctx);
-  MGN_HIP(ctx, hipMemcpyAsync(dst, (const char*)buf->ptr + offset, bytes, hipMemcpyDeviceToHost, ctx->stream));
-  MGN_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  if (const int e = mgn::copy_out(ctx, dst, (const char*)buf->ptr + offset, bytes)) return hip_fail(ctx, "download", (hipError_t)e);
   return check_range_flag(ctx);
 }
 
@@ -482,14 +490,13 @@ mgn_status mgn_weight_create_packed(mgn_ctx* ctx, mgn_fmt fmt, const uint8_t* pa
   if (fmt == MGN_FMT_Q4) {
     // the reference layout is already "all scale|min words, then all nibbles": plain copies, and
     // a pass over the scale words for their range
-    if (e == hipSuccess) e = hipMemcpyAsync(w->meta, packed, w->meta_bytes, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(w->quants, packed + w->meta_bytes, w->quant_bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) e = (hipError_t)mgn::copy_in(ctx, w->meta, packed, w->meta_bytes);
+    if (e == hipSuccess) e = (hipError_t)mgn::copy_in(ctx, w->quants, packed + w->meta_bytes, w->quant_bytes);
     if (e == hipSuccess) e = (hipError_t)mgn::launch_scale_range(ctx->stream, view_of(w), range_words(ctx));
   } else {
     const size_t bytes = w->nb * 36;
     if (e == hipSuccess) e = hipMalloc(&tmp, bytes);
-    if (e == hipSuccess) e = hipMemcpyAsync(tmp, packed, bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) e = (hipError_t)mgn::copy_in(ctx, tmp, packed, bytes);
     if (e == hipSuccess)
       e = (hipError_t)mgn::launch_import_q8(ctx->stream, (const uint8_t*)tmp, w->nb, w->meta, w->quants, range_words(ctx));
   }
@@ -547,7 +554,7 @@ static mgn_status weight_from_host_f32(mgn_ctx* ctx, mgn_fmt fmt, const float* w
     *no_staging = true;
     return MGN_ENOMEM;
   }
-  const hipError_t e = hipMemcpyAsync(staged, wdata, bytes, hipMemcpyHostToDevice, ctx->stream);
+  const hipError_t e = (hipError_t)mgn::copy_in(ctx, staged, wdata, bytes);
   const mgn_status st = e == hipSuccess ? weight_from_device_f32(ctx, fmt, staged, bytes, rows, cols, nk, out)
                                         : hip_fail(ctx, "weight upload", e);
   if (e != hipSuccess || st != MGN_OK) (void)hipStreamSynchronize(ctx->stream);
@@ -629,8 +636,7 @@ mgn_status mgn_weight_dequantize(mgn_ctx* ctx, const mgn_weight* w, float* out_h
   hipError_t e = hipMalloc((void**)&tmp, bytes);
   if (e != hipSuccess) return e == hipErrorOutOfMemory ? fail(ctx, MGN_ENOMEM, "out of device memory") : hip_fail(ctx, "hipMalloc", e);
   e = (hipError_t)mgn::launch_dequantize(ctx->stream, view_of(w), tmp);
-  if (e == hipSuccess) e = hipMemcpyAsync(out_host, tmp, bytes, hipMemcpyDeviceToHost, ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  if (e == hipSuccess) e = (hipError_t)mgn::copy_out(ctx, out_host, tmp, bytes);
   (void)hipFree(tmp);
   if (e != hipSuccess) return hip_fail(ctx, "dequantize", e);
   return MGN_OK;
@@ -641,16 +647,14 @@ mgn_status mgn_weight_export_ref(mgn_ctx* ctx, const mgn_weight* w, uint8_t* out
   hipError_t e = hipSuccess;
   void* tmp = nullptr;
   if (w->fmt == MGN_FMT_Q4) {
-    e = hipMemcpyAsync(out_packed, w->meta, w->meta_bytes, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(out_packed + w->meta_bytes, w->quants, w->quant_bytes, hipMemcpyDeviceToHost, ctx->stream);
+    e = (hipError_t)mgn::copy_out(ctx, out_packed, w->meta, w->meta_bytes);
+    if (e == hipSuccess) e = (hipError_t)mgn::copy_out(ctx, out_packed + w->meta_bytes, w->quants, w->quant_bytes);
   } else {
     const size_t bytes = w->nb * 36;
     e = hipMalloc(&tmp, bytes);
     if (e == hipSuccess) e = (hipError_t)mgn::launch_export_q8(ctx->stream, view_of(w), (uint8_t*)tmp);
-    if (e == hipSuccess) e = hipMemcpyAsync(out_packed, tmp, bytes, hipMemcpyDeviceToHost, ctx->stream);
+    if (e == hipSuccess) e = (hipError_t)mgn::copy_out(ctx, out_packed, tmp, bytes);
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (tmp) (void)hipFree(tmp);
   if (e != hipSuccess) return hip_fail(ctx, "weight export", e);
   return MGN_OK;

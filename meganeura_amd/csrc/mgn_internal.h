@@ -115,6 +115,8 @@ int launch_quantize_nk(ihipStream_t* s, int fmt, const float* w_nk_dev, uint32_t
                        uint32_t* range2_dev);
 // in[rows][cols] -> out[cols][rows] (f32); cols at most 65535 * 32
 int launch_transpose(ihipStream_t* s, const float* in, float* out, uint32_t rows, uint32_t cols);
+// pinned host memory <-> device, both 16-byte aligned, at most 2^32 bytes
+int launch_copy_bytes(ihipStream_t* s, void* dst, const void* src, size_t bytes);
 // measurement aid: one pass of plain reads over the weight's quants and scales
 // two words: shader-clock ticks and 100 MHz ticks over the same ~20 us
 // (num_cus_loaded > 0: that many workgroups of matrix-instruction work run meanwhile; out2_dev then
@@ -174,6 +176,18 @@ int launch_matmul_block_mfma(ihipStream_t* s, const LaunchArgs& a);
 
 }  // namespace mgn
 
+namespace mgn {
+// host_copy.cpp: the pinned memory through which a context's copies from and to ordinary host memory go
+// (made at the first one)
+struct HostStage {
+  char* ring = nullptr;
+  char* ring_dev = nullptr;  // the ring as the device sees it
+  size_t used = 0;  // bytes from the front that copies on the stream may still use
+  ihipEvent_t* done[16] = {};
+  bool refused = false;  // no pinned memory to be had: the runtime copies
+};
+}  // namespace mgn
+
 struct mgn_ctx {
   int device = 0;
   int num_cus = 0;
@@ -196,6 +210,7 @@ struct mgn_ctx {
   void* block_ws = nullptr;             // the blocked kernel's workspace (LaunchArgs::block_ws)
   void* at_stage = nullptr;             // transposed activations of the A^T matmul forms, grown on demand
   size_t at_stage_bytes = 0;
+  mgn::HostStage stage;
   std::vector<struct mgn_chain*> chains;  // live chains: their workspaces are emptied again after a fault
   std::string err;
 };
@@ -213,6 +228,12 @@ struct mgn_chain {
 };
 
 namespace mgn {
+// host -> device on the context's stream: on return the host bytes may change, the device's arrive in
+// stream order.  device -> host: on return they are there.  Both return a hipError_t.
+int copy_in(mgn_ctx* ctx, void* dev, const void* host, size_t bytes);
+int copy_out(mgn_ctx* ctx, void* host, const void* dev, size_t bytes);
+void release_host_stage(mgn_ctx* ctx);  // the stream must be idle
+mgn_status queue_upload(mgn_ctx* ctx, mgn_buf* buf, size_t offset, const void* src, size_t bytes);
 mgn_status reserve_at_stage(mgn_ctx* ctx, size_t bytes);
 // whether mgn_matmul_q_batch would take these weights in one launch (same K and format assumed checked)
 bool batch_plans(const mgn_ctx* ctx, const mgn_weight* const* ws, size_t count, uint32_t m, int pro_kind);

@@ -568,7 +568,8 @@ void Session::set_input(const std::string& name, const float* data, size_t len) 
   for (const auto& ib : plan_.input_buffers) {
     if (ib.first != name) continue;
     if (len * 4 > plan_.buffers[ib.second]) throw std::invalid_argument("input '" + name + "': data exceeds buffer");
-    check(mgn_buf_upload(ctx_, buffers_[ib.second], 0, data, len * 4), "mgn_buf_upload");
+    // not waited for: the step that reads it follows on the stream
+    check(queue_upload(ctx_, buffers_[ib.second], 0, data, len * 4), "input upload");
     return;
   }
   throw std::out_of_range("unknown input: " + name);
