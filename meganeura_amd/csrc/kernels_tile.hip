@@ -759,11 +759,36 @@ constexpr int resident_slices(bool f32a, int r) { return f32a && r == 2 ? 2 : 4;
 // a tile fall into different LDS banks.
 __host__ __device__ constexpr uint32_t meta_stride(int fmt, uint32_t nsl) { return nsl * kSliceBlocks * (fmt == MGN_FMT_Q4 ? 4 : 2) + 16; }
 
-template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false>
+// What a launch has besides its first weight (ROWS form: up to three weights that share their activations,
+// and what the activations go through on their way into the images).
+struct RowsExtra {
+  struct Item {
+    const void *meta, *quants;
+    const float* dres;
+    float* c;
+    uint32_t n, cg_first;  // columns; the weight's first column group
+    AddLift lift;
+  } item[2];
+  uint32_t items;  // 0 .. 2 of them
+  const float* norm_w;
+  float eps;
+};
+constexpr int kRowsPlain = -1;
+
+// ROWS: kRowsPlain, or the activations' prologue (kProNone / kProRmsNorm / kProSwiglu) of a launch that may
+// serve several weights.  A decoder layer of some hundred rows is made of launches that last 10 to 25 us
+// and leave part of the chip idle, with 4 to 6 us ones between them that only rewrite the activations.
+// Every workgroup converts its own rows anyway, so a norm (where the part holds the whole row: one K
+// part) or a SwiGLU costs it a second operand per element and no pass over memory; weights side by side
+// fill the rounds that each would leave open.  Two decoder layers of 333 rows, 1024 wide (Q8), q | k | v, the
+// output projection, gate | up and down with norms and SwiGLU: 18 launches, 213 us -> 8 launches, 161 us (Q4 184
+// -> 139; 128 rows, 576 wide 156 -> 104; 8 rows Q4 138 -> 90).
+template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain>
 __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restrict__ a, const void* __restrict__ meta_arg,
                                                              const void* __restrict__ quants_arg, uint32_t m, uint32_t kdim,
                                                              uint32_t n, uint32_t parts, uint32_t nslices, uint32_t colgroups,
-                                                             TileTail tail) {
+                                                             TileTail tail, RowsExtra extra) {
+  static_assert(ROWS == kRowsPlain || (F32A && R == 1 && !LATE), "the forms that are launched");
   constexpr uint32_t UNITS = image_units(F32A);
   constexpr float kOpScale = FMT == MGN_FMT_Q4 ? 1048576.0f : 16777216.0f;
   constexpr int QB = FMT == MGN_FMT_Q4 ? 16 : 32;
@@ -791,7 +816,17 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   if (rg >= rowgroups) return;            // padding of the grid
   const uint32_t row0 = rg * (R * 16);    // first row of this workgroup's row group
   const uint32_t bpc = kdim / 32;
-  const uint32_t pair0 = (cg * 8 + wave) * Q;  // this wave's first pair of column tiles
+  uint32_t wcg = cg;  // the column group within its weight
+  if constexpr (ROWS != kRowsPlain) {
+#pragma unroll
+    for (uint32_t j = 0; j < 2; j++)
+      if (j < extra.items && cg >= extra.item[j].cg_first) {  // (uniform)
+        meta_arg = extra.item[j].meta, quants_arg = extra.item[j].quants, n = extra.item[j].n;
+        tail.dres = extra.item[j].dres, tail.c = extra.item[j].c, tail.lift = extra.item[j].lift;
+        wcg = cg - extra.item[j].cg_first;
+      }
+  }
+  const uint32_t pair0 = (wcg * 8 + wave) * Q;  // this wave's first pair of column tiles
   const uint32_t sl0 = part * NSL;             // first slice of this part
   uint4* const img = lds4;                     // [NSL][R][UNITS]
   // this wave's scale words: [Q pairs x 32 columns][mstride bytes]
@@ -810,7 +845,16 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
     const uint32_t s = t / R, rr = t % R;
     const uint32_t row = row0 + rr * 16 + cr, k0 = (sl0 + s) * 256 + cl * 8;
     xok[t] = row < m && k0 < kdim;
-    load_task<F32A>(a, xok[t] ? (size_t)row * kdim + k0 : (size_t)0, xin[t]);
+    load_task<F32A>(a, xok[t] ? (size_t)row * (ROWS == kProSwiglu ? 2 * kdim : kdim) + k0 : (size_t)0, xin[t]);
+  }
+  TaskWords<true> xtwo[ROWS == kProRmsNorm || ROWS == kProSwiglu ? NT : 1];  // the norm's weights, or up beside gate
+  if constexpr (ROWS == kProRmsNorm || ROWS == kProSwiglu) {
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      const uint32_t row = row0 + cr, k0 = (sl0 + t) * 256 + cl * 8;
+      if constexpr (ROWS == kProRmsNorm) load_task<true>(extra.norm_w, xok[t] ? (size_t)k0 : (size_t)0, xtwo[t]);
+      else load_task<true>(a, xok[t] ? (size_t)row * 2 * kdim + kdim + k0 : (size_t)0, xtwo[t]);
+    }
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -873,8 +917,31 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   // 10.93 us, 512 x 3072 x 1024 14.22 -> 14.0.  (On half a chip the early request wins: M = 64 on
   // 4096 x 4096, 128 workgroups, 10.2 against 10.45 us; and with f32 activations a later one loses.)
   constexpr int kFirstFetchAfterTask = NT > 1 ? (LATE ? NT - 1 : 1) : 0;
+  auto word = [](uint32_t w) __attribute__((always_inline)) { return __builtin_bit_cast(float, w); };
+  float rinv = 1.0f;
+  if constexpr (ROWS == kProRmsNorm) {
+    // the half-wave's tasks are the whole row (one K part): x / sqrt(mean(x^2) + eps) * weight
+    float ss = 0.0f;
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const float v = xok[t] ? word(xin[t].w[e]) : 0.0f;
+        ss = __fmaf_rn(v, v, ss);
+      }
+#pragma unroll
+    for (int d = 16; d > 0; d >>= 1) ss += __shfl_xor(ss, d, 32);
+    rinv = 1.0f / sqrtf(ss / (float)kdim + extra.eps);
+  }
 #pragma unroll
   for (int t = 0; t < NT; t++) {
+    if constexpr (ROWS == kProRmsNorm) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) xin[t].w[e] = __builtin_bit_cast(uint32_t, word(xin[t].w[e]) * rinv * word(xtwo[t].w[e]));
+    } else if constexpr (ROWS == kProSwiglu) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) xin[t].w[e] = __builtin_bit_cast(uint32_t, swiglu_act(word(xin[t].w[e]), word(xtwo[t].w[e])));
+    }
     convert_task<FMT, F32A>(xin[t], xok[t], img + t * UNITS, cr, cl);
     __builtin_amdgcn_sched_barrier(0);
     if (t >= kFirstFetchAfterTask && t - kFirstFetchAfterTask < DEPTH && t - kFirstFetchAfterTask < STEPS) fetch(t - kFirstFetchAfterTask);
@@ -1041,7 +1108,7 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
         }
         // the tile's place in the output: slot = (pair * kSide + side) * R + row tile of wave src_wave
         const uint32_t tp = slot / (kSide * R), tu = (slot / R) % kSide, tr = slot % R;
-        const uint32_t col = (((cg * 8 + src_wave) * Q + tp) * kSide + tu) * 16 + c;
+        const uint32_t col = (((wcg * 8 + src_wave) * Q + tp) * kSide + tu) * 16 + c;
         if (col < n) {
           if (row0 + R * 16 <= m && !tail.dres && tail.epilogue == 0) {  // (uniform) whole rows, nothing to add or apply
             float* const dst = tail.c + (size_t)(row0 + tr * 16 + 4 * g) * n + col;
@@ -1213,7 +1280,9 @@ bool plan_resident(const LaunchArgs& x, ResidentPlan* out) {
   const uint32_t bpc = x.w.k / 32;
   if ((uint64_t)x.w.n * bpc * 32 >= (1ull << 32)) return false;  // a lane's weight offsets are 32-bit
   const bool f32a = !x.a_is_f16;
-  const uint32_t nslices = (bpc + kSliceBlocks - 1) / kSliceBlocks, n_tiles = (x.w.n + 15) / 16;
+  const uint32_t nslices = (bpc + kSliceBlocks - 1) / kSliceBlocks;
+  for (int j = 0; j < x.n_more; j++)
+    if ((uint64_t)x.more[j].w.n * bpc * 32 >= (1ull << 32)) return false;
   double best = 0;
   ResidentPlan bp{};
   for (uint32_t r = 1; r <= 2; r++) {
@@ -1228,7 +1297,9 @@ bool plan_resident(const LaunchArgs& x, ResidentPlan* out) {
     if (rowgroups > 65535) continue;
     for (uint32_t q = 1; q <= (r == 1 ? 2u : 1u); q++) {
       const uint32_t per_wg = 8 * kSide * q;
-      const uint32_t colgroups = (n_tiles + per_wg - 1) / per_wg;
+      auto groups_of = [&](uint32_t n) { return ((n + 15) / 16 + per_wg - 1) / per_wg; };  // a group lies in one weight
+      uint32_t colgroups = groups_of(x.w.n);
+      for (int j = 0; j < x.n_more; j++) colgroups += groups_of(x.more[j].w.n);
       if (parts > 65535 || (uint64_t)colgroups * rowgroups > 0x7FFFFFF0ull) continue;
       // a workgroup's partial tile: 8 waves x (q kSide r) float4 per lane; the last part keeps its own
       // Every part adds up a share of the tiles when all workgroups are resident at once (every part then
@@ -1262,20 +1333,41 @@ bool plan_resident(const LaunchArgs& x, ResidentPlan* out) {
   return true;
 }
 
-template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false>
+template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain>
 int launch_resident_q(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& p) {
-  auto kern = tile_resident_kernel<FMT, F32A, R, Q, PARK, LATE>;
+  auto kern = tile_resident_kernel<FMT, F32A, R, Q, PARK, LATE, ROWS>;
   static std::atomic<uint64_t> big_lds_done{0};
   if (p.lds > 64 * 1024)
     if (int e = enable_big_lds(kern, x.device, big_lds_done)) return e;
   const TileTail tail{x.d, x.c, (float*)x.scratch, x.counters, x.epilogue, (float*)x.handover, x.spin_limit, x.fault_flag, p.spread ? 1u : 0u, add_lift(x.w)};
+  RowsExtra extra{};
+  if constexpr (ROWS != kRowsPlain) {
+    constexpr uint32_t per_wg = 8 * kSide * Q;
+    uint32_t first = ((x.w.n + 15) / 16 + per_wg - 1) / per_wg;
+    for (int j = 0; j < x.n_more; j++) {
+      const LaunchArgs::More& o = x.more[j];
+      extra.item[j] = {o.w.meta, o.w.quants, o.d, o.c, o.w.n, first, add_lift(o.w)};
+      first += ((o.w.n + 15) / 16 + per_wg - 1) / per_wg;
+    }
+    extra.items = (uint32_t)x.n_more;
+    extra.norm_w = x.pro_weight, extra.eps = x.pro_eps;
+  }
   // (column groups x row groups, K parts); with K parts the first is rounded up to a multiple of 8 (see the kernel)
   const uint64_t groups = (uint64_t)p.colgroups * p.rowgroups;
   const dim3 grid((unsigned)(p.parts > 1 ? (groups + 7) / 8 * 8 : groups), p.parts, 1);
   hipLaunchKernelGGL(kern, grid, dim3(512), p.lds, s, x.a, x.w.meta, x.w.quants, x.m, x.w.k, x.w.n, p.parts, p.nslices,
-                     p.colgroups, tail);
+                     p.colgroups, tail, extra);
   MGN_HIP_LAUNCH_CHECK();
   return 0;
+}
+
+template <int FMT, int Q>
+int launch_resident_rows(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& p) {
+  constexpr bool kPark = Q == 1;
+  if (p.park != kPark) return (int)hipErrorInvalidValue;
+  if (x.pro_kind == kProRmsNorm) return launch_resident_q<FMT, true, 1, Q, kPark, false, kProRmsNorm>(s, x, p);
+  if (x.pro_kind == kProSwiglu) return launch_resident_q<FMT, true, 1, Q, kPark, false, kProSwiglu>(s, x, p);
+  return launch_resident_q<FMT, true, 1, Q, kPark, false, kProNone>(s, x, p);
 }
 
 template <int FMT, bool F32A>
@@ -1503,6 +1595,34 @@ bool tile_mfma_preferred(const LaunchArgs& x) {
   }
   if (rp.r != 1 || rp.nslices < 3) return false;
   return 4 * wgs >= 3 * rounds * (uint64_t)x.num_cus;
+}
+
+// One launch for several weights, a norm or a SwiGLU on the way (more rows than the GEMV takes, f32
+// activations).  Each weight on its own must be this kernel's; the norm needs the whole row in one K part;
+// a prologue is worked out anew by every column group and round, so it rides along only where the
+// launch takes one round; weights join where the rounds' cost of the joint plan is below the sum of theirs.
+bool tile_rows_supported(const LaunchArgs& x) {
+  ResidentPlan joint, own;
+  if (x.a_is_f16 || x.m <= 4 || !use_resident(x, &joint) || joint.r != 1) return false;
+  if (x.pro_kind == kProRmsNorm && joint.parts != 1) return false;
+  const uint64_t wgs = (uint64_t)joint.parts * joint.colgroups * joint.rowgroups;
+  if (x.pro_kind != kProNone && wgs > (uint64_t)x.num_cus) return false;
+  LaunchArgs y = x;
+  y.n_more = 0;
+  double sum = 0;
+  for (int j = 0; j <= x.n_more; j++) {
+    if (j > 0) y.w = x.more[j - 1].w;
+    if (!use_resident(y, &own)) return false;
+    sum += own.cost;
+  }
+  return x.n_more == 0 || joint.cost < sum;
+}
+
+int launch_tile_rows(ihipStream_t* s, const LaunchArgs& x) {
+  ResidentPlan p;
+  if (!tile_rows_supported(x) || !use_resident(x, &p)) return (int)hipErrorInvalidValue;
+  if (x.w.fmt == MGN_FMT_Q4) return p.q == 1 ? launch_resident_rows<MGN_FMT_Q4, 1>(s, x, p) : launch_resident_rows<MGN_FMT_Q4, 2>(s, x, p);
+  return p.q == 1 ? launch_resident_rows<MGN_FMT_Q8, 1>(s, x, p) : launch_resident_rows<MGN_FMT_Q8, 2>(s, x, p);
 }
 
 bool describe_tile_mfma(const LaunchArgs& x, mgn_plan_info* out) {

@@ -863,8 +863,10 @@ mgn_status mgn_matmul_q_swiglu(mgn_ctx* ctx, const mgn_buf* gate_up, const mgn_w
   return matmul_impl(ctx, gate_up, false, w, d, c, m, mgn::kProSwiglu);
 }
 
-mgn_status mgn_matmul_q_batch(mgn_ctx* ctx, const mgn_buf* a, mgn_prologue prologue, const mgn_buf* norm_weight, float eps,
-                              const mgn_matmul_item* items, size_t count, uint32_t m) {
+// The launch arguments of up to three matmuls that share their activations, checked.  MGN_OK with m == 0:
+// there is nothing to launch.
+static mgn_status batch_args(mgn_ctx* ctx, const mgn_buf* a, mgn_prologue prologue, const mgn_buf* norm_weight, float eps,
+                             const mgn_matmul_item* items, size_t count, uint32_t m, mgn::LaunchArgs* out) {
   if (!ctx || !a || !items) return fail(ctx, MGN_EINVAL, "null argument");
   if (count == 0 || count > 3) return fail(ctx, MGN_EINVAL, "a batch holds 1 to 3 matmuls");
   if (prologue < MGN_PROLOGUE_NONE || prologue > MGN_PROLOGUE_SWIGLU) return fail(ctx, MGN_EINVAL, "unknown prologue");
@@ -877,7 +879,8 @@ mgn_status mgn_matmul_q_batch(mgn_ctx* ctx, const mgn_buf* a, mgn_prologue prolo
   if (a->bytes / 4 < (size_t)m * a_cols) return fail(ctx, MGN_EINVAL, "A is smaller than its m rows");
   if (prologue == MGN_PROLOGUE_RMS_NORM && (!norm_weight || norm_weight->bytes / 4 < k))
     return fail(ctx, MGN_EINVAL, "norm weight is missing or shorter than K floats");
-  mgn::LaunchArgs x{view_of(w0), a->ptr, items[0].d ? (const float*)items[0].d->ptr : nullptr, (float*)items[0].c->ptr, m,
+  mgn::LaunchArgs& x = *out;
+  x = mgn::LaunchArgs{view_of(w0), a->ptr, items[0].d ? (const float*)items[0].d->ptr : nullptr, (float*)items[0].c->ptr, m,
                     false, ctx->num_cus};
   for (size_t j = 0; j < count; j++) {
     const mgn_matmul_item& it = items[j];
@@ -900,12 +903,66 @@ mgn_status mgn_matmul_q_batch(mgn_ctx* ctx, const mgn_buf* a, mgn_prologue prolo
   x.pro_kind = (int)prologue;
   x.pro_weight = norm_weight ? (const float*)norm_weight->ptr : nullptr;
   x.pro_eps = eps;
+  return MGN_OK;
+}
+
+mgn_status mgn_matmul_q_batch(mgn_ctx* ctx, const mgn_buf* a, mgn_prologue prologue, const mgn_buf* norm_weight, float eps,
+                              const mgn_matmul_item* items, size_t count, uint32_t m) {
+  mgn::LaunchArgs x{};
+  if (const mgn_status st = batch_args(ctx, a, prologue, norm_weight, eps, items, count, m, &x)) return st;
+  if (m == 0) return MGN_OK;
   if ((ctx->route != MGN_ROUTE_AUTO && ctx->route != MGN_ROUTE_GEMV_MFMA) || !mgn::gemv_mfma_supported(x))
     return fail(ctx, MGN_EUNSUPPORTED, "batched matmul needs the GEMV_MFMA route (f32 activations, M <= 4)");
   const int rc = mgn::launch_matmul_gemv_mfma(ctx->stream, x);
   if (rc != 0) return hip_fail(ctx, "kernel launch", (hipError_t)rc);
   return MGN_OK;
 }
+
+}  // extern "C"
+
+namespace mgn {
+static void rows_args(const mgn_ctx* ctx, LaunchArgs* x) {
+  x->device = ctx->device;
+  x->num_cus = ctx->num_cus;
+  x->shared_device = ctx->shared_device;
+  x->scratch = ctx->scratch;
+  x->scratch_bytes = ctx->scratch_bytes;
+  x->handover = ctx->handover;
+  x->handover_bytes = ctx->handover_bytes;
+  x->block_ws = ctx->block_ws;
+  x->block_ws_bytes = kBlockWsBytes;
+}
+
+bool rows_plans(const mgn_ctx* ctx, const mgn_weight* const* ws, size_t count, uint32_t m, int pro_kind) {
+  if (!ctx || !ws || count == 0 || count > 3 || m <= 4 || ctx->route != MGN_ROUTE_AUTO) return false;
+  LaunchArgs x{view_of(ws[0]), nullptr, nullptr, nullptr, m, false, ctx->num_cus};
+  rows_args(ctx, &x);
+  for (size_t j = 0; j < count; j++) {
+    x.w = view_of(ws[j]);
+    if (auto_route(x, ctx->any_magnitude) != MGN_ROUTE_TILE_MFMA) return false;
+  }
+  x.w = view_of(ws[0]);
+  for (size_t j = 1; j < count; j++) x.more[j - 1] = {view_of(ws[j]), nullptr, nullptr};
+  x.n_more = (int)count - 1;
+  x.pro_kind = pro_kind;
+  return tile_rows_supported(x);
+}
+
+mgn_status matmul_rows(mgn_ctx* ctx, const mgn_buf* a, int pro_kind, const mgn_buf* norm_weight, float eps,
+                       const mgn_matmul_item* items, size_t count, uint32_t m) {
+  LaunchArgs x{};
+  if (const mgn_status st = batch_args(ctx, a, (mgn_prologue)pro_kind, norm_weight, eps, items, count, m, &x)) return st;
+  if (m == 0) return MGN_OK;
+  rows_args(ctx, &x);
+  const mgn_weight* ws[3] = {};
+  for (size_t j = 0; j < count; j++) ws[j] = items[j].w;
+  if (!rows_plans(ctx, ws, count, m, pro_kind)) return fail(ctx, MGN_EUNSUPPORTED, "not one launch's work");
+  const int rc = launch_tile_rows(ctx->stream, x);
+  return rc ? hip_fail(ctx, "kernel launch", (hipError_t)rc) : MGN_OK;
+}
+}  // namespace mgn
+
+extern "C" {
 
 int mgn_matmul_q_can_fuse(mgn_ctx* ctx, const mgn_weight* w, uint32_t m) {
   if (!ctx || !w || m == 0) return 0;

@@ -167,6 +167,9 @@ bool tile_mfma_supported(const LaunchArgs& a);
 bool tile_mfma_preferred(const LaunchArgs& a);
 bool describe_tile_mfma(const LaunchArgs& a, mgn_plan_info* out);
 int launch_matmul_tile_mfma(ihipStream_t* s, const LaunchArgs& a);
+// the same kernel for several weights (LaunchArgs::more) and with a prologue, f32 activations
+bool tile_rows_supported(const LaunchArgs& a);
+int launch_tile_rows(ihipStream_t* s, const LaunchArgs& a);
 // kernels_block.hip: the blocked kernel for many rows (32x32x16 tiles, activations prepared once per call)
 bool block_mfma_supported(const LaunchArgs& a);
 // what it is expected to take on a shape (0: not served)
@@ -235,6 +238,12 @@ int copy_out(mgn_ctx* ctx, void* host, const void* dev, size_t bytes);
 void release_host_stage(mgn_ctx* ctx);  // the stream must be idle
 mgn_status queue_upload(mgn_ctx* ctx, mgn_buf* buf, size_t offset, const void* src, size_t bytes);
 mgn_status reserve_at_stage(mgn_ctx* ctx, size_t bytes);
+// One launch for up to three matmuls of more than four rows that share their activations, and a prologue (a
+// session's own launches: the public forms take up to four rows).  MGN_EUNSUPPORTED where rows_plans
+// says no.
+bool rows_plans(const mgn_ctx* ctx, const mgn_weight* const* ws, size_t count, uint32_t m, int pro_kind);
+mgn_status matmul_rows(mgn_ctx* ctx, const mgn_buf* a, int pro_kind, const mgn_buf* norm_weight, float eps,
+                       const mgn_matmul_item* items, size_t count, uint32_t m);
 // whether mgn_matmul_q_batch would take these weights in one launch (same K and format assumed checked)
 bool batch_plans(const mgn_ctx* ctx, const mgn_weight* const* ws, size_t count, uint32_t m, int pro_kind);
 }  // namespace mgn

@@ -744,7 +744,7 @@ void Session::plan_chains() {
 // Which RmsNorm / SwiGLUConcat dispatches disappear into the matmuls that read them
 // (models/smollm2.rs:340-341,396: norm -> q/k/v and norm -> gate/up; compile.rs:1814-1830:
 // swiglu_concat -> down).  A producer is folded only if every reader of its output is a
-// decode matmul taking it as the activation operand and served by the fusing kernel.
+// matmul taking it as the activation operand and served by a fusing kernel.
 void Session::plan_launches() {
   if (launches_planned_) return;
   const size_t nd = plan_.dispatches.size();
@@ -759,6 +759,10 @@ void Session::plan_launches() {
     for (int b : plan_.dispatches[i].input_buffers) readers[b].push_back((int)i);
   std::vector<char> is_output(plan_.buffers.size(), 0);
   for (int b : plan_.output_buffers) is_output[b] = 1;
+  // a matmul whose launch can take the prologue: up to four rows the GEMV's, beyond the resident kernel's
+  auto fusable = [&](mgn_weight* w, uint32_t m, int kind) {
+    return mgn_matmul_q_can_fuse(ctx_, w, m) == 1 || rows_plans(ctx_, &w, 1, m, kind);
+  };
   for (size_t pi = 0; pi < nd; pi++) {
     const Dispatch& p = plan_.dispatches[pi];
     const bool norm = p.shader == MGN_SHADER_RMS_NORM, swi = p.shader == MGN_SHADER_SWIGLU_CONCAT;
@@ -772,7 +776,7 @@ void Session::plan_launches() {
       mgn_weight* w = is_matmul(c.shader) ? weights_[c.input_buffers[1]] : nullptr;
       ok = ok && (size_t)ci > pi && w && c.input_buffers[0] == out && is_matmul(c.shader) && !is_at(c.shader) && matmul_k(c) == width &&
            (c.input_buffers.size() < 3 || c.input_buffers[2] != out) && fused_[ci].kind == 0 && c.epilogue.empty() &&
-           mgn_matmul_q_can_fuse(ctx_, w, c.params[0]) == 1;
+           fusable(w, c.params[0], norm ? kProRmsNorm : kProSwiglu);
     }
     if (!ok) continue;
     skipped_[pi] = 1;
@@ -790,7 +794,7 @@ void Session::plan_launches() {
     const Dispatch& d = plan_.dispatches[i];
     if (skipped_[i] || !is_matmul(d.shader) || is_at(d.shader) || !d.epilogue.empty()) return false;
     mgn_weight* w = weights_[d.input_buffers[1]];
-    return w && mgn_matmul_q_can_fuse(ctx_, w, d.params[0]) == 1;
+    return w && fusable(w, d.params[0], fused_[i].kind);
   };
   for (size_t i = 0; i < nd; i++) {
     if (!batchable(i)) continue;
@@ -810,7 +814,9 @@ void Session::plan_launches() {
       const mgn_weight* group[3] = {weights_[di.input_buffers[1]], nullptr, nullptr};
       for (int f = 0; f < found; f++) group[1 + f] = weights_[plan_.dispatches[fused_[i].more[f]].input_buffers[1]];
       group[1 + found] = weights_[dj.input_buffers[1]];
-      if (!batch_plans(ctx_, group, (size_t)found + 2, di.params[0], fused_[i].kind)) continue;
+      if (!batch_plans(ctx_, group, (size_t)found + 2, di.params[0], fused_[i].kind) &&
+          !rows_plans(ctx_, group, (size_t)found + 2, di.params[0], fused_[i].kind))
+        continue;
       fused_[i].more[found++] = (int)j;
       skipped_[j] = 1;
     }
@@ -895,7 +901,9 @@ void Session::run_dispatches() {
           const Dispatch* p = f.kind != kProNone ? &plan_.dispatches[f.producer] : nullptr;
           const mgn_buf* act = p ? buffers_[p->input_buffers[0]] : buffers_[d.input_buffers[0]];
           const mgn_buf* nw = f.kind == kProRmsNorm ? buffers_[p->input_buffers[1]] : nullptr;
-          mgn_status st = mgn_matmul_q_batch(ctx_, act, (mgn_prologue)f.kind, nw, p ? p->eps : 0.0f, items, count, d.params[0]);
+          const float eps = p ? p->eps : 0.0f;
+          mgn_status st = d.params[0] <= 4 ? mgn_matmul_q_batch(ctx_, act, (mgn_prologue)f.kind, nw, eps, items, count, d.params[0])
+                                           : matmul_rows(ctx_, act, f.kind, nw, eps, items, count, d.params[0]);
           if (st == MGN_EUNSUPPORTED) {
             // planned as one launch, refused now (the route was changed since): the producer's own
             // dispatch into its own buffer, then one plain matmul per weight
@@ -906,7 +914,10 @@ void Session::run_dispatches() {
           check(st, "mgn_matmul_q_batch");
         } else if (f.kind == kProRmsNorm || f.kind == kProSwiglu) {
           const Dispatch& p = plan_.dispatches[f.producer];
-          mgn_status st = f.kind == kProRmsNorm
+          const mgn_matmul_item item{w, addend, buffers_[d.output_buffer]};
+          mgn_status st = d.params[0] > 4 ? matmul_rows(ctx_, buffers_[p.input_buffers[0]], f.kind,
+                                                        f.kind == kProRmsNorm ? buffers_[p.input_buffers[1]] : nullptr, p.eps, &item, 1, d.params[0])
+                          : f.kind == kProRmsNorm
                               ? mgn_matmul_q_rms_norm(ctx_, buffers_[p.input_buffers[0]], buffers_[p.input_buffers[1]], p.eps, w, addend,
                                                       buffers_[d.output_buffer], d.params[0])
                               : mgn_matmul_q_swiglu(ctx_, buffers_[p.input_buffers[0]], w, addend, buffers_[d.output_buffer], d.params[0]);

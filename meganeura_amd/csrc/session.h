@@ -154,8 +154,9 @@ class Session {
   // are a single graph launch.  Results are identical; only launch overhead changes --
   // less host work per step, but measured slower on the GPU side for chains of tiny kernels.
   void set_graph_replay(bool on);
-  // Fold RmsNorm / SwiGLUConcat dispatches into the decode matmuls that consume them, serve
-  // sibling decode matmuls (same activations, e.g. q/k/v) with one launch and let a matmul's
+  // Fold RmsNorm / SwiGLUConcat dispatches into the matmuls that consume them, serve
+  // sibling matmuls (same activations, e.g. q/k/v) with one launch, up to four rows by the GEMV, beyond where
+  // the resident kernel takes each of them (rows_plans), and let a matmul's
   // launch apply the unary dispatches that follow it (the compiler folds those into tiled
   // matmul entries only, not into the M = 1 ones) (default on).  The plan keeps the reference's dispatch list; only the launches differ.
   void set_fusion(bool on);
