@@ -8,8 +8,8 @@
 //     next chunk while the last one travels; writes need not be waited for (the stream keeps them in
 //     order with the launches that read them); launches, not copy engine commands, move the chunks
 //     (copy_bytes_kernel), except reads on an idle stream;
-//   beyond: the ring as slots of kSlot, up to kWorkers threads with two slots each that take the chunks
-//     in turn (one thread's 29 GB/s is half of what the bus takes: 64 MB 2306 us with one thread, 874
+//   beyond (uploads from kLargeIn on): the ring as slots of kSlot, up to kWorkers threads with two slots
+//     each that take the chunks in turn (one thread's 29 GB/s is half of what the bus takes: 64 MB 2306 us with one thread, 874
 //     with four).  The threads live as long as the call.
 // Measured, before -> after: the eight-layer decode step of a session 147 -> 124 us, two layers of 333
 // rows 460 -> 410 us, a 4096 x 4096 weight from f32 and its packed bytes back 3400 -> 2470 us.
@@ -29,9 +29,14 @@ namespace {
 constexpr size_t kSlot = (size_t)2 << 20, kSlots = 8, kRing = kSlot * kSlots;
 constexpr int kWorkers = (int)kSlots / 2;
 constexpr size_t kSmall = (size_t)4 << 20;
+// Uploads between these two go the runtime's way, which pins the pages: one thread fills the ring at what DRAM
+// gives it, and four cost their start.  Whole upload or weight from f32, ring or slots : runtime, us: 2 MB 108 : 98,
+// 3.5 MB weight 285 : 236, 8 MB weight 460 : 415, 12 MB 410 : 352 from the caches, 438 : 419 from memory,
+// 16 MB 510 : 460 and 531 : 582, 32 MB 863 : 920 and 876 : 1139.
+constexpr size_t kSmallIn = (size_t)2 << 20, kLargeIn = (size_t)16 << 20;
 constexpr size_t kChunk = (size_t)1 << 20, kChunkOut = (size_t)512 << 10;
 constexpr size_t kEvents = sizeof(HostStage::done) / sizeof(ihipEvent_t*);
-static_assert(kSmall / kChunkOut <= kEvents && kSlots <= kEvents, "an event per chunk, and per slot");
+static_assert(kSmallIn <= kSmall && kSmall / kChunkOut <= kEvents && kSlots <= kEvents, "an event per chunk, and per slot");
 
 // The context's ring and events; false: there is no pinned memory to be had.
 bool have_stage(mgn_ctx* ctx) {
@@ -142,12 +147,12 @@ hipError_t ring_piece(mgn_ctx* ctx, size_t bytes, size_t* out) {
 
 int copy_in(mgn_ctx* ctx, void* dev, const void* host, size_t bytes) {
   if (bytes == 0) return 0;
-  if (!pageable(host) || !have_stage(ctx)) {
+  if ((bytes > kSmallIn && bytes < kLargeIn) || !pageable(host) || !have_stage(ctx)) {
     hipError_t e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     return (int)e;
   }
-  if (bytes > kSmall) return (int)copy_large(ctx, (char*)dev, (char*)const_cast<void*>(host), bytes, true);
+  if (bytes > kSmallIn) return (int)copy_large(ctx, (char*)dev, (char*)const_cast<void*>(host), bytes, true);
   size_t piece;
   if (const hipError_t e = ring_piece(ctx, bytes, &piece)) return (int)e;
   for (size_t o = 0; o < bytes; o += kChunk) {

@@ -10,8 +10,8 @@ from meganeura_amd.graph import Graph, build_inference_session
 
 pytestmark = pytest.mark.gpu
 
-CHUNK, SLOT, SMALL = 1 << 20, 2 << 20, 4 << 20  # host_copy.cpp: kChunk, kSlot, kSmall
-SIZES = [1, 3, 4, 2304, (512 << 10) - 1, 512 << 10, (512 << 10) + 1, CHUNK + 1, SMALL - 1, SMALL, SMALL + 1, 5 * SLOT, 8 * SLOT + 7, 33 * SLOT - 5]
+CHUNK, SLOT, SMALL = 1 << 20, 2 << 20, 4 << 20  # host_copy.cpp: kChunk, kSlot and kSmallIn, kSmall; kLargeIn is 8 slots
+SIZES = [1, 3, 4, 2304, (512 << 10) - 1, 512 << 10, (512 << 10) + 1, CHUNK + 1, SLOT, SLOT + 1, SMALL - 1, SMALL, SMALL + 1, 5 * SLOT, 8 * SLOT - 1, 8 * SLOT, 8 * SLOT + 7, 33 * SLOT - 5]
 
 
 def pattern(nbytes, seed):
