@@ -24,7 +24,7 @@
 //   * K parts for different workgroups, where the tiles do not fill the chip, meet in the workspace and are added
 //     in part order by a third launch.
 // Measured (one box, weights from memory; before -> now, us): fp16 2048 x 4096 x 14336 589 -> 299 (805 TFLOP/s),
-// f32 the same 1034 -> 467; f32 512 x 4096 x 14336 295 -> 123; f32 77 x 4096 x 14336 82 -> 44, 77 x 14336 x 4096
+// f32 the same 1034 -> 467; f32 512 x 4096 x 14336 295 -> 123; f32 77 x 4096 x 14336 82 -> 42, 77 x 14336 x 4096
 // 98 -> 46.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.4
 // times its issue cycles (LDS and barrier waits).
 #include <algorithm>
@@ -726,19 +726,21 @@ __global__ __launch_bounds__(256) void add_parts_kernel(const float* __restrict_
 // further round of 256 (tn; where two fit a CU, what the second costs beside the first).
 struct BlockConfig {
   void (*kernel)(BlockArgs);
-  uint32_t rows, cols, threads;
+  uint32_t rows, cols, threads, streams;
   size_t lds;
   double t1, tn;
 };
 
-template <int FMT, bool F32A, int RT, int WM, int WN, int SUBB, int PD, int SD>
+template <int FMT, bool F32A, int RT, int WM, int WN, int SUBB, int PD, int SD, int WK = 1>
 BlockConfig block_config(double t1, double tn) {
-  using S = BlockShape<FMT, F32A, RT, WM, WN, 1, SUBB, PD, SD>;
+  // (fp16 activations are read where they are: a stream without a stage would multiply what lies behind K by zero)
+  static_assert(WK == 1 || F32A, "streams may run out of stages only on prepared activations");
+  using S = BlockShape<FMT, F32A, RT, WM, WN, WK, SUBB, PD, SD>;
   static_assert(S::LDS <= 160 * 1024, "fits a CU");
-  return {block_kernel<FMT, F32A, RT, WM, WN, 1, SUBB, PD, SD>, (uint32_t)S::ROWS, (uint32_t)S::COLS, 64u * S::WAVES, S::LDS, t1, tn};
+  return {block_kernel<FMT, F32A, RT, WM, WN, WK, SUBB, PD, SD>, (uint32_t)S::ROWS, (uint32_t)S::COLS, 64u * S::WAVES, (uint32_t)WK, S::LDS, t1, tn};
 }
 
-constexpr int kBlockConfigs = 7;
+constexpr int kBlockConfigs = 9;  // at most, per format and kind of activations
 const BlockConfig* block_configs(int fmt, bool f32a) {
   static const BlockConfig q4_f16[kBlockConfigs] = {
       block_config<0, false, 4, 2, 4, 2, 2, 1>(5.7, 4.1), block_config<0, false, 3, 2, 4, 2, 2, 2>(4.65, 3.1),
@@ -749,7 +751,8 @@ const BlockConfig* block_configs(int fmt, bool f32a) {
       block_config<0, true, 4, 2, 4, 1, 2, 1>(7.6, 6.7), block_config<0, true, 3, 2, 4, 1, 2, 2>(6.3, 5.2),
       block_config<0, true, 2, 2, 4, 1, 3, 1>(4.7, 3.2), block_config<0, true, 3, 1, 4, 1, 2, 1>(4.4, 2.4),
       block_config<0, true, 2, 1, 4, 1, 3, 1>(2.95, 1.9), block_config<0, true, 1, 1, 4, 1, 4, 1>(2.0, 1.3),
-      block_config<0, true, 1, 2, 2, 1, 3, 1>(1.65, 1.2)};
+      block_config<0, true, 1, 2, 2, 1, 3, 1>(1.65, 1.2), block_config<0, true, 3, 1, 4, 1, 2, 1, 2>(3.55, 3.3),
+      block_config<0, true, 2, 1, 4, 1, 3, 1, 2>(2.45, 2.3)};
   static const BlockConfig q8_f16[kBlockConfigs] = {
       block_config<1, false, 3, 2, 4, 2, 2, 3>(5.3, 3.5), block_config<1, false, 3, 2, 4, 2, 2, 2>(5.4, 3.8),
       block_config<1, false, 2, 2, 4, 2, 2, 3>(4.35, 2.6), block_config<1, false, 3, 1, 4, 2, 2, 3>(3.3, 2.6),
@@ -759,9 +762,17 @@ const BlockConfig* block_configs(int fmt, bool f32a) {
       block_config<1, true, 4, 2, 4, 1, 2, 1>(8.4, 7.6), block_config<1, true, 3, 2, 4, 1, 2, 2>(6.9, 5.5),
       block_config<1, true, 2, 2, 4, 1, 3, 2>(5.4, 3.9), block_config<1, true, 3, 1, 4, 1, 2, 1>(5.25, 2.6),
       block_config<1, true, 2, 1, 4, 1, 3, 2>(3.6, 2.8), block_config<1, true, 1, 1, 4, 1, 4, 2>(2.4, 2.3),
-      block_config<1, true, 1, 2, 2, 1, 3, 2>(2.45, 1.4)};
+      block_config<1, true, 1, 2, 2, 1, 3, 2>(2.45, 1.4), block_config<1, true, 3, 1, 4, 1, 2, 1, 2>(4.1, 3.9)};
   return fmt == MGN_FMT_Q4 ? (f32a ? q4_f32 : q4_f16) : (f32a ? q8_f32 : q8_f16);
 }
+
+// Two streams in one workgroup instead of two workgroups on a CU: the same waves and the same loads, but
+// one set of sums leaves the CU, so a shape takes half the K parts and half the traffic of adding them up
+// (f32, one stream -> two, us: Q4 128 x 4096 x 14336 59.0 -> 50.4, 77 x 4096 x 14336 43.5 -> 42.2, 160 x 14336 x
+// 4096 75.1 -> 70.4; Q8 77 x 4096 x 14336 52.0 -> 47.0, 160 x 2048 x 8192 34.3 -> 32.7).  Not where a stream has
+// fewer stages than this, the start of the rings and the meeting being most of it then (Q4 77 x 4096 x 4096, two
+// stages each, 23.6 -> 25.7; Q8 26.1 -> 27.7), nor with 32 rows (level) or, Q8, 64 (64 x 4096 x 14336 37.2 -> 41.9).
+constexpr uint32_t kStreamStages = 4;
 
 struct BlockPlan {
   const BlockConfig* cfg;
@@ -783,6 +794,7 @@ bool plan_block_rows(const LaunchArgs& x, uint32_t m, BlockPlan* out) {
   double best = 0;
   for (int i = 0; i < kBlockConfigs; i++) {
     const BlockConfig& c = cfgs[i];
+    if (!c.kernel) break;
     const uint32_t rowgroups = (m + c.rows - 1) / c.rows, mpad = rowgroups * c.rows;
     const uint64_t colgroups = (n + c.cols - 1) / c.cols;
     const uint64_t tiles = rowgroups * colgroups;
@@ -795,12 +807,13 @@ bool plan_block_rows(const LaunchArgs& x, uint32_t m, BlockPlan* out) {
     for (uint32_t parts = 1; parts <= stages && parts <= 32; parts++) {
       const uint32_t spp = (stages + parts - 1) / parts;
       if ((stages + spp - 1) / spp != parts) continue;  // same split, already seen
+      if (spp < c.streams * kStreamStages && c.streams > 1) break;
       const size_t partial = parts > 1 ? (size_t)parts * m * n * 4 : 0;
       if (a_bytes + means + inv + partial > x.block_ws_bytes) break;
       const uint64_t wgs = tiles * parts;
-      const double nk = spp * (double)sb / 4.0;
+      const double nk = (spp + c.streams - 1) / c.streams * c.streams * (double)sb / 4.0;
       const double rounds = std::ceil((double)wgs / x.num_cus);
-      double us = nk * (c.t1 + (rounds - 1) * c.tn);
+      double us = nk * (c.t1 + (rounds - 1) * c.tn) + (c.streams > 1 ? rounds : 0.0);  // (the streams' meeting)
       const double mem = (double)bpc * n * (x.w.fmt == MGN_FMT_Q4 ? 20 : 34) / 5.0e6 + (double)m * n * 4 / 4.0e6;
       us = std::max(us, mem) + 3.5 + (double)m * n * 4 / 8.0e6;
       if (parts > 1) us += 3.5 + (2.0 * parts + 1) * m * n * 4 / 5.0e6;

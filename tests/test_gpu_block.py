@@ -135,3 +135,23 @@ def test_rows_beyond_the_workspace_run_in_blocks(ctx, orc):
     for r in range(0, m, 50):
         assert_rows_close(got[r:r + 50], want, x[:50], k)
     wt.free()
+
+
+# Parts that do not share evenly between the two streams of a workgroup: an odd number of stages, a shorter last part,
+# one of a single stage (the second stream has none)
+@pytest.mark.parametrize("fmt,m,k,n", [(Q4, 97, 3168, 9846), (Q4, 65, 3872, 11916), (Q4, 34, 4160, 14866), (Q8, 66, 3616, 6605), (Q8, 65, 2368, 8403),
+                                       (Q8, 66, 2624, 10815)])
+def test_two_streams(ctx, orc, fmt, m, k, n):
+    plan = capi.matmul_block_plan(fmt, m, k, n)
+    assert (plan.threads, plan.cols, plan.rows) == (512, 256, 96 if fmt == Q8 or m == 65 else 64) and plan.k_parts > 1
+    w = synth.normal(2050, k * n, 0.02).reshape(k, n)
+    x = synth.normal(2051, m * k).reshape(m, k)
+    x[3, 256:] *= np.float32(2.0**-30)  # rows whose sums change scale along K, each stream on its own slices
+    x[4, : k - 64] *= np.float32(2.0**-70)
+    x[5, 700:900] *= np.float32(1e-20)
+    wt = ctx.weight(fmt, w)
+    want = x.astype(np.float64) @ orc.dequantize(fmt, orc.quantize(fmt, w), k, n).astype(np.float64)
+    got = run(ctx, x, wt)
+    assert_rows_close(got, want, x, k)
+    assert np.array_equal(bits(run(ctx, x, wt)), bits(got)), "not repeatable"
+    wt.free()
