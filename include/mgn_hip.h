@@ -273,6 +273,9 @@ typedef struct mgn_plan_info {
                            * quads share one more step for (K = 32 * (16 * steps + tail_blocks)) */
   uint64_t workspace_bytes; /* partial sums held in the context's workspace */
 } mgn_plan_info;
+/* (Q8 weights with f32 activations of 33 to 127 rows: the plan of the general tiled kernel, which a forced
+ * MGN_ROUTE_TILE_MFMA runs; the automatic choice takes the form with LDS-resident images where K has at most
+ * four parts.) */
 mgn_status mgn_matmul_q_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus,
                              mgn_plan_info* out);
 

@@ -1520,13 +1520,18 @@ size_t tile_workspace_bytes(const TilePlan& p) { return ((p.partial_bytes + 255)
 // Which of the two kernels takes a call.  Up to 32 rows: the one with LDS-resident images.  Beyond,
 // it runs row groups side by side and still wins where K is short enough for at most four K parts
 // and their partial tiles stay small (f32 512 x 1024 x 3072: 16.5 us against 29 us with images
-// through the workspace; 128 x 4096 x 4096: 21.8 against 28.8), except for Q8 below 128 rows,
-// where too few workgroups carry too much each (64 x 1024 x 3072: 13.9 against 11.2 us), and for
-// wide outputs whose partial tiles dominate (64 x 4096 x 14336: 43 against 40 us).
+// through the workspace; 128 x 4096 x 4096: 21.8 against 28.8), except for wide outputs whose
+// partial tiles dominate (64 x 4096 x 14336: 43 against 40 us).  Q8 of 33 to 127 rows joins with f32
+// activations where the library chooses by itself (LaunchArgs::resident_q8): one launch instead of two, and
+// never the slower one since the kernel starts its weights early (us, general -> resident: 64 x 1024 x 3072 11.2 ->
+// 10.9, 96 rows 17.1 -> 11.0, 64 x 3584 x 1536 19.9 -> 12.8, 33 x 4096 x 4096 22.1 -> 13.9, 96 x 4096 x 1000 23.7 -> 12.8,
+// 96 x 576 x 576 11.5 -> 9.6).
 bool use_resident(const LaunchArgs& x, ResidentPlan* rp) {
   if (!plan_resident(x, rp)) return false;
   if (x.m <= 32) return true;
-  return rp->parts <= 4 && rp->partial_bytes <= ((size_t)8 << 20) && (x.w.fmt == MGN_FMT_Q4 || x.m >= 128);
+  if (rp->parts > 4 || rp->partial_bytes > ((size_t)8 << 20)) return false;
+  if (x.w.fmt == MGN_FMT_Q4 || x.m >= 128) return true;
+  return x.resident_q8 && !x.a_is_f16 && rp->partial_bytes <= ((size_t)4 << 20);  // (what the static workspace holds: one plan for both)
 }
 
 // The general kernel's plan for as many rows per launch as the workspace has room for (partial
@@ -1580,7 +1585,8 @@ bool tile_mfma_supported(const LaunchArgs& x) {
 // against 18.6, 48 x 3072 x 4096 10.3 against 13.2; f32 128 x 4096 x 4096 20.1 against 23.2, but
 // 128 x 3072 x 3072, two pairs of tiles per wave without room to park the quants on 0.56 of the CUs,
 // 20.4 against 19.0);
-// Q8 is between 0.8 and 1.4 of the tiled kernel's time on this one and stays where it was.
+// Q8 is between 0.8 and 1.4 of the tiled kernel's time on this one and stays where it was (beside the
+// rescaling kernels it is always the faster one: see use_resident).
 bool tile_mfma_preferred(const LaunchArgs& x) {
   ResidentPlan rp;
   if (!use_resident(x, &rp)) return false;

@@ -764,6 +764,7 @@ static mgn_status matmul_impl(mgn_ctx* ctx, const mgn_buf* a, bool a_is_f16, con
       return fail(ctx, MGN_EUNSUPPORTED, "fused prologue needs the GEMV_MFMA route (f32 activations, M <= 4)");
     route = MGN_ROUTE_GEMV_MFMA;
   }
+  x.resident_q8 = route == MGN_ROUTE_AUTO;
   if (route == MGN_ROUTE_AUTO) route = auto_route(x, ctx->any_magnitude);
   if (static_workspace) {
     // Same plan as the allocating entry point (the planners see the same workspace limits), run
@@ -931,6 +932,7 @@ static void rows_args(const mgn_ctx* ctx, LaunchArgs* x) {
   x->handover_bytes = ctx->handover_bytes;
   x->block_ws = ctx->block_ws;
   x->block_ws_bytes = kBlockWsBytes;
+  x->resident_q8 = true;  // (rows_plans: the route is the library's choice)
 }
 
 bool rows_plans(const mgn_ctx* ctx, const mgn_weight* const* ws, size_t count, uint32_t m, int pro_kind) {
@@ -1037,6 +1039,7 @@ mgn_status mgn_matmul_q_block_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t
   if (!out || !planned_args(fmt, m, k, n, a_is_f16, num_cus, &x)) return MGN_EINVAL;
   *out = mgn_block_plan{};
   if (!mgn::describe_block_mfma(x, out)) return MGN_EUNSUPPORTED;
+  x.resident_q8 = true;  // (as the automatic choice has it)
   out->taken = auto_route(x, a_is_f16 == 0) == MGN_ROUTE_BLOCK_MFMA ? 1u : 0u;
   return MGN_OK;
 }

@@ -91,6 +91,9 @@ struct LaunchArgs {
   void* block_ws = nullptr;
   size_t block_ws_bytes = 0;
   bool promised_range = false;  // f32 activations were promised to lie in the fp16 range: report those that do not
+  // Q8 of 33 to 127 rows may run on the resident tiled kernel: set where the route is the library's choice (a
+  // forced route and the plan entry know the general form)
+  bool resident_q8 = false;
   // host-visible word a kernel sets when f32 activations leave the range it can represent
   uint32_t* range_flag = nullptr;
   // host-visible word set by a wave that gave up waiting for another workgroup's partial sums

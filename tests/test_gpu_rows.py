@@ -4,7 +4,8 @@ slices, K parts and column groups, with every kind of row that the conversion tr
 import numpy as np
 import pytest
 
-from meganeura_amd import synth
+from helpers import Q8
+from meganeura_amd import capi, synth
 from meganeura_amd.graph import Graph, build_inference_session
 
 pytestmark = pytest.mark.gpu
@@ -114,3 +115,23 @@ def test_swiglu_on_the_way(quant, m, k, n, residual, launches):
     plain = step_outputs(s, [m * n])[0]
     s.close()
     close(fused, plain, m, 1e-5)
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 32, 1), (47, 288, 257), (64, 1056, 70), (127, 4096, 300), (96, 3584, 513), (113, 2080, 1025)])
+def test_q8_of_33_to_127_rows(orc, m, k, n):
+    """The automatic choice against 64 bits; every product carries 22 bits of the row's largest slice and sums are f32:
+    8 (2^-22 + 2^-24) sqrt(K) of the row's largest magnitude times the weights' size (0.02, zero points included 0.06)."""
+    w, x, d = synth.normal(60, k * n, 0.02).reshape(k, n), rows_of(m, k, 61), synth.normal(62, m * n).reshape(m, n)
+    dq = orc.dequantize(Q8, orc.quantize(Q8, w), k, n).astype(np.float64)
+    with capi.Context(0) as ctx:
+        wt, a, c, dd = ctx.weight(Q8, w), ctx.upload(x), ctx.buffer(m * n * 4), ctx.upload(d)
+        bound = 8 * (2.0**-22 + 2.0**-24) * 0.06 * np.sqrt(k) * np.abs(x).max(axis=1, keepdims=True).astype(np.float64)
+        for res in (None, dd):
+            ctx.matmul_q(a, wt, c, m, res)
+            got = c.download(np.float32, m * n).reshape(m, n)
+            want = x.astype(np.float64) @ dq + (d if res else 0)
+            assert (np.abs(got - want) <= bound + 2.0**-23 * np.abs(want)).all()
+            ctx.matmul_q(a, wt, c, m, res)
+            assert np.array_equal(c.download(np.float32, m * n).reshape(m, n), got), "not repeatable"
+        for b in (a, c, dd, wt):
+            b.free()
