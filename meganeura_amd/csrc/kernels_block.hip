@@ -59,10 +59,12 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 }
 
 // 64 x 16 bytes from memory straight into LDS: lane i's bytes land at lds + 16 i.  (In assembly, with the
-// waits counted by hand: the compiler waits for every such load before any LDS read that might alias it.)
+// waits counted by hand: the compiler waits for every such load before any LDS read that might alias it.  Nor does
+// it look in here for the five wait states that a load must keep from the vector unit's write of a scalar it
+// reads, v_readfirstlane's and a spilled scalar's v_readlane among them: the move and the nop are these five.)
 __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t src, uint32_t lane_off, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(lane_off), "s"(src), "s"(__builtin_amdgcn_readfirstlane(off)) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(lane_off), "s"(src), "s"(__builtin_amdgcn_readfirstlane(off)) : "memory", "m0");
 }
 template <int N>
 __device__ __forceinline__ void wait_loads() {
