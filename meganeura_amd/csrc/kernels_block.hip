@@ -631,12 +631,13 @@ __global__ __launch_bounds__(512) void prepare_f32_kernel(const float* __restric
   rmin = -group_max32(-rmin);
   const int er = (int)(__builtin_bit_cast(uint32_t, rmax) >> 23) - 127;
   const bool bad = er >= 100;
-  const int shr = (er <= -100 || bad) ? 0 : kTop - er;
+  const bool scaled = er > -100 && !bad;  // (a flag of its own: a row whose largest is in [2^kTop, 2^(kTop + 1)) has a shift of 0 as well)
+  const int shr = scaled ? kTop - er : 0;
   // One scale for the row, unless a slice would keep fewer than 22 bits of its largest magnitude on it
   // (the low halves end at 2^-24, so below 2^-2): such slices get scales of their own.
   auto shift = [&](float smx) __attribute__((always_inline)) {
     const int es = (int)(__builtin_bit_cast(uint32_t, smx) >> 23) - 127;
-    return !bad && shr != 0 && es > -100 && es + shr < -2 ? min(kTop - es, shr + 60) : shr;
+    return scaled && es > -100 && es + shr < -2 ? min(kTop - es, shr + 60) : shr;
   };
   const bool any_mixed = shift(rmin) != shr;
   auto convert = [&](const floatx4 (&v)[2], uint32_t s) __attribute__((always_inline)) {

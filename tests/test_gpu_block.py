@@ -112,6 +112,29 @@ def test_magnitudes_that_change_along_k(ctx, orc, fmt, k):
 
 
 @pytest.mark.parametrize("fmt", [Q4, Q8])
+def test_small_slices_beside_a_large_one(ctx, orc, fmt):
+    """A slice of 256 elements keeps 22 bits of its own largest magnitude whatever the row's largest is, 2^14 (where the
+    row's scale is 1) and its neighbours among them: seen in a column whose weights are zero over the large slice."""
+    k, n = 1280, 130
+    rows = [(top, small) for top in (2.0**13, 9000.0, 2.0**14, 20000.0, 32767.0, 2.0**15, 40000.0, 1.5, 1e-6, 1e9) for small in (2.0**-15, 2.0**-22, 2.0**-30, 2.0**-40)]
+    m = len(rows)
+    w = synth.normal(2060, k * n, 0.02).reshape(k, n)
+    w[:256, n - 1] = 0.0
+    x = synth.normal(2061, m * k).reshape(m, k)
+    x /= np.abs(x).reshape(m, -1, 256).max(axis=2).repeat(256, axis=1)
+    for r, (top, small) in enumerate(rows):
+        x[r] *= np.float32(top)
+        x[r, 256:] *= np.float32(small)
+    wt = ctx.weight(fmt, w)
+    dq = orc.dequantize(fmt, orc.quantize(fmt, w), k, n).astype(np.float64)
+    assert (dq[:256, n - 1] == 0).all()
+    want, got = x.astype(np.float64) @ dq, run(ctx, x, wt)
+    assert_rows_close(got, want, x, k)
+    assert_rows_close(got[:, n - 1:], want[:, n - 1:], x[:, 256:], k)
+    wt.free()
+
+
+@pytest.mark.parametrize("fmt", [Q4, Q8])
 def test_infinite_rows_of_fp16_activations_stay_on_their_own(ctx, orc, fmt):
     m, k, n = 40, 96, 70  # K ends in the middle of the 64 elements that are loaded at once
     x = synth.normal(2030, m * k).reshape(m, k).astype(np.float16)
