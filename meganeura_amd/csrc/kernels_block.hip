@@ -19,8 +19,8 @@
 //   * everything the multiplication wants to know about the activations is worked out once per call by
 //     a small launch in front (prepare_*): the blocks' means, and for f32 the fp16 pairs on a scale per
 //     row.  One scale for the whole row, so that no accumulator is rescaled on the way: a slice of
-//     256 elements that would keep fewer than 22 bits on it gets its own, and the waves that meet
-//     such a row move their sums from scale to scale;
+//     256 elements that would be held in fewer bits than the tiled kernels hold it gets its own, and the
+//     waves that meet such a row move their sums from scale to scale;
 //   * K parts for different workgroups, where the tiles do not fill the chip, meet in the workspace and are added
 //     in part order by a third launch.
 // Measured (one box, weights from memory; before -> now, us): fp16 2048 x 4096 x 14336 589 -> 299 (805 TFLOP/s),
@@ -574,19 +574,20 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
 constexpr uint32_t kMaxSlices = 256;
 constexpr int kTop = 14;  // a row's largest magnitude is brought into [2^14, 2^15)
 
-__device__ __forceinline__ void store_mean(uint16_t* means, int sb, uint32_t mpad, uint32_t row, uint32_t block, float mean) {
-  const uint32_t mh = pack_rtz(mean, 0.0f);
-  const uint32_t ml = pack_rtz((mean - half_lo(mh)) * 2048.0f, 0.0f);
-  uint16_t* const p = means + ((size_t)(block / sb) * mpad + row) * (sb * 2) + block % sb;
-  p[0] = (uint16_t)mh;
-  p[sb] = (uint16_t)ml;
+__device__ __forceinline__ void store_mean(_Float16* means, int sb, uint32_t mpad, uint32_t row, uint32_t block, float mean) {
+  _Float16* const p = means + ((size_t)(block / sb) * mpad + row) * (sb * 2) + block % sb;
+  p[0] = (_Float16)mean;
+  p[sb] = (_Float16)((mean - (float)p[0]) * 2048.0f);
 }
 
 // grid.x = mpad rows, 512 threads: half-wave w converts the row's slices w, w + 16, ..; HELD of them stay
 // in registers between the search for the row's largest magnitude and the conversion, the rest of a
 // longer row is read twice.
+//
+// Both halves of a pair are rounded to nearest (23 bits and no bias; cut, as the tiled kernels' pairs are, they
+// carry 22 and all results come out 2^-24 to 2^-23 small), and a block's mean is that of its pairs.
 template <int FMT, int HELD>
-__global__ __launch_bounds__(512) void prepare_f32_kernel(const float* __restrict__ a, uint8_t* __restrict__ out, uint16_t* __restrict__ means,
+__global__ __launch_bounds__(512) void prepare_f32_kernel(const float* __restrict__ a, uint8_t* __restrict__ out, _Float16* __restrict__ means,
                                                           float* __restrict__ inv, float* __restrict__ row_scale, uint32_t* __restrict__ mixed,
                                                           uint32_t m, uint32_t k, uint32_t nslices, uint32_t mpad,
                                                           uint32_t* __restrict__ range_flag) {
@@ -633,11 +634,15 @@ __global__ __launch_bounds__(512) void prepare_f32_kernel(const float* __restric
   const bool bad = er >= 100;
   const bool scaled = er > -100 && !bad;  // (a flag of its own: a row whose largest is in [2^kTop, 2^(kTop + 1)) has a shift of 0 as well)
   const int shr = scaled ? kTop - er : 0;
-  // One scale for the row, unless a slice would keep fewer than 22 bits of its largest magnitude on it
-  // (the low halves end at 2^-24, so below 2^-2): such slices get scales of their own.
+  // One scale for the row, unless a slice's largest would come to lie more than a bit below where the tiled kernels
+  // bring every slice's (2^7 with Q4, 2^11 with Q8; the low halves end at 2^-24, and what is rounded there is as close as
+  // what is cut a bit further down): such slices get scales of their own, up to 2^60 times the row's (the sums of
+  // the large slices move along and must stay finite).  Rows that have such slices cost: lognormal activations (sigma
+  // 1.5), a tenth with Q8, nothing to a fiftieth with Q4.
+  constexpr int kLeast = FMT == MGN_FMT_Q4 ? 6 : 10;
   auto shift = [&](float smx) __attribute__((always_inline)) {
     const int es = (int)(__builtin_bit_cast(uint32_t, smx) >> 23) - 127;
-    return scaled && es > -100 && es + shr < -2 ? min(kTop - es, shr + 60) : shr;
+    return scaled && es > -100 && es + shr < kLeast ? min(kTop - es, shr + 60) : shr;
   };
   const bool any_mixed = shift(rmin) != shr;
   auto convert = [&](const floatx4 (&v)[2], uint32_t s) __attribute__((always_inline)) {
@@ -649,18 +654,19 @@ __global__ __launch_bounds__(512) void prepare_f32_kernel(const float* __restric
       if (s == nslices - 1) row_scale[row] = bad ? __builtin_nanf("") : back;
     }
     const floatx4 x0 = v[0] * scale, x1 = v[1] * scale;
-    const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    uint32_t hp[4], lp[4];
+    float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    half8 hi, lo;
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      hp[e] = pack_rtz(x[2 * e], x[2 * e + 1]);
-      lp[e] = pack_rtz(x[2 * e] - half_lo(hp[e]), x[2 * e + 1] - half_hi(hp[e]));
+    for (int e = 0; e < 8; e++) {
+      hi[e] = (_Float16)x[e];
+      lo[e] = (_Float16)(x[e] - (float)hi[e]);
+      x[e] = (float)hi[e] + (float)lo[e];
     }
     float sum = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
     if (live) {
       uint8_t* const dst = out + ((size_t)row * nslices * 8 + s * 8 + (l >> 2)) * 128 + (l & 3) * 16;
-      *(uint4*)dst = make_uint4(hp[0], hp[1], hp[2], hp[3]);
-      *(uint4*)(dst + 64) = make_uint4(lp[0], lp[1], lp[2], lp[3]);
+      *(half8*)dst = hi;
+      *(half8*)(dst + 64) = lo;
     }
     sum += dpp_move<kDppQuadXor1>(sum);
     sum += dpp_move<kDppQuadXor2>(sum);
@@ -681,7 +687,7 @@ __global__ __launch_bounds__(512) void prepare_f32_kernel(const float* __restric
 }
 
 template <int FMT>
-__global__ __launch_bounds__(256) void prepare_f16_kernel(const _Float16* __restrict__ a, uint16_t* __restrict__ means, uint32_t m,
+__global__ __launch_bounds__(256) void prepare_f16_kernel(const _Float16* __restrict__ a, _Float16* __restrict__ means, uint32_t m,
                                                           uint32_t k, uint32_t nslices, uint32_t mpad) {
   constexpr int SB = stage_blocks(FMT);
   const uint32_t row = blockIdx.x;
@@ -853,7 +859,7 @@ int launch_block_rows(ihipStream_t* s, const LaunchArgs& x, const BlockPlan& p) 
   const bool f32a = !x.a_is_f16;
   char* const ws = (char*)x.block_ws;
   uint8_t* const prepared = (uint8_t*)ws;
-  uint16_t* const means = (uint16_t*)(ws + p.a_bytes);
+  _Float16* const means = (_Float16*)(ws + p.a_bytes);
   float* const inv = (float*)(ws + p.a_bytes + p.means_bytes);
   float* const row_scale = inv + (size_t)p.nslices * p.mpad;
   uint32_t* const mixed = (uint32_t*)(row_scale + p.mpad);

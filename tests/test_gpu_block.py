@@ -135,6 +135,46 @@ def test_small_slices_beside_a_large_one(ctx, orc, fmt):
 
 
 @pytest.mark.parametrize("fmt", [Q4, Q8])
+@pytest.mark.parametrize("gap", [0, 3, 4, 7, 8, 12, 16])
+def test_small_elements_of_a_slice(ctx, orc, fmt, gap):
+    """Inside a slice 2^gap below the row's largest: elements far below the slice's own largest are held down to 2^-31 (Q4) or
+    2^-35 (Q8) of that largest, as in the tiled kernels, and rounded, not cut.  The large elements meet blocks of zero
+    weights and all products are positive, so that what every element loses adds up."""
+    m, k, n = 33, 512, 70
+    x = np.abs(synth.normal(2070, m * k)).reshape(m, k).astype(np.float32) + np.float32(0.5)
+    x *= np.float32(2.0 ** (-gap - 20))
+    x[:, :256] *= np.float32(2.0**20)
+    x[:, 5], x[:, 261] = 1.0, 2.0**-gap
+    w = np.abs(synth.normal(2071, k * n, 0.02)).reshape(k, n) + np.float32(0.001)
+    w[:288] = 0.0
+    x[:, :256] = np.minimum(x[:, :256], 1.0)
+    wt = ctx.weight(fmt, w)
+    dq = orc.dequantize(fmt, orc.quantize(fmt, w), k, n).astype(np.float64)
+    assert (dq[:288] == 0).all() and (dq >= 0).all()
+    want, got = x.astype(np.float64) @ dq, run(ctx, x, wt).astype(np.float64)
+    held = 2.0 ** (-gap - (31 if fmt == Q4 else 35)) * dq.sum(axis=0)  # the last bit held of every element that meets a weight, of which it is half off at most
+    # the f32 sums: 16 blocks and their means, 2^-24 each of the products' sum (Q8: of 128 scales per element, before the bias)
+    biased = want if fmt == Q4 else (x[:, 288:].astype(np.float64).sum(axis=1) * 128)[:, None] * (dq.max(axis=0) / 127)
+    assert (np.abs(got - want) <= held / 2 + 2.0**-20 * biased).all()
+    wt.free()
+
+
+@pytest.mark.parametrize("fmt", [Q4, Q8])
+def test_activations_are_rounded_without_a_bias(ctx, orc, fmt):
+    """The pairs that f32 activations enter as are rounded to nearest: over many outputs the errors have no part along the result
+    (cut to 22 bits they have one of 2^-24 to 2^-23)."""
+    m, k, n = 65, 4096, 513
+    w = synth.normal(2080, k * n, 0.02).reshape(k, n)
+    x = synth.normal(2081, m * k).reshape(m, k)
+    wt = ctx.weight(fmt, w)
+    want = x.astype(np.float64) @ orc.dequantize(fmt, orc.quantize(fmt, w), k, n).astype(np.float64)
+    err = run(ctx, x, wt) - want
+    # errors of at most 2^-19 of the result's size (8 x 2^-22), independent over m n outputs, average out to 2^-19 / sqrt(m n)
+    assert abs((err * want).sum() / (want * want).sum()) <= 2.0**-26 + 2.0**-19 / np.sqrt(m * n)
+    wt.free()
+
+
+@pytest.mark.parametrize("fmt", [Q4, Q8])
 def test_infinite_rows_of_fp16_activations_stay_on_their_own(ctx, orc, fmt):
     m, k, n = 40, 96, 70  # K ends in the middle of the 64 elements that are loaded at once
     x = synth.normal(2030, m * k).reshape(m, k).astype(np.float16)
