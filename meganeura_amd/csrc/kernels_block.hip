@@ -2,7 +2,8 @@
 // (prefill, and decode batches of more than some 32 rows on large weights).
 //
 // The arithmetic is that of the other tiled kernels (raw quants as the B operand of the matrix
-// instructions, block scales on their results, block minima as a product of their own), so the vector
+// instructions, block scales on their results, block minima as a product of their own; Q8 with f32 activations
+// multiplies signed bytes and has no such product), so the vector
 // ALU owes 16 multiply-adds per 32 x 32 outputs and quant block whatever the tiling; with the matrix
 // instructions (two of 32 cycles; four with f32 activations, which enter as fp16 pairs hi + lo) that is
 // the bound: measured on one SIMD, v_mfma_f32_32x32x16_f16 occupies its pipe for 32 cycles and the vector
@@ -78,6 +79,23 @@ __device__ __forceinline__ half8 nibbles_in_order(uint32_t w) {
                   __builtin_amdgcn_perm(od, ev, 0x0c060c02u), __builtin_amdgcn_perm(od, ev, 0x0c070c03u));
 }
 
+// Q8 with f32 activations multiplies the bytes as they are; the other forms leave an additive part (Q4's minima, the
+// bias of Q8's bytes) to a product of the blocks' means.  The bias of 128 is several times the bytes: it enters the
+// running sum and leaves it again at every stage, and the sum's roundings are those of its size.  Four packed subtractions
+// per operand keep it out, which the vector unit has room for with four matrix instructions per tile and block (not with
+// fp16's two).  Error against f64 (2-norm, normal activations; the tiled kernels, biased here, signed) and time (biased,
+// signed): 2048 x 14336 x 4096 9.4e-7, 1.03e-6, 2.8e-7, 560 -> 549 us; 77 x 4096 x 14336 7.1e-7, 7.2e-7, 1.1e-7,
+// 43.8 -> 41.9 us.
+constexpr bool has_additive(int fmt, bool f32a) { return fmt == MGN_FMT_Q4 || !f32a; }
+
+// two dwords of int8 -> 8 fp16, the bytes' own values: 1024 + (q + 128) as bits, less 1152
+__device__ __forceinline__ half8 signed_bytes_to_operand(uint32_t w0, uint32_t w1) {
+  const uint32_t u0 = w0 ^ 0x80808080u, u1 = w1 ^ 0x80808080u, k1024 = 0x64646464u;
+  const half8 v = as_half8(__builtin_amdgcn_perm(k1024, u0, 0x04010400u), __builtin_amdgcn_perm(k1024, u0, 0x04030402u),
+                           __builtin_amdgcn_perm(k1024, u1, 0x04010400u), __builtin_amdgcn_perm(k1024, u1, 0x04030402u));
+  return v - (half8)((_Float16)1152.0f);
+}
+
 // the j-th of NM equal shares of acc += dq * d
 template <int NM, int j>
 __device__ __forceinline__ void scale_part(floatx16& acc, const floatx16& d, float dq) {
@@ -126,7 +144,7 @@ struct BlockShape {
   static constexpr int PANELS = SUBB * (F32A ? 128 : 64) / 128;  // 128 bytes of activations per row each
   static constexpr int ARING = PD + 1, SRING = SD + 1;
   static constexpr uint32_t A_BYTES = WK * PANELS * ROWS * 128u, B_BYTES = WK * COLS * 64u, M_BYTES = WK * COLS * 16u;
-  static constexpr uint32_t MEAN_STREAM = (ROWS * SB * 4 + 1023) / 1024 * 1024, S_BYTES = WK * MEAN_STREAM;
+  static constexpr uint32_t MEAN_STREAM = has_additive(FMT, F32A) ? (ROWS * SB * 4 + 1023) / 1024 * 1024 : 0, S_BYTES = WK * MEAN_STREAM;
   static constexpr uint32_t STAGE_BYTES = B_BYTES + M_BYTES + S_BYTES;
   static constexpr int NA = (int)(A_BYTES / 1024), NST = (int)(STAGE_BYTES / 1024);  // loads of 1 KiB
   static constexpr int NAW = (NA + WAVES - 1) / WAVES, NSTW = (NST + WAVES - 1) / WAVES;
@@ -208,11 +226,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
     st_stream[j] = q / (COLS / 16), st_step[j] = 64, st_base[j] = 0;
     const uint32_t bcol = q % (COLS / 16) * 16 + (lane >> 2);
     st_off[j] = min(col0 + bcol, x.n - 1) * (x.bpc * QB) + (((lane & 3) ^ ((bcol >> 2) & 3)) << 4);
-    if (q >= NBL + NML) {
+    if (MEAN_STREAM > 0 && q >= NBL + NML) {
+      constexpr uint32_t KIB = MEAN_STREAM > 0 ? MEAN_STREAM / 1024 : 1;
       const uint32_t p = q - NBL - NML;
       base = x.means, bytes = x.means_bytes;
-      st_stream[j] = p / (MEAN_STREAM / 1024), st_step[j] = x.mpad * (SB * 4), st_base[j] = row0 * (SB * 4);
-      st_off[j] = p % (MEAN_STREAM / 1024) * 1024u + lane * 16u;
+      st_stream[j] = p / KIB, st_step[j] = x.mpad * (SB * 4), st_base[j] = row0 * (SB * 4);
+      st_off[j] = p % KIB * 1024u + lane * 16u;
     } else if (q >= NBL) {
       const uint32_t mcol = (q - NBL) % (COLS / 64) * 64 + lane;
       base = x.meta, bytes = x.meta_bytes;
@@ -291,6 +310,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
     if constexpr (FMT == MGN_FMT_Q4) {
       bop[t][0] = nibbles_in_order(braw[t][0]);
       bop[t][1] = nibbles_in_order(braw[t][1]);
+    } else if constexpr (F32A) {
+      bop[t][0] = signed_bytes_to_operand(braw[t][0], braw[t][1]);
+      bop[t][1] = signed_bytes_to_operand(braw[t][2], braw[t][3]);
     } else {
       bop[t][0] = bytes_to_operand(braw[t][0], braw[t][1]);
       bop[t][1] = bytes_to_operand(braw[t][2], braw[t][3]);
@@ -424,7 +446,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
         });
         dqp = dq[kCT - 1];
       });
-      if constexpr (last) {
+      if constexpr (last && has_additive(FMT, F32A)) {
         // the additive part of the stage's blocks: means times m (Q4) or the scale (Q8)
         half8 bm[kCT];
 #pragma unroll
@@ -638,7 +660,7 @@ __global__ __launch_bounds__(512) void prepare_f32_kernel(const float* __restric
   // bring every slice's (2^7 with Q4, 2^11 with Q8; the low halves end at 2^-24, and what is rounded there is as close as
   // what is cut a bit further down): such slices get scales of their own, up to 2^60 times the row's (the sums of
   // the large slices move along and must stay finite).  Rows that have such slices cost: lognormal activations (sigma
-  // 1.5), a tenth with Q8, nothing to a fiftieth with Q4.
+  // 1.5), Q8 77 x 4096 x 14336 43.5 -> 46.8 us, Q4 level.
   constexpr int kLeast = FMT == MGN_FMT_Q4 ? 6 : 10;
   auto shift = [&](float smx) __attribute__((always_inline)) {
     const int es = (int)(__builtin_bit_cast(uint32_t, smx) >> 23) - 127;
@@ -670,7 +692,7 @@ __global__ __launch_bounds__(512) void prepare_f32_kernel(const float* __restric
     }
     sum += dpp_move<kDppQuadXor1>(sum);
     sum += dpp_move<kDppQuadXor2>(sum);
-    if ((l & 3) == 0) store_mean(means, SB, mpad, row, s * 8 + (l >> 2), sum * 0.03125f);
+    if (has_additive(FMT, true) && (l & 3) == 0) store_mean(means, SB, mpad, row, s * 8 + (l >> 2), sum * 0.03125f);
   };
 #pragma unroll
   for (int i = 0; i < HELD; i++)
@@ -811,7 +833,7 @@ bool plan_block_rows(const LaunchArgs& x, uint32_t m, BlockPlan* out) {
     const size_t a_bytes = f32a ? align256((size_t)m * nslices * 1024) : 0;
     const size_t a_read = f32a ? (size_t)m * nslices * 1024 : (size_t)m * k * 2;
     if (a_read >= (1ull << 32)) continue;
-    const size_t means = align256((size_t)nslices * 8 * mpad * 4 + 4096);
+    const size_t means = has_additive(x.w.fmt, f32a) ? align256((size_t)nslices * 8 * mpad * 4 + 4096) : 0;
     const size_t inv = f32a ? align256((size_t)nslices * mpad * 4 + (size_t)mpad * 8) : 0;
     for (uint32_t parts = 1; parts <= stages && parts <= 32; parts++) {
       const uint32_t spp = (stages + parts - 1) / parts;
@@ -885,12 +907,13 @@ int launch_block_rows(ihipStream_t* s, const LaunchArgs& x, const BlockPlan& p) 
   a.m = x.m, a.mpad = p.mpad, a.n = x.w.n, a.bpc = x.w.k / 32, a.stages = p.stages;
   a.rowgroups = p.rowgroups, a.colgroups = p.colgroups, a.parts = p.parts;
   // The sums run in units of 2^lift / 32 (Q4) or 2^lift / 4096 (Q8) of the result: the additive constants
-  // enter times 2^lift (WeightView::additive_lift), their means as they are.
+  // enter times 2^lift (WeightView::additive_lift), their means as they are.  (Without an additive part: the result's own.)
   const int lift = (int)std::min<uint32_t>(x.w.additive_lift, 15u);
   const float sign = FMT == MGN_FMT_Q4 ? 1.0f : -1.0f;
   a.add_hi = half_pair(sign * std::ldexp(1.0f, lift)), a.add_lo = half_pair(sign * std::ldexp(1.0f, lift - 11));
   a.dscale = std::ldexp(1.0f, (FMT == MGN_FMT_Q4 ? 15 : 12) + lift);
   a.unit = std::ldexp(1.0f, (FMT == MGN_FMT_Q4 ? 5 : 12) - lift);
+  if (!has_additive(FMT, f32a)) a.dscale = a.unit = 1.0f;
   a.dres = x.d, a.c = x.c, a.partial = partial, a.epilogue = x.epilogue;
   if (p.cfg->lds > 64 * 1024) {
     static std::atomic<uint64_t> big_lds_done[4][kBlockConfigs];

@@ -174,6 +174,20 @@ def test_activations_are_rounded_without_a_bias(ctx, orc, fmt):
     wt.free()
 
 
+def test_q8_sums_are_free_of_the_byte_bias(ctx, orc):
+    """Q8 with f32 activations that have a mean: a bias of 128 on the bytes would put sums of some hundred times the result's
+    size into the accumulators.  Without one the error is that of the f32 additions, one per block of 32, each 2^-24
+    of a sum no larger than the result's size, independent of each other."""
+    m, k, n = 65, 4096, 513
+    w = synth.normal(2090, k * n, 0.02).reshape(k, n)
+    x = synth.normal(2091, m * k).reshape(m, k) + np.float32(8.0)
+    wt = ctx.weight(Q8, w)
+    want = x.astype(np.float64) @ orc.dequantize(Q8, orc.quantize(Q8, w), k, n).astype(np.float64)
+    err = run(ctx, x, wt) - want
+    assert np.linalg.norm(err) <= 2.0**-24 * np.sqrt(k / 32) * np.linalg.norm(want)
+    wt.free()
+
+
 @pytest.mark.parametrize("fmt", [Q4, Q8])
 def test_infinite_rows_of_fp16_activations_stay_on_their_own(ctx, orc, fmt):
     m, k, n = 40, 96, 70  # K ends in the middle of the 64 elements that are loaded at once
