@@ -38,7 +38,25 @@ constexpr size_t kChunk = (size_t)1 << 20, kChunkOut = (size_t)512 << 10;
 constexpr size_t kEvents = sizeof(HostStage::done) / sizeof(ihipEvent_t*);
 static_assert(kSmallIn <= kSmall && kSmall / kChunkOut <= kEvents && kSlots <= kEvents, "an event per chunk, and per slot");
 
-// The context's ring and events; false: there is no pinned memory to be had.
+// The context's device while it lives, the caller's afterwards: events belong to the device that is current when they
+// are made, and record on no other device's stream.
+class OnDevice {
+ public:
+  explicit OnDevice(int device) : mine_(device) {
+    if (hipGetDevice(&before_) != hipSuccess) before_ = mine_;
+    if (before_ != mine_) (void)hipSetDevice(mine_);
+  }
+  ~OnDevice() {
+    if (before_ != mine_) (void)hipSetDevice(before_);
+  }
+  OnDevice(const OnDevice&) = delete;
+  OnDevice& operator=(const OnDevice&) = delete;
+
+ private:
+  int mine_, before_ = 0;
+};
+
+// The context's ring and events (its device is current); false: there is no pinned memory to be had.
 bool have_stage(mgn_ctx* ctx) {
   HostStage& st = ctx->stage;
   if (st.ring) return true;
@@ -82,7 +100,7 @@ hipError_t copy_large(mgn_ctx* ctx, char* dev, char* host, size_t bytes, bool in
   std::atomic<size_t> next{0};
   std::atomic<int> error{(int)hipSuccess};
   auto work = [&](int worker) {
-    hipError_t err = hipSetDevice(ctx->device);
+    hipError_t err = worker ? hipSetDevice(ctx->device) : hipSuccess;  // (a thread starts on device 0)
     size_t busy[2] = {0, 0};  // chunk + 1 that travels through the slot
     auto size_of = [&](size_t c) { return std::min(kSlot, bytes - c * kSlot); };
     // waits for what travels through slot s; on the way out, takes it from there
@@ -113,8 +131,6 @@ hipError_t copy_large(mgn_ctx* ctx, char* dev, char* host, size_t bytes, bool in
   const unsigned cpus = std::thread::hardware_concurrency();
   const int wanted = (int)std::min<size_t>({(size_t)kWorkers, (chunks + 1) / 2, cpus ? cpus : 1});
   std::thread helpers[kWorkers - 1];
-  int device = ctx->device;
-  (void)hipGetDevice(&device);
   for (int i = 1; i < wanted; i++) {
     try {
       helpers[i - 1] = std::thread(work, i);
@@ -125,7 +141,6 @@ hipError_t copy_large(mgn_ctx* ctx, char* dev, char* host, size_t bytes, bool in
   work(0);
   for (std::thread& t : helpers)
     if (t.joinable()) t.join();
-  if (device != ctx->device) (void)hipSetDevice(device);
   e = hipStreamSynchronize(ctx->stream);
   return error.load() != (int)hipSuccess ? (hipError_t)error.load() : e;
 }
@@ -147,6 +162,7 @@ hipError_t ring_piece(mgn_ctx* ctx, size_t bytes, size_t* out) {
 
 int copy_in(mgn_ctx* ctx, void* dev, const void* host, size_t bytes) {
   if (bytes == 0) return 0;
+  const OnDevice on(ctx->device);
   if ((bytes > kSmallIn && bytes < kLargeIn) || !pageable(host) || !have_stage(ctx)) {
     hipError_t e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -165,6 +181,7 @@ int copy_in(mgn_ctx* ctx, void* dev, const void* host, size_t bytes) {
 
 int copy_out(mgn_ctx* ctx, void* host, const void* dev, size_t bytes) {
   if (bytes == 0) return (int)hipStreamSynchronize(ctx->stream);
+  const OnDevice on(ctx->device);
   if (!pageable(host) || !have_stage(ctx)) {
     hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);

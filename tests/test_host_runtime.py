@@ -1,0 +1,58 @@
+"""The library's host code on a stand-in for the HIP runtime (host_runtime/fake_hip.cpp), in processes of their own: what one
+device, or a machine with enough memory, does not show.  No device needed."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    where = tmp_path_factory.mktemp("runtime")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-Wno-deprecated-declarations",
+                    os.path.join(HERE, "host_runtime", "fake_hip.cpp"), "-Wl,-soname,libamdhip64.so.7",
+                    "-Wl,--version-script=" + os.path.join(HERE, "host_runtime", "versions.map"), "-o", str(where / "libamdhip64.so.7")], check=True)
+    return where
+
+
+def on(runtime, program):
+    head = """
+        import ctypes, sys
+        import numpy as np
+        from meganeura_amd import capi
+        capi.load()
+        hip = ctypes.CDLL("libamdhip64.so.7")
+        assert hasattr(hip, "fake_launches"), "not the stand-in"
+        hip.fake_refuse_allocations_of.argtypes = [ctypes.c_size_t]
+        def current():
+            d = ctypes.c_int()
+            hip.hipGetDevice(ctypes.byref(d))
+            return d.value
+    """
+    env = dict(os.environ, LD_LIBRARY_PATH=str(runtime), PYTHONPATH=ROOT)
+    r = subprocess.run([sys.executable, "-c", textwrap.dedent(head) + textwrap.dedent(program)], env=env, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                       text=True, timeout=100)
+    assert r.returncode == 0, r.stdout
+
+
+@pytest.mark.parametrize("nbytes", [5, 3 << 20, 20 << 20])  # one piece of the ring, pieces, slots
+def test_copies_belong_to_the_contexts_device(runtime, nbytes):
+    """A context's first copies made while another device is current: its events are made on its own device, and the other device is
+    current again afterwards."""
+    on(runtime, f"""
+        with capi.Context(1) as ctx:
+            b = ctx.buffer({nbytes})
+            hip.hipSetDevice(0)
+            want = np.random.default_rng(1).integers(0, 256, {nbytes}, dtype=np.uint8)
+            for direction in range(2):
+                b.upload(want)
+                assert current() == 0
+                assert np.array_equal(b.download(np.uint8, {nbytes}), want)
+                assert current() == 0
+            b.free()
+    """)
