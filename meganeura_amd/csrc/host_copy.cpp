@@ -18,7 +18,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 #include "mgn_internal.h"
@@ -134,8 +134,8 @@ hipError_t copy_large(mgn_ctx* ctx, char* dev, char* host, size_t bytes, bool in
   for (int i = 1; i < wanted; i++) {
     try {
       helpers[i - 1] = std::thread(work, i);
-    } catch (const std::system_error&) {
-      break;  // no more threads: those there are take all chunks
+    } catch (const std::exception&) {
+      break;  // no more threads, or no memory for one: those there are take all chunks
     }
   }
   work(0);

@@ -11,6 +11,7 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 
 namespace {
@@ -47,9 +48,29 @@ struct ihipEvent_t {
   uint64_t at = 0;
 };
 
-#define LOCK std::lock_guard<std::recursive_mutex> lock(mu)
+// held by every call that changes something; `inside`: the runtime's own allocations are not the ones to fail
+thread_local int inside = 0;
+long failing_new = -1;  // operator new calls left until the one that fails
+struct Locked {
+  Locked() { mu.lock(), inside++; }
+  ~Locked() { inside--, mu.unlock(); }
+};
+#define LOCK Locked lock
+
+void* operator new(size_t n) {
+  if (!inside) {
+    LOCK;
+    if (failing_new >= 0 && failing_new-- == 0) throw std::bad_alloc();
+  }
+  if (void* p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
 extern "C" {
 void fake_refuse_allocations_of(size_t bytes) { refused_bytes = bytes; }
+void fake_fail_allocation(long n) { failing_new = n; }
 long fake_launches(const char* part_of_name) {
   LOCK;
   long n = 0;
@@ -96,7 +117,10 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
 }
 hipError_t hipGetSymbolAddress(void** p, const void* s) { return *p = const_cast<void*>(s), hipSuccess; }
 
-hipError_t hipStreamCreate(hipStream_t* s) { return *s = new ihipStream_t{current, {}}, hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t* s) {
+  LOCK;
+  return *s = new ihipStream_t{current, {}}, hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t s) {
   LOCK;
   s->run_to(s->queued);
@@ -111,7 +135,10 @@ hipError_t hipStreamDestroy(hipStream_t s) {
   delete s;
   return hipSuccess;
 }
-hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return *e = new ihipEvent_t{current}, hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  LOCK;
+  return *e = new ihipEvent_t{current}, hipSuccess;
+}
 hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
 hipError_t hipEventDestroy(hipEvent_t e) { return delete e, hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {

@@ -56,3 +56,22 @@ def test_copies_belong_to_the_contexts_device(runtime, nbytes):
                 assert current() == 0
             b.free()
     """)
+
+
+@pytest.mark.parametrize("nth", [0, 1, 2, 9])
+@pytest.mark.parametrize("upload", [True, False])
+def test_threads_that_cannot_be_made(runtime, nth, upload):
+    """Large copies ask for threads; where the host has no memory for the nth of them, those there are do the work."""
+    on(runtime, f"""
+        with capi.Context(0) as ctx:
+            want = np.random.default_rng(2).integers(0, 256, 20 << 20, dtype=np.uint8)
+            b = ctx.buffer(want.size)
+            if {upload}:
+                hip.fake_fail_allocation(ctypes.c_long({nth}))
+            b.upload(want)
+            if not {upload}:
+                hip.fake_fail_allocation(ctypes.c_long({nth}))
+            assert np.array_equal(b.download(np.uint8, want.size), want)
+            hip.fake_fail_allocation(ctypes.c_long(-1))
+            b.free()
+    """)
