@@ -75,3 +75,31 @@ def test_threads_that_cannot_be_made(runtime, nth, upload):
             hip.fake_fail_allocation(ctypes.c_long(-1))
             b.free()
     """)
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_a_context_without_room_for_the_blocked_kernel(runtime, fmt):
+    """The blocked kernel's 96 MiB workspace is not to be had: the context exists without it, and the calls that would take the kernel
+    run on the ones behind it."""
+    on(runtime, f"""
+        m, k, n = 77, 4096, 14336
+        assert capi.matmul_block_plan({fmt}, m, k, n).taken
+        def run(ctx):
+            w = ctx.weight_from_packed({fmt}, np.zeros(capi.packed_size({fmt}, k, n), np.uint8), k, n)
+            a, c = ctx.buffer(m * k * 4), ctx.buffer(m * n * 4)
+            before = hip.fake_launches(b"12block_kernel"), hip.fake_launches(b"tile_")
+            ctx.matmul_q(a, w, c, m)
+            ctx.sync()
+            return hip.fake_launches(b"12block_kernel") - before[0], hip.fake_launches(b"tile_") - before[1]
+        with capi.Context(0) as ctx:
+            assert run(ctx) == (1, 0)
+        hip.fake_refuse_allocations_of(96 << 20)
+        with capi.Context(0) as ctx:
+            assert run(ctx)[0] == 0 and run(ctx)[1] > 0
+            ctx.set_route(capi.ROUTE_BLOCK_MFMA)
+            try:
+                run(ctx)
+                assert False, "a kernel that has no workspace"
+            except capi.MgnError as e:
+                assert e.status == capi.EINVAL
+    """)
