@@ -213,7 +213,10 @@ mgn_status mgn_matmul_q_f16a(mgn_ctx* ctx, const mgn_buf* a_f16, const mgn_weigh
  * library runs on until the process ends) and calls no hipMalloc / hipFree or any other
  * allocating routine.  Same plan, same kernels and bit-identical results as mgn_matmul_q;
  * MGN_EUNSUPPORTED, with the byte counts in mgn_last_error, when the shape's partial sums or
- * hand-over words do not fit the static array.  All contexts of a device share the array: calls
+ * hand-over words do not fit the static array.  Which shapes it takes is settled by the kernels that
+ * use the array, mgn_matmul_q_plan's; of these, the many-row shapes that mgn_matmul_q gives to the
+ * blocked kernel run on it here too, in the workspace that the context has for it since its
+ * creation.  All contexts of a device share the array: calls
  * that overlap on one device (two contexts, two threads) race; calls on one context are ordered by
  * its stream.  The array keeps the last call's contents: the counters are cleared and the
  * hand-over words a launch will use are set to the empty pattern by a small fill kernel in front

@@ -769,9 +769,10 @@ static mgn_status matmul_impl(mgn_ctx* ctx, const mgn_buf* a, bool a_is_f16, con
   if (route == MGN_ROUTE_AUTO) route = auto_route(x, ctx->any_magnitude);
   if (static_workspace) {
     // Same plan as the allocating entry point (the planners see the same workspace limits), run
-    // on the library's static array if the plan's partial sums fit it; refused otherwise.  (What the
-    // blocked kernel takes is refused or not by the plan behind it; it runs on the context's own
-    // workspace, which is there since the context was created.)
+    // on the library's static array if the plan's partial sums fit it; refused otherwise.  (Of the shapes that the
+    // blocked kernel takes, those that the kernels behind it could run on the array are accepted, as they were
+    // before there was a blocked kernel; it runs on the context's own workspace, which is there since the
+    // context was created.)
     mgn_plan_info plan{};
     const mgn_route taken = route;
     if (route == MGN_ROUTE_BLOCK_MFMA) route = basic_route(x, ctx->any_magnitude);

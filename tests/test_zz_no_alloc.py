@@ -65,6 +65,14 @@ def test_static_workspace_matches_the_allocating_entry_point(ctx, orc, first, se
     both(ctx, orc, *second, seed=907, with_d=False)
 
 
+# many rows: the blocked kernel (fits the array behind it; K in one part, in parts, and an array's limit exactly reached)
+@pytest.mark.parametrize("fmt,m,k,n", [(Q4, 512, 1024, 8192), (Q8, 77, 2048, 9000), (Q8, 512, 2048, 2048)])
+def test_static_entry_runs_the_blocked_kernel_where_the_plain_one_does(ctx, orc, fmt, m, k, n):
+    assert capi.matmul_block_plan(fmt, m, k, n).taken
+    assert capi.matmul_plan(fmt, m, k, n).workspace_bytes <= capi.STATIC_WORKSPACE_BYTES
+    both(ctx, orc, fmt, m, k, n, seed=951, with_d=True)
+
+
 def test_static_workspace_tolerates_what_an_earlier_call_left(ctx, orc):
     """All contexts of a device share the static array and it keeps the last call's contents.  A
     call that gave up half-way (forced here with a zero spin limit) leaves partial sums behind and
