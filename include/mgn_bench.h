@@ -39,6 +39,14 @@ typedef struct mgn_block_plan {
 mgn_status mgn_matmul_q_block_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus,
                                    mgn_block_plan* out);
 
+/* What the automatic choice really launches for a shape, the two cases included in which mgn_matmul_q_plan (arguments as
+ * there) describes the kernel behind it.  Q8 weights with f32 activations of 33 to 127 rows: the resident
+ * form where the choice takes it.  Shapes of the blocked kernel: route MGN_ROUTE_BLOCK_MFMA, grid = (K parts, column groups,
+ * row groups), waves_n = 32-column tiles per workgroup, quads_per_wave = launches over blocks of rows, full_steps = row
+ * tiles of 32 rows per workgroup, and the rest as for the tiled routes or 0. */
+mgn_status mgn_matmul_q_auto_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus,
+                                  mgn_plan_info* out);
+
 /* How many times a wave polls for another workgroup's partial sums before it gives up (kernels whose
  * K parts meet without counters; default 2^20, far beyond any wait of a healthy launch).  With 0 a
  * reading wave looks at nothing and gives up at once, which is how a test makes that path run: the

@@ -249,13 +249,14 @@ mgn_status mgn_matmul_q_at(mgn_ctx* ctx, const mgn_buf* a_t, const mgn_weight* w
                            uint32_t m, const mgn_unary* ops, size_t n_ops);
 
 /* What mgn_matmul_q would launch for a shape, without a device: the kernel family the
- * automatic choice takes (the analogue of reading compile.rs:1390 and runtime.rs:1634 for the
- * reference) and the launch geometry.  For logs, and for checking the planner on the host.
+ * automatic choice takes among those that need no workspace prepared (the analogue of reading compile.rs:1390 and
+ * runtime.rs:1634 for the reference) and the launch geometry; mgn_matmul_q_auto_plan in mgn_bench.h has the choice
+ * among all of them.  For logs, and for checking the planner on the host.
  * `num_cus` is the device's compute-unit count (256 on MI355X); the workspace is assumed to be
  * the one every context owns.  a_is_f16: 0 = f32 activations of any magnitude (a context's
  * default), 1 = fp16 activations, 2 = f32 activations promised to lie in the fp16 range
  * (MGN_ACT_FP16_RANGE).  MGN_EINVAL for shapes no weight can have.  For the many-row shapes that the
- * blocked kernel takes (mgn_matmul_q_block_plan in mgn_bench.h tells), this is the kernel behind it. */
+ * blocked kernel takes, this is the kernel behind it. */
 typedef struct mgn_plan_info {
   int route;              /* mgn_route (never MGN_ROUTE_AUTO) */
   uint32_t grid[3];       /* workgroups: GEMV (column groups, K parts, 1); tiled routes (K parts, column groups, row
@@ -278,7 +279,7 @@ typedef struct mgn_plan_info {
 } mgn_plan_info;
 /* (Q8 weights with f32 activations of 33 to 127 rows: the plan of the general tiled kernel, which a forced
  * MGN_ROUTE_TILE_MFMA runs; the automatic choice takes the form with LDS-resident images where K has at most
- * four parts.) */
+ * four parts and their sums take at most 4 MiB.) */
 mgn_status mgn_matmul_q_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus,
                              mgn_plan_info* out);
 

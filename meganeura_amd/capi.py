@@ -18,7 +18,7 @@ STATIC_WORKSPACE_BYTES = 4 << 20  # MGN_STATIC_WORKSPACE_BYTES
 ROUTE_AUTO, ROUTE_GENERIC, ROUTE_GEMV_VALU, ROUTE_GEMV_MFMA, ROUTE_GEMM_MFMA, ROUTE_TILE_MFMA, ROUTE_BLOCK_MFMA = range(7)
 
 # every symbol include/mgn_hip.h, include/mgn_bench.h and include/mgn_session.h declare
-BENCH_SYMBOLS = ["mgn_ctx_set_route", "mgn_matmul_q_block_plan", "mgn_ctx_set_spin_limit", "mgn_engine_clock_mhz", "mgn_matmul_q_loop", "mgn_weight_read_loop"]
+BENCH_SYMBOLS = ["mgn_ctx_set_route", "mgn_matmul_q_block_plan", "mgn_matmul_q_auto_plan", "mgn_ctx_set_spin_limit", "mgn_engine_clock_mhz", "mgn_matmul_q_loop", "mgn_weight_read_loop"]
 HIP_SYMBOLS = [
     "mgn_ctx_create", "mgn_ctx_destroy", "mgn_last_error", "mgn_sync", "mgn_ctx_set_activation_range", "mgn_ctx_set_shared_device",
     "mgn_buf_alloc", "mgn_buf_free", "mgn_buf_size", "mgn_buf_device_ptr", "mgn_buf_upload",
@@ -122,6 +122,7 @@ def load():
         "mgn_matmul_q_at": (C.c_int, [vp, vp, vp, vp, vp, C.c_uint32, vp, C.c_size_t]),
         "mgn_matmul_q_plan": (C.c_int, [C.c_int, C.c_uint32, C.c_uint64, C.c_uint64, C.c_int, C.c_int, vp]),
         "mgn_matmul_q_block_plan": (C.c_int, [C.c_int, C.c_uint32, C.c_uint64, C.c_uint64, C.c_int, C.c_int, vp]),
+        "mgn_matmul_q_auto_plan": (C.c_int, [C.c_int, C.c_uint32, C.c_uint64, C.c_uint64, C.c_int, C.c_int, vp]),
         "mgn_matmul_q_loop": (C.c_int, [vp, vp, C.c_int, vp, C.c_size_t, vp, vp, C.c_uint32, C.c_uint32]),
         "mgn_weight_read_loop": (C.c_int, [vp, vp, C.c_size_t, C.c_uint32, C.c_int]),
         "mgn_matmul_q_rms_norm": (C.c_int, [vp, vp, vp, C.c_float, vp, vp, vp, C.c_uint32]),
@@ -197,11 +198,11 @@ class PlanInfo(C.Structure):
                 ("workspace_bytes", C.c_uint64)]
 
 
-def matmul_plan(fmt, m, k, n, a_is_f16=False, num_cus=256, fp16_range=False):
-    """What mgn_matmul_q would launch for this shape (no device needed).  fp16_range: f32
-    activations on a context set to ACT_FP16_RANGE."""
+def matmul_plan(fmt, m, k, n, a_is_f16=False, num_cus=256, fp16_range=False, auto=False):
+    """What mgn_matmul_q would launch for this shape (no device needed): among the kernels that need no workspace
+    prepared, or with auto=True among all of them.  fp16_range: f32 activations on a context set to ACT_FP16_RANGE."""
     info = PlanInfo()
-    st = load().mgn_matmul_q_plan(fmt, m, k, n, 1 if a_is_f16 else 2 if fp16_range else 0, num_cus, C.byref(info))
+    st = (load().mgn_matmul_q_auto_plan if auto else load().mgn_matmul_q_plan)(fmt, m, k, n, 1 if a_is_f16 else 2 if fp16_range else 0, num_cus, C.byref(info))
     if st != OK:
         raise MgnError(st, "matmul_plan: no weight has this shape")
     return info

@@ -1024,15 +1024,37 @@ static bool planned_args(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_
   return true;
 }
 
+// The plan of the kernel that `route` names (the scalar ones have none beside their name).
+static void describe_route(const mgn::LaunchArgs& x, mgn_route route, mgn_plan_info* out) {
+  if (route == MGN_ROUTE_GEMV_MFMA && mgn::describe_gemv_mfma(x, out)) return;
+  if (route == MGN_ROUTE_GEMM_MFMA && mgn::describe_gemm_mfma(x, out)) return;
+  if (route == MGN_ROUTE_TILE_MFMA && mgn::describe_tile_mfma(x, out)) return;
+  out->route = route;
+}
+
 mgn_status mgn_matmul_q_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus, mgn_plan_info* out) {
   mgn::LaunchArgs x{};
   if (!out || !planned_args(fmt, m, k, n, a_is_f16, num_cus, &x)) return MGN_EINVAL;
   *out = mgn_plan_info{};
-  const mgn_route route = basic_route(x, a_is_f16 == 0);
-  if (route == MGN_ROUTE_GEMV_MFMA && mgn::describe_gemv_mfma(x, out)) return MGN_OK;
-  if (route == MGN_ROUTE_GEMM_MFMA && mgn::describe_gemm_mfma(x, out)) return MGN_OK;
-  if (route == MGN_ROUTE_TILE_MFMA && mgn::describe_tile_mfma(x, out)) return MGN_OK;
+  describe_route(x, basic_route(x, a_is_f16 == 0), out);
+  return MGN_OK;
+}
+
+mgn_status mgn_matmul_q_auto_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus, mgn_plan_info* out) {
+  mgn::LaunchArgs x{};
+  if (!out || !planned_args(fmt, m, k, n, a_is_f16, num_cus, &x)) return MGN_EINVAL;
+  *out = mgn_plan_info{};
+  x.resident_q8 = true;
+  const mgn_route route = auto_route(x, a_is_f16 == 0);
+  mgn_block_plan b{};
+  if (route != MGN_ROUTE_BLOCK_MFMA || !mgn::describe_block_mfma(x, &b)) {
+    describe_route(x, route, out);
+    return MGN_OK;
+  }
   out->route = route;
+  out->grid[0] = out->k_parts = b.k_parts, out->grid[1] = b.col_groups, out->grid[2] = b.row_groups;
+  out->threads = b.threads, out->lds_bytes = b.lds_bytes, out->workspace_bytes = b.workspace_bytes;
+  out->waves_n = b.cols / 32, out->full_steps = b.rows / 32, out->quads_per_wave = b.launches;
   return MGN_OK;
 }
 

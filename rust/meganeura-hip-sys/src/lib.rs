@@ -188,7 +188,8 @@ pub mod bench {
     #[link(name = "mgn_hip")]
     extern "C" {
         pub fn mgn_matmul_q_block_plan(fmt: mgn_fmt, m: u32, k: u64, n: u64, a_is_f16: c_int, num_cus: c_int, out: *mut mgn_block_plan) -> mgn_status;
-    pub fn mgn_ctx_set_route(ctx: *mut mgn_ctx, route: mgn_route) -> mgn_status;
+        pub fn mgn_matmul_q_auto_plan(fmt: mgn_fmt, m: u32, k: u64, n: u64, a_is_f16: c_int, num_cus: c_int, out: *mut mgn_plan_info) -> mgn_status;
+        pub fn mgn_ctx_set_route(ctx: *mut mgn_ctx, route: mgn_route) -> mgn_status;
         pub fn mgn_ctx_set_spin_limit(ctx: *mut mgn_ctx, polls: u32) -> mgn_status;
         pub fn mgn_engine_clock_mhz(ctx: *mut mgn_ctx, loaded: c_int, mhz: *mut f32, cycles_per_round: *mut f32) -> mgn_status;
         pub fn mgn_matmul_q_loop(ctx: *mut mgn_ctx, a: *const mgn_buf, a_is_f16: c_int, weights: *const *const mgn_weight, count: usize, d: *const mgn_buf, c: *mut mgn_buf, m: u32, steps: u32) -> mgn_status;

@@ -20,6 +20,7 @@ thread_local int current = 0;
 thread_local hipError_t last = hipSuccess;
 std::map<const void*, std::string> kernels;
 std::map<std::string, long> launched;
+std::string launches;  // the names of all launches, in order, one a line
 std::map<uintptr_t, std::pair<size_t, int>> pinned;  // pinned host memory: bytes, device
 size_t refused_bytes = 0;  // allocations of exactly this size fail
 
@@ -71,6 +72,11 @@ void operator delete(void* p, size_t) noexcept { std::free(p); }
 extern "C" {
 void fake_refuse_allocations_of(size_t bytes) { refused_bytes = bytes; }
 void fake_fail_allocation(long n) { failing_new = n; }
+const char* fake_launch_log() {  // since the last time it was asked for
+  LOCK;
+  static std::string given;
+  return given.swap(launches), launches.clear(), given.c_str();
+}
 long fake_launches(const char* part_of_name) {
   LOCK;
   long n = 0;
@@ -166,10 +172,11 @@ hipError_t hipMemcpyAsync(void* d, const void* src, size_t n, hipMemcpyKind kind
   if (host && !is_pinned(host)) s->run_to(s->queued);  // pageable memory is staged before the call returns
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t, hipStream_t s) {
   LOCK;
   const std::string& name = kernels[f];
   launched[name]++;
+  launches += name + " " + std::to_string(grid.x) + " " + std::to_string(grid.y) + " " + std::to_string(grid.z) + " " + std::to_string(block.x) + "\n";
   if (name.find("copy_bytes_kernel") != std::string::npos) {
     void *dst = *(void**)args[0], *src = *(void**)args[1];
     const size_t n = (size_t)*(uint32_t*)args[2] * 16 + *(uint32_t*)args[3];

@@ -29,6 +29,7 @@ def on(runtime, program):
         hip = ctypes.CDLL("libamdhip64.so.7")
         assert hasattr(hip, "fake_launches"), "not the stand-in"
         hip.fake_refuse_allocations_of.argtypes = [ctypes.c_size_t]
+        hip.fake_launch_log.restype = ctypes.c_char_p
         def current():
             d = ctypes.c_int()
             hip.hipGetDevice(ctypes.byref(d))
@@ -102,4 +103,49 @@ def test_a_context_without_room_for_the_blocked_kernel(runtime, fmt):
                 assert False, "a kernel that has no workspace"
             except capi.MgnError as e:
                 assert e.status == capi.EINVAL
+    """)
+
+
+def test_the_automatic_plan_is_what_is_launched(runtime):
+    """mgn_matmul_q_auto_plan against the launches of the calls themselves: the kernel, its grid and its threads, in every range of rows,
+    for both formats and all three kinds of activations."""
+    on(runtime, """
+        KERNELS = {capi.ROUTE_GEMV_MFMA: "gemv", capi.ROUTE_GEMM_MFMA: "gemm_mfma_kernel", capi.ROUTE_TILE_MFMA: "tile_", capi.ROUTE_BLOCK_MFMA: "12block_kernel"}
+        seen = set()
+        with capi.Context(0) as ctx:
+            a, c = ctx.buffer(520 * 4096 * 4), ctx.buffer(520 * 14336 * 4)
+            for fmt in (0, 1):
+                for k, n in ((576, 1536), (1024, 3072), (2048, 2048), (4096, 4096), (4096, 14336), (4096, 1000)):
+                    w = ctx.weight_from_packed(fmt, np.zeros(capi.packed_size(fmt, k, n), np.uint8), k, n)
+                    for m in (1, 4, 5, 16, 17, 33, 40, 64, 96, 127, 128, 200, 512):
+                        for act in ("any", "f16", "range"):
+                            ctx.set_activation_range(act == "range")
+                            hip.fake_launch_log()
+                            (ctx.matmul_q_f16a if act == "f16" else ctx.matmul_q)(a, w, c, m)
+                            log = [l.split() for l in hip.fake_launch_log().decode().splitlines()]
+                            p = capi.matmul_plan(fmt, m, k, n, act == "f16", fp16_range=act == "range", auto=True)
+                            where = (fmt, m, k, n, act, p.route, log)
+                            main = [l for l in log if KERNELS[p.route] in l[0]]
+                            assert main and all(int(l[4]) == p.threads for l in main), where
+                            wgs = p.grid[0] * p.grid[1] * p.grid[2]
+                            got = sum(int(l[1]) * int(l[2]) * int(l[3]) for l in main)
+                            kind = p.route
+                            if p.route == capi.ROUTE_TILE_MFMA:
+                                kind = "resident" if p.quads_per_wave == 0 else "general"
+                                assert ("tile_resident_kernel" in main[0][0]) == (kind == "resident"), where
+                            if p.route == capi.ROUTE_BLOCK_MFMA:
+                                tiles = p.grid[1] * p.grid[2]
+                                assert got == -(-tiles // 8) * 8 * p.grid[0] and p.quads_per_wave == 1, where
+                                assert (p.k_parts > 1) == any("add_parts" in l[0] for l in log), where
+                                b = capi.matmul_block_plan(fmt, m, k, n, act == "f16")
+                                assert b.taken and (b.row_groups, b.col_groups, b.k_parts) == (p.grid[2], p.grid[1], p.grid[0]), where
+                            elif kind == "resident" and p.k_parts > 1:
+                                assert got == -(-p.grid[1] * p.grid[2] // 8) * 8 * p.grid[0], where
+                            elif kind != "general" or p.quads_per_wave == 1:
+                                assert got == wgs, where
+                            seen.add((kind, fmt, act))
+                    w.free()
+            resident_q8 = capi.matmul_plan(1, 64, 1024, 3072, auto=True)
+            assert resident_q8.quads_per_wave == 0 and capi.matmul_plan(1, 64, 1024, 3072).quads_per_wave > 0
+        assert len({s[0] for s in seen}) >= 4, seen
     """)
