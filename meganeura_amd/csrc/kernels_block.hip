@@ -30,7 +30,7 @@
 // times its issue cycles (LDS and barrier waits).
 #include <algorithm>
 #include <cmath>
-
+#include <cstring>
 #include <type_traits>
 #include <utility>
 
@@ -807,22 +807,34 @@ constexpr uint32_t kStreamStages = 4;
 
 struct BlockPlan {
   const BlockConfig* cfg;
-  uint32_t rows_per_launch, rowgroups, colgroups, parts, stages, nslices, mpad;
+  uint32_t rows_per_launch = 0, rowgroups, colgroups, parts, stages, nslices, mpad;
   size_t a_bytes, means_bytes, inv_bytes, partial_bytes;  // in the workspace, in this order (row scales and flags behind inv)
-  double us;
+  double us = 0;
 };
+constexpr double kNoLimit = 1e30;
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-bool plan_block_rows(const LaunchArgs& x, uint32_t m, BlockPlan* out) {
+// The best plan for m rows that is expected to take less than limit_us.  kNone: no shape of workgroup serves them; kSlow:
+// none in that time.  A caller that weighs the kernel against another one pays for the search on calls that end up elsewhere
+// too, so what cannot beat the limit, or the best plan so far, is left out by bounds from below: a shape by its
+// rounds' share of the work, K parts by their traffic.  (Host time of a call with a runtime that does nothing, without
+// this kernel, searched whole, with the bounds, us: 128 x 1024 x 3072 1.2, 1.7 (Q8 2.0), 1.35; 77 x 4096 x 14336, which it
+// takes, 3.4, 7.0, 3.9 with one search for choice and launch.)
+enum class Found { kNone, kSlow, kPlan };
+Found plan_block_rows(const LaunchArgs& x, uint32_t m, double limit_us, BlockPlan* out) {
   const bool f32a = !x.a_is_f16;
   const uint64_t k = x.w.k, n = x.w.n;
   const uint32_t bpc = x.w.k / 32, sb = stage_blocks(x.w.fmt);
   const uint32_t stages = (bpc + sb - 1) / sb, nslices = (bpc + 7) / 8;
-  if (m == 0 || bpc == 0 || nslices > kMaxSlices) return false;
-  if (n * bpc * 32 >= (1ull << 32)) return false;  // a lane's weight offsets are 32-bit
+  if (m == 0 || bpc == 0 || nslices > kMaxSlices) return Found::kNone;
+  if (n * bpc * 32 >= (1ull << 32)) return Found::kNone;  // a lane's weight offsets are 32-bit
   const BlockConfig* const cfgs = block_configs(x.w.fmt, f32a);
-  double best = 0;
+  const double outputs = (double)m * n * 4;
+  const double mem = (double)bpc * n * (x.w.fmt == MGN_FMT_Q4 ? 20 : 34) / 5.0e6 + outputs / 4.0e6;
+  const double fixed = 3.5 + outputs / 8.0e6 + 2.2 + (double)m * k * (f32a ? 8 : 2) / 5.0e6;
+  double best = limit_us;
+  Found found = Found::kNone;
   for (int i = 0; i < kBlockConfigs; i++) {
     const BlockConfig& c = cfgs[i];
     if (!c.kernel) break;
@@ -835,7 +847,14 @@ bool plan_block_rows(const LaunchArgs& x, uint32_t m, BlockPlan* out) {
     if (a_read >= (1ull << 32)) continue;
     const size_t means = has_additive(x.w.fmt, f32a) ? align256((size_t)nslices * 8 * mpad * 4 + 4096) : 0;
     const size_t inv = f32a ? align256((size_t)nslices * mpad * 4 + (size_t)mpad * 8) : 0;
+    if (stages < c.streams * kStreamStages && c.streams > 1) continue;
+    if (a_bytes + means + inv > x.block_ws_bytes) continue;
+    if (found == Found::kNone) found = Found::kSlow;
+    // (nk of a part times its rounds is never less than all of K times the tiles' share of a round, and no round costs less than tn)
+    if (0.999 * ((double)stages * sb / 4.0 * c.tn * tiles / x.num_cus + fixed) >= best) continue;
     for (uint32_t parts = 1; parts <= stages && parts <= 32; parts++) {
+      const double adding = parts > 1 ? 3.5 + (2.0 * parts + 1) * outputs / 5.0e6 : 0.0;
+      if (0.999 * (std::max(mem, c.t1 * sb / 4.0) + fixed + adding) >= best) break;
       const uint32_t spp = (stages + parts - 1) / parts;
       if ((stages + spp - 1) / spp != parts) continue;  // same split, already seen
       if (spp < c.streams * kStreamStages && c.streams > 1) break;
@@ -844,28 +863,25 @@ bool plan_block_rows(const LaunchArgs& x, uint32_t m, BlockPlan* out) {
       const uint64_t wgs = tiles * parts;
       const double nk = (spp + c.streams - 1) / c.streams * c.streams * (double)sb / 4.0;
       const double rounds = std::ceil((double)wgs / x.num_cus);
-      double us = nk * (c.t1 + (rounds - 1) * c.tn) + (c.streams > 1 ? rounds : 0.0);  // (the streams' meeting)
-      const double mem = (double)bpc * n * (x.w.fmt == MGN_FMT_Q4 ? 20 : 34) / 5.0e6 + (double)m * n * 4 / 4.0e6;
-      us = std::max(us, mem) + 3.5 + (double)m * n * 4 / 8.0e6;
-      if (parts > 1) us += 3.5 + (2.0 * parts + 1) * m * n * 4 / 5.0e6;
-      us += 2.2 + (double)m * k * (f32a ? 8 : 2) / 5.0e6;
-      if (best == 0 || us < best) {
+      const double us = std::max(nk * (c.t1 + (rounds - 1) * c.tn) + (c.streams > 1 ? rounds : 0.0), mem) + fixed + adding;  // (rounds: the streams' meeting)
+      if (us < best) {
         best = us;
+        found = Found::kPlan;
         *out = BlockPlan{&c, m, rowgroups, (uint32_t)colgroups, parts, stages, nslices, mpad, a_bytes, means, inv, partial, us};
       }
     }
   }
-  return best != 0;
+  return found;
 }
 
 // As many rows per launch as the workspace has room for: all of them, or blocks of rows one after the other.
-bool plan_block(const LaunchArgs& x, BlockPlan* out) {
+bool plan_block(const LaunchArgs& x, double limit_us, BlockPlan* out) {
   if (!x.block_ws || x.n_more != 0 || x.pro_kind != kProNone) return false;
   for (uint32_t rows = x.m;;) {
-    if (plan_block_rows(x, rows, out)) {
-      out->us *= (x.m + rows - 1) / rows;
-      return true;
-    }
+    const uint32_t launches = (x.m + rows - 1) / rows;
+    const Found f = plan_block_rows(x, rows, limit_us / launches, out);
+    out->us *= launches;
+    if (f != Found::kNone) return f == Found::kPlan;
     if (rows <= 256) return false;
     rows = (rows / 2 + 255) / 256 * 256;
   }
@@ -936,19 +952,17 @@ int launch_block_rows(ihipStream_t* s, const LaunchArgs& x, const BlockPlan& p) 
 
 }  // namespace
 
-bool block_mfma_supported(const LaunchArgs& x) {
+bool choose_block_mfma(const LaunchArgs& x, double limit_us, BlockChoice* out) {
+  static_assert(sizeof(BlockPlan) <= sizeof out->plan && std::is_trivially_copyable_v<BlockPlan>, "a plan travels in a choice");
   BlockPlan p;
-  return plan_block(x, &p);
+  if (!plan_block(x, limit_us > 0 ? limit_us : kNoLimit, &p)) return false;
+  std::memcpy(out->plan, &p, sizeof p);
+  return true;
 }
 
-double block_mfma_us(const LaunchArgs& x) {
+int launch_matmul_block_mfma(ihipStream_t* s, const LaunchArgs& x, const BlockChoice& choice) {
   BlockPlan p;
-  return plan_block(x, &p) ? p.us : 0.0;
-}
-
-int launch_matmul_block_mfma(ihipStream_t* s, const LaunchArgs& x) {
-  BlockPlan p;
-  if (!plan_block(x, &p)) return (int)hipErrorInvalidValue;
+  std::memcpy(&p, choice.plan, sizeof p);
   const uint32_t rows = p.rows_per_launch;
   for (uint32_t r0 = 0; r0 < x.m; r0 += rows) {
     LaunchArgs y = x;
@@ -956,7 +970,7 @@ int launch_matmul_block_mfma(ihipStream_t* s, const LaunchArgs& x) {
     y.a = (const char*)x.a + (size_t)r0 * x.w.k * (x.a_is_f16 ? 2 : 4);
     y.c = x.c + (size_t)r0 * x.w.n;
     y.d = x.d ? x.d + (size_t)r0 * x.w.n : nullptr;
-    if (y.m != rows && !plan_block_rows(y, y.m, &p)) return (int)hipErrorInvalidValue;
+    if (y.m != rows && plan_block_rows(y, y.m, kNoLimit, &p) != Found::kPlan) return (int)hipErrorInvalidValue;
     const int e = x.w.fmt == MGN_FMT_Q4 ? launch_block_rows<MGN_FMT_Q4>(s, y, p) : launch_block_rows<MGN_FMT_Q8>(s, y, p);
     if (e) return e;
   }
@@ -965,7 +979,7 @@ int launch_matmul_block_mfma(ihipStream_t* s, const LaunchArgs& x) {
 
 bool describe_block_mfma(const LaunchArgs& x, mgn_block_plan* out) {
   BlockPlan p;
-  if (!plan_block(x, &p)) return false;
+  if (!plan_block(x, kNoLimit, &p)) return false;
   out->rows = p.cfg->rows, out->cols = p.cfg->cols, out->threads = p.cfg->threads, out->lds_bytes = (uint32_t)p.cfg->lds;
   out->row_groups = p.rowgroups, out->col_groups = p.colgroups, out->k_parts = p.parts;
   out->launches = (x.m + p.rows_per_launch - 1) / p.rows_per_launch;

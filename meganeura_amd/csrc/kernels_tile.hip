@@ -1626,7 +1626,7 @@ bool tile_rows_supported(const LaunchArgs& x) {
 
 int launch_tile_rows(ihipStream_t* s, const LaunchArgs& x) {
   ResidentPlan p;
-  if (!tile_rows_supported(x) || !use_resident(x, &p)) return (int)hipErrorInvalidValue;
+  if (!use_resident(x, &p)) return (int)hipErrorInvalidValue;  // (the caller has asked tile_rows_supported)
   if (x.w.fmt == MGN_FMT_Q4) return p.q == 1 ? launch_resident_rows<MGN_FMT_Q4, 1>(s, x, p) : launch_resident_rows<MGN_FMT_Q4, 2>(s, x, p);
   return p.q == 1 ? launch_resident_rows<MGN_FMT_Q8, 1>(s, x, p) : launch_resident_rows<MGN_FMT_Q8, 2>(s, x, p);
 }

@@ -155,12 +155,11 @@ double basic_us(const mgn::LaunchArgs& x, mgn_route route) {
 // besides, but multiplies two to three times as fast: f32 512 x 4096 x 14336 295 -> 123 us, fp16 2048 x 4096 x
 // 14336 527 -> 283, 77 x 14336 x 4096 83 -> 47 with Q8, while 128 x 1024 x 3072 stays at 10 against 15.  Its own estimate
 // is made for weights that come from memory, the fit above for weights in the caches: hence 0.92.
-// Of the 480 calls 22 end up on a kernel more than 6 % slower than the better one.)
-mgn_route auto_route(const mgn::LaunchArgs& x, bool any_magnitude) {
+// Of the 480 calls 22 end up on a kernel more than 6 % slower than the better one.)  `choice`: the plan, if it does.
+mgn_route auto_route(const mgn::LaunchArgs& x, bool any_magnitude, mgn::BlockChoice* choice) {
   const mgn_route basic = basic_route(x, any_magnitude);
   if (x.m <= 16 || (x.m <= 32 && x.w.fmt == MGN_FMT_Q4)) return basic;
-  const double us = mgn::block_mfma_us(x);
-  return us > 0 && us * 0.92 < basic_us(x, basic) ? MGN_ROUTE_BLOCK_MFMA : basic;
+  return mgn::choose_block_mfma(x, basic_us(x, basic) / 0.92, choice) ? MGN_ROUTE_BLOCK_MFMA : basic;
 }
 
 // After the stream has been synchronised: did a wave give up waiting for another workgroup's
@@ -766,7 +765,11 @@ static mgn_status matmul_impl(mgn_ctx* ctx, const mgn_buf* a, bool a_is_f16, con
     route = MGN_ROUTE_GEMV_MFMA;
   }
   x.resident_q8 = route == MGN_ROUTE_AUTO;
-  if (route == MGN_ROUTE_AUTO) route = auto_route(x, ctx->any_magnitude);
+  mgn::BlockChoice block;
+  if (route == MGN_ROUTE_AUTO)
+    route = auto_route(x, ctx->any_magnitude, &block);
+  else if (route == MGN_ROUTE_BLOCK_MFMA && !mgn::choose_block_mfma(x, 0, &block))
+    return fail(ctx, MGN_EINVAL, "BLOCK_MFMA route does not support this shape");
   if (static_workspace) {
     // Same plan as the allocating entry point (the planners see the same workspace limits), run
     // on the library's static array if the plan's partial sums fit it; refused otherwise.  (Of the shapes that the
@@ -824,8 +827,7 @@ static mgn_status matmul_impl(mgn_ctx* ctx, const mgn_buf* a, bool a_is_f16, con
       rc = mgn::launch_matmul_gemm_mfma(ctx->stream, x);
       break;
     case MGN_ROUTE_BLOCK_MFMA:
-      if (!mgn::block_mfma_supported(x)) return fail(ctx, MGN_EINVAL, "BLOCK_MFMA route does not support this shape");
-      rc = mgn::launch_matmul_block_mfma(ctx->stream, x);
+      rc = mgn::launch_matmul_block_mfma(ctx->stream, x, block);
       break;
     default:
       rc = mgn::launch_matmul_generic(ctx->stream, x);
@@ -866,8 +868,8 @@ mgn_status mgn_matmul_q_swiglu(mgn_ctx* ctx, const mgn_buf* gate_up, const mgn_w
   return matmul_impl(ctx, gate_up, false, w, d, c, m, mgn::kProSwiglu);
 }
 
-// The launch arguments of up to three matmuls that share their activations, checked.  MGN_OK with m == 0:
-// there is nothing to launch.
+// The launch arguments of up to three matmuls that share their activations, checked, into *out as it was
+// constructed.  MGN_OK with m == 0: there is nothing to launch.
 static mgn_status batch_args(mgn_ctx* ctx, const mgn_buf* a, mgn_prologue prologue, const mgn_buf* norm_weight, float eps,
                              const mgn_matmul_item* items, size_t count, uint32_t m, mgn::LaunchArgs* out) {
   if (!ctx || !a || !items) return fail(ctx, MGN_EINVAL, "null argument");
@@ -883,8 +885,8 @@ static mgn_status batch_args(mgn_ctx* ctx, const mgn_buf* a, mgn_prologue prolog
   if (prologue == MGN_PROLOGUE_RMS_NORM && (!norm_weight || norm_weight->bytes / 4 < k))
     return fail(ctx, MGN_EINVAL, "norm weight is missing or shorter than K floats");
   mgn::LaunchArgs& x = *out;
-  x = mgn::LaunchArgs{view_of(w0), a->ptr, items[0].d ? (const float*)items[0].d->ptr : nullptr, (float*)items[0].c->ptr, m,
-                    false, ctx->num_cus};
+  x.w = view_of(w0), x.a = a->ptr, x.d = items[0].d ? (const float*)items[0].d->ptr : nullptr, x.c = (float*)items[0].c->ptr, x.m = m;
+  x.num_cus = ctx->num_cus;
   for (size_t j = 0; j < count; j++) {
     const mgn_matmul_item& it = items[j];
     if (it.w->rows != k || it.w->fmt != w0->fmt) return fail(ctx, MGN_EINVAL, "batched weights must share K and the format");
@@ -941,9 +943,10 @@ bool rows_plans(const mgn_ctx* ctx, const mgn_weight* const* ws, size_t count, u
   if (!ctx || !ws || count == 0 || count > 3 || m <= 4 || ctx->route != MGN_ROUTE_AUTO) return false;
   LaunchArgs x{view_of(ws[0]), nullptr, nullptr, nullptr, m, false, ctx->num_cus};
   rows_args(ctx, &x);
+  BlockChoice block;
   for (size_t j = 0; j < count; j++) {
     x.w = view_of(ws[j]);
-    if (auto_route(x, ctx->any_magnitude) != MGN_ROUTE_TILE_MFMA) return false;
+    if (auto_route(x, ctx->any_magnitude, &block) != MGN_ROUTE_TILE_MFMA) return false;
   }
   x.w = view_of(ws[0]);
   for (size_t j = 1; j < count; j++) x.more[j - 1] = {view_of(ws[j]), nullptr, nullptr};
@@ -1045,7 +1048,8 @@ mgn_status mgn_matmul_q_auto_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t 
   if (!out || !planned_args(fmt, m, k, n, a_is_f16, num_cus, &x)) return MGN_EINVAL;
   *out = mgn_plan_info{};
   x.resident_q8 = true;
-  const mgn_route route = auto_route(x, a_is_f16 == 0);
+  mgn::BlockChoice block;
+  const mgn_route route = auto_route(x, a_is_f16 == 0, &block);
   mgn_block_plan b{};
   if (route != MGN_ROUTE_BLOCK_MFMA || !mgn::describe_block_mfma(x, &b)) {
     describe_route(x, route, out);
@@ -1064,7 +1068,8 @@ mgn_status mgn_matmul_q_block_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t
   *out = mgn_block_plan{};
   if (!mgn::describe_block_mfma(x, out)) return MGN_EUNSUPPORTED;
   x.resident_q8 = true;  // (as the automatic choice has it)
-  out->taken = auto_route(x, a_is_f16 == 0) == MGN_ROUTE_BLOCK_MFMA ? 1u : 0u;
+  mgn::BlockChoice block;
+  out->taken = auto_route(x, a_is_f16 == 0, &block) == MGN_ROUTE_BLOCK_MFMA ? 1u : 0u;
   return MGN_OK;
 }
 

@@ -174,11 +174,14 @@ int launch_matmul_tile_mfma(ihipStream_t* s, const LaunchArgs& a);
 bool tile_rows_supported(const LaunchArgs& a);
 int launch_tile_rows(ihipStream_t* s, const LaunchArgs& a);
 // kernels_block.hip: the blocked kernel for many rows (32x32x16 tiles, activations prepared once per call)
-bool block_mfma_supported(const LaunchArgs& a);
-// what it is expected to take on a shape (0: not served)
-double block_mfma_us(const LaunchArgs& a);
+// A plan that was found, for the launch that follows (its form is the kernel's own).
+struct BlockChoice {
+  alignas(8) unsigned char plan[88];
+};
+// false: the kernel does not serve the call, or is not expected to in less than limit_us (0: however long it takes)
+bool choose_block_mfma(const LaunchArgs& a, double limit_us, BlockChoice* out);
 bool describe_block_mfma(const LaunchArgs& a, mgn_block_plan* out);
-int launch_matmul_block_mfma(ihipStream_t* s, const LaunchArgs& a);
+int launch_matmul_block_mfma(ihipStream_t* s, const LaunchArgs& a, const BlockChoice& choice);
 
 }  // namespace mgn
 
