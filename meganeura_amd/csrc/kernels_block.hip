@@ -785,8 +785,7 @@ const BlockConfig* block_configs(int fmt, bool f32a) {
       block_config<0, true, 1, 2, 2, 1, 3, 1>(1.65, 1.2), block_config<0, true, 3, 1, 4, 1, 2, 1, 2>(3.55, 3.3),
       block_config<0, true, 2, 1, 4, 1, 3, 1, 2>(2.45, 2.3)};
   static const BlockConfig q8_f16[kBlockConfigs] = {
-      block_config<1, false, 3, 2, 4, 2, 2, 3>(5.3, 3.5), block_config<1, false, 3, 2, 4, 2, 2, 2>(5.4, 3.8),
-      block_config<1, false, 2, 2, 4, 2, 2, 3>(4.35, 2.6), block_config<1, false, 3, 1, 4, 2, 2, 3>(3.3, 2.6),
+      block_config<1, false, 3, 2, 4, 2, 2, 3>(5.3, 3.5), block_config<1, false, 2, 2, 4, 2, 2, 3>(4.35, 2.6), block_config<1, false, 3, 1, 4, 2, 2, 3>(3.3, 2.6),
       block_config<1, false, 2, 1, 4, 2, 2, 3>(2.65, 2.2), block_config<1, false, 1, 1, 4, 2, 3, 2>(1.95, 1.9),
       block_config<1, false, 1, 2, 2, 2, 2, 3>(1.6, 1.2)};
   static const BlockConfig q8_f32[kBlockConfigs] = {
