@@ -1,6 +1,9 @@
 """The blocked many-row kernel (MGN_ROUTE_BLOCK_MFMA) against the oracle, at the edges of what it is built
 from: tiles of 32 rows and 64 columns, workgroups of 32 to 256 rows, blocks of 32 / stages of 64 or 128 / slices
 of 256 elements of K, K parts; and rows whose magnitudes change along K."""
+import os
+import re
+
 import numpy as np
 import pytest
 
@@ -43,6 +46,32 @@ def assert_rows_close(got, want, x, k):
     assert np.isfinite(got).all()
     err = np.abs(got - want)
     assert (err <= bound + 2.0**-23 * np.abs(want)).all(), float((err / bound).max())
+
+
+def mixed_rows(x):
+    """Gives rows 3 to 8 slices of very different magnitudes: a large slice in front or at the end, small ones in the middle, and the
+    three octaves around the one in which a row's scale is 1.  Returns the rows whose large part is the first 256 elements."""
+    x[3, 256:] *= np.float32(2.0**-30)
+    x[4, :-64] *= np.float32(2.0**-70)
+    x[5, 700:900] *= np.float32(1e-20)
+    for r, top in ((6, 9000.0), (7, 20000.0), (8, 40000.0)):
+        x[r] *= np.float32(top / np.abs(x[r]).max())
+        x[r, 256:] *= np.float32(2.0**-22)
+    return [3, 6, 7, 8]
+
+
+def tail_slice(k):
+    return (k - 64) // 256 * 256
+
+
+def assert_small_slices(got, want, x, dq, rows, first, last):
+    """The small slices keep their own accuracy: in column `first`, whose weights are zero over the first 256 elements, and (row 4)
+    column `last`, zero from the slice of the last 64 elements on."""
+    k = x.shape[1]
+    end = tail_slice(k)
+    assert (dq[:256, first] == 0).all() and (dq[end:, last] == 0).all()
+    assert_rows_close(got[rows, first][:, None], want[rows, first][:, None], x[rows, 256:], k)
+    assert_rows_close(got[4:5, last][:, None], want[4:5, last][:, None], x[4:5, :end], k)
 
 
 SHAPES = [(1, 32, 1), (31, 64, 63), (33, 96, 65), (32, 128, 64), (64, 160, 128), (65, 288, 257), (97, 992, 300), (129, 1056, 513),
@@ -98,10 +127,9 @@ def test_magnitudes_that_change_along_k(ctx, orc, fmt, k):
     got = run(ctx, x, wt)
     assert_rows_close(got, want, x, k)
     small = np.abs(x[[3, 4]][:, 512:]).max(axis=1)
-    zero = dq[:512, n - 1] == 0  # (Q4 carries zero blocks exactly only up to its minimum's rounding)
-    if zero.all():
-        err = np.abs(got[[3, 4], n - 1] - want[[3, 4], n - 1])
-        assert (err <= 8 * 2.0**-21 * 0.06 * np.sqrt(k) * small).all(), err / small
+    assert (dq[:512, n - 1] == 0).all()
+    err = np.abs(got[[3, 4], n - 1] - want[[3, 4], n - 1])
+    assert (err <= 8 * 2.0**-21 * 0.06 * np.sqrt(k) * small).all(), err / small
     # infinities, NaNs and magnitudes of 2^100 stay in their rows
     y = x.copy()
     y[0, 5], y[1, 700], y[2, 40] = np.inf, np.nan, np.float32(2.0**101)
@@ -222,13 +250,80 @@ def test_two_streams(ctx, orc, fmt, m, k, n):
     plan = capi.matmul_block_plan(fmt, m, k, n)
     assert (plan.threads, plan.cols, plan.rows) == (512, 256, 96 if fmt == Q8 or m == 65 else 64) and plan.k_parts > 1
     w = synth.normal(2050, k * n, 0.02).reshape(k, n)
+    w[:256, n - 1] = w[tail_slice(k):, n - 2] = 0.0
     x = synth.normal(2051, m * k).reshape(m, k)
-    x[3, 256:] *= np.float32(2.0**-30)  # rows whose sums change scale along K, each stream on its own slices
-    x[4, : k - 64] *= np.float32(2.0**-70)
-    x[5, 700:900] *= np.float32(1e-20)
+    small = mixed_rows(x)
     wt = ctx.weight(fmt, w)
-    want = x.astype(np.float64) @ orc.dequantize(fmt, orc.quantize(fmt, w), k, n).astype(np.float64)
+    dq = orc.dequantize(fmt, orc.quantize(fmt, w), k, n).astype(np.float64)
+    want = x.astype(np.float64) @ dq
     got = run(ctx, x, wt)
     assert_rows_close(got, want, x, k)
+    assert_small_slices(got, want, x, dq, small, n - 1, n - 2)
     assert np.array_equal(bits(run(ctx, x, wt)), bits(got)), "not repeatable"
     wt.free()
+
+
+# Every workgroup that is built, with K in one part and in several, at ragged sizes for which the planner takes it:
+# rows x columns x threads, then shape and parts
+WORKGROUPS = {
+    (Q4, False): [(32, 256, 256, 66, 1056, 17126, 1), (32, 256, 256, 67, 4320, 1278, 17), (64, 128, 256, 49, 736, 16625, 1), (64, 128, 256, 34, 6304, 858, 25),
+                  (64, 256, 256, 387, 736, 16657, 1), (64, 256, 256, 34, 4128, 7231, 17), (64, 256, 512, 100, 1056, 16512, 1), (64, 256, 512, 67, 30496, 797, 30),
+                  (96, 256, 256, 271, 736, 20163, 1), (96, 256, 256, 67, 4320, 3623, 17), (96, 256, 512, 844, 928, 4633, 1), (96, 256, 512, 67, 27808, 1552, 28),
+                  (128, 256, 512, 296, 736, 19594, 1), (128, 256, 512, 197, 3232, 3273, 9), (192, 256, 512, 583, 736, 13585, 1), (192, 256, 512, 130, 4192, 5476, 11),
+                  (256, 256, 512, 577, 160, 19639, 1), (256, 256, 512, 195, 3360, 8220, 7)],
+    (Q4, True): [(32, 256, 256, 67, 1056, 12824, 1), (32, 256, 256, 35, 2080, 16322, 2), (64, 128, 256, 905, 736, 2063, 1), (64, 128, 256, 34, 17440, 4091, 23),
+                 (64, 256, 256, 395, 736, 16800, 1), (64, 256, 256, 34, 19488, 4016, 31), (96, 256, 256, 199, 736, 18696, 1), (96, 256, 256, 66, 15136, 3658, 17),
+                 (128, 256, 512, 298, 736, 19605, 1), (128, 256, 512, 98, 12064, 4022, 16), (192, 256, 512, 583, 736, 13572, 1), (192, 256, 512, 163, 15840, 2549, 25),
+                 (256, 256, 512, 523, 160, 21043, 1), (256, 256, 512, 195, 17504, 2638, 23)],
+    (Q8, False): [(32, 256, 256, 51, 736, 16442, 1), (32, 256, 256, 19, 736, 133, 12), (64, 128, 256, 167, 736, 10856, 1), (64, 128, 256, 34, 6880, 1109, 27),
+                  (64, 256, 256, 115, 736, 16405, 1), (64, 256, 256, 34, 6112, 1565, 32), (96, 256, 256, 161, 160, 21882, 1), (96, 256, 256, 68, 3232, 3691, 17),
+                  (96, 256, 512, 203, 736, 16738, 1), (96, 256, 512, 67, 14368, 1293, 29), (128, 256, 512, 326, 736, 16423, 1), (128, 256, 512, 100, 2272, 5405, 9),
+                  (192, 256, 512, 400, 736, 18702, 1), (192, 256, 512, 132, 6240, 2323, 25), (256, 256, 512, 484, 160, 21765, 1), (256, 256, 512, 194, 1568, 10874, 5)],
+    (Q8, True): [(32, 256, 256, 134, 736, 13028, 1), (64, 128, 256, 98, 736, 12724, 1), (64, 128, 256, 35, 8224, 6463, 10), (64, 256, 256, 130, 736, 18829, 1),
+                 (64, 256, 256, 35, 11872, 3790, 17), (96, 256, 256, 198, 736, 17016, 1), (96, 256, 256, 66, 18016, 1977, 32), (128, 256, 512, 387, 736, 13986, 1),
+                 (128, 256, 512, 99, 13088, 2805, 23), (192, 256, 512, 388, 736, 19172, 1), (192, 256, 512, 130, 9568, 3691, 17)],
+}
+
+
+@pytest.mark.parametrize("fmt,f16,rows,cols,threads,m,k,n,parts", [kind + shape for kind, shapes in WORKGROUPS.items() for shape in shapes])
+def test_every_workgroup(ctx, orc, fmt, f16, rows, cols, threads, m, k, n, parts):
+    """Products, rows of mixed scale, infinite and NaN rows beside the others, residuals and epilogues.  The weight's columns
+    repeat after 1499 (no multiple of a tile), so that all outputs have a reference."""
+    plan = capi.matmul_block_plan(fmt, m, k, n, f16)
+    assert (plan.taken, plan.rows, plan.cols, plan.threads, plan.k_parts) == (1, rows, cols, threads, parts)
+    base = min(n, 1499)
+    w = synth.normal(2100, k * base, 0.02).reshape(k, base)
+    x = synth.normal(2101, m * k).reshape(m, k)
+    mixed = not f16 and k >= 512
+    if mixed:
+        w[:256, 5] = w[tail_slice(k):, 7] = 0.0
+        small = mixed_rows(x)
+    x = x.astype(np.float16) if f16 else x
+    wide = np.ascontiguousarray(w[:, np.arange(n) % base])
+    wt = ctx.weight(fmt, wide)
+    del wide
+    dq = orc.dequantize(fmt, orc.quantize(fmt, w), k, base).astype(np.float64)
+    want = (x.astype(np.float64) @ dq)[:, np.arange(n) % base]
+    got = run(ctx, x, wt, f16)
+    assert_rows_close(got, want, x.astype(np.float32), k)
+    if mixed:
+        assert_small_slices(got, want, x, dq, small, 5, 7)
+    y = x.copy()
+    y[0, 0], y[1, k - 1] = np.inf, np.nan
+    bad = run(ctx, y, wt, f16)
+    assert not np.isfinite(bad[:2]).any() and np.array_equal(bits(bad[2:]), bits(got[2:]))
+    d = synth.normal(2102, m * n).reshape(m, n)
+    added = run(ctx, x, wt, f16, d=d)
+    assert np.array_equal(added, got + d)
+    if not f16:
+        assert np.array_equal(run(ctx, x, wt, d=d, ops=(capi.UNARY_NEG, capi.UNARY_RELU)), np.maximum(-added, 0))
+    wt.free()
+
+
+def test_every_workgroup_is_in_the_list():
+    source = open(os.path.join(os.path.dirname(capi.__file__), "csrc", "kernels_block.hip")).read()
+    built = set()
+    for fmt, f32, numbers in re.findall(r"block_config<([01]), (true|false), ([0-9, ]+)>\(", source):
+        rt, wm, wn, _, _, _, wk = [int(v) for v in (numbers + ", 1").split(",")][:7]
+        built.add((int(fmt), f32 == "false", 32 * rt * wm, 64 * wn, 64 * wm * wn * wk))
+    assert built == {kind + shape[:3] for kind, shapes in WORKGROUPS.items() for shape in shapes} and len(built) == 30
