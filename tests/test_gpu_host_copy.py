@@ -31,19 +31,34 @@ def test_round_trip(nbytes):
 
 
 def test_ring_wraps():
-    """More uploads than the pinned ring holds, and nothing overwritten before it has travelled."""
-    with capi.Context(0) as ctx:
-        bufs = [(ctx.buffer(3 << 20), pattern(3 << 20, s)) for s in range(8)]
-        for b, want in bufs:
-            b.upload(want)
-        for b, want in bufs:
-            assert np.array_equal(b.download(np.uint8, want.size), want)
+    """Inputs go through the pinned ring without being waited for: more of them than it holds (16 MiB) in front of one step, pieces of
+    odd lengths, the caller's array changing as soon as set_input returns, and of two writes to an input the later one."""
+    m, k, count = 509, 1023, 12  # 2.08 MB each, just below the largest that takes this way
+    assert (2 << 20) - (16 << 10) < m * k * 4 <= SLOT
+    g = Graph()
+    total = g.input("x0", [m, k])
+    for i in range(1, count):
+        total = g.add(total, g.input(f"x{i}", [m, k]))
+    g.set_outputs([total])
+    s = build_inference_session(g)
+    scratch, ramp = np.empty((m, k), np.float32), np.arange(m * k, dtype=np.float32).reshape(m, k)
+    for step in range(3):
+        for round_ in range(2):
+            for i in np.random.default_rng(10 * step + round_).permutation(count):
+                scratch[:] = ramp * np.float32(i) + np.float32(step + 100 * round_)  # (whole numbers below 2^24: exact)
+                s.set_input(f"x{i}", scratch)
+                scratch[:] = -1
+        s.step()
+        s.wait()
+        want = ramp.astype(np.float64) * sum(range(count)) + count * (step + 100)
+        assert np.abs(s.read_output(m * k).reshape(m, k) - want).max() <= 2.0**-24 * count * want.max()
+    s.close()
 
 
-def test_queued_inputs():
-    """set_input returns before the bytes have arrived: the caller's array may change at once, and inputs that
-    together exceed the ring (16 MiB) still all arrive before the step."""
-    m, k = 1536, 1024  # 6 MiB each
+@pytest.mark.parametrize("m", [256, 1536])  # 1 MiB each, through the ring; 6 MiB, as the runtime copies
+def test_queued_inputs(m):
+    """set_input returns before the step that reads the bytes: the caller's array may change at once."""
+    k = 1024
     g = Graph()
     x, y = g.input("x", [m, k]), g.input("y", [m, k])
     g.set_outputs([g.add(x, y)])
