@@ -24,9 +24,9 @@
 //     waves that meet such a row move their sums from scale to scale;
 //   * K parts for different workgroups, where the tiles do not fill the chip, meet in the workspace and are added
 //     in part order by a third launch.
-// Measured (one box, weights from memory; before -> now, us): fp16 2048 x 4096 x 14336 589 -> 299 (805 TFLOP/s),
-// f32 the same 1034 -> 467; f32 512 x 4096 x 14336 295 -> 123; f32 77 x 4096 x 14336 82 -> 42, 77 x 14336 x 4096
-// 98 -> 46.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.4
+// Measured (weights from memory; before -> now, us, Q4): fp16 2048 x 4096 x 14336 589 -> 291 (827 TFLOP/s),
+// f32 the same 1034 -> 470; f32 512 x 4096 x 14336 295 -> 117; f32 77 x 4096 x 14336 82 -> 40, 77 x 14336 x 4096
+// 98 -> 43.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.4
 // times its issue cycles (LDS and barrier waits).
 #include <algorithm>
 #include <cmath>

@@ -60,7 +60,7 @@ struct LaunchArgs {
   // other work may run on the device beside this launch: no plan whose workgroups all wait for
   // each other (they would have to be resident together, and a second such kernel can take their CUs)
   bool shared_device = false;
-  // further weights served by the same launch (GEMV-MFMA route only): same K, format and
+  // further weights served by the same launch (the MFMA GEMV, and launch_tile_rows): same K, format and
   // activations, each with its own output and optional residual
   struct More {
     WeightView w;
@@ -70,7 +70,7 @@ struct LaunchArgs {
   More more[2] = {};
   int n_more = 0;
   uint32_t epilogue = 0;  // unary operations on the output, four bits each, first in the low bits
-  // fused prologue (GEMV-MFMA route only): what `a` goes through before the matmul
+  // fused prologue (the MFMA GEMV, and launch_tile_rows): what `a` goes through before the matmul
   int pro_kind = 0;                   // kProNone / kProRmsNorm / kProSwiglu
   const float* pro_weight = nullptr;  // norm weight [K]
   float pro_eps = 0.0f;
