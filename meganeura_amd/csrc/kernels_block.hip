@@ -831,7 +831,9 @@ Found plan_block_rows(const LaunchArgs& x, uint32_t m, double limit_us, BlockPla
   const BlockConfig* const cfgs = block_configs(x.w.fmt, f32a);
   const double outputs = (double)m * n * 4;
   const double mem = (double)bpc * n * (x.w.fmt == MGN_FMT_Q4 ? 20 : 34) / 5.0e6 + outputs / 4.0e6;
-  const double fixed = 3.5 + outputs / 8.0e6 + 2.2 + (double)m * k * (f32a ? 8 : 2) / 5.0e6;
+  // (f32: the workgroups that convert a row each are more than the chip holds at once beyond some 512 rows; without that term short
+  // calls of 1024 to 2048 rows measured 2 to 3 us above their estimate)
+  const double fixed = 3.5 + outputs / 8.0e6 + 2.2 + (double)m * k * (f32a ? 8 : 2) / 5.0e6 + (f32a && m > 512 ? (m - 512) * 2.2e-3 : 0.0);
   double best = limit_us;
   Found found = Found::kNone;
   for (int i = 0; i < kBlockConfigs; i++) {

@@ -135,18 +135,24 @@ mgn_route basic_route(const mgn::LaunchArgs& x, bool any_magnitude) {
 
 // What a call of more than 16 rows takes on the kernel of basic_route, in us, fitted to 480 measured
 // calls (M = 20 .. 2048 on twelve shapes from 576 x 1536 to 14336 x 4096 and 576 x 49152, both formats, f32 and fp16
-// activations).  The resident kernel: so much per round of workgroups; the others: a fixed part and a
-// rate over the rows they compute, a multiple of 32.
-double basic_us(const mgn::LaunchArgs& x, mgn_route route) {
+// activations) and, for K below 576, to 600 more.  The resident kernel: so much per round of workgroups, less where K is
+// shorter than the four slices of 256 that a workgroup holds (measured over the four slices' time, medians by format and
+// activations: one slice 0.55 .. 0.72, two 0.79 .. 0.90, three 0.88 .. 1.08, the most with two pairs of tiles per wave); the
+// others: a fixed part and a rate over the rows they compute, a multiple of 32 (K of up to 128: 5.4 to 12 us).  *steady: the resident kernel with one
+// pair of tiles per wave.
+double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool* steady) {
   const bool q4 = x.w.fmt == MGN_FMT_Q4;
   const double flops = 2.0 * ((x.m + 31) / 32 * 32) * x.w.k * x.w.n;
-  if (route == MGN_ROUTE_GEMM_MFMA) return 7.0 + flops / (q4 ? 390e6 : 310e6);
+  *steady = false;
+  if (route == MGN_ROUTE_GEMM_MFMA) return x.w.k <= 128 ? 5.6 + flops / (x.a_is_f16 ? 175e6 : 120e6) : 7.0 + flops / (q4 ? 390e6 : 310e6);
   mgn_plan_info p{};
   if (route != MGN_ROUTE_TILE_MFMA || !mgn::describe_tile_mfma(x, &p)) return 1e9;  // scalar routes
   if (p.quads_per_wave != 0) return 9.0 + flops / (q4 ? 175e6 : 165e6);
-  const double rounds = std::ceil((double)p.grid[0] * p.grid[1] * p.grid[2] / x.num_cus), parts = p.k_parts > 1 ? 1.0 : 0.0;
+  *steady = p.full_steps != 2 && p.waves_n <= 16;
+  const double share = x.w.k <= 256 ? 0.65 : x.w.k <= 512 ? (p.waves_n <= 16 ? 0.82 : 0.9) : x.w.k <= 768 && *steady ? 0.94 : 1.0;
+  const double rounds = std::ceil((double)p.grid[0] * p.grid[1] * p.grid[2] / x.num_cus) * share, parts = p.k_parts > 1 ? 1.0 : 0.0;
   if (p.full_steps == 2) return 10.5 * rounds + parts;
-  if (p.waves_n <= 16) return (q4 ? 9.0 : 10.0) * (x.a_is_f16 ? 0.9 : 1.0) * rounds + parts;
+  if (*steady) return (q4 ? 9.0 : 10.0) * (x.a_is_f16 ? 0.9 : 1.0) * rounds + parts;
   return (q4 ? 15.5 : 22.0) * (x.a_is_f16 ? 0.9 : 1.0) * rounds + (q4 ? 1.0 : 9.0) * parts;
 }
 
@@ -156,10 +162,15 @@ double basic_us(const mgn::LaunchArgs& x, mgn_route route) {
 // 14336 527 -> 283, 77 x 14336 x 4096 83 -> 47 with Q8, while 128 x 1024 x 3072 stays at 10 against 15.  Its own estimate
 // is made for weights that come from memory, the fit above for weights in the caches: hence 0.92.
 // Of the 480 calls 22 end up on a kernel more than 6 % slower than the better one.)  `choice`: the plan, if it does.
+// Not so where the other kernel is the resident one with one pair of tiles per wave: small weights, which take it the
+// same time a round from wherever they come.  (Blocked and resident, us: Q8 f32 22 x 1760 x 1307 14.1, 11.4, 17 x 768 x 579
+// 10.1, 8.8; short K: Q4 f32 470 x 192 x 275 9.6, 6.4, Q4 fp16 145 x 160 x 105 8.6, 4.2.)
 mgn_route auto_route(const mgn::LaunchArgs& x, bool any_magnitude, mgn::BlockChoice* choice) {
   const mgn_route basic = basic_route(x, any_magnitude);
   if (x.m <= 16 || (x.m <= 32 && x.w.fmt == MGN_FMT_Q4)) return basic;
-  return mgn::choose_block_mfma(x, basic_us(x, basic) / 0.92, choice) ? MGN_ROUTE_BLOCK_MFMA : basic;
+  bool steady;
+  const double us = basic_us(x, basic, &steady);
+  return mgn::choose_block_mfma(x, steady ? us : us / 0.92, choice) ? MGN_ROUTE_BLOCK_MFMA : basic;
 }
 
 // After the stream has been synchronised: did a wave give up waiting for another workgroup's

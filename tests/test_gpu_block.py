@@ -268,14 +268,14 @@ def test_two_streams(ctx, orc, fmt, m, k, n):
 WORKGROUPS = {
     (Q4, False): [(32, 256, 256, 66, 1056, 17126, 1), (32, 256, 256, 67, 4320, 1278, 17), (64, 128, 256, 49, 736, 16625, 1), (64, 128, 256, 34, 6304, 858, 25),
                   (64, 256, 256, 387, 736, 16657, 1), (64, 256, 256, 34, 4128, 7231, 17), (64, 256, 512, 100, 1056, 16512, 1), (64, 256, 512, 67, 30496, 797, 30),
-                  (96, 256, 256, 271, 736, 20163, 1), (96, 256, 256, 67, 4320, 3623, 17), (96, 256, 512, 844, 928, 4633, 1), (96, 256, 512, 67, 27808, 1552, 28),
+                  (96, 256, 256, 271, 736, 20163, 1), (96, 256, 256, 67, 4320, 3623, 17), (96, 256, 512, 233, 928, 18803, 1), (96, 256, 512, 67, 27808, 1552, 28),
                   (128, 256, 512, 296, 736, 19594, 1), (128, 256, 512, 197, 3232, 3273, 9), (192, 256, 512, 583, 736, 13585, 1), (192, 256, 512, 130, 4192, 5476, 11),
                   (256, 256, 512, 577, 160, 19639, 1), (256, 256, 512, 195, 3360, 8220, 7)],
-    (Q4, True): [(32, 256, 256, 67, 1056, 12824, 1), (32, 256, 256, 35, 2080, 16322, 2), (64, 128, 256, 905, 736, 2063, 1), (64, 128, 256, 34, 17440, 4091, 23),
+    (Q4, True): [(32, 256, 256, 129, 96, 14369, 1), (32, 256, 256, 35, 2080, 16322, 2), (64, 128, 256, 905, 736, 2063, 1), (64, 128, 256, 34, 17440, 4091, 23),
                  (64, 256, 256, 395, 736, 16800, 1), (64, 256, 256, 34, 19488, 4016, 31), (96, 256, 256, 199, 736, 18696, 1), (96, 256, 256, 66, 15136, 3658, 17),
                  (128, 256, 512, 298, 736, 19605, 1), (128, 256, 512, 98, 12064, 4022, 16), (192, 256, 512, 583, 736, 13572, 1), (192, 256, 512, 163, 15840, 2549, 25),
                  (256, 256, 512, 523, 160, 21043, 1), (256, 256, 512, 195, 17504, 2638, 23)],
-    (Q8, False): [(32, 256, 256, 51, 736, 16442, 1), (32, 256, 256, 19, 736, 133, 12), (64, 128, 256, 167, 736, 10856, 1), (64, 128, 256, 34, 6880, 1109, 27),
+    (Q8, False): [(32, 256, 256, 51, 736, 16442, 1), (32, 256, 256, 39, 1568, 78, 25), (64, 128, 256, 167, 736, 10856, 1), (64, 128, 256, 34, 6880, 1109, 27),
                   (64, 256, 256, 115, 736, 16405, 1), (64, 256, 256, 34, 6112, 1565, 32), (96, 256, 256, 161, 160, 21882, 1), (96, 256, 256, 68, 3232, 3691, 17),
                   (96, 256, 512, 203, 736, 16738, 1), (96, 256, 512, 67, 14368, 1293, 29), (128, 256, 512, 326, 736, 16423, 1), (128, 256, 512, 100, 2272, 5405, 9),
                   (192, 256, 512, 400, 736, 18702, 1), (192, 256, 512, 132, 6240, 2323, 25), (256, 256, 512, 484, 160, 21765, 1), (256, 256, 512, 194, 1568, 10874, 5)],

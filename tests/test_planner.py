@@ -222,3 +222,22 @@ def test_shapes_no_weight_can_have_are_refused():
     for args in ((Q4, 1, 100, 8), (Q4, 0, 64, 8), (Q4, 1, 0, 8), (Q4, 1, 64, 0), (7, 1, 64, 8)):
         with pytest.raises(capi.MgnError):
             capi.matmul_plan(*args)
+
+
+@pytest.mark.parametrize("fmt,m,k,n,f16", [
+    (Q8, 17, 768, 579, False), (Q8, 32, 1920, 810, False), (Q8, 22, 1760, 1307, False), (Q8, 20, 2048, 802, False), (Q8, 82, 320, 321, False),
+    (Q4, 470, 192, 275, False), (Q4, 145, 160, 105, True), (Q4, 333, 256, 768, False), (Q8, 333, 256, 768, False), (Q4, 128, 256, 1024, True),
+    (Q4, 44, 64, 17509, False), (Q8, 818, 128, 599, True)])
+def test_small_calls_stay_with_the_kernel_that_needs_one_launch(fmt, m, k, n, f16):
+    """Short K, and Q8 of 17 to 32 rows on small weights: the blocked kernel's two or three launches take 1.1 to 2 times as long."""
+    p = capi.matmul_plan(fmt, m, k, n, f16, auto=True)
+    assert p.route == (GEMM_MFMA if fmt == Q8 and f16 else TILE_MFMA) and p.quads_per_wave == 0
+    assert not capi.matmul_block_plan(fmt, m, k, n, f16).taken
+
+
+@pytest.mark.parametrize("fmt,m,k,n,f16", [
+    (Q4, 77, 4096, 14336, False), (Q8, 77, 14336, 4096, False), (Q4, 2048, 4096, 14336, True), (Q8, 22, 3296, 14036, False), (Q4, 122, 736, 11506, False),
+    (Q8, 199, 896, 7513, False), (Q4, 454, 832, 4683, True), (Q8, 1359, 384, 2477, True), (Q8, 241, 128, 8416, True)])
+def test_large_calls_take_the_blocked_kernel(fmt, m, k, n, f16):
+    """Calls on which it measured 1.1 to 2.5 times as fast as the kernel behind it."""
+    assert capi.matmul_block_plan(fmt, m, k, n, f16).taken and capi.matmul_plan(fmt, m, k, n, f16, auto=True).route == capi.ROUTE_BLOCK_MFMA
