@@ -24,9 +24,9 @@
 //     waves that meet such a row move their sums from scale to scale;
 //   * K parts for different workgroups, where the tiles do not fill the chip, meet in the workspace and are added
 //     in part order by a third launch.
-// Measured (weights from memory; before -> now, us, Q4): fp16 2048 x 4096 x 14336 589 -> 291 (827 TFLOP/s),
-// f32 the same 1034 -> 470; f32 512 x 4096 x 14336 295 -> 117; f32 77 x 4096 x 14336 82 -> 40, 77 x 14336 x 4096
-// 98 -> 43.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.4
+// Measured (weights from memory; before -> now, us, Q4): fp16 2048 x 4096 x 14336 589 -> 268 (898 TFLOP/s),
+// f32 the same 1034 -> 453; f32 512 x 4096 x 14336 295 -> 118; f32 77 x 4096 x 14336 82 -> 39.6, 77 x 14336 x 4096
+// 98 -> 42.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.3
 // times its issue cycles (LDS and barrier waits).
 #include <algorithm>
 #include <cmath>
@@ -152,21 +152,38 @@ struct BlockShape {
   static constexpr size_t RED = WK > 1 ? (size_t)WM * WN * RT * kCT * 4096 : 0, STRIP = (size_t)WAVES * 4096;
   static constexpr size_t LDS = PIPE > RED ? (PIPE > STRIP ? PIPE : STRIP) : (RED > STRIP ? RED : STRIP);
   // A wave's loads in issue order: in substep i the activations of substep i + PD, then, where it is a
-  // stage's first, the stage SD ahead.  At its end everything that substep i + 1 reads, and the first
-  // block of i + 2, must have landed; the loads issued after the last of those may be in flight.
-  static constexpr int issued(int i) { return NAW + (i % NSUB == 0 ? NSTW : 0); }
+  // stage's first, the stage SD ahead, dealt over the substep's tiles.  The substep's barrier stands in front of
+  // tile TURN of its last block: by then a wave holds all operands of substep i that it has still to multiply, and
+  // what it reads from there to the next barrier is substep i + 1's, and that one's stage.  So these must have
+  // landed; the loads issued after the last of them may be in flight.  (With the barrier behind the last tile, the
+  // next substep's first operands had to have landed a barrier earlier: at PD = 2 the loads of the very substep that
+  // ends, and their whole latency was waited for.  us, weights from memory: Q4 fp16 2048 x 4096 x 14336 292 -> 268, f32
+  // 476 -> 453; 77 x 4096 x 14336 Q4 40.4 -> 39.6, Q8 44.5 -> 41.4; no shape measured slower.)
+  static constexpr int TILES = RT * kCT, SLOTS = SUBB * TILES;
+  static constexpr int TURN = F32A ? TILES - 1 : TILES - 2;
+  static constexpr int issued(int i) { return NAW + ((i + 64 * NSUB) % NSUB == 0 ? NSTW : 0); }
   static constexpr int since(int from, int to) {
     int n = 0;
     for (int i = from; i <= to; i++) n += issued(i);
     return n;
   }
-  static constexpr int in_flight(int u) {
-    const int i = u + 64 * NSUB;
-    const int after_a = (i + 2 - PD) % NSUB == 0 ? NSTW + since(i + 3 - PD, i) : since(i + 3 - PD, i);
-    const int after_stage = since(((i + 2) / NSUB - SD) * NSUB + 1, i);
+  static constexpr int stage_of(int i) { return (i + 64 * NSUB) / NSUB - 64; }
+  static constexpr int requested(int i) { return (stage_of(i) - SD) * NSUB; }  // the substep that asks for substep i's stage
+  static constexpr int behind_a(int i) { return (i - PD + 64 * NSUB) % NSUB == 0 ? NSTW : 0; }  // loads behind substep i's activations in the substep that asks for them
+  static constexpr int in_flight(int i) {
+    const int here = ((SUBB - 1) * TILES + TURN) * issued(i) / SLOTS;
+    const int after_a = behind_a(i + 1) + since(i + 2 - PD, i - 1) + here;
+    const int after_stage = since(requested(i + 1) + 1, i - 1) + here;
     return after_a < after_stage ? after_a : after_stage;
   }
-  static_assert(PD >= 2 && 2 / NSUB <= SD && (NSUB > 1 || SD >= 2), "what a substep waits for has been requested");
+  // In front of the loop, in the same order, what the substeps before the first would have asked for: landed must be
+  // substep 0's activations and its stage.
+  static constexpr int FIRST = -(PD > SD * NSUB ? PD : SD * NSUB);
+  static constexpr int in_flight_first() {
+    const int after_a = behind_a(0) + since(1 - PD, -1), after_stage = since(requested(0) + 1, -1);
+    return after_a < after_stage ? after_a : after_stage;
+  }
+  static_assert(PD >= 2 && requested(NSUB) < NSUB - 1, "what a substep waits for has been requested in whole");
 };
 
 template <int FMT, bool F32A, int RT, int WM, int WN, int WK, int SUBB, int PD, int SD>
@@ -267,15 +284,17 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
   const uint32_t s_rd = B_BYTES + M_BYTES + ks * MEAN_STREAM + (wm * (RT * 32) + c) * (SB * 4u) + h * (SB * 2u);
   const uint32_t addp = h ? x.add_lo : x.add_hi;
 
-  // (in the order of the loop's own requests: stages first that the first substeps read)
+  static_for<-S::FIRST>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = S::FIRST + I, a = i + PD;
+    if constexpr (a >= 0) {
 #pragma unroll
-  for (int i = 0; i < SD; i++)
+      for (int j = 0; j < NAW; j++) load_a(j, min((uint32_t)(a / NSUB), iters - 1), a % NSUB, a);
+    }
+    if constexpr ((i + 64 * NSUB) % NSUB == 0 && S::stage_of(i) + SD >= 0) {
 #pragma unroll
-    for (int j = 0; j < NSTW; j++) load_stage(j, min((uint32_t)i, iters - 1), i);
-#pragma unroll
-  for (int i = 0; i < PD; i++)
-#pragma unroll
-    for (int j = 0; j < NAW; j++) load_a(j, min((uint32_t)(i / NSUB), iters - 1), i % NSUB, i);
+      for (int j = 0; j < NSTW; j++) load_stage(j, min((uint32_t)(S::stage_of(i) + SD), iters - 1), S::stage_of(i) + SD);
+    }
+  });
   bool mixed = false;
   float row_scale[RT];  // of row c of each row tile
   if constexpr (F32A) {
@@ -287,7 +306,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
     }
     mixed = __builtin_amdgcn_ballot_w64(any != 0) != 0;
   }
-  wait_loads<(PD - 2) * NAW>();
+  wait_loads<S::in_flight_first()>();
   lds_barrier();
 
   // What is in registers ahead of its use: the raw quants of the next block, the operands of its first
@@ -360,10 +379,15 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
       }
     }
     if (!F32A && valid > 0 && valid < SB) {
-      // What the loads brought in behind the row's last block is another row's, or nothing's.  (The two
-      // substeps that a stage of fp16 activations has at most have landed; each wave clears the rows that
-      // it reads, so that its own order suffices; waves that share rows write the same zeros.)
-      static_assert(F32A || NSUB <= 2, "one substep ahead has landed");
+      // What the loads brought in behind the row's last block is another row's, or nothing's.  (Each wave clears the
+      // rows that it reads, so that its own order suffices; waves that share rows write the same zeros.  Block 0,
+      // whose first operands are in registers by now, is always the row's own.  Cleared substep by substep, behind the
+      // barriers inside the loop, the branch there costs the 128 x 64 tiles 250 spilled registers.)
+      static_assert(F32A || NSUB <= 2, "one substep ahead has been requested");
+      if constexpr (NSUB > 1) {
+        wait_loads<0>();
+        lds_barrier();
+      }
       for (uint32_t i = lane; i < NSUB * PANELS * RT * 32 * 8; i += 64) {
         const uint32_t unit = i & 7, row = i / 8 % (RT * 32), panel = i / (RT * 32 * 8);  // panels of the stage
         const uint32_t buf = abuf + panel / PANELS >= ARING ? abuf + panel / PANELS - ARING : abuf + panel / PANELS;
@@ -392,6 +416,37 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
         }
       }
     }
+    // the additive part of the stage's blocks: means times m (Q4) or the scale (Q8)
+    auto add_means = [&]() __attribute__((always_inline)) {
+      if constexpr (has_additive(FMT, F32A)) {
+        half8 bm[kCT];
+#pragma unroll
+        for (int t = 0; t < kCT; t++) {
+          uint32_t w0, w1 = 0;
+          const half2_t mulp = __builtin_bit_cast(half2_t, addp);
+          if constexpr (FMT == MGN_FMT_Q4) {
+            w0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(mcur[t][1], mcur[t][0], 0x07060302u)) * mulp);
+            w1 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(mcur[t][3], mcur[t][2], 0x07060302u)) * mulp);
+          } else {
+            w0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, mcur[t][0]) * mulp);
+          }
+          bm[t] = as_half8(w0, w1, 0u, 0u);
+        }
+        const uint8_t* const ps = lds_st + sbuf * STAGE_BYTES + s_rd;
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+          half8 am;
+          if constexpr (FMT == MGN_FMT_Q4) {
+            const uint2 v = *(const uint2*)(ps + r * (32 * SB * 4));
+            am = as_half8(v.x, v.y, 0u, 0u);
+          } else {
+            am = as_half8(*(const uint32_t*)(ps + r * (32 * SB * 4)), 0u, 0u, 0u);
+          }
+#pragma unroll
+          for (int t = 0; t < kCT; t++) acc[r][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm[t], acc[r][t], 0, 0, 0);
+        }
+      }
+    };
     static_for<NSUB>([&](auto U) __attribute__((always_inline)) {
       constexpr int u = U;
       constexpr bool last = u == NSUB - 1;
@@ -407,6 +462,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
         if constexpr (q >= NAW) load_stage(q - NAW, its, sload);
         else load_a(q, ita, usub, aload);
       };
+      if constexpr (last) add_means();
       __builtin_amdgcn_sched_barrier(0);
       static_for<SUBB>([&](auto BL) __attribute__((always_inline)) {
         constexpr int bl = BL, sb = u * SUBB + bl;
@@ -423,6 +479,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
         static_for<TILES>([&](auto TT) __attribute__((always_inline)) {
           constexpr int T = TT, r = T / kCT, t = T % kCT, pr = T ? (T - 1) / kCT : RT - 1, pt = T ? (T - 1) % kCT : kCT - 1;
           constexpr int slot = F32A ? 0 : (sb * RT + r) & 1;
+          constexpr int b_at = ends_sub && S::TURN > 1 ? S::TURN : 1;  // (a substep's first quants are read behind its barrier)
+          if constexpr (ends_sub && T == S::TURN) {
+            wait_loads<S::in_flight(u)>();
+            lds_barrier();
+          }
           static_for<NM>([&](auto J) __attribute__((always_inline)) {
             constexpr int j = J;
             d[T & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aop[slot][j], bop[t][j & 1], j == 0 ? (floatx16)(0.0f) : d[T & 1], 0, 0, 0);
@@ -434,8 +495,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
               else read_a(ns, j, pan, ends_sub ? 0 : bl + 1, 0);
             }
             if constexpr (j == 0 && T == 0) unpack_b(1);
-            if constexpr (j == 0 && T == 1) read_b(0, pbn, ends_stage ? 0 : sb + 1), read_b(1, pbn, ends_stage ? 0 : sb + 1);
-            if constexpr (j == (TILES == 2 ? NM - 1 : 0) && T == TILES - 1) unpack_b(0);
+            if constexpr (j == 0 && T == b_at) read_b(0, pbn, ends_stage ? 0 : sb + 1), read_b(1, pbn, ends_stage ? 0 : sb + 1);
+            if constexpr (j == (TILES == 2 || b_at == TILES - 1 ? NM - 1 : 0) && T == TILES - 1) unpack_b(0);
             scale_part<NM, j>(acc[pr][pt], d[(T + 1) & 1], T ? dq[pt] : dqp);
             if constexpr (j == NM - 1) {
               constexpr int from = (bl * TILES + T) * LOADS / SLOTS, to = (bl * TILES + T + 1) * LOADS / SLOTS;
@@ -446,37 +507,6 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
         });
         dqp = dq[kCT - 1];
       });
-      if constexpr (last && has_additive(FMT, F32A)) {
-        // the additive part of the stage's blocks: means times m (Q4) or the scale (Q8)
-        half8 bm[kCT];
-#pragma unroll
-        for (int t = 0; t < kCT; t++) {
-          uint32_t w0, w1 = 0;
-          const half2_t mulp = __builtin_bit_cast(half2_t, addp);
-          if constexpr (FMT == MGN_FMT_Q4) {
-            w0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(mcur[t][1], mcur[t][0], 0x07060302u)) * mulp);
-            w1 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(mcur[t][3], mcur[t][2], 0x07060302u)) * mulp);
-          } else {
-            w0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, mcur[t][0]) * mulp);
-          }
-          bm[t] = as_half8(w0, w1, 0u, 0u);
-        }
-        const uint8_t* const ps = lds_st + sbuf * STAGE_BYTES + s_rd;
-#pragma unroll
-        for (int r = RT - 1; r >= 0; r--) {
-          half8 am;
-          if constexpr (FMT == MGN_FMT_Q4) {
-            const uint2 v = *(const uint2*)(ps + r * (32 * SB * 4));
-            am = as_half8(v.x, v.y, 0u, 0u);
-          } else {
-            am = as_half8(*(const uint32_t*)(ps + r * (32 * SB * 4)), 0u, 0u, 0u);
-          }
-#pragma unroll
-          for (int t = kCT - 1; t >= 0; t--) acc[r][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm[t], acc[r][t], 0, 0, 0);
-        }
-      }
-      wait_loads<S::in_flight(u)>();
-      lds_barrier();
       abuf = anext;
       if constexpr (last) sbuf = snext;
     });
