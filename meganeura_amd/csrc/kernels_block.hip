@@ -25,8 +25,8 @@
 //   * K parts for different workgroups, where the tiles do not fill the chip, meet in the workspace and are added
 //     in part order by a third launch.
 // Measured (weights from memory; before -> now, us, Q4): fp16 2048 x 4096 x 14336 589 -> 268 (898 TFLOP/s),
-// f32 the same 1034 -> 453; f32 512 x 4096 x 14336 295 -> 118; f32 77 x 4096 x 14336 82 -> 39.6, 77 x 14336 x 4096
-// 98 -> 42.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.3
+// f32 the same 1034 -> 453; f32 512 x 4096 x 14336 295 -> 118; f32 77 x 4096 x 14336 82 -> 38.8, 77 x 14336 x 4096
+// 98 -> 41.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.3
 // times its issue cycles (LDS and barrier waits).
 #include <algorithm>
 #include <cmath>
@@ -149,7 +149,7 @@ struct BlockShape {
   static constexpr int NA = (int)(A_BYTES / 1024), NST = (int)(STAGE_BYTES / 1024);  // loads of 1 KiB
   static constexpr int NAW = (NA + WAVES - 1) / WAVES, NSTW = (NST + WAVES - 1) / WAVES;
   static constexpr size_t PIPE = (size_t)ARING * A_BYTES + (size_t)SRING * STAGE_BYTES;
-  static constexpr size_t RED = WK > 1 ? (size_t)WM * WN * RT * kCT * 4096 : 0, STRIP = (size_t)WAVES * 4096;
+  static constexpr size_t RED = WK > 1 ? (size_t)WAVES * RT * 4096 : 0, STRIP = (size_t)WAVES * 4096;
   static constexpr size_t LDS = PIPE > RED ? (PIPE > STRIP ? PIPE : STRIP) : (RED > STRIP ? RED : STRIP);
   // A wave's loads in issue order: in substep i the activations of substep i + PD, then, where it is a
   // stage's first, the stage SD ahead, dealt over the substep's tiles.  The substep's barrier stands in front of
@@ -552,36 +552,35 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
       for (int t = 0; t < kCT; t++) acc[r][t] *= x.unit;
   }
   if constexpr (WK > 1) {
-    // the streams' sums meet in LDS, in stream order
+    // The streams' sums meet in LDS: each stream keeps one of the two column tiles, hands the other one over and stores
+    // what it kept, so that the exchange and the stores have all waves.  (Before, one stream's waves added up and stored
+    // both tiles when the other's had ended, 3.4 of a workgroup's 28 us.  us, before -> now: Q4 77 x 4096 x 14336 39.7 -> 38.8,
+    // 77 x 14336 x 4096 41.4 -> 40.9, 200 x 2048 x 8192 27.8 -> 27.4; Q8 77 x 4096 x 14336 40.9 -> 40.6; the 64-row shape level.)
+    static_assert(WK == 2 && kCT == 2 && (WM * WN & (WM * WN - 1)) == 0, "a column tile per stream, and the other stream's wave a bit away");
     float* const red = (float*)lds4;
-    constexpr int G = WM * WN;  // waves per stream
-    for (uint32_t s = 1; s < WK; s++) {
-      if (ks == s) {
+    const uint32_t other = wave ^ (WM * WN);
+    if (ks != 0) {
 #pragma unroll
-        for (int r = 0; r < RT; r++)
-#pragma unroll
-          for (int t = 0; t < kCT; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-              *(floatx4*)(red + ((((wave % G) * RT + r) * kCT + t) * 4 + i) * 256 + lane * 4) =
-                  floatx4{acc[r][t][4 * i], acc[r][t][4 * i + 1], acc[r][t][4 * i + 2], acc[r][t][4 * i + 3]};
+      for (int r = 0; r < RT; r++) {
+        const floatx16 kept = acc[r][1];
+        acc[r][1] = acc[r][0], acc[r][0] = kept;
       }
-      lds_barrier();
-      if (ks == 0) {
-#pragma unroll
-        for (int r = 0; r < RT; r++)
-#pragma unroll
-          for (int t = 0; t < kCT; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-              const floatx4 v = *(const floatx4*)(red + ((((wave % G) * RT + r) * kCT + t) * 4 + i) * 256 + lane * 4);
-#pragma unroll
-              for (int e = 0; e < 4; e++) acc[r][t][4 * i + e] += v[e];
-            }
-      }
-      lds_barrier();
     }
-    if (ks > 0) return;
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        *(floatx4*)(red + ((wave * RT + r) * 4 + i) * 256 + lane * 4) =
+            floatx4{acc[r][1][4 * i], acc[r][1][4 * i + 1], acc[r][1][4 * i + 2], acc[r][1][4 * i + 3]};
+    lds_barrier();
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const floatx4 v = *(const floatx4*)(red + ((other * RT + r) * 4 + i) * 256 + lane * 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[r][0][4 * i + e] += v[e];
+      }
   }
   // Stores through a buffer descriptor that ends with the last row: what lies past it is dropped.
   const bool direct = x.parts == 1;
@@ -597,8 +596,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
 #pragma unroll
   for (int r = 0; r < RT; r++)
 #pragma unroll
-    for (int t = 0; t < kCT; t++) {
-      const uint32_t col = col0 + (wn * kCT + t) * 32 + c;
+    for (int t = 0; t < kCT / WK; t++) {
+      const uint32_t col = col0 + (wn * kCT + (WK > 1 ? ks : t)) * 32 + c;
       const uint32_t off = ((row0 + (wm * RT + r) * 32 + h * 4) * x.n + col) * 4u;
       if (col >= x.n) continue;
       if (residual) {

@@ -107,6 +107,21 @@ def test_residual_and_epilogue(ctx, orc, fmt, m, k, n):
     wt.free()
 
 
+@pytest.mark.parametrize("fmt,m,k,n", [(Q4, 65, 1024, 30005), (Q4, 300, 1024, 14369), (Q8, 65, 512, 50017)])
+def test_two_streams_that_store_the_result_themselves(ctx, orc, fmt, m, k, n):
+    """Each stream finishes one of a wave's two column tiles: residual, unary operations and a last column
+    group whose tiles end inside or behind the result."""
+    plan = capi.matmul_block_plan(fmt, m, k, n)
+    assert plan.threads == 512 and plan.rows < 128 and plan.k_parts == 1
+    w = synth.normal(2013, k * n, 0.02).reshape(k, n)
+    x, d = synth.normal(2014, m * k).reshape(m, k), synth.normal(2015, m * n).reshape(m, n)
+    wt = ctx.weight(fmt, w)
+    want = orc.matmul_f32(x, orc.dequantize(fmt, orc.quantize(fmt, w), k, n), d).astype(np.float64)
+    orc.assert_close(run(ctx, x, wt, d=d), want, 1e-3, 1e-4)
+    orc.assert_close(run(ctx, x, wt, d=d, ops=(capi.UNARY_NEG, capi.UNARY_SILU)), -want / (1 + np.exp(want)), 1e-3, 1e-4)
+    wt.free()
+
+
 @pytest.mark.parametrize("fmt", [Q4, Q8])
 @pytest.mark.parametrize("k", [1280, 4128])
 def test_magnitudes_that_change_along_k(ctx, orc, fmt, k):
