@@ -342,3 +342,22 @@ def test_every_workgroup_is_in_the_list():
         rt, wm, wn, _, _, _, wk = [int(v) for v in (numbers + ", 1").split(",")][:7]
         built.add((int(fmt), f32 == "false", 32 * rt * wm, 64 * wn, 64 * wm * wn * wk))
     assert built == {kind + shape[:3] for kind, shapes in WORKGROUPS.items() for shape in shapes} and len(built) == 30
+
+
+@pytest.mark.parametrize("fmt,f16", [(Q4, False), (Q4, True), (Q8, False), (Q8, True)])
+def test_results_that_pass_the_caches_by(ctx, orc, fmt, f16):
+    """Just over 64 MiB of result, ragged in rows and columns.  Rows repeat after 41 and columns after 1499, so that all outputs
+    have a reference."""
+    m, k, n = 1025, 96, 16389
+    assert m * n * 4 > 64 << 20 and capi.matmul_block_plan(fmt, m, k, n, f16).k_parts == 1
+    w = synth.normal(2200, k * 1499, 0.02).reshape(k, 1499)
+    base = synth.normal(2201, 41 * k).reshape(41, k).astype(np.float16 if f16 else np.float32)
+    rows, cols = np.arange(m) % 41, np.arange(n) % 1499
+    wt = ctx.weight(fmt, np.ascontiguousarray(w[:, cols]))
+    want = base.astype(np.float64) @ orc.dequantize(fmt, orc.quantize(fmt, w), k, 1499).astype(np.float64)
+    got = run(ctx, base[rows], wt, f16)
+    # (not bit for bit across tiles: a wave's last tile adds a block's product behind the next blocks' means)
+    assert_rows_close(got, want[rows][:, cols], base[rows].astype(np.float32), k)
+    d = synth.normal(2202, m * n).reshape(m, n)
+    assert np.array_equal(run(ctx, base[rows], wt, f16, d=d), got + d)
+    wt.free()
