@@ -24,9 +24,9 @@
 //     waves that meet such a row move their sums from scale to scale;
 //   * K parts for different workgroups, where the tiles do not fill the chip, meet in the workspace and are added
 //     in part order by a third launch.
-// Measured (weights from memory; before -> now, us, Q4): fp16 2048 x 4096 x 14336 589 -> 268 (898 TFLOP/s),
-// f32 the same 1034 -> 453; f32 512 x 4096 x 14336 295 -> 118; f32 77 x 4096 x 14336 82 -> 38.8, 77 x 14336 x 4096
-// 98 -> 41.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.3
+// Measured (weights from memory; before -> now, us, Q4; machines differ by 3 %): fp16 2048 x 4096 x 14336 589 -> 271
+// (888 TFLOP/s), f32 the same 1034 -> 455; f32 512 x 4096 x 14336 295 -> 120; f32 77 x 4096 x 14336 82 -> 40, 77 x 14336 x
+// 4096 98 -> 42.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.3
 // times its issue cycles (LDS and barrier waits).
 #include <algorithm>
 #include <cmath>
