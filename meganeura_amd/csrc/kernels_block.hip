@@ -24,8 +24,8 @@
 //     waves that meet such a row move their sums from scale to scale;
 //   * K parts for different workgroups, where the tiles do not fill the chip, meet in the workspace and are added
 //     in part order by a third launch.
-// Measured (weights from memory; before -> now, us, Q4; machines differ by 3 %): fp16 2048 x 4096 x 14336 589 -> 271
-// (888 TFLOP/s), f32 the same 1034 -> 455; f32 512 x 4096 x 14336 295 -> 120; f32 77 x 4096 x 14336 82 -> 40, 77 x 14336 x
+// Measured (weights from memory; before -> now, us, Q4; machines differ by 3 %): fp16 2048 x 4096 x 14336 589 -> 277
+// (867 TFLOP/s), f32 the same 1034 -> 455; f32 512 x 4096 x 14336 295 -> 120; f32 77 x 4096 x 14336 82 -> 40, 77 x 14336 x
 // 4096 98 -> 42.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.3
 // times its issue cycles (LDS and barrier waits).
 #include <algorithm>
@@ -52,14 +52,6 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 constexpr int kCT = 2;  // column tiles of 32 columns per wave
-constexpr int kStoreNonTemporal = 2;  // the cache policy operand of a buffer store
-
-// Whether the kernel's stores pass L2 by (non-temporal).  A result of more than 64 MiB, twice the L2s of the chip, is gone from there
-// before anyone reads it, and drives out the activations and quants that the next workgroups share.  With a residual, us, before ->
-// now: 2048 x 4096 x 14336 (117 MB) Q4 f32 476 -> 464, Q4 fp16 296 -> 289, Q8 f32 524 -> 515; Q4 f32 1500 x 1024 x 14336 (86 MB) 118.8 ->
-// 116.2.  At half of that it is level (1024 x 4096 x 14336, 59 MB: Q8 f32 226.9 -> 227.3, fp16 190 -> 191).  Sums of K parts go both ways
-// (Q4 f32 77 x 4096 x 14336 40.9 -> 40.1, 45 x 14336 x 4096 33.4 -> 35.0) and stay.
-bool stream_result(uint64_t m, uint64_t n, uint32_t parts) { return parts == 1 && m * n * 4 > (64u << 20); }
 
 constexpr int stage_blocks(int fmt) { return fmt == MGN_FMT_Q4 ? 4 : 2; }  // 64 bytes of quants per column
 
@@ -130,7 +122,6 @@ struct BlockArgs {
   float* c;
   float* partial;  // [parts][m][n] when parts > 1
   uint32_t epilogue;
-  uint32_t stream_out;  // stores that do not stay in L2 (stream_result)
 };
 
 __device__ __forceinline__ float group_max32(float v) {
@@ -591,7 +582,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
         for (int e = 0; e < 4; e++) acc[r][0][4 * i + e] += v[e];
       }
   }
-  // Stores through a buffer descriptor that ends with the last row: what lies past it is dropped.
+  // Stores through a buffer descriptor that ends with the last row: what lies past it is dropped.  (Stores like any other, also of
+  // results far larger than the L2s: a row whose length is no multiple of 32 words shares its 128-byte lines between
+  // workgroups, and only a cache that keeps them puts them together.  With the non-temporal hint, us, without -> with: fp16
+  // activations 700 x 576 x 49151 Q4 88 -> 148, Q8 87 -> 146; 2048 x 1024 x 14337 Q4 89 -> 143, f32 137 -> 159.  In whole
+  // lines it went both ways, 2048 x 4096 x 14336 Q4 277 -> 271 but 2048 x 576 x 49152 f32 321 -> 328, with a residual 391 -> 441; with a call
+  // behind it that reads the result: 1250 x 1024 -> 14336 -> 1024 221 -> 225, 2048 the like 348 -> 350, 4096 728 -> 705.)
   const bool direct = x.parts == 1;
   const uint32_t bytes = x.m * x.n * 4u;
   const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc((void*)(direct ? x.c : x.partial + (size_t)part * x.m * x.n), 0, bytes, 0x00020000);
@@ -624,13 +620,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[r][t][i] = strip[i * 64];
       }
-      auto store = [&](auto Policy) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 16; i++)
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, (float)acc[r][t][i]), out, off + ((i >> 2) * 8 + (i & 3)) * x.n * 4u, 0, Policy);
-      };
-      if (x.stream_out) store(std::integral_constant<int, kStoreNonTemporal>{});
-      else store(std::integral_constant<int, 0>{});
+      for (int i = 0; i < 16; i++)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, (float)acc[r][t][i]), out, off + ((i >> 2) * 8 + (i & 3)) * x.n * 4u, 0, 0);
     }
 }
 
@@ -974,7 +966,6 @@ int launch_block_rows(ihipStream_t* s, const LaunchArgs& x, const BlockPlan& p) 
   a.unit = std::ldexp(1.0f, (FMT == MGN_FMT_Q4 ? 5 : 12) - lift);
   if (!has_additive(FMT, f32a)) a.dscale = a.unit = 1.0f;
   a.dres = x.d, a.c = x.c, a.partial = partial, a.epilogue = x.epilogue;
-  a.stream_out = stream_result(x.m, x.w.n, p.parts);
   if (p.cfg->lds > 64 * 1024) {
     static std::atomic<uint64_t> big_lds_done[4][kBlockConfigs];
     const BlockConfig* const first = block_configs(FMT, f32a);

@@ -45,6 +45,18 @@ def hazards(lines):
     return bad, loads
 
 
+@pytest.fixture(scope="module")
+def code_objects(tmp_path_factory):
+    """The assembler's lines for each of the library's device code objects, by name."""
+    if not os.path.exists(OBJDUMP) or not os.path.exists(LIB):
+        pytest.skip("no llvm-objdump, or the library is not built")
+    at = tmp_path_factory.mktemp("code")
+    lib = shutil.copy(LIB, at / "lib.so")
+    subprocess.run([OBJDUMP, "--offloading", str(lib)], cwd=at, check=True, stdout=subprocess.DEVNULL)
+    return {name: subprocess.run([OBJDUMP, "-d", "--mcpu=gfx950", name], cwd=at, check=True, stdout=subprocess.PIPE, text=True).stdout.splitlines()
+            for name in sorted(os.listdir(at)) if name.endswith("gfx950")}
+
+
 def test_the_rule_is_recognised():
     after = ["s_mov_b32 m0, s9", "s_nop 0", "buffer_load_dwordx4 v1, s[4:7], s2 offen lds"]
     for first in ("v_readfirstlane_b32 s2, v0", "v_readlane_b32 s6, v0, 3"):
@@ -54,19 +66,26 @@ def test_the_rule_is_recognised():
     assert len(hazards([after[0], after[2]])[0]) == 1
 
 
-def test_loads_into_lds_wait_for_their_scalars(tmp_path):
-    if not os.path.exists(OBJDUMP) or not os.path.exists(LIB):
-        pytest.skip("no llvm-objdump, or the library is not built")
-    lib = shutil.copy(LIB, tmp_path / "lib.so")
-    subprocess.run([OBJDUMP, "--offloading", str(lib)], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
+def test_loads_into_lds_wait_for_their_scalars(code_objects):
     loads = 0
-    for name in sorted(os.listdir(tmp_path)):
-        if not name.endswith("gfx950"):
+    for name, lines in code_objects.items():
+        if not any(" lds" in line for line in lines):
             continue
-        out = subprocess.run([OBJDUMP, "-d", "--mcpu=gfx950", name], cwd=tmp_path, check=True, stdout=subprocess.PIPE, text=True).stdout
-        if " lds " not in out:
-            continue
-        bad, n = hazards(out.splitlines())
+        bad, n = hazards(lines)
         assert not bad, f"{len(bad)} of {n} in {name}, the first: {bad[0]}"
         loads += n
     assert loads > 100, "the blocked kernels' loads were not found"
+
+
+def test_the_blocked_kernel_stores_through_the_caches(code_objects):
+    """Rows whose length is no multiple of 128 bytes share their lines between workgroups: stores with the non-temporal hint
+    write such a line in pieces (up to 1.6 times the call's time)."""
+    kernel, stores = "", 0
+    for line in (line for lines in code_objects.values() for line in lines):
+        text = line.split("//")[0].strip()
+        if text.endswith(">:"):
+            kernel = text
+        elif "block_kernel" in kernel and text.startswith("buffer_store"):
+            assert not re.search(r"\b(nt|sc0|sc1)\b", text), (kernel, text)
+            stores += 1
+    assert stores > 30 * 16, "the blocked kernels' stores were not found"

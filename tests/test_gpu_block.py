@@ -346,7 +346,7 @@ def test_every_workgroup_is_in_the_list():
 
 @pytest.mark.parametrize("fmt,f16", [(Q4, False), (Q4, True), (Q8, False), (Q8, True)])
 def test_results_that_pass_the_caches_by(ctx, orc, fmt, f16):
-    """Just over 64 MiB of result, ragged in rows and columns.  Rows repeat after 41 and columns after 1499, so that all outputs
+    """Just over 64 MiB of result, twice the chip's L2s, ragged in rows and columns.  Rows repeat after 41 and columns after 1499, so that all outputs
     have a reference."""
     m, k, n = 1025, 96, 16389
     assert m * n * 4 > 64 << 20 and capi.matmul_block_plan(fmt, m, k, n, f16).k_parts == 1
