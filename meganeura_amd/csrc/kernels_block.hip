@@ -162,6 +162,7 @@ struct BlockShape {
   static constexpr int TILES = RT * kCT, SLOTS = SUBB * TILES;
   static constexpr int TURN = F32A ? TILES - 1 : TILES - 2;
   static constexpr int issued(int i) { return NAW + ((i + 64 * NSUB) % NSUB == 0 ? NSTW : 0); }
+  static constexpr int issued_before(int i, int slot) { return slot * issued(i) / SLOTS; }  // of them in front of tile `slot` of the substep
   static constexpr int since(int from, int to) {
     int n = 0;
     for (int i = from; i <= to; i++) n += issued(i);
@@ -171,7 +172,7 @@ struct BlockShape {
   static constexpr int requested(int i) { return (stage_of(i) - SD) * NSUB; }  // the substep that asks for substep i's stage
   static constexpr int behind_a(int i) { return (i - PD + 64 * NSUB) % NSUB == 0 ? NSTW : 0; }  // loads behind substep i's activations in the substep that asks for them
   static constexpr int in_flight(int i) {
-    const int here = ((SUBB - 1) * TILES + TURN) * issued(i) / SLOTS;
+    const int here = issued_before(i, (SUBB - 1) * TILES + TURN);
     const int after_a = behind_a(i + 1) + since(i + 2 - PD, i - 1) + here;
     const int after_stage = since(requested(i + 1) + 1, i - 1) + here;
     return after_a < after_stage ? after_a : after_stage;
@@ -184,6 +185,26 @@ struct BlockShape {
     return after_a < after_stage ? after_a : after_stage;
   }
   static_assert(PD >= 2 && requested(NSUB) < NSUB - 1, "what a substep waits for has been requested in whole");
+
+  // The requests of three stages one by one, in the order and number in which the kernel issues them: whether at each of
+  // its waits what may still be in flight holds none that must have landed.
+  static constexpr bool waits_suffice() {
+    int sent = 0, a_end[PD + 4 * NSUB] = {}, st_end[SD + 4] = {};  // requests up to and with the last of a substep's activations, of a stage
+    for (int i = FIRST; i < 3 * NSUB; i++) {
+      const bool first = (i + 64 * NSUB) % NSUB == 0 && stage_of(i) + SD >= 0;
+      auto landed = [&](int in_flight, int sub) { return sent - in_flight >= a_end[sub] && sent - in_flight >= st_end[sub / NSUB]; };
+      if (i == 0 && !landed(in_flight_first(), 0)) return false;
+      const int all = i < 0 ? (i + PD >= 0 ? NAW : 0) + (first ? NSTW : 0) : issued_before(i, SLOTS);
+      const int at_turn = i < 0 ? all : issued_before(i, (SUBB - 1) * TILES + TURN);
+      const int before = sent;
+      if (i + PD >= 0) a_end[i + PD] = before + NAW;
+      if (first) st_end[stage_of(i) + SD] = before + all;
+      sent = before + at_turn;
+      if (i >= 0 && !landed(in_flight(i % NSUB), i + 1)) return false;
+      sent = before + all;
+    }
+    return true;
+  }
 };
 
 template <int FMT, bool F32A, int RT, int WM, int WN, int WK, int SUBB, int PD, int SD>
@@ -195,7 +216,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
   constexpr uint32_t MEAN_STREAM = S::MEAN_STREAM;
   constexpr int QB = FMT == MGN_FMT_Q4 ? 16 : 32, MB = FMT == MGN_FMT_Q4 ? 4 : 2;
   constexpr int NM = F32A ? 4 : 2;             // matrix instructions per tile and block
-  constexpr int TILES = RT * kCT;
+  constexpr int TILES = S::TILES;
   static_assert(F32A || SUBB % 2 == 0, "fp16 activations: two blocks per 128 bytes");
   extern __shared__ uint4 lds4[];
   uint8_t* const lds = (uint8_t*)lds4;
@@ -450,7 +471,6 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
     static_for<NSUB>([&](auto U) __attribute__((always_inline)) {
       constexpr int u = U;
       constexpr bool last = u == NSUB - 1;
-      constexpr int SLOTS = SUBB * TILES, LOADS = S::issued(u);
       constexpr int ahead = (u + PD) / NSUB, usub = (u + PD) % NSUB;  // the activations requested here: iterations ahead, substep
       const uint32_t anext = abuf + 1 == ARING ? 0 : abuf + 1, aload = abuf == 0 ? ARING - 1 : abuf - 1;
       const uint32_t snext = sbuf + 1 == SRING ? 0 : sbuf + 1, sload = sbuf == 0 ? SRING - 1 : sbuf - 1;
@@ -499,7 +519,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
             if constexpr (j == (TILES == 2 || b_at == TILES - 1 ? NM - 1 : 0) && T == TILES - 1) unpack_b(0);
             scale_part<NM, j>(acc[pr][pt], d[(T + 1) & 1], T ? dq[pt] : dqp);
             if constexpr (j == NM - 1) {
-              constexpr int from = (bl * TILES + T) * LOADS / SLOTS, to = (bl * TILES + T + 1) * LOADS / SLOTS;
+              constexpr int from = S::issued_before(u, bl * TILES + T), to = S::issued_before(u, bl * TILES + T + 1);
               static_for<to - from>([&](auto Qn) __attribute__((always_inline)) { issue_load(std::integral_constant<int, from + Qn>{}); });
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -802,6 +822,7 @@ BlockConfig block_config(double t1, double tn) {
   static_assert(WK == 1 || F32A, "streams may run out of stages only on prepared activations");
   using S = BlockShape<FMT, F32A, RT, WM, WN, WK, SUBB, PD, SD>;
   static_assert(S::LDS <= 160 * 1024, "fits a CU");
+  static_assert(S::waits_suffice(), "a wave passes a barrier before its operands have landed");
   return {block_kernel<FMT, F32A, RT, WM, WN, WK, SUBB, PD, SD>, (uint32_t)S::ROWS, (uint32_t)S::COLS, 64u * S::WAVES, (uint32_t)WK, S::LDS, t1, tn};
 }
 
