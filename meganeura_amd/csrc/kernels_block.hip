@@ -157,10 +157,17 @@ struct BlockShape {
   // what it reads from there to the next barrier is substep i + 1's, and that one's stage.  So these must have
   // landed; the loads issued after the last of them may be in flight.  (With the barrier behind the last tile, the
   // next substep's first operands had to have landed a barrier earlier: at PD = 2 the loads of the very substep that
-  // ends, and their whole latency was waited for.  us, weights from memory: Q4 fp16 2048 x 4096 x 14336 292 -> 268, f32
-  // 476 -> 453; 77 x 4096 x 14336 Q4 40.4 -> 39.6, Q8 44.5 -> 41.4; no shape measured slower.)
+  // ends, and their whole latency was waited for.  us, weights from memory: Q4 fp16 2048 x 4096 x 14336 290 -> 267, f32
+  // 478 -> 450; 77 x 4096 x 14336 Q4 40.7 -> 39.5, Q8 45.4 -> 41.3; level where PD is 3 already.)
+  // f32 activations hold the operands of one row tile: the last ones have been read when its first column tile begins, and a
+  // wave may turn there or a tile later.  With PD = 3 the next substep's operands have landed by then, and what the later turn
+  // waits for is the next quants, read behind the barrier and unpacked at the end of the same tile: workgroups of two row tiles per
+  // wave, medians of 8 to 22 sizes, barrier behind the last tile = 1, in front of it, a tile earlier: Q4 64 x 256 1.014, 1.004,
+  // of two streams 1.004, 0.991, 128 x 256 1.001, 0.980; Q8 64 x 256 1.020, 0.998, 128 x 256 1.006, 0.981 (444 x 2176 x 8192 52.3, 54.4,
+  // 52.6 us).  With one row tile the earlier turn is the whole substep's wait (Q4 32 x 256 0.988, 0.998; 64 x 128 0.977, 0.987).  At
+  // PD = 2 both ways: 0.5 to 1 % faster with 96 to 256 rows, but Q8 96 x 256 of two streams 0.915, 0.932.
   static constexpr int TILES = RT * kCT, SLOTS = SUBB * TILES;
-  static constexpr int TURN = F32A ? TILES - 1 : TILES - 2;
+  static constexpr int TURN = F32A && (PD == 2 || RT == 1) ? TILES - 1 : TILES - 2;
   static constexpr int issued(int i) { return NAW + ((i + 64 * NSUB) % NSUB == 0 ? NSTW : 0); }
   static constexpr int issued_before(int i, int slot) { return slot * issued(i) / SLOTS; }  // of them in front of tile `slot` of the substep
   static constexpr int since(int from, int to) {
