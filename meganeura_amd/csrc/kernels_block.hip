@@ -460,9 +460,14 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
           }
           bm[t] = as_half8(w0, w1, 0u, 0u);
         }
+        // (Q8's stages are one substep of two blocks: the products stand between every second block's tiles, and they begin with
+        // the last tile, whose scaling is due next and would wait for the end of them.  fp16, us, with the products behind the
+        // stage's tiles, in front with the first tile's first, with the last tile's first: 437 x 1600 x 7168 33.2, 34.3, 33.0, 444 x 1152 x 6656
+        // 25.6, 26.7, 25.7, 610 x 896 x 5120 22.0, 22.8, 21.9.  Q4 is level but for short K: 1009 x 160 x 19456 39.5 first tile first, 40.6.)
         const uint8_t* const ps = lds_st + sbuf * STAGE_BYTES + s_rd;
 #pragma unroll
-        for (int r = 0; r < RT; r++) {
+        for (int i = 0; i < RT; i++) {
+          const int r = FMT == MGN_FMT_Q8 ? RT - 1 - i : i;
           half8 am;
           if constexpr (FMT == MGN_FMT_Q4) {
             const uint2 v = *(const uint2*)(ps + r * (32 * SB * 4));
@@ -471,7 +476,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
             am = as_half8(*(const uint32_t*)(ps + r * (32 * SB * 4)), 0u, 0u, 0u);
           }
 #pragma unroll
-          for (int t = 0; t < kCT; t++) acc[r][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm[t], acc[r][t], 0, 0, 0);
+          for (int j = 0; j < kCT; j++) {
+            const int t = FMT == MGN_FMT_Q8 ? kCT - 1 - j : j;
+            acc[r][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm[t], acc[r][t], 0, 0, 0);
+          }
         }
       }
     };
