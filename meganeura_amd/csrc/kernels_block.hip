@@ -444,45 +444,47 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
         }
       }
     }
-    // the additive part of the stage's blocks: means times m (Q4) or the scale (Q8)
-    auto add_means = [&]() __attribute__((always_inline)) {
-      if constexpr (has_additive(FMT, F32A)) {
-        half8 bm[kCT];
+    // The additive part of the stage's blocks: means times m (Q4) or the scale (Q8).
+    // Q4's come in front of the stage's last substep.  Q8's stand for a bias of 128 on the bytes, several times the products
+    // themselves, which must be in the sum when they take it out: the subtraction leaves little and rounds nothing, where in front of the
+    // products the matrix unit rounds sums of the bias's size.  (Error against f64, fp16 activations behind a silu, first behind
+    // the stage's products, then in front: 77 x 4096 x 14336 6.9e-7, 8.2e-7, 200 x 2048 x 8192 6.1e-7, 7.1e-7; Q4, whose minima are of
+    // the products' size, 4.0e-7, 3.6e-7 on 2048 x 4096 x 14336.)  They are read in front of the barrier that gives their buffer away.
+    uint32_t means[RT][FMT == MGN_FMT_Q4 ? 2 : 1];
+    auto read_means = [&]() __attribute__((always_inline)) {
+      const uint8_t* const ps = lds_st + sbuf * STAGE_BYTES + s_rd;
 #pragma unroll
-        for (int t = 0; t < kCT; t++) {
-          uint32_t w0, w1 = 0;
-          const half2_t mulp = __builtin_bit_cast(half2_t, addp);
-          if constexpr (FMT == MGN_FMT_Q4) {
-            w0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(mcur[t][1], mcur[t][0], 0x07060302u)) * mulp);
-            w1 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(mcur[t][3], mcur[t][2], 0x07060302u)) * mulp);
-          } else {
-            w0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, mcur[t][0]) * mulp);
-          }
-          bm[t] = as_half8(w0, w1, 0u, 0u);
-        }
-        // (Q8's stages are one substep of two blocks: the products stand between every second block's tiles, and they begin with
-        // the last tile, whose scaling is due next and would wait for the end of them.  fp16, us, with the products behind the
-        // stage's tiles, in front with the first tile's first, with the last tile's first: 437 x 1600 x 7168 33.2, 34.3, 33.0, 444 x 1152 x 6656
-        // 25.6, 26.7, 25.7, 610 x 896 x 5120 22.0, 22.8, 21.9.  Q4 is level but for short K: 1009 x 160 x 19456 39.5 first tile first, 40.6.)
-        const uint8_t* const ps = lds_st + sbuf * STAGE_BYTES + s_rd;
-#pragma unroll
-        for (int i = 0; i < RT; i++) {
-          const int r = FMT == MGN_FMT_Q8 ? RT - 1 - i : i;
-          half8 am;
-          if constexpr (FMT == MGN_FMT_Q4) {
-            const uint2 v = *(const uint2*)(ps + r * (32 * SB * 4));
-            am = as_half8(v.x, v.y, 0u, 0u);
-          } else {
-            am = as_half8(*(const uint32_t*)(ps + r * (32 * SB * 4)), 0u, 0u, 0u);
-          }
-#pragma unroll
-          for (int j = 0; j < kCT; j++) {
-            const int t = FMT == MGN_FMT_Q8 ? kCT - 1 - j : j;
-            acc[r][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm[t], acc[r][t], 0, 0, 0);
-          }
+      for (int r = 0; r < RT; r++) {
+        if constexpr (FMT == MGN_FMT_Q4) {
+          const uint2 v = *(const uint2*)(ps + r * (32 * SB * 4));
+          means[r][0] = v.x, means[r][1] = v.y;
+        } else {
+          means[r][0] = *(const uint32_t*)(ps + r * (32 * SB * 4));
         }
       }
     };
+    auto add_means = [&]() __attribute__((always_inline)) {
+      half8 bm[kCT];
+#pragma unroll
+      for (int t = 0; t < kCT; t++) {
+        uint32_t w0, w1 = 0;
+        const half2_t mulp = __builtin_bit_cast(half2_t, addp);
+        if constexpr (FMT == MGN_FMT_Q4) {
+          w0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(mcur[t][1], mcur[t][0], 0x07060302u)) * mulp);
+          w1 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(mcur[t][3], mcur[t][2], 0x07060302u)) * mulp);
+        } else {
+          w0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, mcur[t][0]) * mulp);
+        }
+        bm[t] = as_half8(w0, w1, 0u, 0u);
+      }
+      // (Q8: the last tile, whose products are still to be scaled, comes first)
+      static_for<TILES>([&](auto TT) __attribute__((always_inline)) {
+        constexpr int T = FMT == MGN_FMT_Q4 ? (int)TT : TILES - 1 - TT, r = T / kCT, t = T % kCT;
+        const half8 am = as_half8(means[r][0], FMT == MGN_FMT_Q4 ? means[r][FMT == MGN_FMT_Q4] : 0u, 0u, 0u);
+        acc[r][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm[t], acc[r][t], 0, 0, 0);
+      });
+    };
+    constexpr bool means_first = FMT == MGN_FMT_Q4, means_last = FMT == MGN_FMT_Q8 && has_additive(FMT, F32A);
     static_for<NSUB>([&](auto U) __attribute__((always_inline)) {
       constexpr int u = U;
       constexpr bool last = u == NSUB - 1;
@@ -497,7 +499,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
         if constexpr (q >= NAW) load_stage(q - NAW, its, sload);
         else load_a(q, ita, usub, aload);
       };
-      if constexpr (last) add_means();
+      if constexpr (last && means_first) read_means(), add_means();
       __builtin_amdgcn_sched_barrier(0);
       static_for<SUBB>([&](auto BL) __attribute__((always_inline)) {
         constexpr int bl = BL, sb = u * SUBB + bl;
@@ -516,6 +518,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
           constexpr int slot = F32A ? 0 : (sb * RT + r) & 1;
           constexpr int b_at = ends_sub && S::TURN > 1 ? S::TURN : 1;  // (a substep's first quants are read behind its barrier)
           if constexpr (ends_sub && T == S::TURN) {
+            if constexpr (last && means_last) read_means();
             wait_loads<S::in_flight(u)>();
             lds_barrier();
           }
@@ -542,6 +545,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
         });
         dqp = dq[kCT - 1];
       });
+      if constexpr (last && means_last) add_means();
       abuf = anext;
       if constexpr (last) sbuf = snext;
     });

@@ -231,6 +231,31 @@ def test_q8_sums_are_free_of_the_byte_bias(ctx, orc):
     wt.free()
 
 
+# (one for each workgroup, K in one part)
+@pytest.mark.parametrize("m,n", [(134, 13028), (98, 12724), (130, 18829), (198, 17016), (387, 13986), (388, 19172)])
+def test_q8_bias_leaves_a_sum_that_holds_it(ctx, orc, m, n):
+    """Q8 with fp16 activations multiplies bytes with a bias of 128 and takes it out of the sum of each two blocks.  Integers for which every
+    sum on the way fits 24 bits if it is taken out when the products (one tile's: all but the last) are in, and none does if
+    it is taken out first: 2^23 a stage, at a running sum of -2^24 + 1.5 x 2^22 and odd."""
+    k, base = 736, 499
+    assert capi.matmul_block_plan(Q8, m, k, n, True).k_parts == 1
+    rng = np.random.default_rng(7)
+    w = rng.integers(-10, 11, (k, base))
+    w[30::32], w[31::32] = 127, -127  # a block's scale is 1
+    w[30:128:32] = -107
+    w[:64], w[64:128] = np.where(w[:64] == -127, -127, -107), np.where(w[64:128] == -127, -127, -51)
+    x = np.full((m, k), 1024)
+    x[np.arange(m), np.arange(m) % 31] += 1  # meets -107: the sums are odd
+    sums = np.cumsum((x[:, :, None] * w[None, :, :1]).reshape(m, -1, 32).sum(axis=2), axis=1)
+    assert ((sums[:, 3:] > 2**22 - 2**24) & (sums[:, 3:] < 2**23 - 2**24) & (sums[:, 3:] % 2 == 1)).all()
+    packed = orc.quantize(Q8, w.astype(np.float32))
+    assert np.array_equal(orc.dequantize(Q8, packed, k, base), w)
+    wt = ctx.weight(Q8, np.ascontiguousarray(w.astype(np.float32)[:, np.arange(n) % base]))
+    got = run(ctx, x.astype(np.float16), wt, True)
+    assert np.array_equal(got, (x @ w).astype(np.float32)[:, np.arange(n) % base])
+    wt.free()
+
+
 @pytest.mark.parametrize("fmt", [Q4, Q8])
 def test_infinite_rows_of_fp16_activations_stay_on_their_own(ctx, orc, fmt):
     m, k, n = 40, 96, 70  # K ends in the middle of the 64 elements that are loaded at once
