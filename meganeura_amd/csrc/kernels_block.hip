@@ -166,8 +166,14 @@ struct BlockShape {
   // of two streams 1.004, 0.991, 128 x 256 1.001, 0.980; Q8 64 x 256 1.020, 0.998, 128 x 256 1.006, 0.981 (444 x 2176 x 8192 52.3, 54.4,
   // 52.6 us).  With one row tile the earlier turn is the whole substep's wait (Q4 32 x 256 0.988, 0.998; 64 x 128 0.977, 0.987).  At
   // PD = 2 both ways: 0.5 to 1 % faster with 96 to 256 rows, but Q8 96 x 256 of two streams 0.915, 0.932.
+  // The barrier stays behind the last tile, with the next block's operands landed as well, where four waves with nothing to
+  // spare (PD = 2) have a CU to themselves: one wave on each SIMD, and nobody works while it waits for what it may read only now.
+  // That is Q8 with fp16 activations, us, behind, in front: 96 x 256 213 x 1472 x 20992 36.3, 38.1, 298 x 1376 x 13824 36.0, 37.6, 64 x 256
+  // 444 x 1152 x 6656 25.7, 26.1; medians of 21 and 12 sizes 1, 1.010 and 1, 0.997.  (Q8 64 x 256 with f32 activations and PD = 3 is level.)
   static constexpr int TILES = RT * kCT, SLOTS = SUBB * TILES;
-  static constexpr int TURN = F32A && (PD == 2 || RT == 1) ? TILES - 1 : TILES - 2;
+  static constexpr bool ALONE = WAVES == 4 && PD == 2 && 2 * LDS > 160 * 1024;
+  static constexpr int TURN = ALONE ? TILES : F32A && (PD == 2 || RT == 1) ? TILES - 1 : TILES - 2;
+  static constexpr int AHEAD = ALONE ? 2 : 1;  // at its barrier, substep i + AHEAD's operands must have landed
   static constexpr int issued(int i) { return NAW + ((i + 64 * NSUB) % NSUB == 0 ? NSTW : 0); }
   static constexpr int issued_before(int i, int slot) { return slot * issued(i) / SLOTS; }  // of them in front of tile `slot` of the substep
   static constexpr int since(int from, int to) {
@@ -179,19 +185,19 @@ struct BlockShape {
   static constexpr int requested(int i) { return (stage_of(i) - SD) * NSUB; }  // the substep that asks for substep i's stage
   static constexpr int behind_a(int i) { return (i - PD + 64 * NSUB) % NSUB == 0 ? NSTW : 0; }  // loads behind substep i's activations in the substep that asks for them
   static constexpr int in_flight(int i) {
-    const int here = issued_before(i, (SUBB - 1) * TILES + TURN);
-    const int after_a = behind_a(i + 1) + since(i + 2 - PD, i - 1) + here;
-    const int after_stage = since(requested(i + 1) + 1, i - 1) + here;
+    const int here = issued_before(i, (SUBB - 1) * TILES + TURN), of = i + AHEAD;
+    const int after_a = behind_a(of) + (of - PD < i ? since(of - PD + 1, i - 1) + here : 0);
+    const int after_stage = since(requested(of) + 1, i - 1) + here;
     return after_a < after_stage ? after_a : after_stage;
   }
   // In front of the loop, in the same order, what the substeps before the first would have asked for: landed must be
-  // substep 0's activations and its stage.
+  // the activations and the stage of the substeps that are read up to the first barrier.
   static constexpr int FIRST = -(PD > SD * NSUB ? PD : SD * NSUB);
   static constexpr int in_flight_first() {
-    const int after_a = behind_a(0) + since(1 - PD, -1), after_stage = since(requested(0) + 1, -1);
+    const int of = AHEAD - 1, after_a = behind_a(of) + since(of - PD + 1, -1), after_stage = since(requested(of) + 1, -1);
     return after_a < after_stage ? after_a : after_stage;
   }
-  static_assert(PD >= 2 && requested(NSUB) < NSUB - 1, "what a substep waits for has been requested in whole");
+  static_assert(PD >= 2 && requested(NSUB - 1 + AHEAD) < NSUB - 1, "what a substep waits for has been requested in whole");
 
   // The requests of three stages one by one, in the order and number in which the kernel issues them: whether at each of
   // its waits what may still be in flight holds none that must have landed.
@@ -200,14 +206,14 @@ struct BlockShape {
     for (int i = FIRST; i < 3 * NSUB; i++) {
       const bool first = (i + 64 * NSUB) % NSUB == 0 && stage_of(i) + SD >= 0;
       auto landed = [&](int in_flight, int sub) { return sent - in_flight >= a_end[sub] && sent - in_flight >= st_end[sub / NSUB]; };
-      if (i == 0 && !landed(in_flight_first(), 0)) return false;
+      if (i == 0 && !landed(in_flight_first(), AHEAD - 1)) return false;
       const int all = i < 0 ? (i + PD >= 0 ? NAW : 0) + (first ? NSTW : 0) : issued_before(i, SLOTS);
       const int at_turn = i < 0 ? all : issued_before(i, (SUBB - 1) * TILES + TURN);
       const int before = sent;
       if (i + PD >= 0) a_end[i + PD] = before + NAW;
       if (first) st_end[stage_of(i) + SD] = before + all;
       sent = before + at_turn;
-      if (i >= 0 && !landed(in_flight(i % NSUB), i + 1)) return false;
+      if (i >= 0 && !landed(in_flight(i % NSUB), i + AHEAD)) return false;
       sent = before + all;
     }
     return true;
@@ -516,7 +522,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
         static_for<TILES>([&](auto TT) __attribute__((always_inline)) {
           constexpr int T = TT, r = T / kCT, t = T % kCT, pr = T ? (T - 1) / kCT : RT - 1, pt = T ? (T - 1) % kCT : kCT - 1;
           constexpr int slot = F32A ? 0 : (sb * RT + r) & 1;
-          constexpr int b_at = ends_sub && S::TURN > 1 ? S::TURN : 1;  // (a substep's first quants are read behind its barrier)
+          constexpr int b_at = ends_sub && !S::ALONE && S::TURN > 1 ? S::TURN : 1;  // (a substep's first quants are read behind its barrier)
           if constexpr (ends_sub && T == S::TURN) {
             if constexpr (last && means_last) read_means();
             wait_loads<S::in_flight(u)>();
@@ -545,7 +551,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
         });
         dqp = dq[kCT - 1];
       });
+      if constexpr (S::ALONE && last && means_last) read_means();
       if constexpr (last && means_last) add_means();
+      if constexpr (S::ALONE) {
+        wait_loads<S::in_flight(u)>();
+        lds_barrier();
+      }
       abuf = anext;
       if constexpr (last) sbuf = snext;
     });
