@@ -116,8 +116,13 @@ def test_two_streams_that_store_the_result_themselves(ctx, orc, fmt, m, k, n):
     w = synth.normal(2013, k * n, 0.02).reshape(k, n)
     x, d = synth.normal(2014, m * k).reshape(m, k), synth.normal(2015, m * n).reshape(m, n)
     wt = ctx.weight(fmt, w)
-    want = orc.matmul_f32(x, orc.dequantize(fmt, orc.quantize(fmt, w), k, n), d).astype(np.float64)
-    orc.assert_close(run(ctx, x, wt, d=d), want, 1e-3, 1e-4)
+    want = x.astype(np.float64) @ orc.dequantize(fmt, orc.quantize(fmt, w), k, n).astype(np.float64)
+    got = run(ctx, x, wt)
+    assert_rows_close(got, want, x, k)
+    added = run(ctx, x, wt, d=d)
+    assert np.array_equal(added, got + d)
+    assert np.array_equal(run(ctx, x, wt, d=d, ops=(capi.UNARY_NEG, capi.UNARY_RELU)), np.maximum(-added, 0))
+    want += d
     orc.assert_close(run(ctx, x, wt, d=d, ops=(capi.UNARY_NEG, capi.UNARY_SILU)), -want / (1 + np.exp(want)), 1e-3, 1e-4)
     wt.free()
 
@@ -256,9 +261,11 @@ def test_q8_bias_leaves_a_sum_that_holds_it(ctx, orc, m, n):
     wt.free()
 
 
+# One, two and three blocks in K's last 128 elements (two halves of a Q4 stage), in the first stage and in later ones, whose ring slots wrap
 @pytest.mark.parametrize("fmt", [Q4, Q8])
-def test_infinite_rows_of_fp16_activations_stay_on_their_own(ctx, orc, fmt):
-    m, k, n = 40, 96, 70  # K ends in the middle of the 64 elements that are loaded at once
+@pytest.mark.parametrize("m,k,n", [(40, 96, 70), (40, 160, 70), (70, 448, 130), (97, 704, 300), (300, 576, 1000), (260, 1248, 500)])
+def test_infinite_rows_of_fp16_activations_stay_on_their_own(ctx, orc, fmt, m, k, n):
+    """K ends inside the elements that are loaded at once: what lies behind a row's end is the beginning of the next."""
     x = synth.normal(2030, m * k).reshape(m, k).astype(np.float16)
     wt = ctx.weight(fmt, synth.normal(2031, k * n, 0.02).reshape(k, n))
     clean = run(ctx, x, wt, True)
@@ -348,10 +355,14 @@ def test_every_workgroup(ctx, orc, fmt, f16, rows, cols, threads, m, k, n, parts
     assert_rows_close(got, want, x.astype(np.float32), k)
     if mixed:
         assert_small_slices(got, want, x, dq, small, 5, 7)
+    # Rows that are not finite, among them some that begin so, which the row in front reads behind its end where K fills no
+    # whole stage: inside a row tile, in the first row of one, at the far end of what is read
     y = x.copy()
-    y[0, 0], y[1, k - 1] = np.inf, np.nan
+    behind = max(1, -k % (128 if fmt == Q4 else 64))
+    y[0, 0], y[1, k - 1], y[5, 0], y[32, 1], y[m - 1, behind - 1] = np.inf, np.nan, np.inf, np.nan, np.inf
     bad = run(ctx, y, wt, f16)
-    assert not np.isfinite(bad[:2]).any() and np.array_equal(bits(bad[2:]), bits(got[2:]))
+    hit = np.isin(np.arange(m), (0, 1, 5, 32, m - 1))
+    assert not np.isfinite(bad[hit]).any() and np.array_equal(bits(bad[~hit]), bits(got[~hit]))
     d = synth.normal(2102, m * n).reshape(m, n)
     added = run(ctx, x, wt, f16, d=d)
     assert np.array_equal(added, got + d)
