@@ -24,9 +24,9 @@
 //     waves that meet such a row move their sums from scale to scale;
 //   * K parts for different workgroups, where the tiles do not fill the chip, meet in the workspace and are added
 //     in part order by a third launch.
-// Measured (weights from memory; before -> now, us, Q4; machines differ by 3 %): fp16 2048 x 4096 x 14336 589 -> 277
-// (867 TFLOP/s), f32 the same 1034 -> 455; f32 512 x 4096 x 14336 295 -> 120; f32 77 x 4096 x 14336 82 -> 40, 77 x 14336 x
-// 4096 98 -> 42.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.3
+// Measured (weights from memory; before -> now, us, Q4; machines differ by 3 %): fp16 2048 x 4096 x 14336 589 -> 263 (914
+// TFLOP/s), f32 the same 1034 -> 444; f32 512 x 4096 x 14336 295 -> 115; f32 77 x 4096 x 14336 82 -> 38, 77 x 14336 x
+// 4096 98 -> 40.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.3
 // times its issue cycles (LDS and barrier waits).
 #include <algorithm>
 #include <cmath>
@@ -157,8 +157,10 @@ struct BlockShape {
   // what it reads from there to the next barrier is substep i + 1's, and that one's stage.  So these must have
   // landed; the loads issued after the last of them may be in flight.  (With the barrier behind the last tile, the
   // next substep's first operands had to have landed a barrier earlier: at PD = 2 the loads of the very substep that
-  // ends, and their whole latency was waited for.  us, weights from memory: Q4 fp16 2048 x 4096 x 14336 290 -> 267, f32
-  // 478 -> 450; 77 x 4096 x 14336 Q4 40.7 -> 39.5, Q8 45.4 -> 41.3; level where PD is 3 already.)
+  // ends, and their whole latency was waited for.  us, weights from memory, both libraries in turn: Q4 fp16 2048 x 4096 x 14336
+  // 291 -> 263, 512 x 4096 x 14336 85 -> 79, f32 2048 471 -> 444; Q8 f32 1024 x 4096 x 14336 260 -> 230.  Over 364 sizes, medians by
+  // workgroup, 0.88 to 1.00 of the time at PD = 2 and 0.96 to 1.004 where PD is 3 or 4 already; single sizes up to 1.02: Q4 64 x 256
+  // f32, K of 160 to 640, and 32 x 256 fp16, K of 320 to 416.)
   // f32 activations hold the operands of one row tile: the last ones have been read when its first column tile begins, and a
   // wave may turn there or a tile later.  With PD = 3 the next substep's operands have landed by then, and what the later turn
   // waits for is the next quants, read behind the barrier and unpacked at the end of the same tile: workgroups of two row tiles per
@@ -416,7 +418,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
       // What the loads brought in behind the row's last block is another row's, or nothing's.  (Each wave clears the
       // rows that it reads, so that its own order suffices; waves that share rows write the same zeros.  Block 0,
       // whose first operands are in registers by now, is always the row's own.  Cleared substep by substep, behind the
-      // barriers inside the loop, the branch there costs the 128 x 64 tiles 250 spilled registers.)
+      // barriers inside the loop, the branch there costs the 128 x 64 tiles 250 spilled registers.  The wait and the barrier
+      // cost a call 0.1 to 0.3 us, which shows where K is short: Q4 32 x 256, 326 x 352 x 7680 12.8 -> 13.0, 1240 x 416 x 3299 15.8 -> 16.0;
+      // to leave in flight what need not have landed, at PD = 3, is level.)
       static_assert(F32A || NSUB <= 2, "one substep ahead has been requested");
       if constexpr (NSUB > 1) {
         wait_loads<0>();
@@ -604,8 +608,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
   if constexpr (WK > 1) {
     // The streams' sums meet in LDS: each stream keeps one of the two column tiles, hands the other one over and stores
     // what it kept, so that the exchange and the stores have all waves.  (Before, one stream's waves added up and stored
-    // both tiles when the other's had ended, 3.4 of a workgroup's 28 us.  us, before -> now: Q4 77 x 4096 x 14336 39.7 -> 38.8,
-    // 77 x 14336 x 4096 41.4 -> 40.9, 200 x 2048 x 8192 27.8 -> 27.4; Q8 77 x 4096 x 14336 40.9 -> 40.6; the 64-row shape level.)
+    // both tiles when the other's had ended, 3.4 of a workgroup's 28 us.  us, this step by itself: Q4 77 x 4096 x 14336 39.7 -> 38.8,
+    // 77 x 14336 x 4096 41.4 -> 40.9; with the barrier in front of the last tile, on another machine, 38.9 -> 37.6, 42.1 -> 40.4, Q8 42.9 -> 39.5,
+    // 43.9 -> 41.1; the 64-row shape level.)
     static_assert(WK == 2 && kCT == 2 && (WM * WN & (WM * WN - 1)) == 0, "a column tile per stream, and the other stream's wave a bit away");
     float* const red = (float*)lds4;
     const uint32_t other = wave ^ (WM * WN);
@@ -838,7 +843,10 @@ __global__ __launch_bounds__(256) void add_parts_kernel(const float* __restrict_
 // ---- plans ----
 // The workgroup shapes that are built, by (format, activations): rows x columns per workgroup and what a
 // stage costs on them, in us per 128 elements of K: one workgroup per CU on all 256 (t1), and each
-// further round of 256 (tn; where two fit a CU, what the second costs beside the first).
+// further round of 256 (tn; where two fit a CU, what the second costs beside the first).  Fitted before the barriers moved in front
+// of the last tiles: the estimates made of them are now, median by workgroup over 364 sizes, 0.97 to 1.27 times what is measured (most
+// of it one workgroup per CU with K in one part; 2048 x 4096 x 14336 Q4 fp16 337 against 263, f32 512 x 4096 x 14336 163, 115,
+// 77 x 4096 x 14336 48, 38, 1500 x 1024 x 14336 110, 106).  An estimate that is too high leaves a call to the kernel behind.
 struct BlockConfig {
   void (*kernel)(BlockArgs);
   uint32_t rows, cols, threads, streams;

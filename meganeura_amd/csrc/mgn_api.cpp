@@ -158,10 +158,12 @@ double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool* steady) {
 
 // The automatic choice: the above, or the blocked kernel where it is expected to be the faster one.  (It
 // costs a launch to prepare the activations, one to add up K parts if there are any, and about 5 us
-// besides, but multiplies two to three times as fast: f32 512 x 4096 x 14336 295 -> 123 us, fp16 2048 x 4096 x
-// 14336 527 -> 283, 77 x 14336 x 4096 83 -> 47 with Q8, while 128 x 1024 x 3072 stays at 10 against 15.  Its own estimate
+// besides, but multiplies two to three times as fast: f32 512 x 4096 x 14336 295 -> 115 us, fp16 2048 x 4096 x
+// 14336 527 -> 263, 77 x 14336 x 4096 83 -> 41 with Q8, while 128 x 1024 x 3072 stays at 10 against 15.  Its own estimate
 // is made for weights that come from memory, the fit above for weights in the caches: hence 0.92.
-// Of the 480 calls 22 end up on a kernel more than 6 % slower than the better one.)  `choice`: the plan, if it does.
+// Of 1652 other calls, 17 to 2048 rows, K 32 to 8192 and N 64 to 30000, 405 take it, 20 of them more than 3 % slower than on the kernel
+// behind, and 77 do not though it is more than 3 % faster: above all narrow results of long K, for which basic_us is far too
+// low, 743 x 5344 x 243 23 against 61.)  `choice`: the plan, if it does.
 // Not so where the other kernel is the resident one with one pair of tiles per wave: small weights, which take it the
 // same time a round from wherever they come.  (Blocked and resident, us: Q8 f32 22 x 1760 x 1307 14.1, 11.4, 17 x 768 x 579
 // 10.1, 8.8; short K: Q4 f32 470 x 192 x 275 9.6, 6.4, Q4 fp16 145 x 160 x 105 8.6, 4.2.)
