@@ -24,7 +24,7 @@
 //     waves that meet such a row move their sums from scale to scale;
 //   * K parts for different workgroups, where the tiles do not fill the chip, meet in the workspace and are added
 //     in part order by a third launch.
-// Measured (weights from memory; before -> now, us, Q4; machines differ by 3 %): fp16 2048 x 4096 x 14336 589 -> 263 (914
+// Measured (weights from memory; before -> now, us, Q4; machines differ by 4 %): fp16 2048 x 4096 x 14336 589 -> 263 (914
 // TFLOP/s), f32 the same 1034 -> 444; f32 512 x 4096 x 14336 295 -> 115; f32 77 x 4096 x 14336 82 -> 38, 77 x 14336 x
 // 4096 98 -> 40.  What remains on the large call: 448 workgroups on 256 CUs are 1.75 rounds, and a SIMD needs 1.3
 // times its issue cycles (LDS and barrier waits).
@@ -844,9 +844,9 @@ __global__ __launch_bounds__(256) void add_parts_kernel(const float* __restrict_
 // The workgroup shapes that are built, by (format, activations): rows x columns per workgroup and what a
 // stage costs on them, in us per 128 elements of K: one workgroup per CU on all 256 (t1), and each
 // further round of 256 (tn; where two fit a CU, what the second costs beside the first).  Fitted before the barriers moved in front
-// of the last tiles: the estimates made of them are now, median by workgroup over 364 sizes, 0.97 to 1.27 times what is measured (most
-// of it one workgroup per CU with K in one part; 2048 x 4096 x 14336 Q4 fp16 337 against 263, f32 512 x 4096 x 14336 163, 115,
-// 77 x 4096 x 14336 48, 38, 1500 x 1024 x 14336 110, 106).  An estimate that is too high leaves a call to the kernel behind.
+// of the last tiles: the estimates made of them are now, median by workgroup over 364 sizes, 0.97 to 1.27 times what is measured
+// (2048 x 4096 x 14336 Q4 fp16 337 against 263, f32 512 x 4096 x 14336 163 against 115, 77 x 4096 x 14336 48 against 38, 1500 x 1024 x 14336
+// 110 against 106).  An estimate that is too high leaves a call to the kernel behind.
 struct BlockConfig {
   void (*kernel)(BlockArgs);
   uint32_t rows, cols, threads, streams;
