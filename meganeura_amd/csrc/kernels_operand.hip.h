@@ -41,27 +41,18 @@ __device__ __forceinline__ half8 bytes_to_operand(uint32_t w0, uint32_t w1) {
                   __builtin_amdgcn_perm(0u, u1, 0x0c010c00u), __builtin_amdgcn_perm(0u, u1, 0x0c030c02u));
 }
 
-// Power of two that brings a row slice's largest magnitude into [2^TOP, 2^(TOP+1)) (1 if the
-// slice is all zero or tiny).  *inv gets the reciprocal.  A slice that holds an infinity or a
-// magnitude of 2^100 and more is not rescaled and its reciprocal is a NaN: the truncating fp16
+// Power of two that brings a row slice's largest magnitude (not negative) into [2^TOP, 2^(TOP+1)) (1 if the
+// slice is all zero or tiny).  *inv gets the reciprocal.  Of a slice that holds an infinity, a NaN or a
+// magnitude of 2^100 and more the reciprocal is a NaN: the truncating fp16
 // conversion would clamp such values to 65504 and the row would come out finite and wrong, so
 // the row's sums over that slice are made non-finite instead (the f32 arithmetic of the
 // reference overflows or loses all precision at that magnitude).
 template <int TOP>
 __device__ __forceinline__ float slice_scale(float amax, float* inv) {
-  const uint32_t bits = __builtin_bit_cast(uint32_t, amax);
-  const int e = (int)(bits >> 23) - 127;  // floor(log2(amax)) for normal values
-  if (bits == 0 || e <= -100) {
-    *inv = 1.0f;
-    return 1.0f;
-  }
-  if (e >= 100) {
-    *inv = __builtin_nanf("");
-    return 1.0f;
-  }
-  const int sh = TOP - e;
-  *inv = __builtin_bit_cast(float, (uint32_t)(127 - sh) << 23);
-  return __builtin_bit_cast(float, (uint32_t)(127 + sh) << 23);
+  const uint32_t e = __builtin_bit_cast(uint32_t, amax) >> 23;  // floor(log2(amax)) + 127 for normal values
+  const uint32_t f = e <= 27 ? 127 + TOP : e;
+  *inv = e >= 227 ? __builtin_nanf("") : __builtin_bit_cast(float, (f - TOP) << 23);
+  return __builtin_bit_cast(float, (254 + TOP - f) << 23);
 }
 
 // Lanes (c, g), c = lane % 16, g = lane / 16: component j of lane (c, g) <- component g of lane (c, j)

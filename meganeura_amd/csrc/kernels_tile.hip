@@ -30,6 +30,11 @@
 //     With f32 activations a slice's P is multiplied by the rows' inverse power-of-two scales
 //     before it is added to the accumulators.
 //
+// What a task of the conversion costs, 120 vector instructions to begin with, is 45 % of a workgroup's life at M = 16: magnitudes
+// compare as integers, rows past M and what lies past K come as zeros from the descriptor instead of by a select per
+// element, and the 16-lane rows meet by a row swap.  100 instructions; us, 512 x 1024 x 3072 Q4 f32 16.9 -> 16.6, 333 x 1024 x 3072
+// Q8 12.8 -> 12.3, 32 x 4096 x 4096 Q4 11.6 -> 11.15, 16 x 4096 x 49152 Q4 38.1 -> 37.6.
+//
 // Two kernels share this arithmetic.
 //   tile_mfma_kernel (any M): image_kernel converts the activations ONCE per call into images
 //     in the workspace, which every workgroup copies into LDS slice by slice, double-buffered.
@@ -69,14 +74,21 @@ struct AddLift {
   }
 };
 
-// max over aligned groups of 32 consecutive lanes (every lane ends with the group's maximum)
-__device__ __forceinline__ float group_max32(float v) {
-  v = fmaxf(v, dpp_move<kDppQuadXor1>(v));
-  v = fmaxf(v, dpp_move<kDppQuadXor2>(v));
-  v = fmaxf(v, dpp_move<kDppRowHalfMirror>(v));
-  v = fmaxf(v, dpp_move<kDppRowMirror>(v));
-  v = fmaxf(v, __shfl_xor(v, 16, 64));
-  return v;
+// max over aligned groups of 32 consecutive lanes (every lane ends with the group's maximum).  Magnitudes compare as the
+// integers they are stored as: no quieting of each operand as with fmaxf, a move and a maximum in one instruction, and the rows of 16
+// lanes meet without a trip through LDS.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t v) {
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ uint32_t group_max32(uint32_t v) {
+  v = dpp_max<kDppQuadXor1>(v);
+  v = dpp_max<kDppQuadXor2>(v);
+  v = dpp_max<kDppRowHalfMirror>(v);
+  v = dpp_max<kDppRowMirror>(v);
+  u32x2_t s = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  asm("" : "+v"(s.x), "+v"(s.y));  // (left alone, the compiler has taken the two results for one)
+  return max(s.x, s.y);
 }
 
 // ---- the activation image ----
@@ -121,25 +133,39 @@ __device__ __forceinline__ void load_task(const void* __restrict__ a, size_t ele
   }
 }
 
+// The same through a buffer descriptor, which gives zeros for what lies past its end.
+template <bool F32A>
+__device__ __forceinline__ void load_task(__amdgpu_buffer_rsrc_t src, uint32_t off, TaskWords<F32A>& x) {
+#pragma unroll
+  for (int j = 0; j < (F32A ? 2 : 1); j++) {
+    const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(src, off + 16 * j, 0, 0);
+    x.w[4 * j] = v.x, x.w[4 * j + 1] = v.y, x.w[4 * j + 2] = v.z, x.w[4 * j + 3] = v.w;
+  }
+}
+
 // One task of the conversion: half-wave lane l = kb * 4 + g turns the 8 activations k0 .. k0 + 7
 // (k0 = 256 slice + 32 kb + 8 g) of row `row` into its piece of the image `img` of that (row tile,
 // slice); r = row % 16.  All 32 lanes of the half-wave (one row of one slice) must call it together.
 template <int FMT, bool F32A>
-__device__ __forceinline__ void convert_task(const TaskWords<F32A>& xin, bool ok, uint4* __restrict__ img, uint32_t r, uint32_t l) {
+__device__ __forceinline__ void convert_task(const TaskWords<F32A>& xin, bool ok, uint4* __restrict__ img, uint32_t r, uint32_t l,
+                                             bool eight_rows = false) {
   constexpr uint32_t HL = F32A ? 2 : 1;
   const uint32_t kb = l >> 2, g = l & 3;
   const uint32_t alane = image_slot(r, g, kb & 1);
   float s, inv = 1.0f;
   if constexpr (F32A) {
     float x[8];
+    uint32_t am = 0;
 #pragma unroll
-    for (int e = 0; e < 8; e++) x[e] = ok ? __builtin_bit_cast(float, xin.w[e]) : 0.0f;
-    // NaN never wins fmaxf; an infinity does and switches scaling off
-    float am = fmaxf(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))),
-                     fmaxf(fmaxf(fabsf(x[4]), fabsf(x[5])), fmaxf(fabsf(x[6]), fabsf(x[7]))));
+    for (int e = 0; e < 8; e++) {
+      const uint32_t w = ok ? xin.w[e] : 0u;
+      x[e] = __builtin_bit_cast(float, w);
+      am = max(am, w & 0x7FFFFFFFu);
+    }
+    // an infinity or a NaN switches scaling off, and the row's sums over the slice come out non-finite
     am = group_max32(am);
     constexpr bool kSplit = FMT == MGN_FMT_Q4;
-    const float scale = slice_scale<kSplit ? 7 : 11>(am, &inv);
+    const float scale = slice_scale<kSplit ? 7 : 11>(__builtin_bit_cast(float, am), &inv);
 #pragma unroll
     for (int e = 0; e < 8; e++) x[e] *= (kSplit && e % 2 == 0) ? scale * 16.0f : scale;
     float p[8];
@@ -190,10 +216,13 @@ __device__ __forceinline__ void convert_task(const TaskWords<F32A>& xin, bool ok
     if (g == 0) extra[(r + 16 * (kb >> 2)) * 4 + (kb & 3)] = (mh & 0xFFFFu) | (pack_rtz((mean - half_lo(mh)) * 2048.0f, 0.0f) << 16);
     return;
   }
-  if (g == 0) extra[(r + 16 * (kb >> 2)) * 4 + (kb & 3)] = (mh & 0xFFFFu) | (pack_rtz(mean - half_lo(mh), 0.0f) << 16);
-  // lanes (row, g' >= 2) of the additive operand stay zero (8 dwords per half-wave lane... 16 rows x 32
-  // lanes cover the 128 dwords); the rows' inverse scales, times the quants' operand scale, follow
-  if (l < 8) extra[32 * 4 + r * 8 + l] = 0u;
+  // lanes (row, g' >= 2) of the additive operand stay zero (128 dwords: 8 from each of 16 rows, or 16 from each of 8 that are
+  // converted); the rows' inverse scales, times the quants' operand scale, follow
+  if (g == 0) {
+    extra[(r + 16 * (kb >> 2)) * 4 + (kb & 3)] = (mh & 0xFFFFu) | (pack_rtz(mean - half_lo(mh), 0.0f) << 16);
+    if (eight_rows) *(uint2*)(extra + 32 * 4 + r * 16 + kb * 2) = make_uint2(0u, 0u);
+    else extra[32 * 4 + r * 8 + kb] = 0u;
+  }
   if (l == 0) ((float*)extra)[64 * 4 + r] = inv * (FMT == MGN_FMT_Q4 ? 1048576.0f : 16777216.0f);
 }
 
@@ -332,6 +361,7 @@ struct TileTail {  // arguments first needed in the epilogue
   uint32_t* fault_flag;
   uint32_t spread;  // resident kernel: every part adds up a share of the tiles (all workgroups of the launch resident)
   AddLift lift;     // (needed in the walk; rides along here)
+  uint32_t rows;    // KS > 1: rows of a row group, 8 or 16
 };
 
 constexpr int park_stride(int fmt) { return fmt == MGN_FMT_Q4 ? 8 * 16 + 16 : 8 * 32 + 16; }  // bytes per parked column
@@ -759,6 +789,92 @@ constexpr int resident_slices(bool f32a, int r) { return f32a && r == 2 ? 2 : 4;
 // a tile fall into different LDS banks.
 __host__ __device__ constexpr uint32_t meta_stride(int fmt, uint32_t nsl) { return nsl * kSliceBlocks * (fmt == MGN_FMT_Q4 ? 4 : 2) + 16; }
 
+// The end of a launch whose waves split K (KS of them share a pair of column tiles; `strip`: this wave's own piece of LDS,
+// which nobody reads any more): the sums meet in LDS, wave w takes tile w of the workgroup and adds up in the order of ks; K parts of
+// other workgroups meet as in the resident kernel's shares (all workgroups of the launch are resident): tile T
+// belongs to part T % parts.  `m`: the end of the workgroup's rows.
+template <int KS>
+__device__ __forceinline__ void split_tail(const floatx4 (&own)[kSide], uint8_t* strip, uint32_t strip_bytes, uint32_t wave, uint32_t lane,
+                                           uint32_t part, uint32_t parts, uint32_t group, uint32_t groups, uint32_t row0, uint32_t col0,
+                                           uint32_t m, uint32_t n, const TileTail& tail) {
+  constexpr uint32_t TILES = 8 / KS * kSide;
+  constexpr int kDeviceScope = 16;
+  const uint32_t c = lane & 15, g = lane >> 4;
+  float dv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto load_residual = [&](uint32_t tile) __attribute__((always_inline)) {
+    const uint32_t col = col0 + tile * 16 + c;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (row0 + 4 * g + i < m && col < n) dv[i] = tail.dres[(size_t)(row0 + 4 * g + i) * n + col];
+  };
+#pragma unroll
+  for (int u = 0; u < kSide; u++) ((floatx4*)strip)[u * 64 + lane] = own[u];
+  if (parts == 1 && tail.dres && wave < TILES) load_residual(wave);  // (travels while the waves meet)
+  lds_barrier();
+  if (wave >= TILES) return;
+  uint32_t tile = wave;
+  const uint8_t* const first = strip - wave * strip_bytes + wave / kSide * KS * strip_bytes;
+  floatx4 sum = ((const floatx4*)first)[wave % kSide * 64 + lane];
+#pragma unroll
+  for (int k = 1; k < KS; k++) sum += ((const floatx4*)(first + k * strip_bytes))[wave % kSide * 64 + lane];
+  if (parts > 1) {
+    const uint32_t part_stride = groups * (TILES * 1024u);
+    const __amdgpu_buffer_rsrc_t all_parts = __builtin_amdgcn_make_buffer_rsrc(tail.handover, 0, parts * part_stride, 0x00020000);
+    u32x4_t v = __builtin_bit_cast(u32x4_t, sum);
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = v[i] == kHandoverEmpty ? 0x7FC00000u : v[i];
+    __builtin_amdgcn_raw_buffer_store_b128(v, all_parts, part * part_stride + (group * TILES + wave) * 1024u + lane * 16u, 0, kDeviceScope);
+    tile = part + wave * parts;  // (the last one of this wave: there are no more waves than tiles)
+    if (tile >= TILES) return;
+    if (tail.dres) load_residual(tile);
+    const uint32_t off = (group * TILES + tile) * 1024u + lane * 16u;
+    sum = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    bool gave_up = false;
+    constexpr uint32_t PG = 4;
+    const u32x4_t empty4 = {kHandoverEmpty, kHandoverEmpty, kHandoverEmpty, kHandoverEmpty};
+    for (uint32_t p0 = 0; p0 < parts; p0 += PG) {
+      uint32_t w[PG][4];  // (scalars, as in the resident kernel's polling loop)
+#pragma unroll
+      for (uint32_t j = 0; j < PG; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) w[j][i] = kHandoverEmpty;
+      for (uint32_t polls = 0;; polls++) {
+        if (polls >= tail.spin_limit) {  // (a limit of 0 looks at nothing: the give-up path, for tests)
+          gave_up = true;
+          break;
+        }
+        bool missing = false;
+#pragma unroll
+        for (uint32_t j = 0; j < PG; j++) {
+          // (the surplus repeats the last part: a branch here would put the loads one behind the other)
+          const u32x4_t x4 = __builtin_amdgcn_raw_buffer_load_b128(all_parts, min(p0 + j, parts - 1) * part_stride + off, 0, kDeviceScope);
+          w[j][0] = x4.x, w[j][1] = x4.y, w[j][2] = x4.z, w[j][3] = x4.w;
+          missing |= x4.x == kHandoverEmpty || x4.y == kHandoverEmpty || x4.z == kHandoverEmpty || x4.w == kHandoverEmpty;
+        }
+        if (!__builtin_amdgcn_ballot_w64(missing)) break;
+        __builtin_amdgcn_s_sleep(1);
+        asm volatile("" ::: "memory");  // the loads are issued anew on every round
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < PG; j++) {
+        if (p0 + j < parts) {  // uniform
+#pragma unroll
+          for (int i = 0; i < 4; i++) sum[i] += __builtin_bit_cast(float, w[j][i]);
+          __builtin_amdgcn_raw_buffer_store_b128(empty4, all_parts, (p0 + j) * part_stride + off, 0, kDeviceScope);
+        }
+      }
+    }
+    if (gave_up && lane == 0 && tail.fault_flag) *tail.fault_flag = 1u;
+  }
+  const uint32_t col = col0 + tile * 16 + c;
+  if (col >= n) return;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint32_t row = row0 + 4 * g + i;
+    if (row < m) tail.c[(size_t)row * n + col] = apply_epilogue(tail.dres ? sum[i] + dv[i] : sum[i], tail.epilogue);
+  }
+}
+
 // What a launch has besides its first weight (ROWS form: up to three weights that share their activations,
 // and what the activations go through on their way into the images).
 struct RowsExtra {
@@ -783,26 +899,28 @@ constexpr int kRowsPlain = -1;
 // fill the rounds that each would leave open.  Two decoder layers of 333 rows, 1024 wide (Q8), q | k | v, the
 // output projection, gate | up and down with norms and SwiGLU: 18 launches, 213 us -> 8 launches, 161 us (Q4 184
 // -> 139; 128 rows, 576 wide 156 -> 104; 8 rows Q4 138 -> 90).
-template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain>
+template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1>
 __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restrict__ a, const void* __restrict__ meta_arg,
                                                              const void* __restrict__ quants_arg, uint32_t m, uint32_t kdim,
                                                              uint32_t n, uint32_t parts, uint32_t nslices, uint32_t colgroups,
                                                              TileTail tail, RowsExtra extra) {
   static_assert(ROWS == kRowsPlain || (F32A && R == 1 && !LATE), "the forms that are launched");
+  static_assert(KS == 1 || (R == 1 && Q == 1 && PARK && !LATE), "the forms that are launched");
   constexpr uint32_t UNITS = image_units(F32A);
   constexpr float kOpScale = FMT == MGN_FMT_Q4 ? 1048576.0f : 16777216.0f;
   constexpr int QB = FMT == MGN_FMT_Q4 ? 16 : 32;
   constexpr int MB = FMT == MGN_FMT_Q4 ? 4 : 2;
   constexpr int NLQ = QB / 8;
   constexpr int NSL = resident_slices(F32A, R);
-  constexpr int STEPS = NSL * Q;  // step f of the walk = (pair f / NSL, slice f % NSL)
-  constexpr int DEPTH = 1;        // steps whose quants are in flight ahead of the one in use
+  constexpr int SPW = NSL / KS;   // slices of the part that a wave walks
+  constexpr int STEPS = SPW * Q;  // step f of the walk = (pair f / NSL, slice f % NSL), or the wave's slice f
+  constexpr int DEPTH = KS > 1 ? STEPS : 1;  // steps whose quants are in flight ahead of the one in use
   constexpr int SLOTS = DEPTH + 1;
   constexpr int NT = NSL * R;     // conversion tasks per half-wave
   // 16-byte units of scale words a lane stages: Q pairs x 32 columns x NSL slices x (32 or 16) bytes / 64 lanes
-  constexpr int MU = Q * NSL * MB / 4;
-  constexpr uint32_t kUnitsPerColumn = NSL * kSliceBlocks * MB / 16;
-  constexpr uint32_t mstride = meta_stride(FMT, NSL);
+  constexpr int MU = (Q * SPW * MB + 3) / 4;
+  constexpr uint32_t kUnitsPerColumn = SPW * kSliceBlocks * MB / 16;
+  constexpr uint32_t mstride = meta_stride(FMT, SPW);
   extern __shared__ uint4 lds4[];
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -812,9 +930,10 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   // one XCD, which their hand-over below measures 0.5 us better than spread over all eight
   const uint32_t part = blockIdx.y;
   const uint32_t rg = blockIdx.x / colgroups, cg = blockIdx.x - rg * colgroups;
-  const uint32_t rowgroups = (m + R * 16 - 1) / (R * 16);
-  if (rg >= rowgroups) return;            // padding of the grid
-  const uint32_t row0 = rg * (R * 16);    // first row of this workgroup's row group
+  const uint32_t group_rows = KS > 1 ? tail.rows : R * 16;
+  const uint32_t rowgroups = (m + group_rows - 1) / group_rows;
+  if (rg >= rowgroups) return;             // padding of the grid
+  const uint32_t row0 = rg * group_rows;   // first row of this workgroup's row group
   const uint32_t bpc = kdim / 32;
   uint32_t wcg = cg;  // the column group within its weight
   if constexpr (ROWS != kRowsPlain) {
@@ -826,7 +945,8 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
         wcg = cg - extra.item[j].cg_first;
       }
   }
-  const uint32_t pair0 = (wcg * 8 + wave) * Q;  // this wave's first pair of column tiles
+  const uint32_t ks = KS > 1 ? wave % KS : 0;  // KS waves share a pair of column tiles, each with a run of the part's slices
+  const uint32_t pair0 = KS > 1 ? wcg * (8 / KS) + wave / KS : (wcg * 8 + wave) * Q;  // this wave's first pair of column tiles
   const uint32_t sl0 = part * NSL;             // first slice of this part
   uint4* const img = lds4;                     // [NSL][R][UNITS]
   // this wave's scale words: [Q pairs x 32 columns][mstride bytes]
@@ -836,24 +956,38 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   uint8_t* const wpark = (uint8_t*)(lds4 + NSL * R * UNITS) + 8 * (Q * 32 * mstride) + wave * (kSide * 16 * kStride);
 
   // ---- the part's activations: loads first, so that nothing queues in front of them ----
-  // Task (s, rr): half-wave r converts row 16 rr + r of slice sl0 + s.
-  const uint32_t cr = tid >> 5, cl = tid & 31;
+  // Task (s, rr): half-wave r converts row 16 rr + r of slice sl0 + s.  (KS > 1: only slices that there are, and of a row
+  // group of up to 8 rows the two half-waves of a wave take the even and the odd slices of one row.)
+  const uint32_t live_slices = min((uint32_t)NSL, nslices - sl0);
+  const uint32_t run = (live_slices + KS - 1) / KS;  // slices of a wave (at most SPW)
+  const uint32_t wsl = KS > 1 ? ks * run : 0;        // the wave's first slice of the part
+  const bool two_per_row = KS > 1 && min(m - row0, group_rows) <= 8;
+  const uint32_t cr = two_per_row ? tid >> 6 : tid >> 5, cl = tid & 31;
+  const uint32_t tasks = KS == 1 ? (uint32_t)NT : two_per_row ? (live_slices + 1) / 2 : live_slices;  // (uniform)
+  auto task_slice = [&](int t) __attribute__((always_inline)) { return two_per_row ? 2 * t + (lane >> 5) : (uint32_t)(t / R); };
+  // (The row group through a descriptor of its own: rows past M and what lies past K read as zeros.)
+  constexpr uint32_t AB = F32A ? 4 : 2, kPast = 0x80000000u;
+  const uint32_t a_pitch = (ROWS == kProSwiglu ? 2 * kdim : kdim) * AB;
+  const __amdgpu_buffer_rsrc_t a_src =
+      __builtin_amdgcn_make_buffer_rsrc((char*)const_cast<void*>(a) + (size_t)row0 * a_pitch, 0, min(m - row0, group_rows) * a_pitch, 0x00020000);
+  auto task_off = [&](int t) __attribute__((always_inline)) {
+    const uint32_t k0 = (sl0 + task_slice(t)) * 256 + cl * 8;
+    return k0 < kdim ? (t % R * 16 + cr) * a_pitch + k0 * AB : kPast;
+  };
   TaskWords<F32A> xin[NT];
-  bool xok[NT];
 #pragma unroll
   for (int t = 0; t < NT; t++) {
-    const uint32_t s = t / R, rr = t % R;
-    const uint32_t row = row0 + rr * 16 + cr, k0 = (sl0 + s) * 256 + cl * 8;
-    xok[t] = row < m && k0 < kdim;
-    load_task<F32A>(a, xok[t] ? (size_t)row * (ROWS == kProSwiglu ? 2 * kdim : kdim) + k0 : (size_t)0, xin[t]);
+    if (KS > 1 && (uint32_t)t >= tasks) break;
+    load_task<F32A>(a_src, task_off(t), xin[t]);
   }
   TaskWords<true> xtwo[ROWS == kProRmsNorm || ROWS == kProSwiglu ? NT : 1];  // the norm's weights, or up beside gate
   if constexpr (ROWS == kProRmsNorm || ROWS == kProSwiglu) {
+    const __amdgpu_buffer_rsrc_t norm_src = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(extra.norm_w), 0, kdim * 4, 0x00020000);
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-      const uint32_t row = row0 + cr, k0 = (sl0 + t) * 256 + cl * 8;
-      if constexpr (ROWS == kProRmsNorm) load_task<true>(extra.norm_w, xok[t] ? (size_t)k0 : (size_t)0, xtwo[t]);
-      else load_task<true>(a, xok[t] ? (size_t)row * 2 * kdim + kdim + k0 : (size_t)0, xtwo[t]);
+      if (KS > 1 && (uint32_t)t >= tasks) break;
+      if constexpr (ROWS == kProRmsNorm) load_task<true>(norm_src, ((sl0 + task_slice(t)) * 256 + cl * 8) * 4, xtwo[t]);
+      else load_task<true>(a_src, task_off(t) + kdim * 4, xtwo[t]);
     }
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -869,7 +1003,7 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
       const uint32_t id = 64 * j + lane;
       const uint32_t wcol = id / kUnitsPerColumn, unit = id % kUnitsPerColumn;
       const uint32_t col = min(pair0 * (kSide * 16) + wcol, n - 1);
-      const uint8_t* src = (const uint8_t*)meta_arg + ((size_t)col * bpc + (size_t)sl0 * kSliceBlocks) * MB + unit * 16;
+      const uint8_t* src = (const uint8_t*)meta_arg + ((size_t)col * bpc + (size_t)(sl0 + wsl) * kSliceBlocks) * MB + unit * 16;
       typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
       const u32x4_a2 v = *(const u32x4_a2*)src;
       mu[j] = u32x4_t{v.x, v.y, v.z, v.w};
@@ -897,7 +1031,9 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
       }
     }
   auto fetch = [&](int f) {  // step f into slot f % SLOTS
-    const uint8_t* const qb = (const uint8_t*)quants_arg + (size_t)((sl0 + f % NSL) * kSliceBlocks) * QB;
+    const uint32_t sl = sl0 + (KS > 1 ? wsl + f : f % NSL);
+    if (KS > 1 && ((uint32_t)f >= run || sl >= nslices)) return;
+    const uint8_t* const qb = (const uint8_t*)quants_arg + (size_t)(sl * kSliceBlocks) * QB;
 #pragma unroll
     for (int u = 0; u < kSide; u++)
 #pragma unroll
@@ -916,7 +1052,13 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   // same the weights requested in between only stand in their way: fp16 512 x 1024 x 3072 11.23 ->
   // 10.93 us, 512 x 3072 x 1024 14.22 -> 14.0.  (On half a chip the early request wins: M = 64 on
   // 4096 x 4096, 128 workgroups, 10.2 against 10.45 us; and with f32 activations a later one loses.)
+  // (KS > 1: a launch that leaves CUs idle; all of a wave's quants are on their way before the conversion.)
   constexpr int kFirstFetchAfterTask = NT > 1 ? (LATE ? NT - 1 : 1) : 0;
+  if constexpr (KS > 1) {
+#pragma unroll
+    for (int f = 0; f < STEPS; f++) fetch(f);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   auto word = [](uint32_t w) __attribute__((always_inline)) { return __builtin_bit_cast(float, w); };
   float rinv = 1.0f;
   if constexpr (ROWS == kProRmsNorm) {
@@ -926,15 +1068,17 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
     for (int t = 0; t < NT; t++)
 #pragma unroll
       for (int e = 0; e < 8; e++) {
-        const float v = xok[t] ? word(xin[t].w[e]) : 0.0f;
+        const float v = (uint32_t)t < tasks ? word(xin[t].w[e]) : 0.0f;
         ss = __fmaf_rn(v, v, ss);
       }
 #pragma unroll
     for (int d = 16; d > 0; d >>= 1) ss += __shfl_xor(ss, d, 32);
+    if (two_per_row) ss += __shfl_xor(ss, 32, 64);
     rinv = 1.0f / sqrtf(ss / (float)kdim + extra.eps);
   }
 #pragma unroll
   for (int t = 0; t < NT; t++) {
+    if (KS > 1 && (uint32_t)t >= tasks) break;
     if constexpr (ROWS == kProRmsNorm) {
 #pragma unroll
       for (int e = 0; e < 8; e++) xin[t].w[e] = __builtin_bit_cast(uint32_t, word(xin[t].w[e]) * rinv * word(xtwo[t].w[e]));
@@ -942,17 +1086,19 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
 #pragma unroll
       for (int e = 0; e < 8; e++) xin[t].w[e] = __builtin_bit_cast(uint32_t, swiglu_act(word(xin[t].w[e]), word(xtwo[t].w[e])));
     }
-    convert_task<FMT, F32A>(xin[t], xok[t], img + t * UNITS, cr, cl);
+    if constexpr (KS > 1) convert_task<FMT, F32A>(xin[t], true, img + task_slice(t) * UNITS, cr, cl, two_per_row);
+    else convert_task<FMT, F32A>(xin[t], true, img + t * UNITS, cr, cl);
     __builtin_amdgcn_sched_barrier(0);
-    if (t >= kFirstFetchAfterTask && t - kFirstFetchAfterTask < DEPTH && t - kFirstFetchAfterTask < STEPS) fetch(t - kFirstFetchAfterTask);
+    if (KS == 1 && t >= kFirstFetchAfterTask && t - kFirstFetchAfterTask < DEPTH && t - kFirstFetchAfterTask < STEPS) fetch(t - kFirstFetchAfterTask);
     __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
-  for (int f = NT - kFirstFetchAfterTask; f < DEPTH && f < STEPS; f++) fetch(f);
+  for (int f = NT - kFirstFetchAfterTask; KS == 1 && f < DEPTH && f < STEPS; f++) fetch(f);
 #pragma unroll
   for (int j = 0; j < MU; j++) {
     const uint32_t id = 64 * j + lane;
-    *(u32x4_t*)(wmeta + (id / kUnitsPerColumn) * mstride + (id % kUnitsPerColumn) * 16) = mu[j];
+    if (Q * 32 * kUnitsPerColumn % 64 == 0 || id < Q * 32 * kUnitsPerColumn)
+      *(u32x4_t*)(wmeta + (id / kUnitsPerColumn) * mstride + (id % kUnitsPerColumn) * 16) = mu[j];
   }
   __builtin_amdgcn_sched_barrier(0);
   lds_barrier();
@@ -968,7 +1114,8 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   const bool pair_live[2] = {pair0 * (kSide * 16) < n, (pair0 + Q - 1) * (kSide * 16) < n};  // uniform over the wave
 #pragma unroll
   for (int f = 0; f < STEPS; f++) {
-    const int slot = f % SLOTS, wp = f / NSL, ws = f % NSL;
+    const int slot = f % SLOTS, wp = f / SPW, wf = f % SPW;
+    const uint32_t ws = KS > 1 ? wsl + f : (uint32_t)wf;  // slice of the part
     __builtin_amdgcn_sched_barrier(0);
     if (f + DEPTH < STEPS) fetch(f + DEPTH);
     __builtin_amdgcn_sched_barrier(0);
@@ -976,7 +1123,7 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
     uint32_t mw[kSide][8];
 #pragma unroll
     for (int u = 0; u < kSide; u++) {
-      const uint8_t* const ms = wmeta + ((wp * kSide + u) * 16 + c) * mstride + ws * (kSliceBlocks * MB);
+      const uint8_t* const ms = wmeta + ((wp * kSide + u) * 16 + c) * mstride + wf * (kSliceBlocks * MB);
       if constexpr (FMT == MGN_FMT_Q4) {
         const u32x4_t m0 = *(const u32x4_t*)ms, m1 = *(const u32x4_t*)(ms + 16);
         mw[u][0] = m0.x, mw[u][1] = m0.y, mw[u][2] = m0.z, mw[u][3] = m0.w;
@@ -1001,7 +1148,7 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
     }
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t sl_raw = sl0 + ws;
-    if (pair_live[wp == 0 ? 0 : 1] && sl_raw < nslices) {  // (with Q = 2, wp is 0 or 1)
+    if (pair_live[wp == 0 ? 0 : 1] && sl_raw < nslices && (KS == 1 || (uint32_t)f < run)) {  // (with Q = 2, wp is 0 or 1)
       const uint32_t kb0 = sl_raw * kSliceBlocks;
       if (kb0 + kSliceBlocks > bpc) {  // last slice of a K that is no multiple of 256
 #pragma unroll
@@ -1024,6 +1171,12 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   }
   __builtin_amdgcn_sched_barrier(0);
 
+  if constexpr (KS > 1) {
+    const floatx4 own[kSide] = {res[0][0][0], res[0][1][0]};
+    split_tail<KS>(own, wpark, kSide * 16 * kStride, wave, lane, part, parts, rg * colgroups + cg, rowgroups * colgroups, row0,
+                   wcg * (8 / KS * kSide * 16), min(m, row0 + group_rows), n, tail);
+    return;
+  }
   if (parts > 1) {
     // K parts of other workgroups.  The parts of a (column group, row group) run on one XCD (see the
     // grid above) and the part with the highest index is dispatched last, when the others are
@@ -1257,6 +1410,8 @@ AddLift add_lift(const WeightView& w) {
 }
 
 struct ResidentPlan {
+  uint32_t ks;  // waves that share a pair of column tiles
+  uint32_t rows;  // of a row group when ks > 1: 16, or 8 in half-empty tiles
   uint32_t r, q, nsl, parts, colgroups, rowgroups, nslices;
   bool park;  // quants through a wave-private LDS strip (if there is room) instead of row swaps
   bool spread;  // the K parts' tiles are added up by all parts, a share each (see the kernel)
@@ -1264,10 +1419,51 @@ struct ResidentPlan {
   double cost;
 };
 
-size_t resident_lds_bytes(int fmt, bool f32a, uint32_t r, uint32_t q, bool park) {
+size_t resident_lds_bytes(int fmt, bool f32a, uint32_t r, uint32_t q, bool park, uint32_t ks = 1) {
   const uint32_t nsl = resident_slices(f32a, r);
-  return (size_t)nsl * r * image_units(f32a) * 16 + (size_t)8 * q * 32 * meta_stride(fmt, nsl) +
+  return (size_t)nsl * r * image_units(f32a) * 16 + (size_t)8 * q * 32 * meta_stride(fmt, nsl / ks) +
          (park ? (size_t)8 * kSide * 16 * park_stride(fmt) : 0);
+}
+
+// A launch that leaves CUs idle spreads over more of them: KS waves share a pair of column tiles and split K between them
+// (KS = 2 or 4, no more than a part has slices), a workgroup has 1 / KS of the columns, and the walk, the longest stretch of
+// a workgroup's life, is 1 / KS as long; and where half as many rows to a row group still fit, the conversion is half as long (the tiles
+// are half empty then, which idle matrix cores do not mind).  In one round of resident workgroups only: every one converts its
+// activations anew.  A workgroup's cycles, 16 x 1024 x 1024 Q4 f32 (requests, wait, conversion, barrier, walk, sums and stores): 1210, 400, 3920,
+// 840, 11090, 1020 before, 1410, 400, 1710, 540, 2930, 1360 with KS = 4 and 8 rows.  us per call, launch included, one launch behind the other:
+// f32 6 x 864 x 3950 Q8 11.5 -> 7.0, 16 x 3328 x 351 Q4 10.3 -> 7.1, 24 x 640 x 272 Q4 8.3 -> 5.2, 40 x 1760 x 606 Q8 13.1 -> 8.6, 289 x 2624 x 211
+// Q4 10.5 -> 8.3; fp16, where it takes over from the 32x32 kernel, 5 x 576 x 7211 Q8 9.9 -> 5.8, 107 x 4000 x 256 Q8 13.0 -> 7.5, 16 x 3072 x 1073
+// Q4 10.1 -> 6.8.  200 drawn calls of 5 to 512 rows, 141 of which change: 0.74 of the time, medians 0.72.
+// KS = 2 gains less, and with K parts, which then meet in twice as many workgroups, it is level with Q4 (0.85 to 1.09, median 0.99) and with
+// Q8 in four parts or more (0.91 to 1.09); Q8 in two or three parts 0.92.  Q8 with fp16 activations and two slices stays on the 32x32
+// kernel: level (0.87 to 1.11), and that kernel's error is up to 3 % smaller there.  (From three slices on the error against f64 is the smaller
+// one here: medians Q4 0.90, behind a silu 0.72; Q8 0.97, 0.89.)
+void split_resident(const LaunchArgs& x, ResidentPlan* p) {
+  const bool f32a = !x.a_is_f16;
+  const uint32_t nsl = resident_slices(f32a, 1), parts = (p->nslices + nsl - 1) / nsl;
+  if (parts > 1 && x.shared_device) return;  // (the parts wait for each other)
+  if (!f32a && x.w.fmt == MGN_FMT_Q8 && p->nslices < 3) return;
+  for (uint32_t ks = 4; ks >= 2; ks /= 2) {
+    if (std::min(nsl, p->nslices) <= ks / 2) continue;
+    if (ks == 2 && parts > (x.w.fmt == MGN_FMT_Q4 ? 1u : 3u)) continue;
+    const uint32_t per_wg = 8 / ks * kSide;
+    auto groups_of = [&](uint32_t n) { return ((n + 15) / 16 + per_wg - 1) / per_wg; };
+    uint64_t colgroups = groups_of(x.w.n);
+    for (int j = 0; j < x.n_more; j++) colgroups += groups_of(x.more[j].w.n);
+    for (uint32_t rows = 8; rows <= 16; rows += 8) {
+      const uint32_t rowgroups = (x.m + rows - 1) / rows;
+      // (resident at once: see plan_resident)
+      if ((colgroups * rowgroups + 7) / 8 * parts > (uint64_t)x.num_cus / 8) continue;
+      const uint64_t partial = parts > 1 ? parts * rowgroups * colgroups * (per_wg * 1024u) : 0;
+      const size_t lds = resident_lds_bytes(x.w.fmt, f32a, 1, 1, true, ks);
+      if (partial > x.handover_bytes || lds > 160 * 1024) continue;
+      p->ks = ks, p->rows = rows, p->r = 1, p->q = 1, p->nsl = nsl, p->parts = parts;
+      p->colgroups = (uint32_t)colgroups, p->rowgroups = rowgroups;
+      p->park = true, p->spread = parts > 1, p->lds = lds, p->partial_bytes = partial;
+      p->cost = 1.5 + 1.0 / ks + (parts > 1 ? 1.0 : 0.0);
+      return;
+    }
+  }
 }
 
 // Row groups of 16 or 32 rows (32 only beyond 16 rows, and then with one pair per wave: registers), Q = 1 or 2 pairs
@@ -1321,7 +1517,7 @@ bool plan_resident(const LaunchArgs& x, ResidentPlan* out) {
       const double cost = std::ceil((double)wgs / x.num_cus) * (1.5 + q * r * nsl / 4.0) * (r == 2 ? 0.9 : 1.0) + (parts > 1 ? 1.0 : 0.0);
       if (best == 0 || cost < best) {
         best = cost;
-        bp.r = r, bp.q = q, bp.nsl = nsl, bp.parts = parts, bp.colgroups = colgroups, bp.rowgroups = rowgroups;
+        bp.ks = 1, bp.r = r, bp.q = q, bp.nsl = nsl, bp.parts = parts, bp.colgroups = colgroups, bp.rowgroups = rowgroups;
         bp.nslices = nslices, bp.partial_bytes = partial, bp.cost = cost, bp.spread = spread;
         bp.park = resident_lds_bytes(x.w.fmt, f32a, r, q, true) <= 160 * 1024;
         bp.lds = resident_lds_bytes(x.w.fmt, f32a, r, q, bp.park);
@@ -1329,20 +1525,21 @@ bool plan_resident(const LaunchArgs& x, ResidentPlan* out) {
     }
   }
   if (best == 0) return false;
+  if (x.split_waves) split_resident(x, &bp);
   *out = bp;
   return true;
 }
 
-template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain>
+template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1>
 int launch_resident_q(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& p) {
-  auto kern = tile_resident_kernel<FMT, F32A, R, Q, PARK, LATE, ROWS>;
+  auto kern = tile_resident_kernel<FMT, F32A, R, Q, PARK, LATE, ROWS, KS>;
   static std::atomic<uint64_t> big_lds_done{0};
   if (p.lds > 64 * 1024)
     if (int e = enable_big_lds(kern, x.device, big_lds_done)) return e;
-  const TileTail tail{x.d, x.c, (float*)x.scratch, x.counters, x.epilogue, (float*)x.handover, x.spin_limit, x.fault_flag, p.spread ? 1u : 0u, add_lift(x.w)};
+  const TileTail tail{x.d, x.c, (float*)x.scratch, x.counters, x.epilogue, (float*)x.handover, x.spin_limit, x.fault_flag, p.spread ? 1u : 0u, add_lift(x.w), p.rows};
   RowsExtra extra{};
   if constexpr (ROWS != kRowsPlain) {
-    constexpr uint32_t per_wg = 8 * kSide * Q;
+    constexpr uint32_t per_wg = 8 / KS * kSide * Q;
     uint32_t first = ((x.w.n + 15) / 16 + per_wg - 1) / per_wg;
     for (int j = 0; j < x.n_more; j++) {
       const LaunchArgs::More& o = x.more[j];
@@ -1361,13 +1558,18 @@ int launch_resident_q(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& 
   return 0;
 }
 
-template <int FMT, int Q>
+template <int FMT, int Q, int KS>
 int launch_resident_rows(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& p) {
   constexpr bool kPark = Q == 1;
   if (p.park != kPark) return (int)hipErrorInvalidValue;
-  if (x.pro_kind == kProRmsNorm) return launch_resident_q<FMT, true, 1, Q, kPark, false, kProRmsNorm>(s, x, p);
-  if (x.pro_kind == kProSwiglu) return launch_resident_q<FMT, true, 1, Q, kPark, false, kProSwiglu>(s, x, p);
-  return launch_resident_q<FMT, true, 1, Q, kPark, false, kProNone>(s, x, p);
+  if (x.pro_kind == kProRmsNorm) return launch_resident_q<FMT, true, 1, Q, kPark, false, kProRmsNorm, KS>(s, x, p);
+  if (x.pro_kind == kProSwiglu) return launch_resident_q<FMT, true, 1, Q, kPark, false, kProSwiglu, KS>(s, x, p);
+  return launch_resident_q<FMT, true, 1, Q, kPark, false, kProNone, KS>(s, x, p);
+}
+template <int FMT>
+int launch_resident_rows(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& p) {
+  if (p.q == 2) return launch_resident_rows<FMT, 2, 1>(s, x, p);
+  return p.ks == 1 ? launch_resident_rows<FMT, 1, 1>(s, x, p) : p.ks == 2 ? launch_resident_rows<FMT, 1, 2>(s, x, p) : launch_resident_rows<FMT, 1, 4>(s, x, p);
 }
 
 template <int FMT, bool F32A>
@@ -1381,6 +1583,8 @@ int launch_resident_fa(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan&
     }
   }
   if (p.r != 1) return (int)hipErrorInvalidValue;
+  if (p.ks == 2) return launch_resident_q<FMT, F32A, 1, 1, true, false, kRowsPlain, 2>(s, x, p);
+  if (p.ks == 4) return launch_resident_q<FMT, F32A, 1, 1, true, false, kRowsPlain, 4>(s, x, p);
   if (p.q == 1)
     return p.park ? launch_resident_q<FMT, F32A, 1, 1, true>(s, x, p) : launch_resident_q<FMT, F32A, 1, 1, false>(s, x, p);
   return p.park ? launch_resident_q<FMT, F32A, 1, 2, true>(s, x, p) : launch_resident_q<FMT, F32A, 1, 2, false>(s, x, p);
@@ -1483,7 +1687,7 @@ int launch_cpt(ihipStream_t* s, const LaunchArgs& x, const TilePlan& p, uint4* i
   static std::atomic<uint64_t> big_lds_done{0};
   if (p.lds > 64 * 1024)
     if (int e = enable_big_lds(kern, x.device, big_lds_done)) return e;
-  const TileTail tail{x.d, x.c, (float*)x.scratch, x.counters, x.epilogue, nullptr, 0, nullptr, 0, add_lift(x.w)};
+  const TileTail tail{x.d, x.c, (float*)x.scratch, x.counters, x.epilogue, nullptr, 0, nullptr, 0, add_lift(x.w), 0};
   hipLaunchKernelGGL(kern, dim3(p.parts, p.colgroups, p.rowgroups), dim3(64 * p.ksc * p.wnc), p.lds, s, image, x.w.meta, x.w.quants,
                      x.m, x.w.k, x.w.n, p.wnc, p.ksc, p.nph, p.parts, p.nslices, tail);
   MGN_HIP_LAUNCH_CHECK();
@@ -1531,7 +1735,7 @@ bool use_resident(const LaunchArgs& x, ResidentPlan* rp) {
   if (x.m <= 32) return true;
   if (rp->parts > 4 || rp->partial_bytes > ((size_t)8 << 20)) return false;
   if (x.w.fmt == MGN_FMT_Q4 || x.m >= 128) return true;
-  return x.resident_q8 && !x.a_is_f16 && rp->partial_bytes <= ((size_t)4 << 20);  // (what the static workspace holds: one plan for both)
+  return x.resident_q8 && (!x.a_is_f16 || rp->ks > 1) && rp->partial_bytes <= ((size_t)4 << 20);  // (what the static workspace holds: one plan for both)
 }
 
 // The general kernel's plan for as many rows per launch as the workspace has room for (partial
@@ -1558,6 +1762,11 @@ bool tile_mfma_supported(const LaunchArgs& x) {
   TilePlan p;
   uint32_t rows;
   return plan_tile_rows(x, &p, &rows);
+}
+
+bool tile_mfma_splits(const LaunchArgs& x) {
+  ResidentPlan rp;
+  return x.split_waves && use_resident(x, &rp) && rp.ks > 1;
 }
 
 // Where the resident kernel measured faster than the 32x32 tiled one, whatever is known about
@@ -1590,6 +1799,7 @@ bool tile_mfma_supported(const LaunchArgs& x) {
 bool tile_mfma_preferred(const LaunchArgs& x) {
   ResidentPlan rp;
   if (!use_resident(x, &rp)) return false;
+  if (rp.ks > 1) return true;
   const uint64_t wgs = (uint64_t)rp.parts * rp.colgroups * rp.rowgroups;
   const uint64_t rounds = (wgs + x.num_cus - 1) / x.num_cus;
   if (x.m > 32)
@@ -1627,8 +1837,7 @@ bool tile_rows_supported(const LaunchArgs& x) {
 int launch_tile_rows(ihipStream_t* s, const LaunchArgs& x) {
   ResidentPlan p;
   if (!use_resident(x, &p)) return (int)hipErrorInvalidValue;  // (the caller has asked tile_rows_supported)
-  if (x.w.fmt == MGN_FMT_Q4) return p.q == 1 ? launch_resident_rows<MGN_FMT_Q4, 1>(s, x, p) : launch_resident_rows<MGN_FMT_Q4, 2>(s, x, p);
-  return p.q == 1 ? launch_resident_rows<MGN_FMT_Q8, 1>(s, x, p) : launch_resident_rows<MGN_FMT_Q8, 2>(s, x, p);
+  return x.w.fmt == MGN_FMT_Q4 ? launch_resident_rows<MGN_FMT_Q4>(s, x, p) : launch_resident_rows<MGN_FMT_Q8>(s, x, p);
 }
 
 bool describe_tile_mfma(const LaunchArgs& x, mgn_plan_info* out) {
@@ -1638,7 +1847,7 @@ bool describe_tile_mfma(const LaunchArgs& x, mgn_plan_info* out) {
     out->grid[0] = rp.parts, out->grid[1] = rp.colgroups, out->grid[2] = rp.rowgroups;
     out->threads = 512;
     out->lds_bytes = (uint32_t)rp.lds;
-    out->waves_n = 8 * kSide * rp.q, out->k_splits = 1, out->k_parts = rp.parts, out->steps = rp.nsl;
+    out->waves_n = 8 / rp.ks * kSide * rp.q, out->k_splits = rp.ks, out->k_parts = rp.parts, out->steps = rp.nsl;
     out->quads_per_wave = 0, out->full_steps = rp.r, out->tail_blocks = 0;
     out->workspace_bytes = rp.partial_bytes;
     return true;

@@ -126,7 +126,10 @@ mgn_status weight_alloc(mgn_ctx* ctx, mgn_fmt fmt, size_t rows, size_t cols, mgn
 // 16x16x32 kernels for everything else.
 mgn_route basic_route(const mgn::LaunchArgs& x, bool any_magnitude) {
   if (mgn::gemv_mfma_supported(x)) return MGN_ROUTE_GEMV_MFMA;
-  if (mgn::tile_mfma_preferred(x)) return MGN_ROUTE_TILE_MFMA;
+  // (f32 activations that were promised to lie in the fp16 range: the 32x32 kernel checks that they do, and keeps its calls)
+  mgn::LaunchArgs whole = x;
+  whole.split_waves = false;
+  if (mgn::tile_mfma_preferred(x.a_is_f16 || any_magnitude ? x : whole)) return MGN_ROUTE_TILE_MFMA;
   if ((x.a_is_f16 || !any_magnitude) && mgn::gemm_mfma_supported(x)) return MGN_ROUTE_GEMM_MFMA;
   if (mgn::tile_mfma_supported(x)) return MGN_ROUTE_TILE_MFMA;
   if (mgn::gemv_supported(x)) return MGN_ROUTE_GEMV_VALU;
@@ -164,14 +167,19 @@ double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool* steady) {
 // Of 1652 other calls, 17 to 2048 rows, K 32 to 8192 and N 64 to 30000, 405 take it, 20 of them more than 3 % slower than on the kernel
 // behind, and 77 do not though it is more than 3 % faster: above all narrow results of long K, for which basic_us is far too
 // low, 743 x 5344 x 243 23 against 61.)  `choice`: the plan, if it does.
+// The estimates are those of workgroups whose waves do not split K: of 217 drawn calls of 17 and more rows on which they may, none was
+// faster blocked, and none is blocked by these estimates (up to 32 rows and on narrow results some would be: Q8 20 x 1504 x 310, blocked 12.0,
+// split 8.3; they are not compared up to there).
 // Not so where the other kernel is the resident one with one pair of tiles per wave: small weights, which take it the
 // same time a round from wherever they come.  (Blocked and resident, us: Q8 f32 22 x 1760 x 1307 14.1, 11.4, 17 x 768 x 579
 // 10.1, 8.8; short K: Q4 f32 470 x 192 x 275 9.6, 6.4, Q4 fp16 145 x 160 x 105 8.6, 4.2.)
 mgn_route auto_route(const mgn::LaunchArgs& x, bool any_magnitude, mgn::BlockChoice* choice) {
   const mgn_route basic = basic_route(x, any_magnitude);
-  if (x.m <= 16 || (x.m <= 32 && x.w.fmt == MGN_FMT_Q4)) return basic;
+  if (x.m <= 16 || (x.m <= 32 && (x.w.fmt == MGN_FMT_Q4 || (basic == MGN_ROUTE_TILE_MFMA && mgn::tile_mfma_splits(x))))) return basic;
+  mgn::LaunchArgs whole = x;
+  whole.split_waves = false;
   bool steady;
-  const double us = basic_us(x, basic, &steady);
+  const double us = basic_us(whole, basic_route(whole, any_magnitude), &steady);
   return mgn::choose_block_mfma(x, steady ? us : us / 0.92, choice) ? MGN_ROUTE_BLOCK_MFMA : basic;
 }
 
@@ -777,7 +785,7 @@ static mgn_status matmul_impl(mgn_ctx* ctx, const mgn_buf* a, bool a_is_f16, con
       return fail(ctx, MGN_EUNSUPPORTED, "fused prologue needs the GEMV_MFMA route (f32 activations, M <= 4)");
     route = MGN_ROUTE_GEMV_MFMA;
   }
-  x.resident_q8 = route == MGN_ROUTE_AUTO;
+  x.resident_q8 = x.split_waves = route == MGN_ROUTE_AUTO;
   mgn::BlockChoice block;
   if (route == MGN_ROUTE_AUTO)
     route = auto_route(x, ctx->any_magnitude, &block);
@@ -788,22 +796,26 @@ static mgn_status matmul_impl(mgn_ctx* ctx, const mgn_buf* a, bool a_is_f16, con
     // on the library's static array if the plan's partial sums fit it; refused otherwise.  (Of the shapes that the
     // blocked kernel takes, those that the kernels behind it could run on the array are accepted, as they were
     // before there was a blocked kernel; it runs on the context's own workspace, which is there since the
-    // context was created.)
-    mgn_plan_info plan{};
-    const mgn_route taken = route;
-    if (route == MGN_ROUTE_BLOCK_MFMA) route = basic_route(x, ctx->any_magnitude);
-    const bool parts = route == MGN_ROUTE_GEMV_MFMA   ? mgn::describe_gemv_mfma(x, &plan)
-                       : route == MGN_ROUTE_GEMM_MFMA ? mgn::describe_gemm_mfma(x, &plan)
-                       : route == MGN_ROUTE_TILE_MFMA ? mgn::describe_tile_mfma(x, &plan)
-                                                      : false;
-    const uint64_t need = parts ? plan.workspace_bytes : 0;
+    // context was created.  Nor does it change what is accepted that the resident kernel's waves may split K.)
+    auto workspace_of = [](const mgn::LaunchArgs& y, mgn_route r) -> uint64_t {
+      mgn_plan_info plan{};
+      const bool parts = r == MGN_ROUTE_GEMV_MFMA   ? mgn::describe_gemv_mfma(y, &plan)
+                         : r == MGN_ROUTE_GEMM_MFMA ? mgn::describe_gemm_mfma(y, &plan)
+                         : r == MGN_ROUTE_TILE_MFMA ? mgn::describe_tile_mfma(y, &plan)
+                                                    : false;
+      return parts ? plan.workspace_bytes : 0;
+    };
+    mgn::LaunchArgs behind = x;
+    behind.split_waves = false;
+    uint64_t need = workspace_of(behind, ctx->route == MGN_ROUTE_AUTO ? basic_route(behind, ctx->any_magnitude) : route);
     if (need > kStaticPartialBytes)
       return fail(ctx, MGN_EUNSUPPORTED,
                   "mgn_matmul_q_static: this shape's K parts need " + std::to_string(need) +
                       " bytes of workspace, the static one holds " + std::to_string(kStaticPartialBytes) +
                       "; use mgn_matmul_q");
-    const bool blocked = taken == MGN_ROUTE_BLOCK_MFMA;
-    route = taken;
+    const bool blocked = route == MGN_ROUTE_BLOCK_MFMA;
+    if (!blocked) need = workspace_of(x, route);  // (at most 4 MiB where waves split K: a round of workgroups, 16 KiB each)
+    if (!blocked && need > kStaticPartialBytes) return fail(ctx, MGN_EUNSUPPORTED, "mgn_matmul_q_static: no room for this plan's K parts");
     x.scratch = ctx->static_scratch;
     x.scratch_capacity = kStaticPartialBytes;  // a launch that would need more than was checked above is refused, not run
     x.counters = (uint32_t*)((char*)ctx->static_scratch + kStaticPartialBytes);
@@ -949,7 +961,7 @@ static void rows_args(const mgn_ctx* ctx, LaunchArgs* x) {
   x->handover_bytes = ctx->handover_bytes;
   x->block_ws = ctx->block_ws;
   x->block_ws_bytes = kBlockWsBytes;
-  x->resident_q8 = true;  // (rows_plans: the route is the library's choice)
+  x->resident_q8 = x->split_waves = true;  // (rows_plans: the route is the library's choice)
 }
 
 bool rows_plans(const mgn_ctx* ctx, const mgn_weight* const* ws, size_t count, uint32_t m, int pro_kind) {
@@ -957,10 +969,12 @@ bool rows_plans(const mgn_ctx* ctx, const mgn_weight* const* ws, size_t count, u
   LaunchArgs x{view_of(ws[0]), nullptr, nullptr, nullptr, m, false, ctx->num_cus};
   rows_args(ctx, &x);
   BlockChoice block;
+  x.split_waves = false;  // (a weight joins where the kernel takes it whole)
   for (size_t j = 0; j < count; j++) {
     x.w = view_of(ws[j]);
     if (auto_route(x, ctx->any_magnitude, &block) != MGN_ROUTE_TILE_MFMA) return false;
   }
+  x.split_waves = true;
   x.w = view_of(ws[0]);
   for (size_t j = 1; j < count; j++) x.more[j - 1] = {view_of(ws[j]), nullptr, nullptr};
   x.n_more = (int)count - 1;
@@ -1060,7 +1074,7 @@ mgn_status mgn_matmul_q_auto_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t 
   mgn::LaunchArgs x{};
   if (!out || !planned_args(fmt, m, k, n, a_is_f16, num_cus, &x)) return MGN_EINVAL;
   *out = mgn_plan_info{};
-  x.resident_q8 = true;
+  x.resident_q8 = x.split_waves = true;
   mgn::BlockChoice block;
   const mgn_route route = auto_route(x, a_is_f16 == 0, &block);
   mgn_block_plan b{};
@@ -1080,7 +1094,7 @@ mgn_status mgn_matmul_q_block_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t
   if (!out || !planned_args(fmt, m, k, n, a_is_f16, num_cus, &x)) return MGN_EINVAL;
   *out = mgn_block_plan{};
   if (!mgn::describe_block_mfma(x, out)) return MGN_EUNSUPPORTED;
-  x.resident_q8 = true;  // (as the automatic choice has it)
+  x.resident_q8 = x.split_waves = true;  // (as the automatic choice has it)
   mgn::BlockChoice block;
   out->taken = auto_route(x, a_is_f16 == 0, &block) == MGN_ROUTE_BLOCK_MFMA ? 1u : 0u;
   return MGN_OK;

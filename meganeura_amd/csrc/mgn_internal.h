@@ -94,6 +94,8 @@ struct LaunchArgs {
   // Q8 of 33 to 127 rows may run on the resident tiled kernel: set where the route is the library's choice (a
   // forced route and the plan entry know the general form)
   bool resident_q8 = false;
+  // The waves of the resident tiled kernel may split K on launches that leave CUs idle: set likewise
+  bool split_waves = false;
   // host-visible word a kernel sets when f32 activations leave the range it can represent
   uint32_t* range_flag = nullptr;
   // host-visible word set by a wave that gave up waiting for another workgroup's partial sums
@@ -168,6 +170,8 @@ int launch_chain(ihipStream_t* s, int device, int fmt, const ChainStageDev* stag
 bool tile_mfma_supported(const LaunchArgs& a);
 // shapes on which the automatic route takes this kernel ahead of the 32x32 tiled one
 bool tile_mfma_preferred(const LaunchArgs& a);
+// a launch of it whose waves split K (LaunchArgs::split_waves)
+bool tile_mfma_splits(const LaunchArgs& a);
 bool describe_tile_mfma(const LaunchArgs& a, mgn_plan_info* out);
 int launch_matmul_tile_mfma(ihipStream_t* s, const LaunchArgs& a);
 // the same kernel for several weights (LaunchArgs::more) and with a prologue, f32 activations
