@@ -1549,9 +1549,17 @@ int launch_resident_q(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& 
     extra.items = (uint32_t)x.n_more;
     extra.norm_w = x.pro_weight, extra.eps = x.pro_eps;
   }
-  // (column groups x row groups, K parts); with K parts the first is rounded up to a multiple of 8 (see the kernel)
-  const uint64_t groups = (uint64_t)p.colgroups * p.rowgroups;
-  const dim3 grid((unsigned)(p.parts > 1 ? (groups + 7) / 8 * 8 : groups), p.parts, 1);
+  // (column groups x row groups, K parts); with K parts the first is rounded up to a multiple of 8 (see the kernel), which gives some
+  // XCDs the parts of one group more than others.  Where that is another round for them (a plan with K parts fills the LDS of
+  // its CUs), the workgroups go out evenly instead, which keeps them all in the rounds that the plan counted, and a group's parts
+  // meet across XCDs.  us, padded -> evenly: 84 groups in 3 parts (33 workgroups on the 32 CUs of four XCDs) 333 x 3072 x 1024 f32 Q4
+  // 20.1 -> 13.4, Q8 22.4 -> 14.3, fp16 660 x 3072 x 1024 25.4 -> 17.7, 31.5 -> 19.8; 17 groups in 14, 16 x 14336 x 4352 22.4 -> 16.4, 26.7 ->
+  // 20.9; 22 in 11, 16 x 11264 x 5632 22.2 -> 16.0, 26.3 -> 21.4.  (Parts that add up shares are planned for the padded grid.)
+  const uint64_t groups = (uint64_t)p.colgroups * p.rowgroups, padded = (groups + 7) / 8 * 8;
+  const uint64_t per_round = std::max<uint64_t>(x.num_cus / 8, 1);
+  auto rounds = [&](uint64_t wgs) { return ((wgs + 7) / 8 + per_round - 1) / per_round; };
+  const bool even = p.parts == 1 || (!p.spread && rounds(groups * p.parts) < rounds(padded * p.parts));
+  const dim3 grid((unsigned)(even ? groups : padded), p.parts, 1);
   hipLaunchKernelGGL(kern, grid, dim3(512), p.lds, s, x.a, x.w.meta, x.w.quants, x.m, x.w.k, x.w.n, p.parts, p.nslices,
                      p.colgroups, tail, extra);
   MGN_HIP_LAUNCH_CHECK();
