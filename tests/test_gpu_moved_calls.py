@@ -1,0 +1,76 @@
+"""Calls that the automatic route gives to the blocked kernel because of what the plan of the kernel behind it says (narrow results of long K, ragged
+rounds): every form of such a call on both kernels, against the oracle's product in f64 and against each other."""
+import numpy as np
+import pytest
+
+from helpers import Q4, Q8, bits
+from meganeura_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = capi.Context(0)
+    yield c
+    c.close()
+
+
+def run(ctx, x, wt, d=None, ops=(), route=capi.ROUTE_AUTO, static=False):
+    m, n = len(x), wt.cols
+    a, c = ctx.upload(x), ctx.upload(np.full(m * n, np.nan, np.float32))
+    db = None if d is None else ctx.upload(d)
+    ctx.set_route(route)
+    try:
+        if x.dtype == np.float16:
+            ctx.matmul_q_f16a(a, wt, c, m, db)
+        elif static:
+            ctx.matmul_q_static(a, wt, c, m, db)
+        else:
+            ctx.matmul_q_epilogue(a, wt, c, m, list(ops), db)
+        return c.download(np.float32, m * n).reshape(m, n)
+    finally:
+        ctx.set_route(capi.ROUTE_AUTO)
+        for h in (a, c, db):
+            if h is not None:
+                h.free()
+
+
+@pytest.mark.parametrize("fmt,m,k,n,f16", [
+    (Q4, 130, 4160, 992, False), (Q4, 51, 5056, 1088, False), (Q4, 399, 6656, 329, False), (Q8, 87, 1376, 11104, False), (Q8, 41, 5248, 1216, False),
+    (Q8, 665, 6912, 575, False), (Q4, 546, 1056, 4423, True), (Q4, 267, 5440, 2279, True), (Q8, 949, 1120, 3090, True), (Q8, 1028, 5728, 911, True)])
+def test_both_kernels_give_the_call_its_result(ctx, orc, fmt, m, k, n, f16):
+    """Rows of ordinary, tiny, large and mixed magnitudes; bound: activations of 22 bits relative to a slice's largest, f32 sums whose roundings of
+    2^-24 grow like a random walk, on sums up to five times the row's size, twice for the two kernels."""
+    behind = capi.matmul_plan(fmt, m, k, n, f16).route
+    assert capi.matmul_plan(fmt, m, k, n, f16, auto=True).route == capi.ROUTE_BLOCK_MFMA != behind
+    w = synth.normal(2 * k + n, k * n, 0.02).reshape(k, n)
+    x, d = synth.normal(m + k, m * k).reshape(m, k).copy(), synth.normal(7, m * n).reshape(m, n)
+    x[0] = 0
+    if f16:
+        x[1] *= 2.0 ** -10
+        x = x.astype(np.float16)
+    else:
+        x[1] *= 1e-12
+        x[m - 1] *= 1e9
+        x[m - 2, : k // 2] *= 1e-4
+    wt = ctx.weight(fmt, w)
+    exact = orc.matmul_f64(x.astype(np.float32), orc.dequantize(fmt, orc.quantize(fmt, w), k, n))
+    bound = 5 * (2.0 ** -22 + 2.0 ** -24 * np.sqrt(k)) * (0.02 * np.linalg.norm(x.astype(np.float64), axis=1) * np.sqrt(n) + 1e-30)
+    got, other = run(ctx, x, wt), run(ctx, x, wt, route=behind)
+    assert (np.linalg.norm(got - exact, axis=1) <= bound).all() and (np.linalg.norm(got.astype(np.float64) - other, axis=1) <= 2 * bound).all()
+    assert (bits(run(ctx, x, wt)) == bits(got)).all()
+    np.testing.assert_array_equal(run(ctx, x, wt, d), got + d)
+    if not f16:
+        np.testing.assert_array_equal(run(ctx, x, wt, d, [capi.UNARY_NEG, capi.UNARY_RELU]), np.maximum(-(got + d), 0))
+        if capi.matmul_plan(fmt, m, k, n).workspace_bytes <= capi.STATIC_WORKSPACE_BYTES:
+            np.testing.assert_array_equal(run(ctx, x, wt, d, static=True), got + d)
+    # what is not finite stays in its rows
+    x[1, 3], x[2, k - 1], x[m - 1, 300] = np.nan, np.inf, -np.inf
+    bad = [1, 2, m - 1]
+    for route in (capi.ROUTE_AUTO, behind):
+        hit = run(ctx, x, wt, route=route)
+        assert not np.isfinite(hit[bad]).any()
+    good = [r for r in range(m) if r not in bad]
+    np.testing.assert_array_equal(run(ctx, x, wt)[good], got[good])
+    wt.free()
