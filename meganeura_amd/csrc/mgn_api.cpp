@@ -142,7 +142,7 @@ mgn_route basic_route(const mgn::LaunchArgs& x, bool any_magnitude) {
 // shorter than the four slices of 256 that a workgroup holds (measured over the four slices' time, medians by format and
 // activations: one slice 0.55 .. 0.72, two 0.79 .. 0.90, three 0.88 .. 1.08, the most with two pairs of tiles per wave); the
 // others: a fixed part and a rate over the rows they compute, a multiple of 32 (K of up to 128: 5.4 to 12 us).  *steady: the resident kernel with one
-// pair of tiles per wave.
+// pair of tiles per wave.  by_plan: as follows.
 // On 240 calls drawn over 17 to 2048 rows, K of 576 to 14336 and 192 to 49152 columns that stayed behind by that rate, the 32x32 kernel (fp16
 // activations) took 1.0 to 2.4 times and the general tiled one 1.1 to 3.8 times as long as it says (medians 1.4 and 1.75), and the blocked kernel was
 // more than 3 % faster on 88 of 150 and 83 of 90 of them: Q8 f32 998 x 6240 x 544 137 against 43 us, Q4 130 x 4160 x 992 39 against 18, Q4 fp16 546 x 1056 x
@@ -150,14 +150,14 @@ mgn_route basic_route(const mgn::LaunchArgs& x, bool any_magnitude) {
 // Q8, where many calls are level: what it moves by mistake would cost more than what it leaves), and half as much again for the general one.
 // Of 6000 drawn calls of more than four rows that moves 169; of 196 such that were measured five were more than 3.5 % slower then (Q4 fp16
 // 102 x 4384 x 2136 16.6 -> 18.1), all together take 0.72 of the time (geometric mean, 0.28 at best).
-double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool* steady) {
+double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool by_plan, bool* steady) {
   const bool q4 = x.w.fmt == MGN_FMT_Q4;
   const double flops = 2.0 * ((x.m + 31) / 32 * 32) * x.w.k * x.w.n;
   *steady = false;
   mgn_plan_info p{};
   if (route == MGN_ROUTE_GEMM_MFMA) {
     const double rate = x.w.k <= 128 ? 5.6 + flops / (x.a_is_f16 ? 175e6 : 120e6) : 7.0 + flops / (q4 ? 390e6 : 310e6);
-    if (!x.a_is_f16 || x.w.k <= 512 || !mgn::describe_gemm_mfma(x, &p)) return rate;
+    if (!by_plan || !x.a_is_f16 || x.w.k <= 512 || !mgn::describe_gemm_mfma(x, &p)) return rate;
     // That rate is the full rounds' of many rows.  With few columns or a ragged last round the launch takes its chunks of K
     // (256 or 512 elements a workgroup), each partly by how many workgroups the CUs share out and partly by the rounds.
     const double wgs = (double)p.grid[0] * p.grid[1] * p.grid[2] / x.num_cus, rounds = std::ceil(wgs);
@@ -166,7 +166,7 @@ double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool* steady) {
     return std::max(rate, plan);
   }
   if (route != MGN_ROUTE_TILE_MFMA || !mgn::describe_tile_mfma(x, &p)) return 1e9;  // scalar routes
-  if (p.quads_per_wave != 0) return 1.5 * (9.0 + flops / (q4 ? 175e6 : 165e6));
+  if (p.quads_per_wave != 0) return (by_plan ? 1.5 : 1.0) * (9.0 + flops / (q4 ? 175e6 : 165e6));
   *steady = p.full_steps != 2 && p.waves_n <= 16;
   const double share = x.w.k <= 256 ? 0.65 : x.w.k <= 512 ? (p.waves_n <= 16 ? 0.82 : 0.9) : x.w.k <= 768 && *steady ? 0.94 : 1.0;
   const double rounds = std::ceil((double)p.grid[0] * p.grid[1] * p.grid[2] / x.num_cus) * share, parts = p.k_parts > 1 ? 1.0 : 0.0;
@@ -183,16 +183,21 @@ double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool* steady) {
 // Of 1652 other calls, 17 to 2048 rows, K 32 to 8192 and N 64 to 30000, 405 took it by the rates alone, 20 of them more than 3 % slower than on the
 // kernel behind, and 77 did not though it was more than 3 % faster, above all the narrow results of long K that the plans above find.)
 // `choice`: the plan, if it does.
-// A launch whose waves split K is not compared: of 217 drawn calls of 17 and more rows on which they may, none was faster blocked
-// (Q8 20 x 1504 x 310, blocked 12.0, split 8.3; fp16 35 x 704 x 1797 9.8, 5.0).
+// A launch whose waves split K is faster than the unsplit one it is compared as, by that one's rate: of 217 drawn calls of 17 and more rows on which
+// they may, none was faster blocked (up to 32 rows they are not compared; Q8 20 x 1504 x 310, blocked 12.0, split 8.3; fp16 35 x 704 x 1797
+// 9.8, 5.0), and 5 of 6000 are blocked by these estimates.
 // Not so where the other kernel is the resident one with one pair of tiles per wave: small weights, which take it the
 // same time a round from wherever they come.  (Blocked and resident, us: Q8 f32 22 x 1760 x 1307 14.1, 11.4, 17 x 768 x 579
 // 10.1, 8.8; short K: Q4 f32 470 x 192 x 275 9.6, 6.4, Q4 fp16 145 x 160 x 105 8.6, 4.2.)
 mgn_route auto_route(const mgn::LaunchArgs& x, bool any_magnitude, mgn::BlockChoice* choice) {
   const mgn_route basic = basic_route(x, any_magnitude);
-  if (x.m <= 16 || (x.m <= 32 && x.w.fmt == MGN_FMT_Q4) || (basic == MGN_ROUTE_TILE_MFMA && mgn::tile_mfma_splits(x))) return basic;
+  if (x.m <= 16) return basic;
+  const bool splits = basic == MGN_ROUTE_TILE_MFMA && mgn::tile_mfma_splits(x);
+  if (x.m <= 32 && (splits || x.w.fmt == MGN_FMT_Q4)) return basic;
+  mgn::LaunchArgs whole = x;
+  whole.split_waves = false;
   bool steady;
-  const double us = basic_us(x, basic, &steady);
+  const double us = basic_us(whole, splits ? basic_route(whole, any_magnitude) : basic, !splits, &steady);
   return mgn::choose_block_mfma(x, steady ? us : us / 0.92, choice) ? MGN_ROUTE_BLOCK_MFMA : basic;
 }
 
