@@ -891,6 +891,13 @@ struct RowsExtra {
 };
 constexpr int kRowsPlain = -1;
 
+// NSL: the slices a part holds, 4 where nothing is said.  A K of one to three slices, and the parts of one that is cut into 5, 6 or 9
+// (3 + 2, 3 + 3, 3 + 3 + 3 instead of 4 + 1, 4 + 2, 4 + 4 + 1), asked for, converted and walked slices that are not there, or waited for a part
+// with four.  Counted at compile time: bounds tested on the way cost a whole part of four 4 to 6 %.  us, NSL = 4 -> as many as there are:
+// f32 Q4 204 x 256 x 2656 6.5 -> 4.5, 224 x 320 x 2976 7.4 -> 6.1, 234 x 544 x 2240 8.7 -> 8.1, 67 x 1536 x 1664 10.8 -> 9.0, Q8 326 x 1152 x 1472
+// 12.9 -> 11.1, 375 x 2304 x 608 12.5 -> 11.0; fp16 Q4 406 x 1408 x 308 9.0 -> 7.8; with two waves to a pair of tiles, K of 288 to 512, 40 calls
+// of 4.7 to 6.2 us 0.93 to 0.96.
+
 // ROWS: kRowsPlain, or the activations' prologue (kProNone / kProRmsNorm / kProSwiglu) of a launch that may
 // serve several weights.  A decoder layer of some hundred rows is made of launches that last 10 to 25 us
 // and leave part of the chip idle, with 4 to 6 us ones between them that only rewrite the activations.
@@ -899,19 +906,19 @@ constexpr int kRowsPlain = -1;
 // fill the rounds that each would leave open.  Two decoder layers of 333 rows, 1024 wide (Q8), q | k | v, the
 // output projection, gate | up and down with norms and SwiGLU: 18 launches, 213 us -> 8 launches, 161 us (Q4 184
 // -> 139; 128 rows, 576 wide 156 -> 104; 8 rows Q4 138 -> 90).
-template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1>
+template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1, int NSL = resident_slices(F32A, R)>
 __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restrict__ a, const void* __restrict__ meta_arg,
                                                              const void* __restrict__ quants_arg, uint32_t m, uint32_t kdim,
                                                              uint32_t n, uint32_t parts, uint32_t nslices, uint32_t colgroups,
                                                              TileTail tail, RowsExtra extra) {
   static_assert(ROWS == kRowsPlain || (F32A && R == 1 && !LATE), "the forms that are launched");
   static_assert(KS == 1 || (R == 1 && Q == 1 && PARK && !LATE), "the forms that are launched");
+  static_assert(NSL == resident_slices(F32A, R) || (R == 1 && Q == 1 && PARK && !LATE && (KS == 1 || (KS == 2 && NSL == 2))), "the forms that are launched");
   constexpr uint32_t UNITS = image_units(F32A);
   constexpr float kOpScale = FMT == MGN_FMT_Q4 ? 1048576.0f : 16777216.0f;
   constexpr int QB = FMT == MGN_FMT_Q4 ? 16 : 32;
   constexpr int MB = FMT == MGN_FMT_Q4 ? 4 : 2;
   constexpr int NLQ = QB / 8;
-  constexpr int NSL = resident_slices(F32A, R);
   constexpr int SPW = NSL / KS;   // slices of the part that a wave walks
   constexpr int STEPS = SPW * Q;  // step f of the walk = (pair f / NSL, slice f % NSL), or the wave's slice f
   constexpr int DEPTH = KS > 1 ? STEPS : 1;  // steps whose quants are in flight ahead of the one in use
@@ -1419,8 +1426,7 @@ struct ResidentPlan {
   double cost;
 };
 
-size_t resident_lds_bytes(int fmt, bool f32a, uint32_t r, uint32_t q, bool park, uint32_t ks = 1) {
-  const uint32_t nsl = resident_slices(f32a, r);
+size_t resident_lds_bytes(int fmt, bool f32a, uint32_t r, uint32_t q, bool park, uint32_t nsl, uint32_t ks = 1) {
   return (size_t)nsl * r * image_units(f32a) * 16 + (size_t)8 * q * 32 * meta_stride(fmt, nsl / ks) +
          (park ? (size_t)8 * kSide * 16 * park_stride(fmt) : 0);
 }
@@ -1455,9 +1461,10 @@ void split_resident(const LaunchArgs& x, ResidentPlan* p) {
       // (resident at once: see plan_resident)
       if ((colgroups * rowgroups + 7) / 8 * parts > (uint64_t)x.num_cus / 8) continue;
       const uint64_t partial = parts > 1 ? parts * rowgroups * colgroups * (per_wg * 1024u) : 0;
-      const size_t lds = resident_lds_bytes(x.w.fmt, f32a, 1, 1, true, ks);
+      const uint32_t held = ks == 2 && p->nslices <= 2 ? 2 : nsl;
+      const size_t lds = resident_lds_bytes(x.w.fmt, f32a, 1, 1, true, held, ks);
       if (partial > x.handover_bytes || lds > 160 * 1024) continue;
-      p->ks = ks, p->rows = rows, p->r = 1, p->q = 1, p->nsl = nsl, p->parts = parts;
+      p->ks = ks, p->rows = rows, p->r = 1, p->q = 1, p->nsl = held, p->parts = parts;
       p->colgroups = (uint32_t)colgroups, p->rowgroups = rowgroups;
       p->park = true, p->spread = parts > 1, p->lds = lds, p->partial_bytes = partial;
       p->cost = 1.5 + 1.0 / ks + (parts > 1 ? 1.0 : 0.0);
@@ -1519,20 +1526,33 @@ bool plan_resident(const LaunchArgs& x, ResidentPlan* out) {
         best = cost;
         bp.ks = 1, bp.r = r, bp.q = q, bp.nsl = nsl, bp.parts = parts, bp.colgroups = colgroups, bp.rowgroups = rowgroups;
         bp.nslices = nslices, bp.partial_bytes = partial, bp.cost = cost, bp.spread = spread;
-        bp.park = resident_lds_bytes(x.w.fmt, f32a, r, q, true) <= 160 * 1024;
-        bp.lds = resident_lds_bytes(x.w.fmt, f32a, r, q, bp.park);
+        bp.park = resident_lds_bytes(x.w.fmt, f32a, r, q, true, nsl) <= 160 * 1024;
+        bp.lds = resident_lds_bytes(x.w.fmt, f32a, r, q, bp.park, nsl);
       }
     }
   }
   if (best == 0) return false;
   if (x.split_waves) split_resident(x, &bp);
+  if (bp.ks == 1 && bp.r == 1 && bp.q == 1 && bp.park) {  // (the other forms are built for four slices)
+    bp.nsl = (nslices + bp.parts - 1) / bp.parts;
+    bp.lds = resident_lds_bytes(x.w.fmt, f32a, 1, 1, true, bp.nsl);
+  }
   *out = bp;
   return true;
 }
 
-template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1>
+template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1, int NSL = resident_slices(F32A, R)>
 int launch_resident_q(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& p) {
-  auto kern = tile_resident_kernel<FMT, F32A, R, Q, PARK, LATE, ROWS, KS>;
+  if constexpr (R == 1 && Q == 1 && PARK && !LATE && KS == 1 && NSL == resident_slices(F32A, R)) {
+    if (p.nsl == 3) return launch_resident_q<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, 3>(s, x, p);
+    if (p.nsl == 2) return launch_resident_q<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, 2>(s, x, p);
+    if (p.nsl == 1) return launch_resident_q<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, 1>(s, x, p);
+  }
+  if constexpr (KS == 2 && NSL == resident_slices(F32A, R)) {
+    if (p.nsl == 2) return launch_resident_q<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, 2>(s, x, p);
+  }
+  if (p.nsl != NSL) return (int)hipErrorInvalidValue;
+  auto kern = tile_resident_kernel<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, NSL>;
   static std::atomic<uint64_t> big_lds_done{0};
   if (p.lds > 64 * 1024)
     if (int e = enable_big_lds(kern, x.device, big_lds_done)) return e;
@@ -1855,7 +1875,7 @@ bool describe_tile_mfma(const LaunchArgs& x, mgn_plan_info* out) {
     out->grid[0] = rp.parts, out->grid[1] = rp.colgroups, out->grid[2] = rp.rowgroups;
     out->threads = 512;
     out->lds_bytes = (uint32_t)rp.lds;
-    out->waves_n = 8 / rp.ks * kSide * rp.q, out->k_splits = rp.ks, out->k_parts = rp.parts, out->steps = rp.nsl;
+    out->waves_n = 8 / rp.ks * kSide * rp.q, out->k_splits = rp.ks, out->k_parts = rp.parts, out->steps = (uint32_t)resident_slices(!x.a_is_f16, rp.r);  // slices of a part at most
     out->quads_per_wave = 0, out->full_steps = rp.r, out->tail_blocks = 0;
     out->workspace_bytes = rp.partial_bytes;
     return true;

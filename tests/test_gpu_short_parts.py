@@ -1,0 +1,51 @@
+"""The resident kernel's parts of fewer than four slices: K of one to three slices, and of 5, 6 and 9, which is cut evenly (one block, whole slices,
+a block more), with one wave and with two to a pair of tiles, against the oracle's product in f64."""
+import numpy as np
+import pytest
+
+from helpers import Q4, Q8, bits
+from meganeura_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = capi.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("fmt", [Q4, Q8])
+@pytest.mark.parametrize("m,n", [(16, 257), (33, 600)])
+@pytest.mark.parametrize("k", [32, 256, 288, 512, 544, 768, 1024, 1056, 1280, 1312, 1536, 2080, 2304])
+def test_short_parts(ctx, orc, fmt, m, n, k):
+    """Bound: activations cut to 22 bits relative to their slice's largest (fp16 exactly), all towards zero, so K of them add up like sqrt(K) of that
+    largest's size; f32 sums whose roundings of 2^-24 grow like a random walk; both on quants whose sums are up to five times the product's."""
+    w = synth.normal(k + n, k * n, 0.02).reshape(k, n)
+    x, d = synth.normal(m + k, m * k).reshape(m, k).copy(), synth.normal(7, m * n).reshape(m, n)
+    x[0], x[1], x[2, : k // 2] = 0, x[1] * 2.0 ** -10, x[2, : k // 2] * 2.0 ** -6
+    dq = orc.dequantize(fmt, orc.quantize(fmt, w), k, n)
+    wt, db, c = ctx.weight(fmt, w), ctx.upload(d), ctx.buffer(m * n * 4)
+    # (forced: one wave to a pair; the library's choice: two or four where the launch leaves CUs idle; fp16: row groups of 16 only up to 16 rows)
+    for dtype, route in ((np.float32, capi.ROUTE_TILE_MFMA), (np.float32, capi.ROUTE_AUTO), (np.float16, capi.ROUTE_TILE_MFMA)):
+        xa = x.astype(dtype)
+        exact = orc.matmul_f64(xa.astype(np.float32), dq)
+        largest, norm = np.abs(xa.astype(np.float64)).max(axis=1), np.linalg.norm(xa.astype(np.float64), axis=1)
+        cut = 0.0 if dtype == np.float16 else 2.0 ** -22 * largest * np.sqrt(k)
+        bound = 5 * 0.02 * np.sqrt(n) * (cut + (2.0 ** -23 + 2.0 ** -24 * np.sqrt(k)) * norm) + 1e-30
+        a = ctx.upload(xa)
+        ctx.set_route(route)
+        try:
+            got = []
+            for res in (None, None, db):
+                (ctx.matmul_q_f16a if dtype == np.float16 else ctx.matmul_q)(a, wt, c, m, res)
+                got.append(c.download(np.float32, m * n).reshape(m, n))
+        finally:
+            ctx.set_route(capi.ROUTE_AUTO)
+            a.free()
+        assert (np.linalg.norm(got[0] - exact, axis=1) <= bound).all(), (dtype, route)
+        assert (bits(got[0]) == bits(got[1])).all()
+        np.testing.assert_array_equal(got[2], got[0] + d)
+    for h in (wt, db, c):
+        h.free()
