@@ -660,18 +660,18 @@ constexpr int kSide = 2;            // column tiles a wave multiplies side by si
 // rstride bytes apart).
 // PARK: the quants are not in q but parked in LDS, column by column (park_stride apart, tile u
 // 16 columns on): park_rd is this lane's piece of block 0 of its column of tile 0.
-template <int FMT, bool F32A, int R, bool PARK>
-__device__ __forceinline__ void slice_mac_side(const u32x4_t (&q)[kSide][FMT == MGN_FMT_Q4 ? 2 : 4], const uint8_t* park_rd,
-                                               const uint32_t (&mw)[kSide][8], const uint8_t* ib, uint32_t rstride, uint32_t g,
-                                               uint32_t lane, AddLift lift, floatx4 (&acc)[kSide][R]) {
+template <int FMT, bool F32A, int R, bool PARK, int SIDE>
+__device__ __forceinline__ void slice_mac_side(const u32x4_t (&q)[SIDE][FMT == MGN_FMT_Q4 ? 2 : 4], const uint8_t* park_rd,
+                                               const uint32_t (&mw)[SIDE][8], const uint8_t* ib, uint32_t rstride, uint32_t g,
+                                               uint32_t lane, AddLift lift, floatx4 (&acc)[SIDE][R]) {
   constexpr uint32_t HL = F32A ? 2 : 1;
   const uint32_t slot_off[2] = {image_slot(lane & 15, g, 0) * 16, image_slot(lane & 15, g, 1) * 16};
   u32x4_t aop[3][R][HL];
-  uint32_t bq[3][kSide][FMT == MGN_FMT_Q4 ? 1 : 2];  // PARK: the lane's quants of a block
-  floatx4 dsum[2][kSide][R];
-  floatx4 P[kSide][R];
+  uint32_t bq[3][SIDE][FMT == MGN_FMT_Q4 ? 1 : 2];  // PARK: the lane's quants of a block
+  floatx4 dsum[2][SIDE][R];
+  floatx4 P[SIDE][R];
 #pragma unroll
-  for (int u = 0; u < kSide; u++)
+  for (int u = 0; u < SIDE; u++)
 #pragma unroll
     for (int r = 0; r < R; r++) P[u][r] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
   auto lds_reads = [&](int s) {
@@ -681,7 +681,7 @@ __device__ __forceinline__ void slice_mac_side(const u32x4_t (&q)[kSide][FMT == 
       for (uint32_t h = 0; h < HL; h++) aop[s % 3][r][h] = *(const u32x4_t*)(ib + slot_off[s & 1] + r * rstride + (s * HL + h) * 64 * 16);
     if constexpr (PARK) {
 #pragma unroll
-      for (int u = 0; u < kSide; u++) {
+      for (int u = 0; u < SIDE; u++) {
         const uint8_t* src = park_rd + u * 16 * park_stride(FMT) + s * (FMT == MGN_FMT_Q4 ? 16 : 32);
         if constexpr (FMT == MGN_FMT_Q4) {
           bq[s % 3][u][0] = *(const uint32_t*)src;
@@ -694,7 +694,7 @@ __device__ __forceinline__ void slice_mac_side(const u32x4_t (&q)[kSide][FMT == 
   };
   auto mfmas = [&](int s) {
 #pragma unroll
-    for (int u = 0; u < kSide; u++) {
+    for (int u = 0; u < SIDE; u++) {
       half8 bop;
       if constexpr (PARK) {
         if constexpr (FMT == MGN_FMT_Q4) bop = nibbles_to_operand<F32A>(bq[s % 3][u][0]);
@@ -715,7 +715,7 @@ __device__ __forceinline__ void slice_mac_side(const u32x4_t (&q)[kSide][FMT == 
   };
   auto scale = [&](int s) {
 #pragma unroll
-    for (int u = 0; u < kSide; u++) {
+    for (int u = 0; u < SIDE; u++) {
       const float dq = half_bits_to_float(mw[u][s] & 0xFFFFu);
 #pragma unroll
       for (int r = 0; r < R; r++)
@@ -740,9 +740,9 @@ __device__ __forceinline__ void slice_mac_side(const u32x4_t (&q)[kSide][FMT == 
   // additive part of the slice's 8 blocks (see slice_mac)
   const uint32_t upper = 0u - (g & 1u);  // all ones in the lanes that take blocks 4..7
   const float kAdd = additive_constant<FMT>() * lift.down;
-  half8 bm[kSide];
+  half8 bm[SIDE];
 #pragma unroll
-  for (int u = 0; u < kSide; u++) {
+  for (int u = 0; u < SIDE; u++) {
     uint32_t bw[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -759,7 +759,7 @@ __device__ __forceinline__ void slice_mac_side(const u32x4_t (&q)[kSide][FMT == 
       // the rows' inverse slice scales (times 2^20 or 2^24)
       const float4 inv = *(const float4*)(ir - lane * 16 + 64 * 16 + g * 16);
 #pragma unroll
-      for (int u = 0; u < kSide; u++) {
+      for (int u = 0; u < SIDE; u++) {
         const floatx4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bm[u], floatx4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
         acc[u][r][0] = __fmaf_rn(__fmaf_rn(kAdd, d[0], P[u][r][0]), inv.x, acc[u][r][0]);
         acc[u][r][1] = __fmaf_rn(__fmaf_rn(kAdd, d[1], P[u][r][1]), inv.y, acc[u][r][1]);
@@ -771,7 +771,7 @@ __device__ __forceinline__ void slice_mac_side(const u32x4_t (&q)[kSide][FMT == 
       half8 ah, al;
       mean_operands(ir - lane * 16, lane, g, &ah, &al);
 #pragma unroll
-      for (int u = 0; u < kSide; u++) {
+      for (int u = 0; u < SIDE; u++) {
         const floatx4 dh = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bm[u], floatx4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
         const floatx4 dl = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bm[u], floatx4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 #pragma unroll
@@ -793,11 +793,11 @@ __host__ __device__ constexpr uint32_t meta_stride(int fmt, uint32_t nsl) { retu
 // which nobody reads any more): the sums meet in LDS, wave w takes tile w of the workgroup and adds up in the order of ks; K parts of
 // other workgroups meet as in the resident kernel's shares (all workgroups of the launch are resident): tile T
 // belongs to part T % parts.  `m`: the end of the workgroup's rows.
-template <int KS>
-__device__ __forceinline__ void split_tail(const floatx4 (&own)[kSide], uint8_t* strip, uint32_t strip_bytes, uint32_t wave, uint32_t lane,
+template <int KS, int SIDE>
+__device__ __forceinline__ void split_tail(const floatx4 (&own)[SIDE], uint8_t* strip, uint32_t strip_bytes, uint32_t wave, uint32_t lane,
                                            uint32_t part, uint32_t parts, uint32_t group, uint32_t groups, uint32_t row0, uint32_t col0,
                                            uint32_t m, uint32_t n, const TileTail& tail) {
-  constexpr uint32_t TILES = 8 / KS * kSide;
+  constexpr uint32_t TILES = 8 / KS * SIDE;
   constexpr int kDeviceScope = 16;
   const uint32_t c = lane & 15, g = lane >> 4;
   float dv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -808,15 +808,15 @@ __device__ __forceinline__ void split_tail(const floatx4 (&own)[kSide], uint8_t*
       if (row0 + 4 * g + i < m && col < n) dv[i] = tail.dres[(size_t)(row0 + 4 * g + i) * n + col];
   };
 #pragma unroll
-  for (int u = 0; u < kSide; u++) ((floatx4*)strip)[u * 64 + lane] = own[u];
+  for (int u = 0; u < SIDE; u++) ((floatx4*)strip)[u * 64 + lane] = own[u];
   if (parts == 1 && tail.dres && wave < TILES) load_residual(wave);  // (travels while the waves meet)
   lds_barrier();
   if (wave >= TILES) return;
   uint32_t tile = wave;
-  const uint8_t* const first = strip - wave * strip_bytes + wave / kSide * KS * strip_bytes;
-  floatx4 sum = ((const floatx4*)first)[wave % kSide * 64 + lane];
+  const uint8_t* const first = strip - wave * strip_bytes + wave / SIDE * KS * strip_bytes;
+  floatx4 sum = ((const floatx4*)first)[wave % SIDE * 64 + lane];
 #pragma unroll
-  for (int k = 1; k < KS; k++) sum += ((const floatx4*)(first + k * strip_bytes))[wave % kSide * 64 + lane];
+  for (int k = 1; k < KS; k++) sum += ((const floatx4*)(first + k * strip_bytes))[wave % SIDE * 64 + lane];
   if (parts > 1) {
     const uint32_t part_stride = groups * (TILES * 1024u);
     const __amdgpu_buffer_rsrc_t all_parts = __builtin_amdgcn_make_buffer_rsrc(tail.handover, 0, parts * part_stride, 0x00020000);
@@ -906,7 +906,7 @@ constexpr int kRowsPlain = -1;
 // fill the rounds that each would leave open.  Two decoder layers of 333 rows, 1024 wide (Q8), q | k | v, the
 // output projection, gate | up and down with norms and SwiGLU: 18 launches, 213 us -> 8 launches, 161 us (Q4 184
 // -> 139; 128 rows, 576 wide 156 -> 104; 8 rows Q4 138 -> 90).
-template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1, int NSL = resident_slices(F32A, R)>
+template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1, int NSL = resident_slices(F32A, R), int SIDE = kSide>
 __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restrict__ a, const void* __restrict__ meta_arg,
                                                              const void* __restrict__ quants_arg, uint32_t m, uint32_t kdim,
                                                              uint32_t n, uint32_t parts, uint32_t nslices, uint32_t colgroups,
@@ -914,6 +914,7 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   static_assert(ROWS == kRowsPlain || (F32A && R == 1 && !LATE), "the forms that are launched");
   static_assert(KS == 1 || (R == 1 && Q == 1 && PARK && !LATE), "the forms that are launched");
   static_assert(NSL == resident_slices(F32A, R) || (R == 1 && Q == 1 && PARK && !LATE && (KS == 1 || (KS == 2 && NSL == 2))), "the forms that are launched");
+  static_assert(SIDE == kSide || (KS == 4 || (KS == 2 && NSL == 2)), "the forms that are launched");
   constexpr uint32_t UNITS = image_units(F32A);
   constexpr float kOpScale = FMT == MGN_FMT_Q4 ? 1048576.0f : 16777216.0f;
   constexpr int QB = FMT == MGN_FMT_Q4 ? 16 : 32;
@@ -924,8 +925,8 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   constexpr int DEPTH = KS > 1 ? STEPS : 1;  // steps whose quants are in flight ahead of the one in use
   constexpr int SLOTS = DEPTH + 1;
   constexpr int NT = NSL * R;     // conversion tasks per half-wave
-  // 16-byte units of scale words a lane stages: Q pairs x 32 columns x NSL slices x (32 or 16) bytes / 64 lanes
-  constexpr int MU = (Q * SPW * MB + 3) / 4;
+  // 16-byte units of scale words a lane stages: Q x SIDE tiles of 16 columns x SPW slices x (32 or 16) bytes / 64 lanes
+  constexpr int MU = (Q * SIDE * SPW * MB + 7) / 8;
   constexpr uint32_t kUnitsPerColumn = SPW * kSliceBlocks * MB / 16;
   constexpr uint32_t mstride = meta_stride(FMT, SPW);
   extern __shared__ uint4 lds4[];
@@ -957,10 +958,10 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   const uint32_t sl0 = part * NSL;             // first slice of this part
   uint4* const img = lds4;                     // [NSL][R][UNITS]
   // this wave's scale words: [Q pairs x 32 columns][mstride bytes]
-  uint8_t* const wmeta = (uint8_t*)(lds4 + NSL * R * UNITS) + wave * (Q * 32 * mstride);
-  // PARK: this wave's strip for the quants of the step at hand, kSide x 16 columns
+  uint8_t* const wmeta = (uint8_t*)(lds4 + NSL * R * UNITS) + wave * (Q * SIDE * 16 * mstride);
+  // PARK: this wave's strip for the quants of the step at hand, SIDE x 16 columns
   constexpr int kStride = park_stride(FMT);
-  uint8_t* const wpark = (uint8_t*)(lds4 + NSL * R * UNITS) + 8 * (Q * 32 * mstride) + wave * (kSide * 16 * kStride);
+  uint8_t* const wpark = (uint8_t*)(lds4 + NSL * R * UNITS) + 8 * (Q * SIDE * 16 * mstride) + wave * (SIDE * 16 * kStride);
 
   // ---- the part's activations: loads first, so that nothing queues in front of them ----
   // Task (s, rr): half-wave r converts row 16 rr + r of slice sl0 + s.  (KS > 1: only slices that there are, and of a row
@@ -1009,7 +1010,7 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
     for (int j = 0; j < MU; j++) {
       const uint32_t id = 64 * j + lane;
       const uint32_t wcol = id / kUnitsPerColumn, unit = id % kUnitsPerColumn;
-      const uint32_t col = min(pair0 * (kSide * 16) + wcol, n - 1);
+      const uint32_t col = min(pair0 * (SIDE * 16) + wcol, n - 1);
       const uint8_t* src = (const uint8_t*)meta_arg + ((size_t)col * bpc + (size_t)(sl0 + wsl) * kSliceBlocks) * MB + unit * 16;
       typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
       const u32x4_a2 v = *(const u32x4_a2*)src;
@@ -1021,20 +1022,20 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   // ---- weight slices ----
   // Slices past the end of K (last part) and columns past N read the pad behind the weights or
   // a neighbour's data; their products are dropped.
-  u32x4_t wq[SLOTS][kSide][NLQ];
+  u32x4_t wq[SLOTS][SIDE][NLQ];
   constexpr uint32_t LPC = QB / 2, CPL = 64 / LPC;  // PARK: lanes per column, columns per load
   const uint32_t lane_part = FMT == MGN_FMT_Q4 ? g * 16 : (g & 1) * 32 + (g >> 1) * 16;
-  uint32_t q_off[Q][kSide][PARK ? NLQ : 1];
+  uint32_t q_off[Q][SIDE][PARK ? NLQ : 1];
 #pragma unroll
   for (int p = 0; p < Q; p++)
 #pragma unroll
-    for (int u = 0; u < kSide; u++) {
+    for (int u = 0; u < SIDE; u++) {
       if constexpr (PARK) {
 #pragma unroll
         for (int j = 0; j < NLQ; j++)
-          q_off[p][u][j] = min(((pair0 + p) * kSide + u) * 16 + CPL * j + lane / LPC, n - 1) * bpc * QB + (lane % LPC) * 16;
+          q_off[p][u][j] = min(((pair0 + p) * SIDE + u) * 16 + CPL * j + lane / LPC, n - 1) * bpc * QB + (lane % LPC) * 16;
       } else {
-        q_off[p][u][0] = min(((pair0 + p) * kSide + u) * 16 + c, n - 1) * bpc * QB + lane_part;
+        q_off[p][u][0] = min(((pair0 + p) * SIDE + u) * 16 + c, n - 1) * bpc * QB + lane_part;
       }
     }
   auto fetch = [&](int f) {  // step f into slot f % SLOTS
@@ -1042,7 +1043,7 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
     if (KS > 1 && ((uint32_t)f >= run || sl >= nslices)) return;
     const uint8_t* const qb = (const uint8_t*)quants_arg + (size_t)(sl * kSliceBlocks) * QB;
 #pragma unroll
-    for (int u = 0; u < kSide; u++)
+    for (int u = 0; u < SIDE; u++)
 #pragma unroll
       for (int j = 0; j < NLQ; j++)
         wq[f % SLOTS][u][j] = __builtin_nontemporal_load(
@@ -1104,21 +1105,21 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
 #pragma unroll
   for (int j = 0; j < MU; j++) {
     const uint32_t id = 64 * j + lane;
-    if (Q * 32 * kUnitsPerColumn % 64 == 0 || id < Q * 32 * kUnitsPerColumn)
+    if (Q * SIDE * 16 * kUnitsPerColumn % 64 == 0 || id < Q * SIDE * 16 * kUnitsPerColumn)
       *(u32x4_t*)(wmeta + (id / kUnitsPerColumn) * mstride + (id % kUnitsPerColumn) * 16) = mu[j];
   }
   __builtin_amdgcn_sched_barrier(0);
   lds_barrier();
   __builtin_amdgcn_sched_barrier(0);
 
-  floatx4 res[Q][kSide][R];
+  floatx4 res[Q][SIDE][R];
 #pragma unroll
   for (int p = 0; p < Q; p++)
 #pragma unroll
-    for (int u = 0; u < kSide; u++)
+    for (int u = 0; u < SIDE; u++)
 #pragma unroll
       for (int r = 0; r < R; r++) res[p][u][r] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  const bool pair_live[2] = {pair0 * (kSide * 16) < n, (pair0 + Q - 1) * (kSide * 16) < n};  // uniform over the wave
+  const bool pair_live[2] = {pair0 * (SIDE * 16) < n, (pair0 + Q - 1) * (SIDE * 16) < n};  // uniform over the wave
 #pragma unroll
   for (int f = 0; f < STEPS; f++) {
     const int slot = f % SLOTS, wp = f / SPW, wf = f % SPW;
@@ -1127,10 +1128,10 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
     if (f + DEPTH < STEPS) fetch(f + DEPTH);
     __builtin_amdgcn_sched_barrier(0);
     // the slot's quants into B operand order, the step's scale words from LDS
-    uint32_t mw[kSide][8];
+    uint32_t mw[SIDE][8];
 #pragma unroll
-    for (int u = 0; u < kSide; u++) {
-      const uint8_t* const ms = wmeta + ((wp * kSide + u) * 16 + c) * mstride + wf * (kSliceBlocks * MB);
+    for (int u = 0; u < SIDE; u++) {
+      const uint8_t* const ms = wmeta + ((wp * SIDE + u) * 16 + c) * mstride + wf * (kSliceBlocks * MB);
       if constexpr (FMT == MGN_FMT_Q4) {
         const u32x4_t m0 = *(const u32x4_t*)ms, m1 = *(const u32x4_t*)(ms + 16);
         mw[u][0] = m0.x, mw[u][1] = m0.y, mw[u][2] = m0.z, mw[u][3] = m0.w;
@@ -1159,11 +1160,11 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
       const uint32_t kb0 = sl_raw * kSliceBlocks;
       if (kb0 + kSliceBlocks > bpc) {  // last slice of a K that is no multiple of 256
 #pragma unroll
-        for (int u = 0; u < kSide; u++)
+        for (int u = 0; u < SIDE; u++)
 #pragma unroll
           for (int e = 0; e < 8; e++) mw[u][e] = kb0 + e < bpc ? mw[u][e] : 0u;
       }
-      slice_mac_side<FMT, F32A, R, PARK>(wq[slot], wpark + c * kStride + g * (QB / 4), mw, (const uint8_t*)(img + ws * R * UNITS),
+      slice_mac_side<FMT, F32A, R, PARK, SIDE>(wq[slot], wpark + c * kStride + g * (QB / 4), mw, (const uint8_t*)(img + ws * R * UNITS),
                                          UNITS * 16, g, lane, tail.lift, res[wp]);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1172,16 +1173,18 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
 #pragma unroll
     for (int p = 0; p < Q; p++)
 #pragma unroll
-      for (int u = 0; u < kSide; u++)
+      for (int u = 0; u < SIDE; u++)
 #pragma unroll
         for (int r = 0; r < R; r++) res[p][u][r] *= kOpScale;
   }
   __builtin_amdgcn_sched_barrier(0);
 
   if constexpr (KS > 1) {
-    const floatx4 own[kSide] = {res[0][0][0], res[0][1][0]};
-    split_tail<KS>(own, wpark, kSide * 16 * kStride, wave, lane, part, parts, rg * colgroups + cg, rowgroups * colgroups, row0,
-                   wcg * (8 / KS * kSide * 16), min(m, row0 + group_rows), n, tail);
+    floatx4 own[SIDE];
+#pragma unroll
+    for (int u = 0; u < SIDE; u++) own[u] = res[0][u][0];
+    split_tail<KS, SIDE>(own, wpark, SIDE * 16 * kStride, wave, lane, part, parts, rg * colgroups + cg, rowgroups * colgroups, row0,
+                   wcg * (8 / KS * SIDE * 16), min(m, row0 + group_rows), n, tail);
     return;
   }
   if (parts > 1) {
@@ -1198,8 +1201,8 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
     // fault word, which the next synchronising call reports, and goes on with what it has.
     // The partial tiles travel in register order: the float4 a lane holds for (pair, side, row tile)
     // goes out and comes back as one 128-bit access, 1 KiB per wave and instruction, at
-    //   (((part * row groups + row group) * column groups + column group) * 8 + wave) * Q * kSide * R + slot
-    constexpr uint32_t kSlots = Q * kSide * R;
+    //   (((part * row groups + row group) * column groups + column group) * 8 + wave) * Q * SIDE * R + slot
+    constexpr uint32_t kSlots = Q * SIDE * R;
     constexpr int kDeviceScope = 16;  // the sc1 bit of a buffer instruction's cache policy
     const uint32_t wgs_per_part = rowgroups * colgroups;
     const uint32_t part_stride = wgs_per_part * (8u * kSlots * 1024u);
@@ -1218,13 +1221,13 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
 #pragma unroll
       for (int p = 0; p < Q; p++)
 #pragma unroll
-        for (int u = 0; u < kSide; u++)
+        for (int u = 0; u < SIDE; u++)
 #pragma unroll
           for (int r = 0; r < R; r++) {
             u32x4_t v = __builtin_bit_cast(u32x4_t, res[p][u][r]);
 #pragma unroll
             for (int i = 0; i < 4; i++) v[i] = v[i] == kHandoverEmpty ? 0x7FC00000u : v[i];
-            __builtin_amdgcn_raw_buffer_store_b128(v, all_parts, part * part_stride + my_off + ((p * kSide + u) * R + r) * 1024u, 0,
+            __builtin_amdgcn_raw_buffer_store_b128(v, all_parts, part * part_stride + my_off + ((p * SIDE + u) * R + r) * 1024u, 0,
                                                    kDeviceScope);
           }
       bool gave_up = false;
@@ -1266,9 +1269,9 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
             }
           }
         }
-        // the tile's place in the output: slot = (pair * kSide + side) * R + row tile of wave src_wave
-        const uint32_t tp = slot / (kSide * R), tu = (slot / R) % kSide, tr = slot % R;
-        const uint32_t col = (((wcg * 8 + src_wave) * Q + tp) * kSide + tu) * 16 + c;
+        // the tile's place in the output: slot = (pair * SIDE + side) * R + row tile of wave src_wave
+        const uint32_t tp = slot / (SIDE * R), tu = (slot / R) % SIDE, tr = slot % R;
+        const uint32_t col = (((wcg * 8 + src_wave) * Q + tp) * SIDE + tu) * 16 + c;
         if (col < n) {
           if (row0 + R * 16 <= m && !tail.dres && tail.epilogue == 0) {  // (uniform) whole rows, nothing to add or apply
             float* const dst = tail.c + (size_t)(row0 + tr * 16 + 4 * g) * n + col;
@@ -1293,13 +1296,13 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
 #pragma unroll
       for (int p = 0; p < Q; p++)
 #pragma unroll
-        for (int u = 0; u < kSide; u++)
+        for (int u = 0; u < SIDE; u++)
 #pragma unroll
           for (int r = 0; r < R; r++) {
             u32x4_t v = __builtin_bit_cast(u32x4_t, res[p][u][r]);
 #pragma unroll
             for (int i = 0; i < 4; i++) v[i] = v[i] == kHandoverEmpty ? 0x7FC00000u : v[i];
-            __builtin_amdgcn_raw_buffer_store_b128(v, partials, part * part_stride + my_off + ((p * kSide + u) * R + r) * 1024u, 0,
+            __builtin_amdgcn_raw_buffer_store_b128(v, partials, part * part_stride + my_off + ((p * SIDE + u) * R + r) * 1024u, 0,
                                                    kDeviceScope);
           }
       return;
@@ -1356,9 +1359,9 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
 #pragma unroll
     for (int p = 0; p < Q; p++)
 #pragma unroll
-      for (int u = 0; u < kSide; u++)
+      for (int u = 0; u < SIDE; u++)
 #pragma unroll
-        for (int r = 0; r < R; r++) res[p][u][r] = sum[(p * kSide + u) * R + r] + res[p][u][r];
+        for (int r = 0; r < R; r++) res[p][u][r] = sum[(p * SIDE + u) * R + r] + res[p][u][r];
     if (gave_up && lane == 0 && tail.fault_flag) *tail.fault_flag = 1u;
   }
   // The stores end every wave's life, with nothing left to hide them behind: a row group that lies
@@ -1368,8 +1371,8 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
 #pragma unroll
   for (int p = 0; p < Q; p++)
 #pragma unroll
-    for (int u = 0; u < kSide; u++) {
-      const uint32_t col = ((pair0 + p) * kSide + u) * 16 + c;
+    for (int u = 0; u < SIDE; u++) {
+      const uint32_t col = ((pair0 + p) * SIDE + u) * 16 + c;
       if (col < n) {
         if (whole_rows) {
           const size_t first = (size_t)(row0 + 4 * g) * n + col;
@@ -1418,6 +1421,7 @@ AddLift add_lift(const WeightView& w) {
 
 struct ResidentPlan {
   uint32_t ks;  // waves that share a pair of column tiles
+  uint32_t side;  // column tiles of a wave: kSide, or one where ks > 1 and the launch has room for twice the workgroups
   uint32_t rows;  // of a row group when ks > 1: 16, or 8 in half-empty tiles
   uint32_t r, q, nsl, parts, colgroups, rowgroups, nslices;
   bool park;  // quants through a wave-private LDS strip (if there is room) instead of row swaps
@@ -1426,9 +1430,9 @@ struct ResidentPlan {
   double cost;
 };
 
-size_t resident_lds_bytes(int fmt, bool f32a, uint32_t r, uint32_t q, bool park, uint32_t nsl, uint32_t ks = 1) {
-  return (size_t)nsl * r * image_units(f32a) * 16 + (size_t)8 * q * 32 * meta_stride(fmt, nsl / ks) +
-         (park ? (size_t)8 * kSide * 16 * park_stride(fmt) : 0);
+size_t resident_lds_bytes(int fmt, bool f32a, uint32_t r, uint32_t q, bool park, uint32_t nsl, uint32_t ks = 1, uint32_t side = kSide) {
+  return (size_t)nsl * r * image_units(f32a) * 16 + (size_t)8 * q * side * 16 * meta_stride(fmt, nsl / ks) +
+         (park ? (size_t)8 * side * 16 * park_stride(fmt) : 0);
 }
 
 // A launch that leaves CUs idle spreads over more of them: KS waves share a pair of column tiles and split K between them
@@ -1444,6 +1448,10 @@ size_t resident_lds_bytes(int fmt, bool f32a, uint32_t r, uint32_t q, bool park,
 // Q8 in four parts or more (0.91 to 1.09); Q8 in two or three parts 0.92.  Q8 with fp16 activations and two slices stays on the 32x32
 // kernel: level (0.87 to 1.11), and that kernel's error is up to 3 % smaller there.  (From three slices on the error against f64 is the smaller
 // one here: medians Q4 0.90, behind a silu 0.72; Q8 0.97, 0.89.)
+// Where twice the workgroups still fit, a wave has one column tile instead of two side by side: half the requests, and half the walk, whose
+// reads of the activations it no longer shares, which half the columns per CU leave room for.  Fewer rows come first (the conversion is
+// the longer stretch then).  75 drawn calls of 4.2 to 7.1 us, two tiles -> one: 0.77 to 1.004 of the time, median 0.87, the same bits: Q8
+// 12 x 960 x 2336 5.9 -> 4.8, 43 x 2688 x 346 7.1 -> 5.9, 348 x 288 x 288 5.35 -> 4.5, Q4 12 x 1024 x 1024 5.1 -> 4.5, 5 x 2048 x 2033 6.0 -> 5.4.
 void split_resident(const LaunchArgs& x, ResidentPlan* p) {
   const bool f32a = !x.a_is_f16;
   const uint32_t nsl = resident_slices(f32a, 1), parts = (p->nslices + nsl - 1) / nsl;
@@ -1452,19 +1460,21 @@ void split_resident(const LaunchArgs& x, ResidentPlan* p) {
   for (uint32_t ks = 4; ks >= 2; ks /= 2) {
     if (std::min(nsl, p->nslices) <= ks / 2) continue;
     if (ks == 2 && parts > (x.w.fmt == MGN_FMT_Q4 ? 1u : 3u)) continue;
-    const uint32_t per_wg = 8 / ks * kSide;
-    auto groups_of = [&](uint32_t n) { return ((n + 15) / 16 + per_wg - 1) / per_wg; };
-    uint64_t colgroups = groups_of(x.w.n);
-    for (int j = 0; j < x.n_more; j++) colgroups += groups_of(x.more[j].w.n);
-    for (uint32_t rows = 8; rows <= 16; rows += 8) {
+    for (uint32_t form = 0; form < 4; form++) {
+      const uint32_t rows = form < 2 ? 8 : 16, side = form % 2 ? kSide : 1;
+      const uint32_t held = ks == 2 && p->nslices <= 2 ? 2 : nsl;
+      if (side == 1 && ks == 2 && held != 2) continue;
+      const uint32_t per_wg = 8 / ks * side;
+      auto groups_of = [&](uint32_t n) { return ((n + 15) / 16 + per_wg - 1) / per_wg; };
+      uint64_t colgroups = groups_of(x.w.n);
+      for (int j = 0; j < x.n_more; j++) colgroups += groups_of(x.more[j].w.n);
       const uint32_t rowgroups = (x.m + rows - 1) / rows;
       // (resident at once: see plan_resident)
       if ((colgroups * rowgroups + 7) / 8 * parts > (uint64_t)x.num_cus / 8) continue;
       const uint64_t partial = parts > 1 ? parts * rowgroups * colgroups * (per_wg * 1024u) : 0;
-      const uint32_t held = ks == 2 && p->nslices <= 2 ? 2 : nsl;
-      const size_t lds = resident_lds_bytes(x.w.fmt, f32a, 1, 1, true, held, ks);
+      const size_t lds = resident_lds_bytes(x.w.fmt, f32a, 1, 1, true, held, ks, side);
       if (partial > x.handover_bytes || lds > 160 * 1024) continue;
-      p->ks = ks, p->rows = rows, p->r = 1, p->q = 1, p->nsl = held, p->parts = parts;
+      p->ks = ks, p->side = side, p->rows = rows, p->r = 1, p->q = 1, p->nsl = held, p->parts = parts;
       p->colgroups = (uint32_t)colgroups, p->rowgroups = rowgroups;
       p->park = true, p->spread = parts > 1, p->lds = lds, p->partial_bytes = partial;
       p->cost = 1.5 + 1.0 / ks + (parts > 1 ? 1.0 : 0.0);
@@ -1524,7 +1534,7 @@ bool plan_resident(const LaunchArgs& x, ResidentPlan* out) {
       const double cost = std::ceil((double)wgs / x.num_cus) * (1.5 + q * r * nsl / 4.0) * (r == 2 ? 0.9 : 1.0) + (parts > 1 ? 1.0 : 0.0);
       if (best == 0 || cost < best) {
         best = cost;
-        bp.ks = 1, bp.r = r, bp.q = q, bp.nsl = nsl, bp.parts = parts, bp.colgroups = colgroups, bp.rowgroups = rowgroups;
+        bp.ks = 1, bp.side = kSide, bp.r = r, bp.q = q, bp.nsl = nsl, bp.parts = parts, bp.colgroups = colgroups, bp.rowgroups = rowgroups;
         bp.nslices = nslices, bp.partial_bytes = partial, bp.cost = cost, bp.spread = spread;
         bp.park = resident_lds_bytes(x.w.fmt, f32a, r, q, true, nsl) <= 160 * 1024;
         bp.lds = resident_lds_bytes(x.w.fmt, f32a, r, q, bp.park, nsl);
@@ -1541,7 +1551,7 @@ bool plan_resident(const LaunchArgs& x, ResidentPlan* out) {
   return true;
 }
 
-template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1, int NSL = resident_slices(F32A, R)>
+template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1, int NSL = resident_slices(F32A, R), int SIDE = kSide>
 int launch_resident_q(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& p) {
   if constexpr (R == 1 && Q == 1 && PARK && !LATE && KS == 1 && NSL == resident_slices(F32A, R)) {
     if (p.nsl == 3) return launch_resident_q<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, 3>(s, x, p);
@@ -1551,15 +1561,18 @@ int launch_resident_q(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& 
   if constexpr (KS == 2 && NSL == resident_slices(F32A, R)) {
     if (p.nsl == 2) return launch_resident_q<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, 2>(s, x, p);
   }
-  if (p.nsl != NSL) return (int)hipErrorInvalidValue;
-  auto kern = tile_resident_kernel<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, NSL>;
+  if constexpr (SIDE == kSide && (KS == 4 || (KS == 2 && NSL == 2))) {
+    if (p.side == 1) return launch_resident_q<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, NSL, 1>(s, x, p);
+  }
+  if (p.nsl != NSL || p.side != SIDE) return (int)hipErrorInvalidValue;
+  auto kern = tile_resident_kernel<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, NSL, SIDE>;
   static std::atomic<uint64_t> big_lds_done{0};
   if (p.lds > 64 * 1024)
     if (int e = enable_big_lds(kern, x.device, big_lds_done)) return e;
   const TileTail tail{x.d, x.c, (float*)x.scratch, x.counters, x.epilogue, (float*)x.handover, x.spin_limit, x.fault_flag, p.spread ? 1u : 0u, add_lift(x.w), p.rows};
   RowsExtra extra{};
   if constexpr (ROWS != kRowsPlain) {
-    constexpr uint32_t per_wg = 8 / KS * kSide * Q;
+    constexpr uint32_t per_wg = 8 / KS * SIDE * Q;
     uint32_t first = ((x.w.n + 15) / 16 + per_wg - 1) / per_wg;
     for (int j = 0; j < x.n_more; j++) {
       const LaunchArgs::More& o = x.more[j];
@@ -1875,7 +1888,7 @@ bool describe_tile_mfma(const LaunchArgs& x, mgn_plan_info* out) {
     out->grid[0] = rp.parts, out->grid[1] = rp.colgroups, out->grid[2] = rp.rowgroups;
     out->threads = 512;
     out->lds_bytes = (uint32_t)rp.lds;
-    out->waves_n = 8 / rp.ks * kSide * rp.q, out->k_splits = rp.ks, out->k_parts = rp.parts, out->steps = (uint32_t)resident_slices(!x.a_is_f16, rp.r);  // slices of a part at most
+    out->waves_n = 8 / rp.ks * rp.side * rp.q, out->k_splits = rp.ks, out->k_parts = rp.parts, out->steps = (uint32_t)resident_slices(!x.a_is_f16, rp.r);  // slices of a part at most
     out->quads_per_wave = 0, out->full_steps = rp.r, out->tail_blocks = 0;
     out->workspace_bytes = rp.partial_bytes;
     return true;
