@@ -639,7 +639,8 @@ __global__ __launch_bounds__(512) void tile_mfma_kernel(const uint4* __restrict_
 // That form touches half a cache line per column and instruction, twice as many lines per byte,
 // and the CU's memory pipeline charges per line: M = 16 on 4096 x 14336 takes 14.0 us with it and
 // 13.3 us parked (Q8: 18.9 and 16.6 us).  It remains for the plans whose LDS is full (two pairs
-// of tiles per wave with f32 activations).
+// of tiles per wave with f32 activations and four slices; strips for half a slice at a time, which do fit, went both ways: us, f32 Q4
+// 20 x 10208 x 5410 31.3 -> 26.4, 80 x 3872 x 8224 47.4 -> 41.1, but 412 x 1024 x 2752 16.5 -> 18.5, 120 x 2656 x 3904 19.1 -> 21.1).
 // The scale words are wanted by all four lanes of a column; loading them per lane would ask the
 // memory pipeline for every word four times.  Each wave instead loads the words of all its
 // columns and slices once, in whole cache lines, parks them in its own LDS strip and reads a
@@ -896,7 +897,8 @@ constexpr int kRowsPlain = -1;
 // with four.  Counted at compile time: bounds tested on the way cost a whole part of four 4 to 6 %.  us, NSL = 4 -> as many as there are:
 // f32 Q4 204 x 256 x 2656 6.5 -> 4.5, 224 x 320 x 2976 7.4 -> 6.1, 234 x 544 x 2240 8.7 -> 8.1, 67 x 1536 x 1664 10.8 -> 9.0, Q8 326 x 1152 x 1472
 // 12.9 -> 11.1, 375 x 2304 x 608 12.5 -> 11.0; fp16 Q4 406 x 1408 x 308 9.0 -> 7.8; with two waves to a pair of tiles, K of 288 to 512, 40 calls
-// of 4.7 to 6.2 us 0.93 to 0.96.
+// of 4.7 to 6.2 us 0.93 to 0.96; two pairs of tiles per wave, whose quants then find room in strips, f32 Q4 66 x 1472 x 9344 21.5 -> 16.8,
+// 307 x 1184 x 1760 19.8 -> 16.5, 1899 x 1472 x 370 19.5 -> 16.7.
 
 // ROWS: kRowsPlain, or the activations' prologue (kProNone / kProRmsNorm / kProSwiglu) of a launch that may
 // serve several weights.  A decoder layer of some hundred rows is made of launches that last 10 to 25 us
@@ -913,7 +915,7 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
                                                              TileTail tail, RowsExtra extra) {
   static_assert(ROWS == kRowsPlain || (F32A && R == 1 && !LATE), "the forms that are launched");
   static_assert(KS == 1 || (R == 1 && Q == 1 && PARK && !LATE), "the forms that are launched");
-  static_assert(NSL == resident_slices(F32A, R) || (R == 1 && Q == 1 && PARK && !LATE && (KS == 1 || (KS == 2 && NSL == 2))), "the forms that are launched");
+  static_assert(NSL == resident_slices(F32A, R) || (R == 1 && PARK && !LATE && (KS == 1 || (KS == 2 && NSL == 2))), "the forms that are launched");
   static_assert(SIDE == kSide || (KS == 4 || (KS == 2 && NSL == 2)), "the forms that are launched");
   constexpr uint32_t UNITS = image_units(F32A);
   constexpr float kOpScale = FMT == MGN_FMT_Q4 ? 1048576.0f : 16777216.0f;
@@ -1543,9 +1545,10 @@ bool plan_resident(const LaunchArgs& x, ResidentPlan* out) {
   }
   if (best == 0) return false;
   if (x.split_waves) split_resident(x, &bp);
-  if (bp.ks == 1 && bp.r == 1 && bp.q == 1 && bp.park) {  // (the other forms are built for four slices)
+  if (bp.ks == 1 && bp.r == 1) {  // (the other forms are built for four slices)
     bp.nsl = (nslices + bp.parts - 1) / bp.parts;
-    bp.lds = resident_lds_bytes(x.w.fmt, f32a, 1, 1, true, bp.nsl);
+    bp.park = resident_lds_bytes(x.w.fmt, f32a, 1, bp.q, true, bp.nsl) <= 160 * 1024;
+    bp.lds = resident_lds_bytes(x.w.fmt, f32a, 1, bp.q, bp.park, bp.nsl);
   }
   *out = bp;
   return true;
@@ -1553,7 +1556,7 @@ bool plan_resident(const LaunchArgs& x, ResidentPlan* out) {
 
 template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1, int NSL = resident_slices(F32A, R), int SIDE = kSide>
 int launch_resident_q(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& p) {
-  if constexpr (R == 1 && Q == 1 && PARK && !LATE && KS == 1 && NSL == resident_slices(F32A, R)) {
+  if constexpr (R == 1 && PARK && !LATE && KS == 1 && NSL == resident_slices(F32A, R)) {
     if (p.nsl == 3) return launch_resident_q<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, 3>(s, x, p);
     if (p.nsl == 2) return launch_resident_q<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, 2>(s, x, p);
     if (p.nsl == 1) return launch_resident_q<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, 1>(s, x, p);
@@ -1564,7 +1567,7 @@ int launch_resident_q(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& 
   if constexpr (SIDE == kSide && (KS == 4 || (KS == 2 && NSL == 2))) {
     if (p.side == 1) return launch_resident_q<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, NSL, 1>(s, x, p);
   }
-  if (p.nsl != NSL || p.side != SIDE) return (int)hipErrorInvalidValue;
+  if (p.nsl != NSL || p.side != SIDE || p.park != PARK) return (int)hipErrorInvalidValue;
   auto kern = tile_resident_kernel<FMT, F32A, R, Q, PARK, LATE, ROWS, KS, NSL, SIDE>;
   static std::atomic<uint64_t> big_lds_done{0};
   if (p.lds > 64 * 1024)
@@ -1599,18 +1602,27 @@ int launch_resident_q(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& 
   return 0;
 }
 
-template <int FMT, int Q, int KS>
+// (f32 activations, two pairs of tiles per wave: strips fit beside up to three slices, and four go without)
+template <int FMT, bool F32A, int ROWS>
+int launch_resident_two(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& p) {
+  if (p.nsl == 1) return launch_resident_q<FMT, F32A, 1, 2, true, false, ROWS, 1, 1>(s, x, p);
+  if (p.nsl == 2) return launch_resident_q<FMT, F32A, 1, 2, true, false, ROWS, 1, 2>(s, x, p);
+  if (p.nsl == 3) return launch_resident_q<FMT, F32A, 1, 2, true, false, ROWS, 1, 3>(s, x, p);
+  return launch_resident_q<FMT, F32A, 1, 2, !F32A, false, ROWS>(s, x, p);
+}
+
+template <int FMT, int ROWS>
 int launch_resident_rows(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& p) {
-  constexpr bool kPark = Q == 1;
-  if (p.park != kPark) return (int)hipErrorInvalidValue;
-  if (x.pro_kind == kProRmsNorm) return launch_resident_q<FMT, true, 1, Q, kPark, false, kProRmsNorm, KS>(s, x, p);
-  if (x.pro_kind == kProSwiglu) return launch_resident_q<FMT, true, 1, Q, kPark, false, kProSwiglu, KS>(s, x, p);
-  return launch_resident_q<FMT, true, 1, Q, kPark, false, kProNone, KS>(s, x, p);
+  if (p.q == 2) return launch_resident_two<FMT, true, ROWS>(s, x, p);
+  return p.ks == 1   ? launch_resident_q<FMT, true, 1, 1, true, false, ROWS>(s, x, p)
+         : p.ks == 2 ? launch_resident_q<FMT, true, 1, 1, true, false, ROWS, 2>(s, x, p)
+                     : launch_resident_q<FMT, true, 1, 1, true, false, ROWS, 4>(s, x, p);
 }
 template <int FMT>
 int launch_resident_rows(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan& p) {
-  if (p.q == 2) return launch_resident_rows<FMT, 2, 1>(s, x, p);
-  return p.ks == 1 ? launch_resident_rows<FMT, 1, 1>(s, x, p) : p.ks == 2 ? launch_resident_rows<FMT, 1, 2>(s, x, p) : launch_resident_rows<FMT, 1, 4>(s, x, p);
+  if (x.pro_kind == kProRmsNorm) return launch_resident_rows<FMT, kProRmsNorm>(s, x, p);
+  if (x.pro_kind == kProSwiglu) return launch_resident_rows<FMT, kProSwiglu>(s, x, p);
+  return launch_resident_rows<FMT, kProNone>(s, x, p);
 }
 
 template <int FMT, bool F32A>
@@ -1626,9 +1638,8 @@ int launch_resident_fa(ihipStream_t* s, const LaunchArgs& x, const ResidentPlan&
   if (p.r != 1) return (int)hipErrorInvalidValue;
   if (p.ks == 2) return launch_resident_q<FMT, F32A, 1, 1, true, false, kRowsPlain, 2>(s, x, p);
   if (p.ks == 4) return launch_resident_q<FMT, F32A, 1, 1, true, false, kRowsPlain, 4>(s, x, p);
-  if (p.q == 1)
-    return p.park ? launch_resident_q<FMT, F32A, 1, 1, true>(s, x, p) : launch_resident_q<FMT, F32A, 1, 1, false>(s, x, p);
-  return p.park ? launch_resident_q<FMT, F32A, 1, 2, true>(s, x, p) : launch_resident_q<FMT, F32A, 1, 2, false>(s, x, p);
+  if (p.q == 1) return launch_resident_q<FMT, F32A, 1, 1, true>(s, x, p);
+  return launch_resident_two<FMT, F32A, kRowsPlain>(s, x, p);
 }
 
 struct TilePlan {

@@ -1,5 +1,5 @@
 """The resident kernel's parts of fewer than four slices: K of one to three slices, and of 5, 6 and 9, which is cut evenly (one block, whole slices,
-a block more), with one wave and with two to a pair of tiles, against the oracle's product in f64."""
+a block more), with one wave and with two to a pair of tiles and with two pairs to a wave, against the oracle's product in f64."""
 import numpy as np
 import pytest
 
@@ -49,3 +49,34 @@ def test_short_parts(ctx, orc, fmt, m, n, k):
         np.testing.assert_array_equal(got[2], got[0] + d)
     for h in (wt, db, c):
         h.free()
+
+
+@pytest.mark.parametrize("fmt", [Q4, Q8])
+@pytest.mark.parametrize("m,k,n,f16", [(400, 256, 2700, False), (401, 288, 2700, False), (400, 544, 2690, False), (389, 1056, 2182, False), (385, 1536, 2177, False),
+                                       (390, 1024, 2700, False), (5, 288, 66000, True)])
+def test_two_pairs_of_tiles_per_wave(ctx, orc, fmt, m, k, n, f16):
+    """The bound above."""
+    if not f16:
+        p = capi.matmul_plan(fmt, m, k, n)
+        assert p.route == capi.ROUTE_TILE_MFMA and p.waves_n == 32 and p.quads_per_wave == 0
+    w = synth.normal(k + n, k * n, 0.02).reshape(k, n)
+    x, d = synth.normal(m + k, m * k).reshape(m, k).copy(), synth.normal(7, m * n).reshape(m, n)
+    x[0], x[1] = 0, x[1] * 2.0 ** -10
+    x = x.astype(np.float16) if f16 else x
+    exact = orc.matmul_f64(x.astype(np.float32), orc.dequantize(fmt, orc.quantize(fmt, w), k, n))
+    wt, a, c, db = ctx.weight(fmt, w), ctx.upload(x), ctx.buffer(m * n * 4), ctx.upload(d)
+    ctx.set_route(capi.ROUTE_TILE_MFMA)
+    try:
+        got = []
+        for res in (None, None, db):
+            (ctx.matmul_q_f16a if f16 else ctx.matmul_q)(a, wt, c, m, res)
+            got.append(c.download(np.float32, m * n).reshape(m, n))
+    finally:
+        ctx.set_route(capi.ROUTE_AUTO)
+        for h in (wt, a, c, db):
+            h.free()
+    cut = 0.0 if f16 else 2.0 ** -20
+    bound = 5 * 0.02 * np.sqrt(n) * (cut + 2.0 ** -23 + 2.0 ** -24 * np.sqrt(k)) * np.linalg.norm(x.astype(np.float64), axis=1) + 1e-30
+    assert (np.linalg.norm(got[0] - exact, axis=1) <= bound).all()
+    assert (bits(got[0]) == bits(got[1])).all()
+    np.testing.assert_array_equal(got[2], got[0] + d)
