@@ -906,7 +906,7 @@ constexpr int kRowsPlain = -1;
 // Every workgroup converts its own rows anyway, so a norm (where the part holds the whole row: one K
 // part) or a SwiGLU costs it a second operand per element and no pass over memory; weights side by side
 // fill the rounds that each would leave open.  Two decoder layers of 333 rows, 1024 wide (Q8), q | k | v, the
-// output projection, gate | up and down with norms and SwiGLU: 18 launches, 213 us -> 8 launches, 161 us (Q4 184
+// output projection, gate | up and down with norms and SwiGLU: 18 launches, 213 us -> 8 launches, 161 us, 138 since K parts go out evenly (Q4 184
 // -> 139; 128 rows, 576 wide 156 -> 104; 8 rows Q4 138 -> 90).
 template <int FMT, bool F32A, int R, int Q, bool PARK, bool LATE = false, int ROWS = kRowsPlain, int KS = 1, int NSL = resident_slices(F32A, R), int SIDE = kSide>
 __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restrict__ a, const void* __restrict__ meta_arg,
