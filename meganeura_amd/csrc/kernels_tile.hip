@@ -1848,12 +1848,22 @@ bool tile_mfma_splits(const LaunchArgs& x) {
 // 20.4 against 19.0);
 // Q8 is between 0.8 and 1.4 of the tiled kernel's time on this one and stays where it was (beside the
 // rescaling kernels it is always the faster one: see use_resident).
+// fp16 activations in one round of workgroups, K of three slices and more (the 32x32 kernel starts its weights later, and its K parts
+// meet through a counter; us, 32x32 -> here, 108 drawn calls): up to 16 rows with one pair of tiles per wave (35 calls 0.59 to 0.85, Q4 11 x 7808 x 4000 17.7 ->
+// 10.4, Q8 11 x 11680 x 1490 18.3 -> 11.3; two pairs 1.01, 1.08); Q4 of 17 to 32 rows in three K parts and more (0.70 to 1.00; in two 1.04 and 1.14; Q8 0.84 to 1.31, no rule); Q8
+// from 128 rows on (17 calls 0.59 to 0.97, 308 x 3072 x 909 19.7 -> 12.7), with row groups of 32 up to 512 rows and in K parts (beyond 0.87, 1.11,
+// 1.13; in one part 0.83 to 1.00, where it stays behind); a second round costs up to 1.7 times there.
 bool tile_mfma_preferred(const LaunchArgs& x) {
   ResidentPlan rp;
   if (!use_resident(x, &rp)) return false;
   if (rp.ks > 1) return true;
   const uint64_t wgs = (uint64_t)rp.parts * rp.colgroups * rp.rowgroups;
   const uint64_t rounds = (wgs + x.num_cus - 1) / x.num_cus;
+  if (x.a_is_f16 && rounds == 1 && rp.nslices >= 3) {
+    if (x.m <= 16 && rp.q == 1) return true;
+    if (x.m <= 32 && x.w.fmt == MGN_FMT_Q4 && rp.parts >= 3) return true;
+    if (x.m >= 128 && x.w.fmt == MGN_FMT_Q8 && (rp.r == 1 || (x.m <= 512 && rp.parts > 1))) return true;
+  }
   if (x.m > 32)
     return x.w.fmt == MGN_FMT_Q4 && (rp.parts == 1 || (rp.park && rounds == 1) || 4 * wgs >= 3 * rounds * (uint64_t)x.num_cus);
   if (x.m > 16) {

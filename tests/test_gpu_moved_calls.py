@@ -1,5 +1,6 @@
 """Calls that the automatic route gives to the blocked kernel because of what the plan of the kernel behind it says (narrow results of long K, ragged
-rounds): every form of such a call on both kernels, against the oracle's product in f64 and against each other."""
+rounds), and calls with fp16 activations that it gives to the resident kernel in one round instead of the 32x32 one: every form of such a call on both
+kernels, against the oracle's product in f64 and against each other."""
 import numpy as np
 import pytest
 
@@ -73,4 +74,38 @@ def test_both_kernels_give_the_call_its_result(ctx, orc, fmt, m, k, n, f16):
         assert not np.isfinite(hit[bad]).any()
     good = [r for r in range(m) if r not in bad]
     np.testing.assert_array_equal(run(ctx, x, wt)[good], got[good])
+    wt.free()
+
+
+@pytest.mark.parametrize("fmt,m,k,n", [
+    (Q4, 5, 8864, 1795), (Q4, 11, 7808, 4000), (Q4, 16, 1152, 21430), (Q4, 17, 10688, 2103), (Q4, 32, 3808, 2833), (Q8, 9, 4256, 5268), (Q8, 16, 1888, 17030),
+    (Q8, 152, 3296, 394), (Q8, 308, 3072, 909), (Q8, 374, 1856, 1918)])
+def test_fp16_activations_on_the_resident_kernel(ctx, orc, fmt, m, k, n):
+    """fp16 activations enter exactly: f32 sums of K products and block means carried with 22 bits, on the same sums as above."""
+    p = capi.matmul_plan(fmt, m, k, n, True, auto=True)
+    assert p.route == capi.ROUTE_TILE_MFMA and p.k_splits == 1 and p.quads_per_wave == 0
+    w = synth.normal(2 * k + n, k * n, 0.02).reshape(k, n)
+    x, d = synth.normal(m + k, m * k).reshape(m, k).astype(np.float16), synth.normal(7, m * n).reshape(m, n)
+    x[0], x[1] = 0, x[1] * np.float16(2.0 ** -10)
+    wt = ctx.weight(fmt, w)
+    exact = orc.matmul_f64(x.astype(np.float32), orc.dequantize(fmt, orc.quantize(fmt, w), k, n))
+    bound = 5 * (2.0 ** -22 + 2.0 ** -24 * np.sqrt(k)) * (0.02 * np.linalg.norm(x.astype(np.float64), axis=1) * np.sqrt(n) + 1e-30)
+    got, other = run(ctx, x, wt), run(ctx, x, wt, route=capi.ROUTE_GEMM_MFMA)
+    assert (np.linalg.norm(got - exact, axis=1) <= bound).all() and (np.linalg.norm(got.astype(np.float64) - other, axis=1) <= 2 * bound).all()
+    assert (bits(run(ctx, x, wt)) == bits(got)).all()
+    np.testing.assert_array_equal(run(ctx, x, wt, d), got + d)
+    x[1, 3], x[2, k - 1], x[m - 1, 300] = np.nan, np.inf, -np.inf
+    bad = [1, 2, m - 1]
+    hit = run(ctx, x, wt)
+    assert not np.isfinite(hit[bad]).any()
+    good = [r for r in range(m) if r not in bad]
+    np.testing.assert_array_equal(hit[good], got[good])
+    # other work on the device: no parts that wait for each other
+    ctx.set_shared_device(True)
+    try:
+        x[bad] = 0
+        shared = run(ctx, x, wt)
+        np.testing.assert_allclose(shared[good], got[good], rtol=0, atol=float(2 * bound.max()))
+    finally:
+        ctx.set_shared_device(False)
     wt.free()
