@@ -1859,13 +1859,16 @@ bool tile_mfma_preferred(const LaunchArgs& x) {
   if (rp.ks > 1) return true;
   const uint64_t wgs = (uint64_t)rp.parts * rp.colgroups * rp.rowgroups;
   const uint64_t rounds = (wgs + x.num_cus - 1) / x.num_cus;
+  // (parked beside four slices, the form that was measured here: two pairs per wave of f32 activations have strips beside up to three, and
+  // the 32x32 kernel, which checks what was promised about the activations, keeps those calls)
+  const bool parked = resident_lds_bytes(x.w.fmt, !x.a_is_f16, rp.r, rp.q, true, resident_slices(!x.a_is_f16, rp.r)) <= 160 * 1024;
   if (x.a_is_f16 && rounds == 1 && rp.nslices >= 3) {
     if (x.m <= 16 && rp.q == 1) return true;
     if (x.m <= 32 && x.w.fmt == MGN_FMT_Q4 && rp.parts >= 3) return true;
     if (x.m >= 128 && x.w.fmt == MGN_FMT_Q8 && (rp.r == 1 || (x.m <= 512 && rp.parts > 1))) return true;
   }
   if (x.m > 32)
-    return x.w.fmt == MGN_FMT_Q4 && (rp.parts == 1 || (rp.park && rounds == 1) || 4 * wgs >= 3 * rounds * (uint64_t)x.num_cus);
+    return x.w.fmt == MGN_FMT_Q4 && (rp.parts == 1 || (parked && rounds == 1) || 4 * wgs >= 3 * rounds * (uint64_t)x.num_cus);
   if (x.m > 16) {
     if (x.a_is_f16 || wgs > (uint64_t)x.num_cus) return false;
     if (x.w.fmt == MGN_FMT_Q4) return !(rp.q == 2 && rp.parts == 1);

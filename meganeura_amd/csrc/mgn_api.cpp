@@ -192,7 +192,8 @@ double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool by_plan, bool* s
 mgn_route auto_route(const mgn::LaunchArgs& x, bool any_magnitude, mgn::BlockChoice* choice) {
   const mgn_route basic = basic_route(x, any_magnitude);
   if (x.m <= 16) return basic;
-  const bool splits = basic == MGN_ROUTE_TILE_MFMA && mgn::tile_mfma_splits(x);
+  // (not where f32 activations were promised to lie in the fp16 range: the blocked kernel checks that they do, and keeps its calls as well)
+  const bool splits = basic == MGN_ROUTE_TILE_MFMA && (x.a_is_f16 || any_magnitude) && mgn::tile_mfma_splits(x);
   if (x.m <= 32 && (splits || x.w.fmt == MGN_FMT_Q4)) return basic;
   mgn::LaunchArgs whole = x;
   whole.split_waves = false;

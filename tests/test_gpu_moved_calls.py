@@ -109,3 +109,21 @@ def test_fp16_activations_on_the_resident_kernel(ctx, orc, fmt, m, k, n):
     finally:
         ctx.set_shared_device(False)
     wt.free()
+
+
+@pytest.mark.parametrize("fmt,m,k,n", [(Q4, 547, 1216, 778), (Q4, 136, 1152, 4810), (Q8, 20, 1824, 479)])
+def test_a_promise_that_does_not_hold_is_reported(ctx, fmt, m, k, n):
+    """On a context that was promised activations in the fp16 range, these calls are the 32x32 and the blocked kernel's, which check them."""
+    x = synth.normal(m + k, m * k).reshape(m, k).copy()
+    wt = ctx.weight(fmt, synth.normal(2 * k + n, k * n, 0.02).reshape(k, n))
+    ctx.set_activation_range(True)
+    try:
+        assert np.isfinite(run(ctx, x, wt)).all()
+        x[m // 2, k - 1] = np.float32(70000.0)
+        with pytest.raises(capi.MgnError) as e:
+            run(ctx, x, wt)
+        assert e.value.status == capi.ERANGE
+        ctx.sync()  # reported once
+    finally:
+        ctx.set_activation_range(False)
+    wt.free()

@@ -251,3 +251,12 @@ def test_the_plan_of_the_other_kernel_decides(fmt, m, k, n, f16, blocked):
     """Narrow results, ragged rounds and waves that split K: 0.3 to 0.75 of the time on the blocked kernel, or 1.1 to 2 times."""
     assert (capi.matmul_plan(fmt, m, k, n, f16, auto=True).route == capi.ROUTE_BLOCK_MFMA) == blocked
     assert bool(capi.matmul_block_plan(fmt, m, k, n, f16).taken) == blocked
+
+
+@pytest.mark.parametrize("fmt,m,k,n,route", [
+    (Q4, 136, 1152, 4810, GEMM_MFMA), (Q4, 46, 1504, 13816, GEMM_MFMA), (Q4, 547, 1216, 778, GEMM_MFMA), (Q4, 370, 1120, 1529, GEMM_MFMA),
+    (Q4, 124, 1088, 4194, GEMM_MFMA), (Q4, 16, 1024, 1024, GEMM_MFMA), (Q8, 20, 1824, 479, capi.ROUTE_BLOCK_MFMA), (Q8, 25, 1888, 17, capi.ROUTE_BLOCK_MFMA)])
+def test_a_promised_range_stays_with_the_kernels_that_check_it(fmt, m, k, n, route):
+    """f32 activations promised to lie in the fp16 range: neither strips that short parts have room for nor waves that split K take a call from
+    the 32x32 or the blocked kernel, which report a promise that does not hold."""
+    assert capi.matmul_plan(fmt, m, k, n, fp16_range=True, auto=True).route == route
