@@ -826,14 +826,14 @@ static mgn_status matmul_impl(mgn_ctx* ctx, const mgn_buf* a, bool a_is_f16, con
     };
     mgn::LaunchArgs behind = x;
     behind.split_waves = false;
-    uint64_t need = workspace_of(behind, ctx->route == MGN_ROUTE_AUTO ? basic_route(behind, ctx->any_magnitude) : route);
+    const bool blocked = route == MGN_ROUTE_BLOCK_MFMA;
+    uint64_t need = workspace_of(behind, blocked || ctx->route == MGN_ROUTE_AUTO ? basic_route(behind, ctx->any_magnitude) : route);
     if (need > kStaticPartialBytes)
       return fail(ctx, MGN_EUNSUPPORTED,
                   "mgn_matmul_q_static: this shape's K parts need " + std::to_string(need) +
                       " bytes of workspace, the static one holds " + std::to_string(kStaticPartialBytes) +
                       "; use mgn_matmul_q");
-    const bool blocked = route == MGN_ROUTE_BLOCK_MFMA;
-    if (!blocked) need = workspace_of(x, route);  // (at most 4 MiB where waves split K: a round of workgroups, 16 KiB each)
+    if (!blocked) need = workspace_of(x, route);  // (where waves split K: a round of workgroups, 8 KiB each at most)
     if (!blocked && need > kStaticPartialBytes) return fail(ctx, MGN_EUNSUPPORTED, "mgn_matmul_q_static: no room for this plan's K parts");
     x.scratch = ctx->static_scratch;
     x.scratch_capacity = kStaticPartialBytes;  // a launch that would need more than was checked above is refused, not run

@@ -149,3 +149,24 @@ def test_the_automatic_plan_is_what_is_launched(runtime):
             assert resident_q8.quads_per_wave == 0 and capi.matmul_plan(1, 64, 1024, 3072).quads_per_wave > 0
         assert len({s[0] for s in seen}) >= 4, seen
     """)
+
+
+@pytest.mark.parametrize("fmt,m,k,n,taken", [(0, 77, 14336, 4096, False), (1, 77, 14336, 4096, False), (0, 33, 8192, 7168, False), (1, 33, 8192, 7168, False),
+                                             (0, 512, 1024, 8192, True), (1, 512, 2048, 2048, True)])
+def test_the_static_entry_takes_the_same_calls_on_a_forced_blocked_route(runtime, fmt, m, k, n, taken):
+    """Of the blocked kernel's calls, those that the kernels behind it could run on the library's array: by the automatic choice and by force."""
+    on(runtime, f"""
+        assert (capi.matmul_plan({fmt}, {m}, {k}, {n}).workspace_bytes <= capi.STATIC_WORKSPACE_BYTES) == {taken}
+        assert capi.matmul_block_plan({fmt}, {m}, {k}, {n}).taken
+        with capi.Context(0) as ctx:
+            w = ctx.weight_from_packed({fmt}, np.zeros(capi.packed_size({fmt}, {k}, {n}), np.uint8), {k}, {n})
+            a, c = ctx.buffer({m * k * 4}), ctx.buffer({m * n * 4})
+            for route in (capi.ROUTE_AUTO, capi.ROUTE_BLOCK_MFMA):
+                ctx.set_route(route)
+                before = hip.fake_launches(b"12block_kernel")
+                try:
+                    ctx.matmul_q_static(a, w, c, {m})
+                    assert {taken} and hip.fake_launches(b"12block_kernel") == before + 1, route
+                except capi.MgnError as e:
+                    assert not {taken} and e.status == capi.EUNSUPPORTED and hip.fake_launches(b"12block_kernel") == before, route
+    """)
