@@ -39,9 +39,10 @@ typedef struct mgn_block_plan {
 mgn_status mgn_matmul_q_block_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus,
                                    mgn_block_plan* out);
 
-/* What the automatic choice really launches for a shape, the two cases included in which mgn_matmul_q_plan (arguments as
- * there) describes the kernel behind it.  Q8 weights with f32 activations of 33 to 127 rows: the resident
- * form where the choice takes it.  Shapes of the blocked kernel: route MGN_ROUTE_BLOCK_MFMA, grid = (K parts, column groups,
+/* What the automatic choice really launches for a shape, the three cases included in which mgn_matmul_q_plan (arguments as
+ * there) describes another launch.  Q8 weights with f32 activations of 33 to 127 rows: the resident
+ * form where the choice takes it.  Small calls whose waves split K: route MGN_ROUTE_TILE_MFMA, k_splits = 2 or 4 waves to a pair of column
+ * tiles.  In the resident form `steps` is the slices of K that a wave walks, as launched: those of a part, or of its share.  Shapes of the blocked kernel: route MGN_ROUTE_BLOCK_MFMA, grid = (K parts, column groups,
  * row groups), waves_n = 32-column tiles per workgroup, quads_per_wave = launches over blocks of rows, full_steps = row
  * tiles of 32 rows per workgroup, and the rest as for the tiled routes or 0. */
 mgn_status mgn_matmul_q_auto_plan(mgn_fmt fmt, uint32_t m, uint64_t k, uint64_t n, int a_is_f16, int num_cus,

@@ -256,23 +256,28 @@ mgn_status mgn_matmul_q_at(mgn_ctx* ctx, const mgn_buf* a_t, const mgn_weight* w
  * the one every context owns.  a_is_f16: 0 = f32 activations of any magnitude (a context's
  * default), 1 = fp16 activations, 2 = f32 activations promised to lie in the fp16 range
  * (MGN_ACT_FP16_RANGE).  MGN_EINVAL for shapes no weight can have.  For the many-row shapes that the
- * blocked kernel takes, this is the kernel behind it. */
+ * blocked kernel takes, this is the kernel behind it; for the small calls whose waves split K (5 rows and more on launches
+ * that leave compute units idle), it is the launch without the split, or the 32x32 kernel that fp16 activations take then. */
 typedef struct mgn_plan_info {
   int route;              /* mgn_route (never MGN_ROUTE_AUTO) */
   uint32_t grid[3];       /* workgroups: GEMV (column groups, K parts, 1); tiled routes (K parts, column groups, row
                            * groups) -- the LDS-resident MGN_ROUTE_TILE_MFMA form launches them as (column groups x
-                           * row groups, rounded up to a multiple of 8 when K is in parts; K parts) */
+                           * row groups; K parts), the first rounded up to a multiple of 8 when K is in parts, unless
+                           * one part reads the others' sums and that would be one more round of workgroups */
   uint32_t threads;       /* per workgroup */
   uint32_t lds_bytes;     /* dynamic LDS per workgroup */
   uint32_t waves_n;       /* column quads (GEMV), 32-column tiles (MGN_ROUTE_GEMM_MFMA) or 16-column tiles
                            * (MGN_ROUTE_TILE_MFMA) per workgroup */
   uint32_t k_splits;      /* waves that share a quad / tile inside a workgroup */
   uint32_t k_parts;       /* workgroups that share a column group; > 1: partial sums through the workspace */
-  uint32_t steps;         /* GEMV: 16-block steps per wave; tiled: 8-block chunks (slices of 256 elements) per wave and part */
+  uint32_t steps;         /* GEMV: 16-block steps per wave; tiled: 8-block chunks (slices of 256 elements) per wave and part; the
+                           * LDS-resident MGN_ROUTE_TILE_MFMA form: 4, by which K is cut into parts (a part holds
+                           * ceil(slices / k_parts) of them) -- mgn_matmul_q_auto_plan has what a wave walks at most */
   uint32_t quads_per_wave; /* GEMV: column quads per wave; MGN_ROUTE_TILE_MFMA: 0 for the form that keeps the
                             * activation images in LDS, else the launches the rows are spread over
                             * (more than one when their activation images exceed the workspace) */
-  uint32_t full_steps;    /* GEMV: 1 when no step needs masking; MGN_ROUTE_TILE_MFMA: row tiles of 16 rows per workgroup */
+  uint32_t full_steps;    /* GEMV: 1 when no step needs masking; MGN_ROUTE_TILE_MFMA: row tiles of 16 rows per workgroup (where
+                           * waves split K, a tile may hold a row group of 8: row groups = ceil(M / 8) then) */
   uint32_t tail_blocks;   /* GEMV only: 0, or the K blocks per column beyond `steps` full steps that the wave's
                            * quads share one more step for (K = 32 * (16 * steps + tail_blocks)) */
   uint64_t workspace_bytes; /* partial sums held in the context's workspace */

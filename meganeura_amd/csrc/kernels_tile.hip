@@ -1912,7 +1912,9 @@ bool describe_tile_mfma(const LaunchArgs& x, mgn_plan_info* out) {
     out->grid[0] = rp.parts, out->grid[1] = rp.colgroups, out->grid[2] = rp.rowgroups;
     out->threads = 512;
     out->lds_bytes = (uint32_t)rp.lds;
-    out->waves_n = 8 / rp.ks * rp.side * rp.q, out->k_splits = rp.ks, out->k_parts = rp.parts, out->steps = (uint32_t)resident_slices(!x.a_is_f16, rp.r);  // slices of a part at most
+    out->waves_n = 8 / rp.ks * rp.side * rp.q, out->k_splits = rp.ks, out->k_parts = rp.parts;
+    // as launched for the library's own choice (LaunchArgs::split_waves); the four slices that K parts are cut by where a plan is asked for
+    out->steps = x.split_waves ? rp.nsl / rp.ks : (uint32_t)resident_slices(!x.a_is_f16, rp.r);
     out->quads_per_wave = 0, out->full_steps = rp.r, out->tail_blocks = 0;
     out->workspace_bytes = rp.partial_bytes;
     return true;

@@ -170,3 +170,24 @@ def test_the_static_entry_takes_the_same_calls_on_a_forced_blocked_route(runtime
                 except capi.MgnError as e:
                     assert not {taken} and e.status == capi.EUNSUPPORTED and hip.fake_launches(b"12block_kernel") == before, route
     """)
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("m,k,n,groups,launched", [(333, 3072, 1024, 84, 84), (320, 2080, 1024, 80, 80), (16, 14336, 4352, 17, 17), (250, 2080, 800, 64, 64),
+                                                   (300, 2080, 800, 76, 80)])
+def test_the_grid_of_k_parts(runtime, fmt, m, k, n, groups, launched):
+    """Column groups x row groups of a resident launch with K parts: rounded up to a multiple of 8 where the rounds stay the same, as they are
+    where they would not."""
+    on(runtime, f"""
+        with capi.Context(0) as ctx:
+            w = ctx.weight_from_packed({fmt}, np.zeros(capi.packed_size({fmt}, {k}, {n}), np.uint8), {k}, {n})
+            a, c = ctx.buffer({m * k * 4}), ctx.buffer({m * n * 4})
+            ctx.set_route(capi.ROUTE_TILE_MFMA)
+            p = capi.matmul_plan({fmt}, {m}, {k}, {n})
+            assert p.quads_per_wave == 0 and p.k_parts > 1 and p.grid[1] * p.grid[2] == {groups}, (p.quads_per_wave, p.k_parts, list(p.grid))
+            hip.fake_launch_log()
+            ctx.matmul_q(a, w, c, {m})
+            log = [l.split() for l in hip.fake_launch_log().decode().splitlines()]
+            got = [l for l in log if "tile_resident_kernel" in l[0]]
+            assert len(got) == 1 and [int(v) for v in got[0][1:4]] == [{launched}, p.k_parts, 1], log
+    """)

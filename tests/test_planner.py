@@ -260,3 +260,14 @@ def test_a_promised_range_stays_with_the_kernels_that_check_it(fmt, m, k, n, rou
     """f32 activations promised to lie in the fp16 range: neither strips that short parts have room for nor waves that split K take a call from
     the 32x32 or the blocked kernel, which report a promise that does not hold."""
     assert capi.matmul_plan(fmt, m, k, n, fp16_range=True, auto=True).route == route
+
+
+@pytest.mark.parametrize("fmt,m,k,n,f16,splits,parts,steps", [
+    (Q4, 8, 1024, 1024, True, 4, 1, 1), (Q4, 12, 1024, 1024, False, 4, 1, 1), (Q8, 300, 544, 33, False, 4, 1, 1), (Q4, 16, 320, 1856, False, 2, 1, 1),
+    (Q8, 101, 672, 2561, False, 2, 1, 2), (Q8, 76, 1312, 1796, False, 2, 2, 2), (Q4, 204, 256, 2656, False, 1, 1, 1), (Q4, 333, 544, 2240, False, 1, 1, 3),
+    (Q8, 326, 1152, 1472, False, 1, 2, 3), (Q4, 512, 1024, 3072, False, 1, 1, 4), (Q4, 512, 1024, 3072, True, 1, 1, 4)])
+def test_the_automatic_plan_tells_the_slices_that_a_wave_walks(fmt, m, k, n, f16, splits, parts, steps):
+    """As launched: a part holds as many of K's slices of 256 as there are, evenly cut, and waves that split them take 1 / k_splits of those."""
+    p = capi.matmul_plan(fmt, m, k, n, f16, auto=True)
+    assert (p.route, p.quads_per_wave, p.k_splits, p.k_parts, p.steps) == (TILE_MFMA, 0, splits, parts, steps)
+    assert p.k_parts * p.k_splits * p.steps >= ceil_div(k, 256)
