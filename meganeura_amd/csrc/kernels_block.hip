@@ -245,11 +245,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void block_kernel(BlockArgs x
   // groups, then parts.  (Before, an eighth of the tiles, rounded up, with all their parts: plans are made for full
   // rounds of the CUs, and that rounding was one more round on some XCDs for every sixth call that comes here.  us: f32 Q8 96 x 8544 x
   // 2606, 11 tiles in 17 parts, 45.4 -> 29.0, 508 x 3456 x 5248, 84 in 3, 85.6 -> 59.0, Q4 118 x 13056 x 1600 35.7 -> 28.8, fp16 641 x 9280 x
-  // 4274 137 -> 95; 16 calls whose tiles divide by 8 0.97 to 1.017, median 0.997.)
+  // 4274 137 -> 95; 16 calls whose tiles divide by 8 0.97 to 1.017, median 0.997.  With as many workgroups launched as that takes, 192
+  // for those 11 tiles where 272 had been, 36 ragged calls 0.98 to 1.02, median 0.996, 8 whose tiles divide by 8 0.97 to 1.01: those that returned at once cost nothing that shows.)
   const uint32_t tiles = x.rowgroups * x.colgroups;
   const uint32_t all = tiles * x.parts, per = (all + 7) / 8;
   const uint32_t at = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if ((blockIdx.x >> 3) >= per || at >= all) return;
+  if (at >= all) return;  // (a grid of 8 * per workgroups)
   const uint32_t part = at / tiles, tile = at - part * tiles;
   const uint32_t rg = tile % x.rowgroups, cg = tile / x.rowgroups;
   const uint32_t row0 = rg * ROWS, col0 = cg * COLS;
@@ -1034,8 +1035,7 @@ int launch_block_rows(ihipStream_t* s, const LaunchArgs& x, const BlockPlan& p) 
     const BlockConfig* const first = block_configs(FMT, f32a);
     if (int e = enable_big_lds(p.cfg->kernel, x.device, big_lds_done[FMT * 2 + f32a][p.cfg - first])) return e;
   }
-  const uint32_t tiles = p.rowgroups * p.colgroups;
-  hipLaunchKernelGGL(p.cfg->kernel, dim3((tiles + 7) / 8 * 8 * p.parts), dim3(p.cfg->threads), p.cfg->lds, s, a);
+  hipLaunchKernelGGL(p.cfg->kernel, dim3((p.rowgroups * p.colgroups * p.parts + 7) / 8 * 8), dim3(p.cfg->threads), p.cfg->lds, s, a);
   MGN_HIP_LAUNCH_CHECK();
   if (p.parts > 1) {
     const uint64_t count = (uint64_t)x.m * x.w.n;

@@ -191,3 +191,23 @@ def test_the_grid_of_k_parts(runtime, fmt, m, k, n, groups, launched):
             got = [l for l in log if "tile_resident_kernel" in l[0]]
             assert len(got) == 1 and [int(v) for v in got[0][1:4]] == [{launched}, p.k_parts, 1], log
     """)
+
+
+@pytest.mark.parametrize("fmt,m,k,n,f16", [(1, 96, 8544, 2606, False), (1, 42, 8096, 253, False), (0, 118, 13056, 1600, False), (0, 641, 9280, 4274, True),
+                                           (1, 508, 3456, 5248, False)])
+def test_the_blocked_kernel_launches_the_workgroups_that_there_are(runtime, fmt, m, k, n, f16):
+    """The tiles of all K parts, dealt out evenly over eight XCDs, and no workgroup more than that takes."""
+    on(runtime, f"""
+        with capi.Context(0) as ctx:
+            w = ctx.weight_from_packed({fmt}, np.zeros(capi.packed_size({fmt}, {k}, {n}), np.uint8), {k}, {n})
+            a, c = ctx.buffer({m * k * 4}), ctx.buffer({m * n * 4})
+            ctx.set_route(capi.ROUTE_BLOCK_MFMA)
+            p = capi.matmul_block_plan({fmt}, {m}, {k}, {n}, {f16})
+            tiles = p.row_groups * p.col_groups
+            assert p.k_parts > 1 and tiles % 8 and p.launches == 1
+            hip.fake_launch_log()
+            (ctx.matmul_q_f16a if {f16} else ctx.matmul_q)(a, w, c, {m})
+            log = [l.split() for l in hip.fake_launch_log().decode().splitlines()]
+            got = [l for l in log if "12block_kernel" in l[0]]
+            assert len(got) == 1 and [int(v) for v in got[0][1:4]] == [-(-tiles * p.k_parts // 8) * 8, 1, 1], log
+    """)
