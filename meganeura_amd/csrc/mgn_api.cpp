@@ -136,17 +136,13 @@ mgn_route basic_route(const mgn::LaunchArgs& x, bool any_magnitude) {
   return MGN_ROUTE_GENERIC;
 }
 
-// What a call of more than 16 rows takes on the kernel of basic_route, in us.
-// The resident kernel: fitted to 2071 measured calls (K of 1 to 56 slices of 256, 17 to 2048 rows, both formats, f32 and fp16 activations, those near
-// the blocked kernel's estimate before all; mean of weights in the caches and from memory; of what is measured 0.8 to 1.25 (5th to 95th percentile), medians
-// 0.95 to 1.05 by the slices of a part): a launch, and per round of workgroups a fixed part and one for each slice that its parts really
-// hold, of which some is shared by as many workgroups as there are; K parts that meet; and more where the quants have no strips (f32 activations,
-// two pairs of tiles per wave, four slices).  Row groups of 32: so much per round, less for short K.
-// On 243 other calls of 33 to 2048 rows near the boundary the faster of the two kernels was missed by more than 3 % on 15 (50 by K alone, at one to four
-// slices alike), and all together take 1.005 times the faster one's time (1.044).
-// The others, fitted to 480 calls (M = 20 .. 2048 on twelve shapes from 576 x 1536 to 14336 x 4096 and 576 x 49152, both formats, f32 and fp16
-// activations) and, for K below 576, to 600 more: a fixed part and a rate over the rows they compute, a multiple of 32 (K of up to 128:
-// 5.4 to 12 us), or what the plan says, as follows.
+// What a call of more than 16 rows takes on the kernel of basic_route, in us, fitted to 480 measured
+// calls (M = 20 .. 2048 on twelve shapes from 576 x 1536 to 14336 x 4096 and 576 x 49152, both formats, f32 and fp16
+// activations) and, for K below 576, to 600 more.  The resident kernel: so much per round of workgroups, less where K is
+// shorter than the four slices of 256 that a workgroup holds (measured over the four slices' time, medians by format and
+// activations: one slice 0.55 .. 0.72, two 0.79 .. 0.90, three 0.88 .. 1.08, the most with two pairs of tiles per wave); the
+// others: a fixed part and a rate over the rows they compute, a multiple of 32 (K of up to 128: 5.4 to 12 us).  *steady: the resident kernel with one
+// pair of tiles per wave.  by_plan: as follows.
 // On 240 calls drawn over 17 to 2048 rows, K of 576 to 14336 and 192 to 49152 columns that stayed behind by that rate, the 32x32 kernel (fp16
 // activations) took 1.0 to 2.4 times and the general tiled one 1.1 to 3.8 times as long as it says (medians 1.4 and 1.75), and the blocked kernel was
 // more than 3 % faster on 88 of 150 and 83 of 90 of them: Q8 f32 998 x 6240 x 544 137 against 43 us, Q4 130 x 4160 x 992 39 against 18, Q4 fp16 546 x 1056 x
@@ -154,15 +150,14 @@ mgn_route basic_route(const mgn::LaunchArgs& x, bool any_magnitude) {
 // Q8, where many calls are level: what it moves by mistake would cost more than what it leaves), and half as much again for the general one.
 // Of 6000 drawn calls of more than four rows that moves 169; of 196 such that were measured five were more than 3.5 % slower then (Q4 fp16
 // 102 x 4384 x 2136 16.6 -> 18.1), all together take 0.72 of the time (geometric mean, 0.28 at best).
-// *low: what the blocked kernel's estimate is multiplied by beside this one.
-double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool promised, double* low) {
+double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool by_plan, bool* steady) {
   const bool q4 = x.w.fmt == MGN_FMT_Q4;
   const double flops = 2.0 * ((x.m + 31) / 32 * 32) * x.w.k * x.w.n;
-  *low = 0.92;
+  *steady = false;
   mgn_plan_info p{};
   if (route == MGN_ROUTE_GEMM_MFMA) {
     const double rate = x.w.k <= 128 ? 5.6 + flops / (x.a_is_f16 ? 175e6 : 120e6) : 7.0 + flops / (q4 ? 390e6 : 310e6);
-    if (!x.a_is_f16 || x.w.k <= 512 || !mgn::describe_gemm_mfma(x, &p)) return rate;
+    if (!by_plan || !x.a_is_f16 || x.w.k <= 512 || !mgn::describe_gemm_mfma(x, &p)) return rate;
     // That rate is the full rounds' of many rows.  With few columns or a ragged last round the launch takes its chunks of K
     // (256 or 512 elements a workgroup), each partly by how many workgroups the CUs share out and partly by the rounds.
     const double wgs = (double)p.grid[0] * p.grid[1] * p.grid[2] / x.num_cus, rounds = std::ceil(wgs);
@@ -171,56 +166,40 @@ double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool promised, double
     return std::max(rate, plan);
   }
   if (route != MGN_ROUTE_TILE_MFMA || !mgn::describe_tile_mfma(x, &p)) return 1e9;  // scalar routes
-  if (p.quads_per_wave != 0) return 1.5 * (9.0 + flops / (q4 ? 175e6 : 165e6));
-  const double wgs = (double)p.grid[0] * p.grid[1] * p.grid[2] / x.num_cus, rounds = std::ceil(wgs), parts = p.k_parts > 1 ? 1.0 : 0.0;
-  const bool one = p.waves_n <= 16, groups32 = p.full_steps == 2, steady = one && !groups32;  // one pair of tiles per wave
-  const double share = x.w.k <= 256 ? 0.65 : x.w.k <= 512 ? (one ? 0.82 : 0.9) : x.w.k <= 768 && steady ? 0.94 : 1.0;
-  if (groups32) return 10.5 * share * rounds + parts;
-  if (promised) {
-    // The rates by which these calls were first divided between the two kernels: the blocked one checks what was promised, the resident one
-    // has no need to, and a call that is checked stays so.
-    if (one) *low = 1.0;
-    return one ? (q4 ? 9.0 : 10.0) * share * rounds + parts : (q4 ? 15.5 : 22.0) * share * rounds + (q4 ? 1.0 : 9.0) * parts;
-  }
-  // (the blocked kernel's estimate is that much of what it takes beside these calls, by the slices of a part)
-  static constexpr double kLow[5] = {0.91, 1.03, 0.97, 0.94, 0.91};
-  const bool two = !one;
-  const uint32_t nslices = (x.w.k + 255) / 256, slices = std::min((nslices + p.k_parts - 1) / p.k_parts, 4u);
-  *low = kLow[slices];
-  // `far`: on top of round_slice for what the 4 MB of an XCD's L2 don't hold of the weights, all of it from 5 MB on.
-  struct Cost { double launch, round, round_slice, wgs_slice, parts, far; };
-  static constexpr Cost kCost[2][2][2] = {  // [Q8][fp16 activations][two pairs]  (Q8, fp16, two pairs, of which there are few: 0.9 of f32)
-      {{{1.7, 1.3, 1.0, 0.9, 1.3, 0.3}, {1.8, 2.3, 2.0, 1.4, 1.7, 0.8}}, {{0.3, 2.4, 1.1, 0.6, 1.6, 0.2}, {1.7, 1.9, 0.0, 3.3, 4.1, 0.7}}},
-      {{{1.4, 1.9, 0.8, 1.4, 0.7, 0.9}, {2.0, 2.1, 2.4, 1.6, 2.0, 1.1}}, {{3.5, 2.1, 0.9, 0.3, 0.9, 0.7}, {1.8, 1.9, 2.2, 1.4, 1.8, 1.0}}}};
-  static constexpr Cost kUnparkedQ8 = {2.9, 1.2, 1.9, 2.2, 3.5, 2.9};
-  const bool unparked = two && !x.a_is_f16 && slices == 4;  // no room for strips
-  const Cost& t = unparked && !q4 ? kUnparkedQ8 : kCost[!q4][x.a_is_f16][two];
-  const double far = t.far * std::min(1.0, (double)x.w.k * x.w.n * (q4 ? 20 : 34) / 32 / 5e6);
-  return t.launch + rounds * (t.round + (t.round_slice + far) * slices) + t.wgs_slice * slices * wgs + t.parts * parts + (unparked && q4 ? 1.1 * wgs : 0.0);
+  if (p.quads_per_wave != 0) return (by_plan ? 1.5 : 1.0) * (9.0 + flops / (q4 ? 175e6 : 165e6));
+  *steady = p.full_steps != 2 && p.waves_n <= 16;
+  const double share = x.w.k <= 256 ? 0.65 : x.w.k <= 512 ? (p.waves_n <= 16 ? 0.82 : 0.9) : x.w.k <= 768 && *steady ? 0.94 : 1.0;
+  const double rounds = std::ceil((double)p.grid[0] * p.grid[1] * p.grid[2] / x.num_cus) * share, parts = p.k_parts > 1 ? 1.0 : 0.0;
+  if (p.full_steps == 2) return 10.5 * rounds + parts;
+  if (*steady) return (q4 ? 9.0 : 10.0) * (x.a_is_f16 ? 0.9 : 1.0) * rounds + parts;
+  return (q4 ? 15.5 : 22.0) * (x.a_is_f16 ? 0.9 : 1.0) * rounds + (q4 ? 1.0 : 9.0) * parts;
 }
 
 // The automatic choice: the above, or the blocked kernel where it is expected to be the faster one.  (It
 // costs a launch to prepare the activations, one to add up K parts if there are any, and about 5 us
 // besides, but multiplies two to three times as fast: f32 512 x 4096 x 14336 295 -> 115 us, fp16 2048 x 4096 x
-// 14336 527 -> 263, 77 x 14336 x 4096 83 -> 41 with Q8, while 128 x 1024 x 3072 stays at 10 against 15.  The fit of the 32x32, the general
-// tiled kernel and row groups of 32 is for weights in the caches, its own estimate for weights from memory: hence 0.92 there.
+// 14336 527 -> 263, 77 x 14336 x 4096 83 -> 41 with Q8, while 128 x 1024 x 3072 stays at 10 against 15.  Its own estimate
+// is made for weights that come from memory, the fit above for weights in the caches: hence 0.92.
 // Of 1652 other calls, 17 to 2048 rows, K 32 to 8192 and N 64 to 30000, 405 took it by the rates alone, 20 of them more than 3 % slower than on the
 // kernel behind, and 77 did not though it was more than 3 % faster, above all the narrow results of long K that the plans above find.)
 // `choice`: the plan, if it does.
-// A launch whose waves split K never does: of 397 drawn calls of 17 and more rows none was faster blocked (at the nearest Q8 fp16 82 x 1408 x 2581,
-// 13.6 to 14.0 against 9.3 to 12.1; Q8 20 x 1504 x 310 12.0, 8.3; fp16 35 x 704 x 1797 9.8, 5.0).
+// A launch whose waves split K is faster than the unsplit one it is compared as, by that one's rate: of 217 drawn calls of 17 and more rows on which
+// they may, none was faster blocked (up to 32 rows they are not compared; Q8 20 x 1504 x 310, blocked 12.0, split 8.3; fp16 35 x 704 x 1797
+// 9.8, 5.0), and 5 of 6000 are blocked by these estimates.
+// Not so where the other kernel is the resident one with one pair of tiles per wave: small weights, which take it the
+// same time a round from wherever they come.  (Blocked and resident, us: Q8 f32 22 x 1760 x 1307 14.1, 11.4, 17 x 768 x 579
+// 10.1, 8.8; short K: Q4 f32 470 x 192 x 275 9.6, 6.4, Q4 fp16 145 x 160 x 105 8.6, 4.2.)
 mgn_route auto_route(const mgn::LaunchArgs& x, bool any_magnitude, mgn::BlockChoice* choice) {
   const mgn_route basic = basic_route(x, any_magnitude);
   if (x.m <= 16) return basic;
   // (not where f32 activations were promised to lie in the fp16 range: the blocked kernel checks that they do, and keeps its calls as well)
-  const bool promised = !x.a_is_f16 && !any_magnitude;
-  if (basic == MGN_ROUTE_TILE_MFMA && !promised && mgn::tile_mfma_splits(x)) return basic;
-  if (x.m <= 32 && x.w.fmt == MGN_FMT_Q4) return basic;
+  const bool splits = basic == MGN_ROUTE_TILE_MFMA && (x.a_is_f16 || any_magnitude) && mgn::tile_mfma_splits(x);
+  if (x.m <= 32 && (splits || x.w.fmt == MGN_FMT_Q4)) return basic;
   mgn::LaunchArgs whole = x;
   whole.split_waves = false;
-  double low;
-  const double us = basic_us(whole, basic, promised, &low);
-  return mgn::choose_block_mfma(x, us / low, choice) ? MGN_ROUTE_BLOCK_MFMA : basic;
+  bool steady;
+  const double us = basic_us(whole, splits ? basic_route(whole, any_magnitude) : basic, !splits, &steady);
+  return mgn::choose_block_mfma(x, steady ? us : us / 0.92, choice) ? MGN_ROUTE_BLOCK_MFMA : basic;
 }
 
 // After the stream has been synchronised: did a wave give up waiting for another workgroup's

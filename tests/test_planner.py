@@ -271,17 +271,3 @@ def test_the_automatic_plan_tells_the_slices_that_a_wave_walks(fmt, m, k, n, f16
     p = capi.matmul_plan(fmt, m, k, n, f16, auto=True)
     assert (p.route, p.quads_per_wave, p.k_splits, p.k_parts, p.steps) == (TILE_MFMA, 0, splits, parts, steps)
     assert p.k_parts * p.k_splits * p.steps >= ceil_div(k, 256)
-
-
-@pytest.mark.parametrize("fmt,m,k,n,f16,blocked", [
-    (Q8, 385, 1536, 2177, False, False), (Q8, 389, 1056, 2182, False, False), (Q8, 738, 1440, 675, False, False), (Q4, 403, 512, 3325, False, False),
-    (Q4, 752, 32, 2513, False, False), (Q8, 502, 224, 3873, False, False), (Q8, 2030, 96, 896, False, False), (Q4, 90, 416, 12979, False, False),
-    (Q4, 46, 32, 40728, True, False), (Q8, 215, 1120, 18, False, False), (Q8, 264, 1952, 21, True, False), (Q8, 1502, 1632, 1248, False, True),
-    (Q8, 218, 1024, 18472, False, True), (Q4, 262, 1472, 7180, True, True)])
-def test_the_slices_that_a_part_holds_decide(fmt, m, k, n, f16, blocked):
-    """Parts of the resident kernel that hold one to three slices and park their quants, waves that split K, and four slices of large Q8 weights
-    without strips: 1.1 to 2 times as long on the other kernel.  Q8 calls whose f32 activations were promised to lie in the fp16 range stay where
-    that is checked."""
-    assert (capi.matmul_plan(fmt, m, k, n, f16, auto=True).route == capi.ROUTE_BLOCK_MFMA) == blocked
-    if fmt == Q8 and not f16:
-        assert capi.matmul_plan(fmt, m, k, n, fp16_range=True, auto=True).route in (GEMM_MFMA, capi.ROUTE_BLOCK_MFMA)
