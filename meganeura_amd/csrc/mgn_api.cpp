@@ -139,9 +139,9 @@ mgn_route basic_route(const mgn::LaunchArgs& x, bool any_magnitude) {
 // What a call of more than 16 rows takes on the kernel of basic_route, in us, fitted to 480 measured
 // calls (M = 20 .. 2048 on twelve shapes from 576 x 1536 to 14336 x 4096 and 576 x 49152, both formats, f32 and fp16
 // activations) and, for K below 576, to 600 more.  The resident kernel: so much per round of workgroups, less where K is
-// shorter than the four slices of 256 that a workgroup holds (measured over the four slices' time, medians by format and
-// activations: one slice 0.55 .. 0.72, two 0.79 .. 0.90, three 0.88 .. 1.08, the most with two pairs of tiles per wave); the
-// others: a fixed part and a rate over the rows they compute, a multiple of 32 (K of up to 128: 5.4 to 12 us).  *steady: the resident kernel with one
+// shorter than the four slices of 256 that a workgroup holds (measured over the four slices' time when a workgroup walked four
+// whatever there were, medians by format and activations: one slice 0.55 .. 0.72, two 0.79 .. 0.90, three 0.88 .. 1.08, the most with two pairs of tiles
+// per wave); the others: a fixed part and a rate over the rows they compute, a multiple of 32 (K of up to 128: 5.4 to 12 us).  *steady: the resident kernel with one
 // pair of tiles per wave.  by_plan: as follows.
 // On 240 calls drawn over 17 to 2048 rows, K of 576 to 14336 and 192 to 49152 columns that stayed behind by that rate, the 32x32 kernel (fp16
 // activations) took 1.0 to 2.4 times and the general tiled one 1.1 to 3.8 times as long as it says (medians 1.4 and 1.75), and the blocked kernel was
@@ -150,6 +150,11 @@ mgn_route basic_route(const mgn::LaunchArgs& x, bool any_magnitude) {
 // Q8, where many calls are level: what it moves by mistake would cost more than what it leaves), and half as much again for the general one.
 // Of 6000 drawn calls of more than four rows that moves 169; of 196 such that were measured five were more than 3.5 % slower then (Q4 fp16
 // 102 x 4384 x 2136 16.6 -> 18.1), all together take 0.72 of the time (geometric mean, 0.28 at best).
+// Parts of one to three slices take less than this by now (Q8 f32 385 x 1536 x 2177 20.2 us, 33.7 here, blocked 27.3), among them those of K of 1056 to 1536
+// and 2080 to 2304.  The rates stay: they also say which calls have the blocked kernel's accuracy, whose error against f64 with f32 activations is a
+// tenth (Q4) or a fifth (Q8) of the resident kernel's (1811 x 672 x 1689 2.4e-7, 3.1e-6; 162 x 32 x 6529 7.6e-8, 4.7e-7; 67 calls, behind a silu an
+// eighth to a tenth).  Estimates by slices, fitted to 2071 calls, took 1.005 times the faster kernel's time on 243 calls near the boundary
+// where these take 1.044 (15 against 50 more than 3 % slower than on the other kernel), and gave 4.5 % of the f32 calls drawn to the less exact one.
 double basic_us(const mgn::LaunchArgs& x, mgn_route route, bool by_plan, bool* steady) {
   const bool q4 = x.w.fmt == MGN_FMT_Q4;
   const double flops = 2.0 * ((x.m + 31) / 32 * 32) * x.w.k * x.w.n;

@@ -127,3 +127,16 @@ def test_a_promise_that_does_not_hold_is_reported(ctx, fmt, m, k, n):
     finally:
         ctx.set_activation_range(False)
     wt.free()
+
+
+@pytest.mark.parametrize("fmt,m,k,n", [(Q8, 385, 1536, 2177), (Q8, 502, 224, 3873), (Q4, 403, 512, 3325), (Q4, 752, 32, 2513)])
+def test_the_blocked_kernel_keeps_the_calls_that_it_answers_more_exactly(ctx, orc, fmt, m, k, n):
+    """Calls on which the resident kernel would be the faster one, whose pairs of fp16 numbers are cut; the blocked kernel's are rounded to nearest.
+    Measured 4 to 13 times the error; twice is asked for."""
+    assert capi.matmul_plan(fmt, m, k, n, auto=True).route == capi.ROUTE_BLOCK_MFMA
+    w, x = synth.normal(k + n, k * n, 0.02).reshape(k, n), synth.normal(m, m * k).reshape(m, k)
+    wt = ctx.weight(fmt, w)
+    exact = orc.matmul_f64(x, orc.dequantize(fmt, orc.quantize(fmt, w), k, n))
+    error = [np.linalg.norm(run(ctx, x, wt, route=r) - exact) for r in (capi.ROUTE_AUTO, capi.ROUTE_TILE_MFMA)]
+    assert 2 * error[0] <= error[1] <= 1e-5 * np.linalg.norm(exact)
+    wt.free()

@@ -239,7 +239,7 @@ def test_small_calls_stay_with_the_kernel_that_needs_one_launch(fmt, m, k, n, f1
     (Q4, 77, 4096, 14336, False), (Q8, 77, 14336, 4096, False), (Q4, 2048, 4096, 14336, True), (Q8, 22, 3296, 14036, False), (Q4, 122, 736, 11506, False),
     (Q8, 199, 896, 7513, False), (Q4, 454, 832, 4683, True), (Q8, 1359, 384, 2477, True), (Q8, 241, 128, 8416, True)])
 def test_large_calls_take_the_blocked_kernel(fmt, m, k, n, f16):
-    """Calls on which it measured 1.1 to 2.5 times as fast as the kernel behind it."""
+    """Calls on which it measured 1.1 to 2.5 times as fast as the kernel behind it (Q4 122 x 736 x 11506 level by now)."""
     assert capi.matmul_block_plan(fmt, m, k, n, f16).taken and capi.matmul_plan(fmt, m, k, n, f16, auto=True).route == capi.ROUTE_BLOCK_MFMA
 
 
@@ -271,3 +271,12 @@ def test_the_automatic_plan_tells_the_slices_that_a_wave_walks(fmt, m, k, n, f16
     p = capi.matmul_plan(fmt, m, k, n, f16, auto=True)
     assert (p.route, p.quads_per_wave, p.k_splits, p.k_parts, p.steps) == (TILE_MFMA, 0, splits, parts, steps)
     assert p.k_parts * p.k_splits * p.steps >= ceil_div(k, 256)
+
+
+@pytest.mark.parametrize("fmt,m,k,n", [(Q8, 385, 1536, 2177), (Q8, 389, 1056, 2182), (Q8, 167, 1120, 3286), (Q8, 502, 224, 3873), (Q4, 403, 512, 3325),
+                                       (Q4, 752, 32, 2513), (Q4, 90, 416, 12979), (Q4, 1811, 672, 1689)])
+def test_calls_that_the_blocked_kernel_answers_more_exactly_stay_with_it(fmt, m, k, n):
+    """Short parts of the resident kernel, which is as fast or up to 1.4 times as fast there, but 4 to 13 times as far from f64."""
+    assert capi.matmul_plan(fmt, m, k, n, auto=True).route == capi.ROUTE_BLOCK_MFMA
+    behind = capi.matmul_plan(fmt, m, k, n)
+    assert behind.route == TILE_MFMA and behind.quads_per_wave == 0
