@@ -96,6 +96,49 @@ def test_fp16_activations(ctx, orc, fmt, m, k, n):
     wt.free()
 
 
+def check(ctx, orc, fmt, x, n):
+    """Results, repeats, residual and rows that are not finite, against f64 and against the kernel without the split; bounds as above."""
+    m, k = x.shape
+    w, d = synth.normal(2 * k + n, k * n, 0.02).reshape(k, n), synth.normal(7, m * n).reshape(m, n)
+    wt = ctx.weight(fmt, w)
+    exact = orc.matmul_f64(x.astype(np.float32), orc.dequantize(fmt, orc.quantize(fmt, w), k, n))
+    size = 0.02 * np.linalg.norm(x.astype(np.float64), axis=1) * np.sqrt(n) + 1e-30
+    got = run(ctx, x, wt)
+    for want in (exact, run(ctx, x, wt, route=capi.ROUTE_TILE_MFMA).astype(np.float64)):
+        assert (np.linalg.norm(got - want, axis=1) <= 5 * (2.0 ** -22 + 2.0 ** -24 * np.sqrt(k)) * size).all()
+    for _ in range(2):
+        assert (bits(run(ctx, x, wt)) == bits(got)).all()
+    np.testing.assert_array_equal(run(ctx, x, wt, d), got + d)
+    y = x.copy()
+    y[1, 3], y[2, k - 1], y[m - 1, 300] = np.nan, np.inf, -np.inf
+    wrong, bad = run(ctx, y, wt), [1, 2, m - 1]
+    good = [r for r in range(m) if r not in bad]
+    assert not np.isfinite(wrong[bad]).any()
+    np.testing.assert_array_equal(wrong[good], got[good])
+    wt.free()
+
+
+@pytest.mark.parametrize("fmt,m,k,n,f16,parts", [
+    (Q4, 101, 704, 2409, False, 1), (Q4, 200, 928, 1418, False, 1), (Q8, 101, 704, 2561, False, 1), (Q8, 200, 992, 1457, False, 1),
+    (Q8, 76, 1312, 1796, False, 2), (Q8, 200, 1056, 588, False, 2), (Q8, 101, 2080, 1029, False, 3), (Q8, 76, 2528, 1098, False, 3),
+    (Q4, 50, 576, 5580, True, 1), (Q4, 101, 1024, 2764, True, 1), (Q8, 200, 576, 1600, True, 1), (Q8, 200, 896, 1600, True, 1),
+    (Q8, 101, 1184, 1293, True, 2), (Q8, 101, 1536, 1243, True, 2), (Q8, 101, 2240, 825, True, 3), (Q8, 101, 2336, 1184, True, 3)])
+def test_two_waves_of_two_slices(ctx, orc, fmt, m, k, n, f16, parts):
+    """Two waves to a pair of tiles, more than one slice each: parts of three (two and one) and four slices, the last of them two to four."""
+    p = capi.matmul_plan(fmt, m, k, n, f16, auto=True)
+    assert (p.route, p.k_splits, p.k_parts, p.steps) == (capi.ROUTE_TILE_MFMA, 2, parts, 2)
+    x = rows_of(m, k, m + k) if not f16 else synth.normal(m, m * k).reshape(m, k).astype(np.float16)
+    check(ctx, orc, fmt, x, n)
+
+
+@pytest.mark.parametrize("fmt", [Q4, Q8])
+@pytest.mark.parametrize("m,k,n", [(5, 544, 64), (18, 2080, 201), (107, 4000, 256)])
+def test_four_waves_with_fp16_activations(ctx, orc, fmt, m, k, n):
+    p = capi.matmul_plan(fmt, m, k, n, True, auto=True)
+    assert p.route == capi.ROUTE_TILE_MFMA and p.k_splits == 4
+    check(ctx, orc, fmt, synth.normal(m, m * k).reshape(m, k).astype(np.float16), n)
+
+
 @pytest.mark.parametrize("fmt", [Q4, Q8])
 @pytest.mark.parametrize("m,k", [(6, 544), (16, 1056), (20, 768)])
 def test_values_that_are_not_finite_stay_in_their_rows(ctx, orc, fmt, m, k):
