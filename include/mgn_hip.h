@@ -103,7 +103,8 @@ typedef enum mgn_act_range { MGN_ACT_ANY = 0, MGN_ACT_FP16_RANGE = 1 } mgn_act_r
 /* Whether other work runs on the device beside this context's launches (other contexts, other
  * processes).  Two kinds of launch let all their workgroups wait for each other, which needs them
  * resident on the device together: a chain (mgn_chain_*), and a matmul whose K parts are added up
- * by all parts, a share each.  Two such kernels at once can take each other's compute units and
+ * by all parts, a share each (which the automatic route gives ordinary calls of five rows and more as well,
+ * with f32 and with fp16 activations, wherever K is cut into parts: mgn_matmul_q_auto_plan, k_parts).  Two such kernels at once can take each other's compute units and
  * both stall until their bounded waits give up (MGN_ETIMEOUT at the next synchronising call, no
  * hang, results not to be used).  shared = 0 (default): the context has the device to itself while
  * it computes, and both are used.  shared != 0: neither is; chains are refused with

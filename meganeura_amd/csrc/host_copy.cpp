@@ -9,7 +9,7 @@
 //     order with the launches that read them); launches, not copy engine commands, move the chunks
 //     (copy_bytes_kernel), except reads on an idle stream;
 //   beyond (uploads from kLargeIn on): the ring as slots of kSlot, up to kWorkers threads with two slots
-//     each that take the chunks in turn (one thread's 29 GB/s is half of what the bus takes: 64 MB 2306 us with one thread, 874
+//     each that take the chunks in turn (one thread's 29 GB/s is half of what the bus takes: 64 MB 2650 us with one thread, 1590
 //     with four).  The threads live as long as the call.
 // Measured, before -> after: the eight-layer decode step of a session 147 -> 124 us, two layers of 333
 // rows 460 -> 410 us, a 4096 x 4096 weight from f32 and its packed bytes back 3400 -> 2470 us.

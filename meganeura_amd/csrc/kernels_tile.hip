@@ -162,7 +162,7 @@ __device__ __forceinline__ void convert_task(const TaskWords<F32A>& xin, bool ok
       x[e] = __builtin_bit_cast(float, w);
       am = max(am, w & 0x7FFFFFFFu);
     }
-    // an infinity or a NaN switches scaling off, and the row's sums over the slice come out non-finite
+    // (of a slice that holds an infinity or a NaN the reciprocal is a NaN, and the row's sums over the slice come out non-finite)
     am = group_max32(am);
     constexpr bool kSplit = FMT == MGN_FMT_Q4;
     const float scale = slice_scale<kSplit ? 7 : 11>(__builtin_bit_cast(float, am), &inv);
@@ -935,9 +935,9 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t c = lane & 15, g = lane >> 4;
-  // grid = (column groups x row groups, rounded up to a multiple of 8; K parts): workgroups go to the
-  // eight XCDs in turn by their linear index, so the K parts of a (column group, row group) run on
-  // one XCD, which their hand-over below measures 0.5 us better than spread over all eight
+  // grid = (column groups x row groups; K parts), the first rounded up to a multiple of 8 unless that would be another
+  // round: workgroups go to the eight XCDs in turn by their linear index, so, rounded up, the K parts of a (column group,
+  // row group) run on one XCD, which their hand-over below measures 0.5 us better than spread over all eight
   const uint32_t part = blockIdx.y;
   const uint32_t rg = blockIdx.x / colgroups, cg = blockIdx.x - rg * colgroups;
   const uint32_t group_rows = KS > 1 ? tail.rows : R * 16;
@@ -1190,8 +1190,8 @@ __global__ __launch_bounds__(512) void tile_resident_kernel(const void* __restri
     return;
   }
   if (parts > 1) {
-    // K parts of other workgroups.  The parts of a (column group, row group) run on one XCD (see the
-    // grid above) and the part with the highest index is dispatched last, when the others are
+    // K parts of other workgroups.  The parts of a (column group, row group) mostly run on one XCD (see the
+    // grid above; the stores and polls have device scope, so they need not) and the part with the highest index is dispatched last, when the others are
     // already running or done; it is the one that adds them up, in part order, its own sums last.
     // There is no counter and no barrier: the hand-over workspace holds kHandoverEmpty in every word
     // between launches, a part stores its tiles over it and is done (write-through stores, device
